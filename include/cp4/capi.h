@@ -434,6 +434,38 @@ cp4_status cp4_pointer_is_device(const void* ptr, int* is_device);
 cp4_status cp4_stream_synchronize(cp4_stream);
 cp4_status cp4_device_synchronize(void);
 
+/* ---- a whole layer: y = act(conv + bias), forward and backward -----------------
+ * The layer the reference builds from its op plus framework ops for bias and activation
+ * (test/layers.py:264-282), for activations of any cp4_dtype in memory (factors, bias,
+ * gradients of both and all arithmetic fp32).  `geometry` NULL: the reference's geometry
+ * (stride 1, shape->pad zeros on every side, 2 * pad = Y - 1 = X - 1 for the gradients to be
+ * the forward's); else as in the _ex entry points (fp32 activations only), shape->pad unused.
+ * Shapes that the 16-bit passes do not take run on fp32 copies in the workspace.
+ *
+ * cp4_layer_backward computes whichever of dx, (dFK, dFC, dFH, dFW) - all or none of the
+ * four - and dbias are not NULL, from the layer's input, its output y (used with
+ * CP4_ACT_RELU only: dy counts where y > 0) and the output gradient.  The workspaces
+ * (device memory on a 256-byte boundary; the sizes depend on the arguments given) are
+ * scratch: nothing in them has to survive the call. */
+typedef enum cp4_dtype { CP4_DTYPE_F32 = 0, CP4_DTYPE_BF16 = 1, CP4_DTYPE_F16 = 2 } cp4_dtype;
+enum {                        /* `wanted` of cp4_layer_backward_workspace_bytes */
+  CP4_WANT_DX = 1, CP4_WANT_FACTORS = 2, CP4_WANT_BIAS = 4
+};
+size_t cp4_layer_forward_workspace_bytes(const cp4_shape* shape, const cp4_geometry* geometry,
+                                         int dtype);
+cp4_status cp4_layer_forward(const cp4_shape* shape, const cp4_geometry* geometry, int dtype,
+                             const void* x, const float* FK, const float* FC, const float* FH,
+                             const float* FW, const float* bias, int activation, void* y,
+                             void* workspace, size_t workspace_bytes, cp4_stream stream);
+size_t cp4_layer_backward_workspace_bytes(const cp4_shape* shape, const cp4_geometry* geometry,
+                                          int dtype, int activation, int wanted);
+cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* geometry, int dtype,
+                              const void* x, const void* y, const void* dy, const float* FK,
+                              const float* FC, const float* FH, const float* FW, int activation,
+                              void* dx, float* dFK, float* dFC, float* dFH, float* dFW,
+                              float* dbias, void* workspace, size_t workspace_bytes,
+                              cp4_stream stream);
+
 /* ---- 3-factor CP sibling op ------------------------------------------------
  * Stands where the reference registers its TensorFlow op Conv2dCpFusedNchw
  * (Kernels/cp_fused_nchw.cc:6-30, launcher Conv2dCpFusedNchwKernelLauncher :33):

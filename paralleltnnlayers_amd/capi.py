@@ -154,6 +154,16 @@ def lib():
     L.cp4_recompose.argtypes = [_S, _F, _F, _F, _F, _F, ctypes.c_void_p]
     L.cp3_expand_factors.argtypes = [_S] + [_F] * 7 + [ctypes.c_void_p]
     L.cp3_fold_gradients.argtypes = [_S] + [_F] * 6 + [ctypes.c_void_p]
+    L.cp4_layer_forward_workspace_bytes.restype = ctypes.c_size_t
+    L.cp4_layer_forward_workspace_bytes.argtypes = [_S, _G, ctypes.c_int]
+    L.cp4_layer_forward.argtypes = ([_S, _G, ctypes.c_int, ctypes.c_void_p] + [_F] * 5 +
+                                    [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
+                                     ctypes.c_void_p])
+    L.cp4_layer_backward_workspace_bytes.restype = ctypes.c_size_t
+    L.cp4_layer_backward_workspace_bytes.argtypes = [_S, _G] + [ctypes.c_int] * 3
+    L.cp4_layer_backward.argtypes = ([_S, _G, ctypes.c_int] + [ctypes.c_void_p] * 3 + [_F] * 4 +
+                                     [ctypes.c_int] + [ctypes.c_void_p] * 6 +
+                                     [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p])
     L.cp3_conv2d_forward_workspace_bytes.restype = ctypes.c_size_t
     L.cp3_conv2d_forward_workspace_bytes.argtypes = [_S]
     L.cp3_conv2d_forward.argtypes = [_S] + [_F] * 5 + [ctypes.c_void_p, ctypes.c_size_t,
@@ -450,6 +460,55 @@ def conv2d_backward_filter_f16(x, dy, FK, FC, FH, FW, pad=1, workspace=None, str
         _ptr(FH), _ptr(FW), *[_ptr(o) for o in outs], ctypes.c_void_p(ws.data_ptr()), ws_bytes,
         _stream(stream)))
     return tuple(outs)
+
+
+_DTYPES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}     # cp4_dtype
+_WANT_DX, _WANT_FACTORS, _WANT_BIAS = 1, 2, 4
+
+
+def _ptr_any(t):
+    if t is None:
+        return None
+    assert t.is_cuda and t.is_contiguous()
+    return ctypes.c_void_p(t.data_ptr())
+
+
+def _scratch(nbytes, device):
+    """`nbytes` of device memory (the allocator's blocks start on 512-byte boundaries)."""
+    return torch.empty(nbytes, device=device, dtype=torch.uint8) if nbytes else None
+
+
+def layer_forward(s, g, x, FK, FC, FH, FW, bias=None, activation=None, stream=None):
+    """y = act(conv(x) + bias) in x's element type; g: a Geometry or None."""
+    dtype = _DTYPES[x.dtype]
+    gp = ctypes.byref(g) if g is not None else None
+    oh, ow = (g.out_h, g.out_w) if g is not None else (s.H, s.W)
+    y = torch.empty((s.N, s.T, oh, ow), device=x.device, dtype=x.dtype)
+    need = lib().cp4_layer_forward_workspace_bytes(ctypes.byref(s), gp, dtype)
+    ws = _scratch(need, x.device)
+    check(lib().cp4_layer_forward(ctypes.byref(s), gp, dtype, _ptr_any(x), _ptr(FK), _ptr(FC),
+                                  _ptr(FH), _ptr(FW), _ptr(bias), ACTIVATIONS[activation],
+                                  _ptr_any(y), _ptr_any(ws), need, _stream(stream)))
+    return y
+
+
+def layer_backward(s, g, x, y, dy, FK, FC, FH, FW, activation=None, want_dx=True,
+                   want_factors=True, want_bias=True, stream=None):
+    """(dx, (dFK, dFC, dFH, dFW), dbias) of layer_forward, None where not wanted."""
+    dtype, act = _DTYPES[x.dtype], ACTIVATIONS[activation]
+    gp = ctypes.byref(g) if g is not None else None
+    dx = torch.empty_like(x) if want_dx else None
+    grads = [torch.empty_like(f) if want_factors else None for f in (FK, FC, FH, FW)]
+    dbias = torch.empty(s.T, device=x.device, dtype=torch.float32) if want_bias else None
+    need = lib().cp4_layer_backward_workspace_bytes(
+        ctypes.byref(s), gp, dtype, act,
+        _WANT_DX * want_dx | _WANT_FACTORS * want_factors | _WANT_BIAS * want_bias)
+    ws = _scratch(need, x.device)
+    check(lib().cp4_layer_backward(
+        ctypes.byref(s), gp, dtype, _ptr_any(x), _ptr_any(y), _ptr_any(dy), _ptr(FK), _ptr(FC),
+        _ptr(FH), _ptr(FW), act, _ptr_any(dx), *[_ptr(t) for t in grads], _ptr(dbias),
+        _ptr_any(ws), need, _stream(stream)))
+    return dx, tuple(grads), dbias
 
 
 def conv2d_backward_data(dy, FK, FC, FH, FW, pad=1, out=None, stream=None):

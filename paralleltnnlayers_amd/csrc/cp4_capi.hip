@@ -1415,6 +1415,15 @@ Canvas canvas_of(const cp4_shape& s, const cp4_geometry& g) {
 }
 }  // namespace
 
+}  // extern "C"
+namespace cp4 {
+cp4_status check_layer_shape(const cp4_shape* s) { return check_shape(s); }
+cp4_status check_layer_geometry(const cp4_shape* s, const cp4_geometry* g) { return check_geometry(s, g); }
+cp4_status fail_with(cp4_status st, const char* what) { return fail(st, what); }
+cp4_status fail_hip(hipError_t e, const char* where) { return hip_fail(e, where); }
+}  // namespace cp4
+extern "C" {
+
 cp4_status cp4_geometry_same(const cp4_shape* s, unsigned sh, unsigned sw, cp4_geometry* g) {
   cp4_status rc = check_shape(s);
   if (rc != CP4_OK) return rc;

@@ -75,6 +75,13 @@ inline Geometry geometry_of(const FwdArgs& a) {
   return Geometry{a.sh, a.sw, a.pt, a.pl, a.Ho, a.Wo};
 }
 
+// The C ABI's argument checks and its error record (cp4_last_error_message), for entry points
+// in other files.
+cp4_status check_layer_shape(const cp4_shape*);
+cp4_status check_layer_geometry(const cp4_shape*, const cp4_geometry*);
+cp4_status fail_with(cp4_status, const char* what);
+cp4_status fail_hip(hipError_t, const char* where);
+
 // Compute units of the current device (256 when no device can be asked).
 int num_compute_units();
 
@@ -144,6 +151,16 @@ hipError_t fwd_pipe_taps2d_launch(const FwdArgs&, hipStream_t);
 // In-place y[n,k,:] = act(y[n,k,:] + bias[k]) for variants without the epilogue.
 hipError_t bias_act_launch(float* y, const float* bias, int act, size_t N, size_t K, size_t HW,
                            hipStream_t);
+
+// Backward of the epilogue: out = dy where y > 0 (y null: dy itself; out null: not wanted, in
+// `dtype` or widened to fp32) and dbias[t] = its sum over images and pixels (null: not wanted;
+// `part`: T * act_grad_segments floats of scratch).  dtype: a cp4_dtype.
+int act_grad_segments(int N, int T, size_t HW, int dtype);
+hipError_t act_grad_launch(const void* y, const void* dy, void* out, int dtype, bool out_f32,
+                           float* dbias, float* part, int N, int T, size_t HW, hipStream_t);
+// Element-wise conversion between fp32 and a 16-bit type (cp4_dtype), round to nearest even.
+hipError_t convert_launch(const void* src, int src_dtype, void* dst, int dst_dtype, size_t n,
+                          hipStream_t);
 
 // Backward-filter (factor gradients).
 struct BwdFilterArgs {

@@ -1,0 +1,231 @@
+// C ABI of a whole layer, y = act(conv + bias): which passes a call needs, on which element
+// type each runs, and where their intermediates lie in the caller's workspace.
+#include <array>
+#include <map>
+#include <mutex>
+
+#include "cp4_internal.h"
+
+namespace {
+
+size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Where the parts of a backward call lie in its workspace (byte offsets; a part that the
+// call does not need has no bytes) and which passes run on 16-bit activations as they are.
+struct BackwardPlan {
+  bool dx16, filter16;       // that pass on the 16-bit activations (16-bit layers only)
+  bool act16, act32;         // dy behind the activation is written in the layer's type / as fp32
+  size_t act16_at, act32_at; // ... here
+  size_t x32_at, dx32_at;    // widened x, fp32 dx before it is rounded
+  size_t bias_at, pass_at;   // partial bias sums, the passes' own workspace
+  size_t pass_bytes, total;
+};
+
+size_t elements(const cp4_shape& s, unsigned channels) {
+  return (size_t)s.N * channels * s.H * s.W;
+}
+size_t out_elements(const cp4_shape& s, const cp4_geometry* g) {
+  return (size_t)s.N * s.T * (g ? (size_t)g->out_h * g->out_w : (size_t)s.H * s.W);
+}
+
+BackwardPlan make_backward_plan(const cp4_shape& s, const cp4_geometry* g, int dtype, int act,
+                                int wanted) {
+  BackwardPlan p{};
+  const bool half = dtype != CP4_DTYPE_F32;
+  const bool dx = wanted & CP4_WANT_DX, filter = wanted & CP4_WANT_FACTORS;
+  const size_t ny = out_elements(s, g), nx = elements(s, s.C);
+  p.dx16 = half && dx && cp4_bf16_supported(&s, 1);
+  p.filter16 = half && filter && cp4_bf16_backward_filter_supported(&s);
+  const bool dx32 = half && dx && !p.dx16, filter32 = half && filter && !p.filter16;
+  // (fp32 layers: the "16" part is dy in the layer's own type)
+  p.act16 = act != CP4_ACT_NONE && (half ? p.dx16 || p.filter16 : dx || filter);
+  p.act32 = dx32 || filter32;
+  size_t at = 0;
+  auto take = [&](bool needed, size_t bytes) {
+    const size_t here = at;
+    if (needed) at += align256(bytes);
+    return here;
+  };
+  p.act16_at = take(p.act16, ny * (half ? 2 : 4));
+  p.act32_at = take(p.act32, ny * 4);
+  p.x32_at = take(filter32, nx * 4);
+  p.dx32_at = take(dx32, nx * 4);
+  const int seg = cp4::act_grad_segments((int)s.N, (int)s.T, ny / ((size_t)s.N * s.T), dtype);
+  p.bias_at = take((wanted & CP4_WANT_BIAS) && seg > 1, (size_t)s.T * seg * 4);
+  p.pass_at = at;
+  if (g) p.pass_bytes = dx || filter ? cp4_conv2d_backward_ex_workspace_bytes(&s, g) : 0;
+  else p.pass_bytes = filter ? cp4_conv2d_backward_filter_workspace_bytes(&s) : 0;
+  p.total = at + align256(p.pass_bytes);
+  return p;
+}
+
+// The plan of a call, remembered: planning asks the backward-filter kernels for theirs,
+// several microseconds of host time that every step of a small layer would wait for.
+BackwardPlan backward_plan(const cp4_shape& s, const cp4_geometry* g, int dtype, int act,
+                           int wanted) {
+  using Key = std::array<unsigned, 18>;
+  static std::mutex mu;
+  static std::map<Key, BackwardPlan> plans;
+  const cp4_geometry none{0, 0, 0, 0, 0, 0};
+  const cp4_geometry& gg = g ? *g : none;
+  const Key key{s.N, s.H, s.W, s.pad, s.T, s.C, s.Y, s.X, s.Rank, gg.stride_h, gg.stride_w,
+                gg.pad_top, gg.pad_left, gg.out_h, gg.out_w, (unsigned)dtype, (unsigned)act,
+                (unsigned)wanted};
+  std::lock_guard<std::mutex> lk(mu);
+  auto it = plans.find(key);
+  if (it != plans.end()) return it->second;
+  if (plans.size() > 4096) plans.clear();
+  return plans[key] = make_backward_plan(s, g, dtype, act, wanted);
+}
+
+cp4_status check_layer(const cp4_shape* s, const cp4_geometry* g, int dtype, int act) {
+  cp4_status rc = g ? cp4::check_layer_geometry(s, g) : cp4::check_layer_shape(s);
+  if (rc != CP4_OK) return rc;
+  if (act != CP4_ACT_NONE && act != CP4_ACT_RELU)
+    return cp4::fail_with(CP4_ERR_UNSUPPORTED, "activation must be CP4_ACT_NONE or CP4_ACT_RELU");
+  if (dtype != CP4_DTYPE_F32 && dtype != CP4_DTYPE_BF16 && dtype != CP4_DTYPE_F16)
+    return cp4::fail_with(CP4_ERR_UNSUPPORTED, "dtype must be a cp4_dtype");
+  if (g && dtype != CP4_DTYPE_F32)
+    return cp4::fail_with(CP4_ERR_UNSUPPORTED, "a layer with a geometry takes fp32 activations");
+  return CP4_OK;
+}
+
+#define CP4_TRY(call)                     \
+  do {                                    \
+    const cp4_status rc_ = (call);        \
+    if (rc_ != CP4_OK) return rc_;        \
+  } while (0)
+#define CP4_LAUNCH(call)                                      \
+  do {                                                        \
+    const hipError_t e_ = (call);                             \
+    if (e_ != hipSuccess) return cp4::fail_hip(e_, #call);    \
+  } while (0)
+
+}  // namespace
+
+extern "C" {
+
+size_t cp4_layer_forward_workspace_bytes(const cp4_shape* shape, const cp4_geometry* g, int dtype) {
+  if (check_layer(shape, g, dtype, CP4_ACT_NONE) != CP4_OK || shape->N == 0) return 0;
+  if (dtype == CP4_DTYPE_F32 || cp4_bf16_supported(shape, 0)) return 0;
+  return align256(elements(*shape, shape->C) * 4) + align256(elements(*shape, shape->T) * 4);
+}
+
+cp4_status cp4_layer_forward(const cp4_shape* shape, const cp4_geometry* g, int dtype,
+                             const void* x, const float* FK, const float* FC, const float* FH,
+                             const float* FW, const float* bias, int activation, void* y,
+                             void* workspace, size_t workspace_bytes, cp4_stream stream) {
+  CP4_TRY(check_layer(shape, g, dtype, activation));
+  if (dtype == CP4_DTYPE_F32) {
+    const float* xf = static_cast<const float*>(x);
+    float* yf = static_cast<float*>(y);
+    return g ? cp4_conv2d_forward_ex(shape, g, xf, FK, FC, FH, FW, bias, activation, yf, stream)
+             : cp4_conv2d_forward_bias_act(shape, xf, FK, FC, FH, FW, bias, activation, yf, stream);
+  }
+  if (shape->N == 0) return CP4_OK;
+  if (cp4_bf16_supported(shape, 0))
+    return dtype == CP4_DTYPE_BF16
+               ? cp4_conv2d_forward_bf16(shape, x, FK, FC, FH, FW, bias, activation, y, stream)
+               : cp4_conv2d_forward_f16(shape, x, FK, FC, FH, FW, bias, activation, y, stream);
+  if (!x || !y) return cp4::fail_with(CP4_ERR_NULL_POINTER, "x or y is NULL");
+  if (!workspace || workspace_bytes < cp4_layer_forward_workspace_bytes(shape, g, dtype))
+    return cp4::fail_with(CP4_ERR_WORKSPACE, "workspace smaller than cp4_layer_forward_workspace_bytes");
+  const size_t nx = elements(*shape, shape->C), ny = elements(*shape, shape->T);
+  float* x32 = static_cast<float*>(workspace);
+  float* y32 = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + align256(nx * 4));
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  CP4_LAUNCH(cp4::convert_launch(x, dtype, x32, CP4_DTYPE_F32, nx, st));
+  CP4_TRY(cp4_conv2d_forward_bias_act(shape, x32, FK, FC, FH, FW, bias, activation, y32, stream));
+  CP4_LAUNCH(cp4::convert_launch(y32, CP4_DTYPE_F32, y, dtype, ny, st));
+  return CP4_OK;
+}
+
+size_t cp4_layer_backward_workspace_bytes(const cp4_shape* shape, const cp4_geometry* g, int dtype,
+                                          int activation, int wanted) {
+  if (check_layer(shape, g, dtype, activation) != CP4_OK || shape->N == 0) return 0;
+  return backward_plan(*shape, g, dtype, activation, wanted).total;
+}
+
+cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* g, int dtype,
+                              const void* x, const void* y, const void* dy, const float* FK,
+                              const float* FC, const float* FH, const float* FW, int activation,
+                              void* dx, float* dFK, float* dFC, float* dFH, float* dFW,
+                              float* dbias, void* workspace, size_t workspace_bytes,
+                              cp4_stream stream) {
+  CP4_TRY(check_layer(shape, g, dtype, activation));
+  const cp4_shape& s = *shape;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const bool filter = dFK || dFC || dFH || dFW;
+  if (filter && (!dFK || !dFC || !dFH || !dFW))
+    return cp4::fail_with(CP4_ERR_NULL_POINTER, "all four factor gradients or none");
+  if (s.N == 0) {            // empty batch: the gradients of the parameters are zero
+    if (filter)
+      CP4_TRY(cp4_conv2d_backward_filter(shape, nullptr, nullptr, FK, FC, FH, FW, dFK, dFC, dFH,
+                                         dFW, nullptr, 0, stream));
+    if (dbias) CP4_LAUNCH(cp4::zero_f32_launch(dbias, s.T, st));
+    return CP4_OK;
+  }
+  if (!dy || (filter && !x) || (activation != CP4_ACT_NONE && !y))
+    return cp4::fail_with(CP4_ERR_NULL_POINTER, "dy, x (factor gradients) or y (activation) is NULL");
+  const int wanted =
+      (dx ? CP4_WANT_DX : 0) | (filter ? CP4_WANT_FACTORS : 0) | (dbias ? CP4_WANT_BIAS : 0);
+  const BackwardPlan p = backward_plan(s, g, dtype, activation, wanted);
+  if (p.total && (!workspace || workspace_bytes < p.total ||
+                  (reinterpret_cast<uintptr_t>(workspace) & 255)))
+    return cp4::fail_with(CP4_ERR_WORKSPACE, "workspace smaller than "
+                          "cp4_layer_backward_workspace_bytes or not on a 256-byte boundary");
+  unsigned char* ws = static_cast<unsigned char*>(workspace);
+  const size_t plane = out_elements(s, g) / ((size_t)s.N * s.T);
+  const int N = (int)s.N, T = (int)s.T;
+  const bool half = dtype != CP4_DTYPE_F32;
+  const void* ym = activation == CP4_ACT_NONE ? nullptr : y;
+  // 1. dy behind the activation, with the bias gradient
+  const void* dya = dy;                                     // in the layer's type
+  const float* dy32 = reinterpret_cast<const float*>(ws + p.act32_at);
+  float* parts = reinterpret_cast<float*>(ws + p.bias_at);
+  if (p.act16) {
+    CP4_LAUNCH(cp4::act_grad_launch(ym, dy, ws + p.act16_at, dtype, false, dbias, parts, N, T, plane, st));
+    dya = ws + p.act16_at;
+  }
+  if (p.act32)
+    CP4_LAUNCH(cp4::act_grad_launch(ym, dy, ws + p.act32_at, dtype, true, p.act16 ? nullptr : dbias,
+                                    parts, N, T, plane, st));
+  if (!p.act16 && !p.act32 && dbias)
+    CP4_LAUNCH(cp4::act_grad_launch(ym, dy, nullptr, dtype, false, dbias, parts, N, T, plane, st));
+  // 2. the input gradient
+  void* pass_ws = ws + p.pass_at;
+  if (dx && g)
+    CP4_TRY(cp4_conv2d_backward_data_ex(shape, g, static_cast<const float*>(dya), FK, FC, FH, FW,
+                                        static_cast<float*>(dx), pass_ws, p.pass_bytes, stream));
+  else if (dx && !half)
+    CP4_TRY(cp4_conv2d_backward_data(shape, static_cast<const float*>(dya), FK, FC, FH, FW,
+                                     static_cast<float*>(dx), stream));
+  else if (dx && p.dx16)
+    CP4_TRY((dtype == CP4_DTYPE_BF16 ? cp4_conv2d_backward_data_bf16 : cp4_conv2d_backward_data_f16)(
+        shape, dya, FK, FC, FH, FW, dx, stream));
+  else if (dx) {
+    float* dx32 = reinterpret_cast<float*>(ws + p.dx32_at);
+    CP4_TRY(cp4_conv2d_backward_data(shape, dy32, FK, FC, FH, FW, dx32, stream));
+    CP4_LAUNCH(cp4::convert_launch(dx32, CP4_DTYPE_F32, dx, dtype, elements(s, s.C), st));
+  }
+  if (!filter) return CP4_OK;
+  // 3. the factor gradients
+  if (g)
+    return cp4_conv2d_backward_filter_ex(shape, g, static_cast<const float*>(x),
+                                         static_cast<const float*>(dya), FK, FC, FH, FW, dFK, dFC,
+                                         dFH, dFW, pass_ws, p.pass_bytes, stream);
+  if (!half)
+    return cp4_conv2d_backward_filter(shape, static_cast<const float*>(x),
+                                      static_cast<const float*>(dya), FK, FC, FH, FW, dFK, dFC,
+                                      dFH, dFW, pass_ws, p.pass_bytes, stream);
+  if (p.filter16)
+    return (dtype == CP4_DTYPE_BF16 ? cp4_conv2d_backward_filter_bf16
+                                    : cp4_conv2d_backward_filter_f16)(
+        shape, x, dya, FK, FC, FH, FW, dFK, dFC, dFH, dFW, pass_ws, p.pass_bytes, stream);
+  float* x32 = reinterpret_cast<float*>(ws + p.x32_at);
+  CP4_LAUNCH(cp4::convert_launch(x, dtype, x32, CP4_DTYPE_F32, elements(s, s.C), st));
+  return cp4_conv2d_backward_filter(shape, x32, dy32, FK, FC, FH, FW, dFK, dFC, dFH, dFW, pass_ws,
+                                    p.pass_bytes, stream);
+}
+
+}  // extern "C"

@@ -50,130 +50,42 @@ def _after_backward():
 
 
 class CP4Conv2dFunction(torch.autograd.Function):
-    """y = act(cp4conv2d(x, FK, FC, FH, FW, pad) + bias).
+    """y = act(cp4conv2d(x, FK, FC, FH, FW) + bias), forward and backward each one call of
+    the library's layer entry points.
 
-    A bfloat16 ``x`` selects the library's bfloat16-activation entry points
-    (y and the input gradient are bfloat16 then; factors, bias and their
-    gradients stay float32); shapes those do not take are widened to float32.
+    ``geom`` None: stride 1 and ``pad`` zeros on every side, in x's type (float32, bfloat16
+    or float16; factors, bias and their gradients stay float32).  A ``geom`` is a layer with
+    a stride, explicit padding or an output plane of its own; float32 only.
     """
 
     @staticmethod
-    def forward(ctx, x, FK, FC, FH, FW, pad, bias=None, activation=None):
-        if 2 * pad + 1 != FH.shape[0] or 2 * pad + 1 != FW.shape[0]:
+    def forward(ctx, x, FK, FC, FH, FW, pad, bias=None, activation=None, geom=None):
+        if geom is None and (2 * pad + 1 != FH.shape[0] or 2 * pad + 1 != FW.shape[0]):
             raise ValueError("autograd binding needs 2*pad = Y-1 = X-1 (the reference's "
                              "backward-data pass is the adjoint only then)")
         FK, FC, FH, FW = (t.contiguous().float() for t in (FK, FC, FH, FW))
         if bias is not None:
             bias = bias.contiguous().float()
+        x = x.contiguous()
+        if geom is not None or x.dtype not in (torch.bfloat16, torch.float16):
+            x = x.float()
         s = capi.shape_for(x.shape, FK, FC, FH, FW, pad)
-        ctx.half = x.dtype == torch.float16
-        if ctx.half:
-            # half-precision activations: all three passes on the library's float16 entry
-            # points where they take the shape, else on widened copies
-            x = x.contiguous()
-            ctx.pad, ctx.bf16, ctx.shape = pad, False, s
-            ctx.relu = capi.ACTIVATIONS[activation] == 1
-            if capi.bf16_supported(s):
-                y = capi.conv2d_forward_f16(x, FK, FC, FH, FW, bias, activation, pad=pad)
-            else:
-                y = capi.conv2d_forward_bias_act(x.float(), FK, FC, FH, FW, bias, activation,
-                                                 pad=pad).half()
-            ctx.save_for_backward(x, FK, FC, FH, FW, y if ctx.relu else None)
-            return y
-        ctx.bf16 = x.dtype == torch.bfloat16
-        ctx.fwd16 = ctx.bf16 and capi.bf16_supported(s)
-        x = x.contiguous() if ctx.bf16 else x.contiguous().float()
-        ctx.pad = pad
-        if ctx.fwd16:
-            y = capi.conv2d_forward_bf16(x, FK, FC, FH, FW, bias, activation, pad=pad)
-        else:
-            y = capi.conv2d_forward_bias_act(x.float(), FK, FC, FH, FW, bias, activation, pad=pad)
-            if ctx.bf16:
-                y = y.to(torch.bfloat16)
-        ctx.relu = capi.ACTIVATIONS[activation] == 1
-        ctx.shape = s
-        ctx.save_for_backward(x, FK, FC, FH, FW, y if ctx.relu else None)
+        y = capi.layer_forward(s, geom, x, FK, FC, FH, FW, bias, activation)
+        ctx.shape, ctx.geom, ctx.activation = s, geom, activation
+        relu = capi.ACTIVATIONS[activation] == 1
+        ctx.save_for_backward(x, FK, FC, FH, FW, y if relu else None)
         return y
 
     @staticmethod
     def backward(ctx, dy):
         x, FK, FC, FH, FW, y = ctx.saved_tensors
-        s = ctx.shape
-        dy = dy.contiguous()
-        if ctx.relu:
-            dy = dy * (y > 0)
-        dbias = dy.float().sum(dim=(0, 2, 3)) if ctx.needs_input_grad[6] else None
-        dy16 = ctx.bf16 and dy.dtype == torch.bfloat16
-        dx = None
-        if ctx.half:
-            if ctx.needs_input_grad[0]:
-                if dy.dtype == torch.float16 and capi.bf16_supported(s, backward_data=True):
-                    dx = capi.conv2d_backward_data_f16(dy, FK, FC, FH, FW, pad=ctx.pad)
-                else:
-                    dx = capi.conv2d_backward_data(dy.float(), FK, FC, FH, FW, pad=ctx.pad).half()
-            grads = (None, None, None, None)
-            if any(ctx.needs_input_grad[1:5]):
-                if dy.dtype == torch.float16 and capi.bf16_backward_filter_supported(s):
-                    grads = capi.conv2d_backward_filter_f16(x, dy, FK, FC, FH, FW, pad=ctx.pad)
-                else:
-                    grads = capi.conv2d_backward_filter(x.float(), dy.float(), FK, FC, FH, FW,
-                                                        pad=ctx.pad)
-                grads = tuple(g if need else None
-                              for g, need in zip(grads, ctx.needs_input_grad[1:5]))
-            _after_backward()
-            return (dx,) + grads + (None, dbias, None)
-        if ctx.needs_input_grad[0]:
-            if dy16 and capi.bf16_supported(s, backward_data=True):
-                dx = capi.conv2d_backward_data_bf16(dy, FK, FC, FH, FW, pad=ctx.pad)
-            else:
-                dx = capi.conv2d_backward_data(dy.float(), FK, FC, FH, FW, pad=ctx.pad)
-                if ctx.bf16:
-                    dx = dx.to(torch.bfloat16)
-        grads = (None, None, None, None)
-        if any(ctx.needs_input_grad[1:5]):
-            if dy16 and capi.bf16_backward_filter_supported(s):
-                grads = capi.conv2d_backward_filter_bf16(x, dy, FK, FC, FH, FW, pad=ctx.pad)
-            else:
-                grads = capi.conv2d_backward_filter(x.float(), dy.float(), FK, FC, FH, FW,
-                                                    pad=ctx.pad)
-            grads = tuple(g if need else None
-                          for g, need in zip(grads, ctx.needs_input_grad[1:5]))
+        need = ctx.needs_input_grad
+        dx, grads, dbias = capi.layer_backward(
+            ctx.shape, ctx.geom, x, y, dy.contiguous().to(x.dtype), FK, FC, FH, FW, ctx.activation,
+            want_dx=need[0], want_factors=any(need[1:5]), want_bias=need[6])
+        grads = tuple(g if n else None for g, n in zip(grads, need[1:5]))
         _after_backward()
-        return (dx,) + grads + (None, dbias, None)
-
-
-class CP4Conv2dGeometryFunction(torch.autograd.Function):
-    """The layer with a stride, explicit padding or an output plane of its own
-    (cp4_conv2d_forward_ex and its two gradients; float32)."""
-
-    @staticmethod
-    def forward(ctx, x, FK, FC, FH, FW, geom, bias=None, activation=None):
-        x, FK, FC, FH, FW = (t.contiguous().float() for t in (x, FK, FC, FH, FW))
-        if bias is not None:
-            bias = bias.contiguous().float()
-        y = capi.conv2d_forward_ex(x, FK, FC, FH, FW, geom, bias, activation)
-        ctx.geom = geom
-        ctx.relu = capi.ACTIVATIONS[activation] == 1
-        ctx.save_for_backward(x, FK, FC, FH, FW, y if ctx.relu else None)
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        x, FK, FC, FH, FW, y = ctx.saved_tensors
-        dy = dy.contiguous().float()
-        if ctx.relu:
-            dy = dy * (y > 0)
-        dbias = dy.sum(dim=(0, 2, 3)) if ctx.needs_input_grad[6] else None
-        dx = None
-        if ctx.needs_input_grad[0]:
-            dx = capi.conv2d_backward_data_ex(dy, x.shape[2:], FK, FC, FH, FW, ctx.geom)
-        grads = (None, None, None, None)
-        if any(ctx.needs_input_grad[1:5]):
-            grads = capi.conv2d_backward_filter_ex(x, dy, FK, FC, FH, FW, ctx.geom)
-            grads = tuple(g if need else None
-                          for g, need in zip(grads, ctx.needs_input_grad[1:5]))
-        _after_backward()
-        return (dx,) + grads + (None, dbias, None)
+        return (dx,) + grads + (None, dbias, None, None)
 
 
 def cp4_conv2d(x, FK, FC, FH, FW, pad, bias=None, activation=None, stride=1, padding=None):
@@ -197,7 +109,7 @@ def cp4_conv2d(x, FK, FC, FH, FW, pad, bias=None, activation=None, stride=1, pad
         return CP4Conv2dFunction.apply(x, FK, FC, FH, FW, y_taps // 2, bias, activation)
     s = capi.shape_for(x.shape, FK, FC, FH, FW, 0)
     geom = capi.geometry(s, stride, padding)
-    return CP4Conv2dGeometryFunction.apply(x, FK, FC, FH, FW, geom, bias, activation)
+    return CP4Conv2dFunction.apply(x, FK, FC, FH, FW, 0, bias, activation, geom)
 
 
 class CP4Conv2d(torch.nn.Module):

@@ -1,0 +1,70 @@
+"""The layer entry points (cp4_layer_forward / cp4_layer_backward): what the activation's
+backward and the bias gradient do at the edges of their kernel - planes that are no multiple
+of a 16-byte piece, channels of one and of many segments, every element type - against
+float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def capi():
+    import paralleltnnlayers_amd.capi as c
+    c.lib()
+    assert torch.cuda.is_available()
+    return c
+
+
+# (N, T, H, W): one pixel / odd plane / a piece and one / several batches per lane / segments
+# that end inside a plane / more channels than workgroups per segment
+@pytest.mark.parametrize("dims", [(1, 1, 1, 1), (3, 5, 7, 7), (2, 3, 3, 3), (4, 2, 55, 55),
+                                  (3, 2, 129, 130), (2, 600, 9, 16)],
+                         ids=lambda d: "x".join(map(str, d)))
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16],
+                         ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("relu", [True, False], ids=["relu", "linear"])
+def test_bias_and_activation_gradient(capi, dims, dtype, relu):
+    N, T, H, W = dims
+    C, R = 4, 2
+    gen = torch.Generator(device="cuda").manual_seed(sum(dims))
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, dy = mk(N, C, H, W).to(dtype), mk(N, T, H, W).to(dtype)
+    fac = [mk(d, R) for d in (T, C, 1, 1)]
+    bias = mk(T)
+    s = capi.shape_for(x.shape, *fac, 0)
+    act = "relu" if relu else None
+    y = capi.layer_forward(s, None, x, *fac, bias, act)
+    dx, grads, dbias = capi.layer_backward(s, None, x, y, dy, *fac, act)
+    masked = torch.where(y > 0, dy, torch.zeros_like(dy)) if relu else dy
+    want = masked.double().sum(dim=(0, 2, 3))
+    # fp32 sums of N * H * W terms: 2^-24 each step, as a random walk over the terms
+    tol = 2.0 ** -22 * (masked.double() ** 2).sum(dim=(0, 2, 3)).sqrt() * (1 + (N * H * W) ** 0.5 / 64)
+    assert ((dbias.double() - want).abs() <= tol + 1e-30).all()
+    # the gradients are those of the masked dy: 1x1 filter, so the layer is a matrix product
+    K = torch.einsum("tr,cr,r->tc", fac[0].double(), fac[1].double(),
+                     (fac[2][0] * fac[3][0]).double())
+    want_dx = torch.einsum("tc,nthw->nchw", K, masked.double())
+    eps = {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    bound = eps * want_dx.abs() * 1.01 + 1e-5 * want_dx.abs().max()
+    assert ((dx.double() - want_dx).abs() <= bound).all()
+    dK = torch.einsum("nthw,nchw->tc", masked.double(), x.double())
+    want_dFK = dK @ (fac[1] * fac[2][0] * fac[3][0]).double()
+    assert (grads[0].double() - want_dFK).abs().max() <= 1e-4 * want_dFK.abs().max() + 1e-6
+
+
+def test_parts_on_their_own(capi):
+    """Each gradient alone is the one of the whole call; what is not wanted is not computed."""
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, dy = mk(2, 16, 9, 11), mk(2, 24, 9, 11)
+    fac = [mk(d, 8) for d in (24, 16, 3, 3)]
+    s = capi.shape_for(x.shape, *fac, 1)
+    y = capi.layer_forward(s, None, x, *fac, mk(24), "relu")
+    dx, grads, db = capi.layer_backward(s, None, x, y, dy, *fac, "relu")
+    only_dx = capi.layer_backward(s, None, x, y, dy, *fac, "relu", True, False, False)
+    only_f = capi.layer_backward(s, None, x, y, dy, *fac, "relu", False, True, False)
+    only_b = capi.layer_backward(s, None, x, y, dy, *fac, "relu", False, False, True)
+    assert torch.equal(only_dx[0], dx) and only_dx[2] is None and only_dx[1][0] is None
+    assert all(torch.equal(a, b) for a, b in zip(only_f[1], grads)) and only_f[0] is None
+    assert torch.equal(only_b[2], db)
