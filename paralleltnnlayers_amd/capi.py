@@ -43,6 +43,16 @@ class RcpDims(ctypes.Structure):
     _fields_ = [(k, ctypes.c_uint) for k in ("S0", "S1", "T0", "T1")]
 
 
+try:
+    from . import _binding as _native
+    _native.set_error(Cp4Error)
+except ImportError as _e:                    # not built: reported at the first call
+    class _Missing:
+        def __getattr__(self, name, _why=str(_e)):
+            raise ImportError(f"paralleltnnlayers_amd._binding is missing ({_why}): build it with "
+                              "`python -c 'import __graft_entry__ as g; g.build()'`")
+    _native = _Missing()
+
 # status codes of cp4_status
 (OK, ERR_NULL_POINTER, ERR_SHAPE, ERR_HIP, ERR_WORKSPACE, ERR_UNSUPPORTED,
  ERR_DEVICE) = range(7)
@@ -224,14 +234,7 @@ def shape_for(x_or_dy_shape, FK, FC, FH, FW, pad):
 
 
 def conv2d_forward(x, FK, FC, FH, FW, pad=1, out=None, variant=-1, stream=None):
-    s = shape_for(x.shape, FK, FC, FH, FW, pad)
-    assert x.shape[1] == s.C and FC.shape[1] == s.Rank
-    y = out if out is not None else torch.empty((s.N, s.T, s.H, s.W), device=x.device,
-                                                dtype=torch.float32)
-    check(lib().cp4_conv2d_forward_variant(ctypes.byref(s), _ptr(x), _ptr(FK), _ptr(FC),
-                                           _ptr(FH), _ptr(FW), _ptr(y), variant,
-                                           _stream(stream)))
-    return y
+    return _native.forward(x, FK, FC, FH, FW, pad, out, variant, stream)
 
 
 ACTIVATIONS = {None: 0, "none": 0, "relu": 1}
@@ -512,13 +515,7 @@ def layer_backward(s, g, x, y, dy, FK, FC, FH, FW, activation=None, want_dx=True
 
 
 def conv2d_backward_data(dy, FK, FC, FH, FW, pad=1, out=None, stream=None):
-    s = shape_for(dy.shape, FK, FC, FH, FW, pad)
-    assert dy.shape[1] == s.T
-    dx = out if out is not None else torch.empty((s.N, s.C, s.H, s.W), device=dy.device,
-                                                 dtype=torch.float32)
-    check(lib().cp4_conv2d_backward_data(ctypes.byref(s), _ptr(dy), _ptr(FK), _ptr(FC),
-                                         _ptr(FH), _ptr(FW), _ptr(dx), _stream(stream)))
-    return dx
+    return _native.backward_data(dy, FK, FC, FH, FW, pad, out, stream)
 
 
 def backward_filter_workspace_bytes(s):
@@ -538,15 +535,7 @@ def _workspace(s, device, workspace):
 def conv2d_backward_filter(x, dy, FK, FC, FH, FW, pad=1, workspace=None, stream=None,
                            variant=-1):
     """Returns (dFK, dFC, dFH, dFW)."""
-    s = shape_for(x.shape, FK, FC, FH, FW, pad)
-    assert tuple(dy.shape) == (s.N, s.T, s.H, s.W) and x.shape[1] == s.C
-    outs = [torch.empty_like(f) for f in (FK, FC, FH, FW)]
-    ws, ws_bytes = _workspace(s, x.device, workspace)
-    check(lib().cp4_conv2d_backward_filter_variant(
-        ctypes.byref(s), _ptr(x), _ptr(dy), _ptr(FK), _ptr(FC), _ptr(FH), _ptr(FW),
-        *[_ptr(o) for o in outs], ctypes.c_void_p(ws.data_ptr()), ws_bytes, variant,
-        _stream(stream)))
-    return tuple(outs)
+    return _native.backward_filter(x, dy, FK, FC, FH, FW, pad, workspace, stream, variant)
 
 
 def conv2d_backward_filter_noalloc(x, dy, FK, FC, FH, FW, outs, pad=1, stream=None):

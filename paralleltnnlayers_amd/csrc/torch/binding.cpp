@@ -1,0 +1,383 @@
+// PyTorch binding of the C ABI (module paralleltnnlayers_amd._binding): the three passes and
+// the differentiable layer as native calls.
+//
+// A small layer's pass takes 4 - 8 us on the device; through ctypes and a Python
+// autograd.Function one call cost 11 us (a pass), 20 us (a layer's inference) and some 150 us
+// of a training step (forward and backward, each with its own tensors, workspace query and
+// argument conversions).  Here the arguments are parsed in place, outputs come straight from
+// the caching allocator and the layer is a C++ autograd function, whose backward runs without
+// the interpreter.
+//
+// The semantics are the Python functions' of capi.py / torch_ops.py that call this module.
+// Stands where the reference registers its op with a framework (Kernels/cp4_conv_nchw.cc:6-108).
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/core/grad_mode.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <atomic>
+#include <optional>
+#include <string>
+
+#include "cp4/capi.h"
+
+namespace {
+
+using at::Tensor;
+
+PyObject* g_error = nullptr;                    // capi.Cp4Error(status, message)
+std::atomic<bool> g_check_backward{false};      // torch_ops.set_device_checks
+
+// ---- errors ---------------------------------------------------------------------
+
+void set_status_error(cp4_status rc) {
+  const std::string text =
+      std::string(cp4_status_string(rc)) + ": " + cp4_last_error_message();
+  PyObject* args = Py_BuildValue("(is)", (int)rc, text.c_str());
+  PyObject* err = args && g_error ? PyObject_CallObject(g_error, args) : nullptr;
+  Py_XDECREF(args);
+  if (err) {
+    PyErr_SetObject(g_error, err);
+    Py_DECREF(err);
+  } else if (!PyErr_Occurred()) {
+    PyErr_SetString(PyExc_RuntimeError, text.c_str());
+  }
+}
+// From any thread, with or without the interpreter lock (the autograd engine's threads run
+// without it): the Python exception travels through the engine as it is.
+void check(cp4_status rc) {
+  if (rc == CP4_OK) return;
+  PyGILState_STATE gil = PyGILState_Ensure();
+  set_status_error(rc);
+  python_error e;
+  e.persist();
+  PyGILState_Release(gil);
+  throw e;
+}
+[[noreturn]] void fail(PyObject* type, const char* what) {
+  PyErr_SetString(type, what);
+  python_error e;
+  e.persist();
+  throw e;
+}
+void require(bool ok, const char* what = "") {
+  if (!ok) fail(PyExc_AssertionError, what);
+}
+
+// ---- arguments --------------------------------------------------------------------
+
+const Tensor& tensor(PyObject* o) {
+  if (!THPVariable_Check(o)) fail(PyExc_AssertionError, "expected a tensor");
+  return THPVariable_Unpack(o);
+}
+long integer(PyObject* o) {
+  const long v = PyLong_AsLong(o);
+  if (v == -1 && PyErr_Occurred()) throw python_error();
+  return v;
+}
+float* f32(const Tensor& t) {
+  require(t.is_cuda() && t.scalar_type() == at::kFloat && t.is_contiguous(),
+          "expected a contiguous float32 device tensor");
+  return static_cast<float*>(t.data_ptr());
+}
+void* stream_of(PyObject* o) {
+  if (o && o != Py_None) {
+    PyObject* h = PyObject_GetAttrString(o, "cuda_stream");
+    if (!h) throw python_error();
+    void* s = PyLong_AsVoidPtr(h);
+    Py_DECREF(h);
+    return s;
+  }
+  return c10::hip::getCurrentHIPStream().stream();
+}
+Tensor empty(at::IntArrayRef sizes, at::ScalarType type, const Tensor& like) {
+  return at::detail::empty_cuda(sizes, type, like.device(), std::nullopt);
+}
+// Device memory of `bytes` (the allocator's blocks lie on 512-byte boundaries); undefined for 0.
+Tensor scratch(size_t bytes, const Tensor& like) {
+  return bytes ? empty({(int64_t)bytes}, at::kByte, like) : Tensor();
+}
+void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+struct Factors {
+  const Tensor &FK, &FC, &FH, &FW;
+};
+// tensor_shape as CP::Conv2dForward / Conv2dBackwardData derive it (Cuda_kernels/cp4Conv2d.cu:21-30)
+cp4_shape shape_for(const Tensor& act, const Factors& f, long pad) {
+  require(act.dim() == 4 && f.FK.dim() == 2 && f.FC.dim() == 2 && f.FH.dim() == 2 && f.FW.dim() == 2);
+  cp4_shape s;
+  s.N = (unsigned)act.size(0); s.H = (unsigned)act.size(2); s.W = (unsigned)act.size(3);
+  s.pad = (unsigned)pad;
+  s.T = (unsigned)f.FK.size(0); s.C = (unsigned)f.FC.size(0); s.Y = (unsigned)f.FH.size(0);
+  s.X = (unsigned)f.FW.size(0); s.Rank = (unsigned)f.FK.size(1);
+  return s;
+}
+
+// ---- the three passes (capi.conv2d_forward, _backward_data, _backward_filter) --------
+
+// (x, FK, FC, FH, FW, pad, out, variant, stream) -> y
+PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  require(n == 9);
+  const Tensor& x = tensor(a[0]);
+  const Factors f{tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4])};
+  const cp4_shape s = shape_for(x, f, integer(a[5]));
+  require(x.size(1) == s.C && f.FC.size(1) == s.Rank);
+  const float *px = f32(x), *pK = f32(f.FK), *pC = f32(f.FC), *pH = f32(f.FH), *pW = f32(f.FW);
+  Tensor y = a[6] != Py_None ? tensor(a[6]) : empty({s.N, s.T, s.H, s.W}, at::kFloat, x);
+  check(cp4_conv2d_forward_variant(&s, px, pK, pC, pH, pW, f32(y), (int)integer(a[7]),
+                                   stream_of(a[8])));
+  return THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
+// (dy, FK, FC, FH, FW, pad, out, stream) -> dx
+PyObject* backward_data(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  require(n == 8);
+  const Tensor& dy = tensor(a[0]);
+  const Factors f{tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4])};
+  const cp4_shape s = shape_for(dy, f, integer(a[5]));
+  require(dy.size(1) == s.T);
+  const float *pdy = f32(dy), *pK = f32(f.FK), *pC = f32(f.FC), *pH = f32(f.FH), *pW = f32(f.FW);
+  Tensor dx = a[6] != Py_None ? tensor(a[6]) : empty({s.N, s.C, s.H, s.W}, at::kFloat, dy);
+  check(cp4_conv2d_backward_data(&s, pdy, pK, pC, pH, pW, f32(dx), stream_of(a[7])));
+  return THPVariable_Wrap(std::move(dx));
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* wrap_four(Tensor (&t)[4]) {
+  PyObject* out = PyTuple_New(4);
+  if (!out) throw python_error();
+  for (int i = 0; i < 4; ++i) PyTuple_SET_ITEM(out, i, THPVariable_Wrap(std::move(t[i])));
+  return out;
+}
+
+// (x, dy, FK, FC, FH, FW, pad, workspace, stream, variant) -> (dFK, dFC, dFH, dFW)
+PyObject* backward_filter(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  require(n == 10);
+  const Tensor &x = tensor(a[0]), &dy = tensor(a[1]);
+  const Factors f{tensor(a[2]), tensor(a[3]), tensor(a[4]), tensor(a[5])};
+  const cp4_shape s = shape_for(x, f, integer(a[6]));
+  require(dy.dim() == 4 && dy.size(0) == s.N && dy.size(1) == s.T && dy.size(2) == s.H &&
+          dy.size(3) == s.W && x.size(1) == s.C);
+  const float *px = f32(x), *pdy = f32(dy), *pK = f32(f.FK), *pC = f32(f.FC), *pH = f32(f.FH),
+              *pW = f32(f.FW);
+  Tensor grads[4];
+  const Tensor* fac[4] = {&f.FK, &f.FC, &f.FH, &f.FW};
+  for (int i = 0; i < 4; ++i) grads[i] = empty(fac[i]->sizes(), at::kFloat, x);
+  Tensor ws;
+  if (a[7] != Py_None) {
+    ws = tensor(a[7]);
+    require(ws.is_cuda() && ws.is_contiguous(), "the workspace must be a contiguous device tensor");
+  } else {
+    const size_t need = cp4_conv2d_backward_filter_workspace_bytes(&s);
+    ws = scratch(need ? need : 4, x);
+  }
+  check(cp4_conv2d_backward_filter_variant(
+      &s, px, pdy, pK, pC, pH, pW, f32(grads[0]), f32(grads[1]), f32(grads[2]), f32(grads[3]), ws.data_ptr(), (size_t)ws.numel() * ws.element_size(),
+      (int)integer(a[9]), stream_of(a[8])));
+  return wrap_four(grads);
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- the differentiable layer (torch_ops.cp4_conv2d) -----------------------------------
+
+struct LayerSpec {
+  cp4_shape shape;
+  cp4_geometry geometry;
+  bool has_geometry, has_bias;
+  int dtype, activation;
+  const cp4_geometry* g() const { return has_geometry ? &geometry : nullptr; }
+};
+
+Tensor as_f32(const Tensor& t) {
+  if (t.scalar_type() == at::kFloat && t.is_contiguous()) return t;
+  return t.contiguous().to(at::kFloat);
+}
+
+Tensor layer_forward(const LayerSpec& l, const Tensor& x, const Factors& f, const Tensor& bias) {
+  const cp4_shape& s = l.shape;
+  const int64_t oh = l.has_geometry ? l.geometry.out_h : s.H, ow = l.has_geometry ? l.geometry.out_w : s.W;
+  Tensor y = empty({s.N, s.T, oh, ow}, x.scalar_type(), x);
+  const size_t need = l.dtype == CP4_DTYPE_F32
+                          ? 0 : cp4_layer_forward_workspace_bytes(&s, l.g(), l.dtype);
+  const Tensor ws = scratch(need, x);
+  check(cp4_layer_forward(&s, l.g(), l.dtype, x.data_ptr(), f32(f.FK), f32(f.FC), f32(f.FH),
+                          f32(f.FW), bias.defined() ? f32(bias) : nullptr, l.activation,
+                          y.data_ptr(), ptr(ws), need,
+                          c10::hip::getCurrentHIPStream(x.device().index()).stream()));
+  return y;
+}
+
+struct LayerFunction : torch::autograd::Function<LayerFunction> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& FK,
+                        const Tensor& FC, const Tensor& FH, const Tensor& FW,
+                        const std::optional<Tensor>& bias, LayerSpec l) {
+    const Factors f{as_f32(FK), as_f32(FC), as_f32(FH), as_f32(FW)};
+    const Tensor b = bias ? as_f32(*bias) : Tensor();
+    Tensor y = layer_forward(l, x, f, b);
+    const bool relu = l.activation == CP4_ACT_RELU;
+    ctx->save_for_backward({x, f.FK, f.FC, f.FH, f.FW, relu ? y : Tensor()});
+    ctx->saved_data["spec"] = c10::IValue(std::string(reinterpret_cast<const char*>(&l), sizeof l));
+    return y;
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grad) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &FK = saved[1], &FC = saved[2], &FH = saved[3], &FW = saved[4];
+    LayerSpec l;
+    {
+      const std::string& raw = ctx->saved_data["spec"].toStringRef();
+      memcpy(&l, raw.data(), sizeof l);
+    }
+    torch::autograd::variable_list out(7);
+    if (!grad[0].defined()) return out;
+    Tensor dy = grad[0].contiguous();
+    if (dy.scalar_type() != x.scalar_type()) dy = dy.to(x.scalar_type());
+    const bool want_dx = ctx->needs_input_grad(0), want_bias = l.has_bias && ctx->needs_input_grad(5);
+    bool want_factor[4], want_factors = false;
+    for (int i = 0; i < 4; ++i) want_factors |= want_factor[i] = ctx->needs_input_grad(1 + i);
+    const Tensor* fac[4] = {&FK, &FC, &FH, &FW};
+    Tensor dx, grads[4], dbias;
+    if (want_dx) dx = empty(x.sizes(), x.scalar_type(), x);
+    if (want_factors)
+      for (int i = 0; i < 4; ++i) grads[i] = empty(fac[i]->sizes(), at::kFloat, x);
+    if (want_bias) dbias = empty({(int64_t)l.shape.T}, at::kFloat, x);
+    const int wanted = (want_dx ? CP4_WANT_DX : 0) | (want_factors ? CP4_WANT_FACTORS : 0) |
+                       (want_bias ? CP4_WANT_BIAS : 0);
+    const size_t need =
+        cp4_layer_backward_workspace_bytes(&l.shape, l.g(), l.dtype, l.activation, wanted);
+    const Tensor ws = scratch(need, x);
+    void* st = c10::hip::getCurrentHIPStream(x.device().index()).stream();
+    check(cp4_layer_backward(&l.shape, l.g(), l.dtype, x.data_ptr(), ptr(saved[5]), dy.data_ptr(),
+                             f32(FK), f32(FC), f32(FH), f32(FW), l.activation, ptr(dx),
+                             static_cast<float*>(ptr(grads[0])), static_cast<float*>(ptr(grads[1])),
+                             static_cast<float*>(ptr(grads[2])), static_cast<float*>(ptr(grads[3])),
+                             static_cast<float*>(ptr(dbias)), ptr(ws), need, st));
+    if (g_check_backward.load(std::memory_order_relaxed)) check(cp4_device_status(st, nullptr));
+    out[0] = dx;
+    for (int i = 0; i < 4; ++i)
+      if (want_factor[i]) out[1 + i] = grads[i];
+    out[5] = dbias;
+    return out;
+  }
+};
+
+int activation_of(PyObject* o) {
+  if (o == Py_None) return CP4_ACT_NONE;
+  if (PyUnicode_Check(o)) {
+    if (PyUnicode_CompareWithASCIIString(o, "relu") == 0) return CP4_ACT_RELU;
+    if (PyUnicode_CompareWithASCIIString(o, "none") == 0) return CP4_ACT_NONE;
+  }
+  PyErr_SetObject(PyExc_KeyError, o);
+  throw python_error();
+}
+
+// An int or a pair of ints.
+void int_pair(PyObject* o, long* h, long* w) {
+  if (PyLong_Check(o)) {
+    *h = *w = integer(o);
+    return;
+  }
+  PyObject* seq = PySequence_Fast(o, "expected an int or an (h, w) pair");
+  if (!seq) throw python_error();
+  const bool two = PySequence_Fast_GET_SIZE(seq) == 2;
+  if (two) {
+    *h = PyLong_AsLong(PySequence_Fast_GET_ITEM(seq, 0));
+    *w = PyLong_AsLong(PySequence_Fast_GET_ITEM(seq, 1));
+  }
+  Py_DECREF(seq);
+  if (PyErr_Occurred()) throw python_error();
+  if (!two) fail(PyExc_ValueError, "expected an int or an (h, w) pair");
+}
+
+// (x, FK, FC, FH, FW, pad, bias, activation, stride, padding) -> y; see torch_ops.cp4_conv2d
+PyObject* layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  require(n == 10);
+  const Tensor& x_in = tensor(a[0]);
+  const Factors f{tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4])};
+  LayerSpec l{};
+  l.activation = activation_of(a[7]);
+  PyObject* padding = a[9] == Py_None ? a[5] : a[9];
+  const bool same = PyUnicode_Check(padding) && PyUnicode_CompareWithASCIIString(padding, "same") == 0;
+  const bool valid = PyUnicode_Check(padding) && PyUnicode_CompareWithASCIIString(padding, "valid") == 0;
+  long sh, sw;
+  int_pair(a[8], &sh, &sw);
+  l.shape = shape_for(x_in, f, 0);
+  const long Y = l.shape.Y, X = l.shape.X;
+  // the reference's own layer runs its three passes as they are
+  bool plain = PyLong_Check(a[8]) && sh == 1 && Y == X;
+  if (plain && PyLong_Check(padding)) plain = 2 * integer(padding) + 1 == Y;
+  else plain = plain && same && Y % 2 == 1;
+  if (plain) {
+    l.shape.pad = (unsigned)(Y / 2);
+  } else {
+    l.has_geometry = true;
+    if (same) {
+      check(cp4_geometry_same(&l.shape, (unsigned)sh, (unsigned)sw, &l.geometry));
+    } else if (valid) {
+      check(cp4_geometry_valid(&l.shape, (unsigned)sh, (unsigned)sw, &l.geometry));
+    } else {
+      long ph, pw;
+      int_pair(padding, &ph, &pw);
+      check(cp4_geometry_symmetric(&l.shape, (unsigned)sh, (unsigned)sw, (unsigned)ph, (unsigned)pw,
+                                   &l.geometry));
+    }
+  }
+  const at::ScalarType t = x_in.scalar_type();
+  const bool half = plain && (t == at::kBFloat16 || t == at::kHalf);
+  l.dtype = !half ? CP4_DTYPE_F32 : t == at::kBFloat16 ? CP4_DTYPE_BF16 : CP4_DTYPE_F16;
+  const Tensor x = half ? x_in.contiguous() : as_f32(x_in);
+  require(x.is_cuda() && x.size(1) == l.shape.C && f.FC.size(1) == l.shape.Rank,
+          "expected a device tensor [N, C, H, W] that matches the factors");
+  std::optional<Tensor> bias;
+  if (a[6] != Py_None) {
+    bias = tensor(a[6]);
+    require(bias->dim() == 1 && bias->size(0) == l.shape.T);
+    l.has_bias = true;
+  }
+  const c10::DeviceGuard guard(x.device());
+  const bool track = at::GradMode::is_enabled() &&
+                     (x.requires_grad() || f.FK.requires_grad() || f.FC.requires_grad() ||
+                      f.FH.requires_grad() || f.FW.requires_grad() || (bias && bias->requires_grad()));
+  if (track) return THPVariable_Wrap(LayerFunction::apply(x, f.FK, f.FC, f.FH, f.FW, bias, l));
+  const Tensor FK = as_f32(f.FK), FC = as_f32(f.FC), FH = as_f32(f.FH), FW = as_f32(f.FW);
+  return THPVariable_Wrap(layer_forward(l, x, Factors{FK, FC, FH, FW}, bias ? as_f32(*bias) : Tensor()));
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* set_error(PyObject*, PyObject* type) {
+  Py_XINCREF(type);
+  Py_XSETREF(g_error, type);
+  Py_RETURN_NONE;
+}
+PyObject* set_check_backward(PyObject*, PyObject* on) {
+  g_check_backward.store(PyObject_IsTrue(on) == 1);
+  Py_RETURN_NONE;
+}
+
+#define FAST(fn) reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(fn)), METH_FASTCALL
+PyMethodDef kMethods[] = {
+    {"forward", FAST(forward), nullptr},
+    {"backward_data", FAST(backward_data), nullptr},
+    {"backward_filter", FAST(backward_filter), nullptr},
+    {"layer", FAST(layer), nullptr},
+    {"set_error", set_error, METH_O, nullptr},
+    {"set_check_backward", set_check_backward, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_binding", nullptr, -1, kMethods,
+                       nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__binding(void) { return PyModule_Create(&kModule); }

@@ -28,13 +28,15 @@ import torch
 
 from . import capi
 
-_check_every_backward = os.environ.get("CP4_CHECK_DEVICE", "0") not in ("", "0")
-
 
 def set_device_checks(on):
     """Check the device's fault record at the end of every backward pass (synchronises)."""
     global _check_every_backward
     _check_every_backward = bool(on)
+    capi._native.set_check_backward(_check_every_backward)
+
+
+set_device_checks(os.environ.get("CP4_CHECK_DEVICE", "0") not in ("", "0"))
 
 
 def check_device(stream=None):
@@ -49,43 +51,21 @@ def _after_backward():
         capi.device_status()
 
 
-class CP4Conv2dFunction(torch.autograd.Function):
-    """y = act(cp4conv2d(x, FK, FC, FH, FW) + bias), forward and backward each one call of
-    the library's layer entry points.
+class CP4Conv2dFunction:
+    """y = act(cp4conv2d(x, FK, FC, FH, FW, pad) + bias), differentiable; the autograd
+    function itself is native (csrc/torch/binding.cpp).
 
-    ``geom`` None: stride 1 and ``pad`` zeros on every side, in x's type (float32, bfloat16
-    or float16; factors, bias and their gradients stay float32).  A ``geom`` is a layer with
-    a stride, explicit padding or an output plane of its own; float32 only.
+    A bfloat16 or float16 ``x`` selects the library's 16-bit activations (y and the input
+    gradient are of x's type then; factors, bias and their gradients stay float32); shapes
+    those do not take run on widened copies.
     """
 
     @staticmethod
-    def forward(ctx, x, FK, FC, FH, FW, pad, bias=None, activation=None, geom=None):
-        if geom is None and (2 * pad + 1 != FH.shape[0] or 2 * pad + 1 != FW.shape[0]):
+    def apply(x, FK, FC, FH, FW, pad, bias=None, activation=None):
+        if 2 * pad + 1 != FH.shape[0] or 2 * pad + 1 != FW.shape[0]:
             raise ValueError("autograd binding needs 2*pad = Y-1 = X-1 (the reference's "
                              "backward-data pass is the adjoint only then)")
-        FK, FC, FH, FW = (t.contiguous().float() for t in (FK, FC, FH, FW))
-        if bias is not None:
-            bias = bias.contiguous().float()
-        x = x.contiguous()
-        if geom is not None or x.dtype not in (torch.bfloat16, torch.float16):
-            x = x.float()
-        s = capi.shape_for(x.shape, FK, FC, FH, FW, pad)
-        y = capi.layer_forward(s, geom, x, FK, FC, FH, FW, bias, activation)
-        ctx.shape, ctx.geom, ctx.activation = s, geom, activation
-        relu = capi.ACTIVATIONS[activation] == 1
-        ctx.save_for_backward(x, FK, FC, FH, FW, y if relu else None)
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        x, FK, FC, FH, FW, y = ctx.saved_tensors
-        need = ctx.needs_input_grad
-        dx, grads, dbias = capi.layer_backward(
-            ctx.shape, ctx.geom, x, y, dy.contiguous().to(x.dtype), FK, FC, FH, FW, ctx.activation,
-            want_dx=need[0], want_factors=any(need[1:5]), want_bias=need[6])
-        grads = tuple(g if n else None for g, n in zip(grads, need[1:5]))
-        _after_backward()
-        return (dx,) + grads + (None, dbias, None, None)
+        return capi._native.layer(x, FK, FC, FH, FW, pad, bias, activation, 1, None)
 
 
 def cp4_conv2d(x, FK, FC, FH, FW, pad, bias=None, activation=None, stride=1, padding=None):
@@ -99,17 +79,7 @@ def cp4_conv2d(x, FK, FC, FH, FW, pad, bias=None, activation=None, stride=1, pad
     after the image than before it), "valid", an int or an (h, w) pair run the
     strided kernels: only the kept outputs are computed.
     """
-    if padding is None:
-        padding = pad
-    y_taps, x_taps = FH.shape[0], FW.shape[0]
-    plain = stride == 1 and (
-        (isinstance(padding, int) and 2 * padding + 1 == y_taps == x_taps) or
-        (padding == "same" and y_taps == x_taps and y_taps % 2 == 1))
-    if plain:
-        return CP4Conv2dFunction.apply(x, FK, FC, FH, FW, y_taps // 2, bias, activation)
-    s = capi.shape_for(x.shape, FK, FC, FH, FW, 0)
-    geom = capi.geometry(s, stride, padding)
-    return CP4Conv2dFunction.apply(x, FK, FC, FH, FW, 0, bias, activation, geom)
+    return capi._native.layer(x, FK, FC, FH, FW, pad, bias, activation, stride, padding)
 
 
 class CP4Conv2d(torch.nn.Module):
@@ -139,8 +109,8 @@ class CP4Conv2d(torch.nn.Module):
         self.stride = stride
 
     def forward(self, x):
-        return cp4_conv2d(x, self.FK, self.FC, self.FH, self.FW, self.pad, self.bias,
-                          self.activation, self.stride, self.padding)
+        return capi._native.layer(x, self.FK, self.FC, self.FH, self.FW, self.pad, self.bias,
+                                  self.activation, self.stride, self.padding)
 
     @staticmethod
     def check_device(stream=None):
