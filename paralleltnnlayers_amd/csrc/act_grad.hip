@@ -43,6 +43,10 @@ struct F16 {
   }
 };
 
+// dy behind a ReLU: the product with the comparison's 0 or 1, so that an infinite or NaN
+// gradient at a clipped output stays visible (NaN) to whoever watches the gradients for it.
+__device__ __forceinline__ float masked(float d, float y) { return d * (y > 0.f ? 1.f : 0.f); }
+
 // V elements at any element-aligned address (planes of an odd number of pixels start
 // anywhere): one 16-byte access, which the memory pipeline takes at such addresses too.
 template <class T, int V>
@@ -102,7 +106,7 @@ __global__ __launch_bounds__(kThreads) void act_grad_kernel(ActGradArgs a) {
 #pragma unroll
         for (int e = 0; e < V; ++e) {
           const float d = In::up(vd[b][e]);
-          const float m = MASK ? (In::up(vy[b][e]) > 0.f ? d : 0.f) : d;
+          const float m = MASK ? masked(d, In::up(vy[b][e])) : d;
           sum += m;
           o[e] = Out::down(m);
         }
@@ -110,7 +114,7 @@ __global__ __launch_bounds__(kThreads) void act_grad_kernel(ActGradArgs a) {
       } else {
         for (unsigned e = 0; e < left[b]; ++e) {       // a plane's last, short piece
           const float d = In::up(dy[at[b] + e]);
-          const float m = MASK ? (In::up(y[at[b] + e]) > 0.f ? d : 0.f) : d;
+          const float m = MASK ? masked(d, In::up(y[at[b] + e])) : d;
           sum += m;
           if (out) out[at[b] + e] = Out::down(m);
         }

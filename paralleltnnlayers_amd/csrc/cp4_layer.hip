@@ -60,17 +60,18 @@ BackwardPlan make_backward_plan(const cp4_shape& s, const cp4_geometry* g, int d
 }
 
 // The plan of a call, remembered: planning asks the backward-filter kernels for theirs,
-// several microseconds of host time that every step of a small layer would wait for.
+// several microseconds of host time that every step of a small layer would wait for.  (It
+// depends on the device by its compute units.)
 BackwardPlan backward_plan(const cp4_shape& s, const cp4_geometry* g, int dtype, int act,
                            int wanted) {
-  using Key = std::array<unsigned, 18>;
+  using Key = std::array<unsigned, 19>;
   static std::mutex mu;
   static std::map<Key, BackwardPlan> plans;
   const cp4_geometry none{0, 0, 0, 0, 0, 0};
   const cp4_geometry& gg = g ? *g : none;
   const Key key{s.N, s.H, s.W, s.pad, s.T, s.C, s.Y, s.X, s.Rank, gg.stride_h, gg.stride_w,
                 gg.pad_top, gg.pad_left, gg.out_h, gg.out_w, (unsigned)dtype, (unsigned)act,
-                (unsigned)wanted};
+                (unsigned)wanted, (unsigned)cp4::num_compute_units()};
   std::lock_guard<std::mutex> lk(mu);
   auto it = plans.find(key);
   if (it != plans.end()) return it->second;

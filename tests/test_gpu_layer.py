@@ -68,3 +68,19 @@ def test_parts_on_their_own(capi):
     assert torch.equal(only_dx[0], dx) and only_dx[2] is None and only_dx[1][0] is None
     assert all(torch.equal(a, b) for a, b in zip(only_f[1], grads)) and only_f[0] is None
     assert torch.equal(only_b[2], db)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16],
+                         ids=["f32", "bf16", "f16"])
+def test_non_finite_gradient_behind_a_clipped_output_is_seen(capi, dtype):
+    """The mask is a product, as dy * (y > 0): an infinite dy at a clipped output gives NaN."""
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, fac = mk(2, 8, 9, 11).to(dtype), [mk(d, 4) for d in (12, 8, 1, 1)]
+    s = capi.shape_for(x.shape, *fac, 0)
+    y = capi.layer_forward(s, None, x, *fac, mk(12), "relu")
+    n, t, h, w = (int(v) for v in (y == 0).nonzero()[0])
+    dy = torch.zeros_like(y)
+    dy[n, t, h, w] = float("inf")
+    dbias = capi.layer_backward(s, None, x, y, dy, *fac, "relu", False, False, True)[2]
+    assert torch.isnan(dbias[t]) and int(torch.isfinite(dbias).sum()) == 11
