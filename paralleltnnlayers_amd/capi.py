@@ -43,15 +43,22 @@ class RcpDims(ctypes.Structure):
     _fields_ = [(k, ctypes.c_uint) for k in ("S0", "S1", "T0", "T1")]
 
 
+class _Missing:
+    """Stands for the binding until it is built: every call of it says so."""
+
+    def __init__(self, why):
+        self._why = why
+
+    def __getattr__(self, name):
+        raise ImportError(f"paralleltnnlayers_amd._binding is missing ({self._why}): build it "
+                          "with `python -c 'import __graft_entry__ as g; g.build()'`")
+
+
 try:
     from . import _binding as _native
     _native.set_error(Cp4Error)
-except ImportError as _e:                    # not built: reported at the first call
-    class _Missing:
-        def __getattr__(self, name, _why=str(_e)):
-            raise ImportError(f"paralleltnnlayers_amd._binding is missing ({_why}): build it with "
-                              "`python -c 'import __graft_entry__ as g; g.build()'`")
-    _native = _Missing()
+except ImportError as _e:
+    _native = _Missing(str(_e))
 
 # status codes of cp4_status
 (OK, ERR_NULL_POINTER, ERR_SHAPE, ERR_HIP, ERR_WORKSPACE, ERR_UNSUPPORTED,

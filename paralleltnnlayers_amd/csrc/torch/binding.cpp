@@ -61,14 +61,23 @@ void check(cp4_status rc) {
   throw e;
 }
 [[noreturn]] void fail(PyObject* type, const char* what) {
+  PyGILState_STATE gil = PyGILState_Ensure();
   PyErr_SetString(type, what);
   python_error e;
   e.persist();
+  PyGILState_Release(gil);
   throw e;
 }
 void require(bool ok, const char* what = "") {
   if (!ok) fail(PyExc_AssertionError, what);
 }
+
+// The interpreter lock is given up around allocations and launches, as a ctypes call does: a
+// launch that waits for room in a full queue must not keep other Python threads from running.
+struct NoGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
 
 // ---- arguments --------------------------------------------------------------------
 
@@ -129,10 +138,15 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Factors f{tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4])};
   const cp4_shape s = shape_for(x, f, integer(a[5]));
   require(x.size(1) == s.C && f.FC.size(1) == s.Rank);
-  const float *px = f32(x), *pK = f32(f.FK), *pC = f32(f.FC), *pH = f32(f.FH), *pW = f32(f.FW);
-  Tensor y = a[6] != Py_None ? tensor(a[6]) : empty({s.N, s.T, s.H, s.W}, at::kFloat, x);
-  check(cp4_conv2d_forward_variant(&s, px, pK, pC, pH, pW, f32(y), (int)integer(a[7]),
-                                   stream_of(a[8])));
+  const int variant = (int)integer(a[7]);
+  void* st = stream_of(a[8]);
+  Tensor y = a[6] != Py_None ? tensor(a[6]) : Tensor();
+  {
+    NoGil unlocked;
+    const float *px = f32(x), *pK = f32(f.FK), *pC = f32(f.FC), *pH = f32(f.FH), *pW = f32(f.FW);
+    if (!y.defined()) y = empty({s.N, s.T, s.H, s.W}, at::kFloat, x);
+    check(cp4_conv2d_forward_variant(&s, px, pK, pC, pH, pW, f32(y), variant, st));
+  }
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
 }
@@ -145,9 +159,14 @@ PyObject* backward_data(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Factors f{tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4])};
   const cp4_shape s = shape_for(dy, f, integer(a[5]));
   require(dy.size(1) == s.T);
-  const float *pdy = f32(dy), *pK = f32(f.FK), *pC = f32(f.FC), *pH = f32(f.FH), *pW = f32(f.FW);
-  Tensor dx = a[6] != Py_None ? tensor(a[6]) : empty({s.N, s.C, s.H, s.W}, at::kFloat, dy);
-  check(cp4_conv2d_backward_data(&s, pdy, pK, pC, pH, pW, f32(dx), stream_of(a[7])));
+  void* st = stream_of(a[7]);
+  Tensor dx = a[6] != Py_None ? tensor(a[6]) : Tensor();
+  {
+    NoGil unlocked;
+    const float *pdy = f32(dy), *pK = f32(f.FK), *pC = f32(f.FC), *pH = f32(f.FH), *pW = f32(f.FW);
+    if (!dx.defined()) dx = empty({s.N, s.C, s.H, s.W}, at::kFloat, dy);
+    check(cp4_conv2d_backward_data(&s, pdy, pK, pC, pH, pW, f32(dx), st));
+  }
   return THPVariable_Wrap(std::move(dx));
   END_HANDLE_TH_ERRORS
 }
@@ -168,22 +187,27 @@ PyObject* backward_filter(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const cp4_shape s = shape_for(x, f, integer(a[6]));
   require(dy.dim() == 4 && dy.size(0) == s.N && dy.size(1) == s.T && dy.size(2) == s.H &&
           dy.size(3) == s.W && x.size(1) == s.C);
-  const float *px = f32(x), *pdy = f32(dy), *pK = f32(f.FK), *pC = f32(f.FC), *pH = f32(f.FH),
-              *pW = f32(f.FW);
+  const int variant = (int)integer(a[9]);
+  void* st = stream_of(a[8]);
+  Tensor ws = a[7] != Py_None ? tensor(a[7]) : Tensor();
   Tensor grads[4];
-  const Tensor* fac[4] = {&f.FK, &f.FC, &f.FH, &f.FW};
-  for (int i = 0; i < 4; ++i) grads[i] = empty(fac[i]->sizes(), at::kFloat, x);
-  Tensor ws;
-  if (a[7] != Py_None) {
-    ws = tensor(a[7]);
-    require(ws.is_cuda() && ws.is_contiguous(), "the workspace must be a contiguous device tensor");
-  } else {
-    const size_t need = cp4_conv2d_backward_filter_workspace_bytes(&s);
-    ws = scratch(need ? need : 4, x);
+  {
+    NoGil unlocked;
+    const float *px = f32(x), *pdy = f32(dy), *pK = f32(f.FK), *pC = f32(f.FC), *pH = f32(f.FH),
+                *pW = f32(f.FW);
+    const Tensor* fac[4] = {&f.FK, &f.FC, &f.FH, &f.FW};
+    for (int i = 0; i < 4; ++i) grads[i] = empty(fac[i]->sizes(), at::kFloat, x);
+    if (ws.defined()) {
+      require(ws.is_cuda() && ws.is_contiguous(), "the workspace must be a contiguous device tensor");
+    } else {
+      const size_t need = cp4_conv2d_backward_filter_workspace_bytes(&s);
+      ws = scratch(need ? need : 4, x);
+    }
+    check(cp4_conv2d_backward_filter_variant(&s, px, pdy, pK, pC, pH, pW, f32(grads[0]),
+                                             f32(grads[1]), f32(grads[2]), f32(grads[3]),
+                                             ws.data_ptr(), (size_t)ws.numel() * ws.element_size(),
+                                             variant, st));
   }
-  check(cp4_conv2d_backward_filter_variant(
-      &s, px, pdy, pK, pC, pH, pW, f32(grads[0]), f32(grads[1]), f32(grads[2]), f32(grads[3]), ws.data_ptr(), (size_t)ws.numel() * ws.element_size(),
-      (int)integer(a[9]), stream_of(a[8])));
   return wrap_four(grads);
   END_HANDLE_TH_ERRORS
 }
@@ -248,12 +272,15 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
     for (int i = 0; i < 4; ++i) want_factors |= want_factor[i] = ctx->needs_input_grad(1 + i);
     const Tensor* fac[4] = {&FK, &FC, &FH, &FW};
     Tensor dx, grads[4], dbias;
+    // create_graph: the bias gradient is linear in dy and stays differentiable (the other
+    // gradients are the library's and are not)
+    const bool bias_graph = want_bias && at::GradMode::is_enabled() && grad[0].requires_grad();
     if (want_dx) dx = empty(x.sizes(), x.scalar_type(), x);
     if (want_factors)
       for (int i = 0; i < 4; ++i) grads[i] = empty(fac[i]->sizes(), at::kFloat, x);
-    if (want_bias) dbias = empty({(int64_t)l.shape.T}, at::kFloat, x);
+    if (want_bias && !bias_graph) dbias = empty({(int64_t)l.shape.T}, at::kFloat, x);
     const int wanted = (want_dx ? CP4_WANT_DX : 0) | (want_factors ? CP4_WANT_FACTORS : 0) |
-                       (want_bias ? CP4_WANT_BIAS : 0);
+                       (dbias.defined() ? CP4_WANT_BIAS : 0);
     const size_t need =
         cp4_layer_backward_workspace_bytes(&l.shape, l.g(), l.dtype, l.activation, wanted);
     const Tensor ws = scratch(need, x);
@@ -264,6 +291,10 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
                              static_cast<float*>(ptr(grads[2])), static_cast<float*>(ptr(grads[3])),
                              static_cast<float*>(ptr(dbias)), ptr(ws), need, st));
     if (g_check_backward.load(std::memory_order_relaxed)) check(cp4_device_status(st, nullptr));
+    if (bias_graph) {
+      const Tensor d = saved[5].defined() ? grad[0] * (saved[5] > 0) : grad[0];
+      dbias = d.to(at::kFloat).sum(at::IntArrayRef{0, 2, 3});
+    }
     out[0] = dx;
     for (int i = 0; i < 4; ++i)
       if (want_factor[i]) out[1 + i] = grads[i];
@@ -347,12 +378,23 @@ PyObject* layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     l.has_bias = true;
   }
   const c10::DeviceGuard guard(x.device());
-  const bool track = at::GradMode::is_enabled() &&
-                     (x.requires_grad() || f.FK.requires_grad() || f.FC.requires_grad() ||
-                      f.FH.requires_grad() || f.FW.requires_grad() || (bias && bias->requires_grad()));
-  if (track) return THPVariable_Wrap(LayerFunction::apply(x, f.FK, f.FC, f.FH, f.FW, bias, l));
-  const Tensor FK = as_f32(f.FK), FC = as_f32(f.FC), FH = as_f32(f.FH), FW = as_f32(f.FW);
-  return THPVariable_Wrap(layer_forward(l, x, Factors{FK, FC, FH, FW}, bias ? as_f32(*bias) : Tensor()));
+  // What carries a forward-mode tangent goes through the autograd function too, which refuses it.
+  auto tracked = [](const Tensor& t) {
+    return (at::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(0).defined();
+  };
+  const bool track = tracked(x) || tracked(f.FK) || tracked(f.FC) || tracked(f.FH) ||
+                     tracked(f.FW) || (bias && tracked(*bias));
+  Tensor y;
+  {
+    NoGil unlocked;
+    if (track) {
+      y = LayerFunction::apply(x, f.FK, f.FC, f.FH, f.FW, bias, l);
+    } else {
+      const Tensor FK = as_f32(f.FK), FC = as_f32(f.FC), FH = as_f32(f.FH), FW = as_f32(f.FW);
+      y = layer_forward(l, x, Factors{FK, FC, FH, FW}, bias ? as_f32(*bias) : Tensor());
+    }
+  }
+  return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
 }
 

@@ -33,7 +33,8 @@ def set_device_checks(on):
     """Check the device's fault record at the end of every backward pass (synchronises)."""
     global _check_every_backward
     _check_every_backward = bool(on)
-    capi._native.set_check_backward(_check_every_backward)
+    if not isinstance(capi._native, capi._Missing):
+        capi._native.set_check_backward(_check_every_backward)
 
 
 set_device_checks(os.environ.get("CP4_CHECK_DEVICE", "0") not in ("", "0"))
@@ -51,9 +52,11 @@ def _after_backward():
         capi.device_status()
 
 
-class CP4Conv2dFunction:
-    """y = act(cp4conv2d(x, FK, FC, FH, FW, pad) + bias), differentiable; the autograd
-    function itself is native (csrc/torch/binding.cpp).
+class CP4Conv2dFunction(torch.autograd.Function):
+    """y = act(cp4conv2d(x, FK, FC, FH, FW, pad) + bias) as a Python autograd function, forward
+    and backward each one call of the library's layer entry points.  ``cp4_conv2d`` runs the
+    native one (csrc/torch/binding.cpp); this one stands for it where a call has to be seen
+    as an operator: in a trace.
 
     A bfloat16 or float16 ``x`` selects the library's 16-bit activations (y and the input
     gradient are of x's type then; factors, bias and their gradients stay float32); shapes
@@ -61,11 +64,70 @@ class CP4Conv2dFunction:
     """
 
     @staticmethod
-    def apply(x, FK, FC, FH, FW, pad, bias=None, activation=None):
+    def forward(ctx, x, FK, FC, FH, FW, pad, bias=None, activation=None):
         if 2 * pad + 1 != FH.shape[0] or 2 * pad + 1 != FW.shape[0]:
             raise ValueError("autograd binding needs 2*pad = Y-1 = X-1 (the reference's "
                              "backward-data pass is the adjoint only then)")
-        return capi._native.layer(x, FK, FC, FH, FW, pad, bias, activation, 1, None)
+        x = x.contiguous()
+        if x.dtype not in (torch.bfloat16, torch.float16):
+            x = x.float()
+        return _layer_forward(ctx, x, FK, FC, FH, FW, pad, None, bias, activation)
+
+    @staticmethod
+    def backward(ctx, dy):
+        return _layer_backward(ctx, dy)
+
+
+class CP4Conv2dGeometryFunction(torch.autograd.Function):
+    """The same for a layer with a stride, explicit padding or an output plane of its own
+    (``geom``: a ``capi.Geometry``; float32)."""
+
+    @staticmethod
+    def forward(ctx, x, FK, FC, FH, FW, geom, bias=None, activation=None):
+        return _layer_forward(ctx, x.contiguous().float(), FK, FC, FH, FW, 0, geom, bias,
+                              activation)
+
+    @staticmethod
+    def backward(ctx, dy):
+        return _layer_backward(ctx, dy)
+
+
+def _layer_forward(ctx, x, FK, FC, FH, FW, pad, geom, bias, activation):
+    FK, FC, FH, FW = (t.contiguous().float() for t in (FK, FC, FH, FW))
+    if bias is not None:
+        bias = bias.contiguous().float()
+    s = capi.shape_for(x.shape, FK, FC, FH, FW, pad)
+    y = capi.layer_forward(s, geom, x, FK, FC, FH, FW, bias, activation)
+    ctx.shape, ctx.geom, ctx.activation = s, geom, activation
+    ctx.save_for_backward(x, FK, FC, FH, FW, y if capi.ACTIVATIONS[activation] == 1 else None)
+    return y
+
+
+def _layer_backward(ctx, dy):
+    x, FK, FC, FH, FW, y = ctx.saved_tensors
+    need = ctx.needs_input_grad
+    # create_graph: the bias gradient is linear in dy and stays differentiable
+    bias_graph = need[6] and torch.is_grad_enabled() and dy.requires_grad
+    dx, grads, dbias = capi.layer_backward(
+        ctx.shape, ctx.geom, x, y, dy.contiguous().to(x.dtype), FK, FC, FH, FW, ctx.activation,
+        want_dx=need[0], want_factors=any(need[1:5]), want_bias=need[6] and not bias_graph)
+    if bias_graph:
+        dbias = (dy if y is None else dy * (y > 0)).float().sum(dim=(0, 2, 3))
+    grads = tuple(g if n else None for g, n in zip(grads, need[1:5]))
+    _after_backward()
+    return (dx,) + grads + (None, dbias, None)
+
+
+def _traced_layer(x, FK, FC, FH, FW, pad, bias, activation, stride, padding):
+    if padding is None:
+        padding = pad
+    y_taps, x_taps = FH.shape[0], FW.shape[0]
+    if stride == 1 and (
+            (isinstance(padding, int) and 2 * padding + 1 == y_taps == x_taps) or
+            (padding == "same" and y_taps == x_taps and y_taps % 2 == 1)):
+        return CP4Conv2dFunction.apply(x, FK, FC, FH, FW, y_taps // 2, bias, activation)
+    geom = capi.geometry(capi.shape_for(x.shape, FK, FC, FH, FW, 0), stride, padding)
+    return CP4Conv2dGeometryFunction.apply(x, FK, FC, FH, FW, geom, bias, activation)
 
 
 def cp4_conv2d(x, FK, FC, FH, FW, pad, bias=None, activation=None, stride=1, padding=None):
@@ -79,7 +141,9 @@ def cp4_conv2d(x, FK, FC, FH, FW, pad, bias=None, activation=None, stride=1, pad
     after the image than before it), "valid", an int or an (h, w) pair run the
     strided kernels: only the kept outputs are computed.
     """
-    return capi._native.layer(x, FK, FC, FH, FW, pad, bias, activation, stride, padding)
+    # torch.jit.trace records operators: the native call would leave a constant in the graph
+    run = capi._native.layer if torch._C._get_tracing_state() is None else _traced_layer
+    return run(x, FK, FC, FH, FW, pad, bias, activation, stride, padding)
 
 
 class CP4Conv2d(torch.nn.Module):
@@ -109,8 +173,8 @@ class CP4Conv2d(torch.nn.Module):
         self.stride = stride
 
     def forward(self, x):
-        return capi._native.layer(x, self.FK, self.FC, self.FH, self.FW, self.pad, self.bias,
-                                  self.activation, self.stride, self.padding)
+        return cp4_conv2d(x, self.FK, self.FC, self.FH, self.FW, self.pad, self.bias,
+                          self.activation, self.stride, self.padding)
 
     @staticmethod
     def check_device(stream=None):

@@ -140,3 +140,57 @@ def test_bfloat16_activations_through_autograd(ops):
     assert (x.grad.double() - xd.grad).abs().max() <= 2.0 ** -7 * xd.grad.abs().max()
     for name, a, b in zip(("dFK", "dFC", "dFH", "dFW"), [f.grad for f in fac], [f.grad for f in fd]):
         assert (a.double() - b).abs().max() <= 1e-3 * b.abs().max(), name
+
+
+def _small_layer(ops, **kw):
+    layer = ops.CP4Conv2d(8, 12, 3, 4, bias=True, activation="relu", **kw)
+    torch.manual_seed(5)
+    with torch.no_grad():
+        layer.bias.normal_()
+    return layer, torch.randn(2, 8, 9, 10, device="cuda")
+
+
+@pytest.mark.parametrize("kw", [{}, {"stride": 2, "padding": "same"}], ids=["plain", "stride"])
+def test_traced_layer_computes_from_its_inputs(ops, kw):
+    """A trace holds the layer as an operator: run on another input it gives that input's result."""
+    layer, x = _small_layer(ops, **kw)
+    traced = torch.jit.trace(layer, x, check_trace=False)
+    other = torch.randn_like(x)
+    assert torch.equal(traced(other), layer(other))
+
+
+@pytest.mark.parametrize("kw", [{}, {"stride": 2, "padding": "same"}], ids=["plain", "stride"])
+def test_python_autograd_function_matches_the_native_one(ops, kw):
+    layer, x = _small_layer(ops, **kw)
+    dy = torch.randn_like(layer(x))
+
+    def grads(run):
+        xi = x.clone().requires_grad_()
+        layer.zero_grad(set_to_none=True)
+        y = run(xi)
+        y.backward(dy)
+        return [y.detach(), xi.grad] + [p.grad for p in layer.parameters()]
+
+    args = lambda xi: (xi, layer.FK, layer.FC, layer.FH, layer.FW, layer.pad, layer.bias,
+                       layer.activation, layer.stride, layer.padding)
+    for a, b in zip(grads(lambda xi: ops._traced_layer(*args(xi))), grads(layer)):
+        assert torch.equal(a, b)
+
+
+def test_forward_mode_tangents_are_refused(ops):
+    import torch.autograd.forward_ad as fwd
+    layer, x = _small_layer(ops)
+    with torch.no_grad(), fwd.dual_level():
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            layer(fwd.make_dual(x, torch.ones_like(x)))
+
+
+def test_bias_gradient_under_create_graph(ops):
+    """The bias gradient is linear in dy: its own gradient with respect to dy is the mask."""
+    layer, x = _small_layer(ops)
+    y = layer(x)
+    dy = torch.randn_like(y).requires_grad_()
+    (db,) = torch.autograd.grad(y, layer.bias, dy, create_graph=True)
+    assert torch.allclose(db, (dy * (y > 0)).sum(dim=(0, 2, 3)), rtol=1e-4, atol=1e-4)
+    (gg,) = torch.autograd.grad(db.sum(), dy)
+    assert torch.equal(gg, (y > 0).float())
