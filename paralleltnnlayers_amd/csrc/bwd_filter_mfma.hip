@@ -1481,6 +1481,19 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs& a, hipStream_t st) {
   }
 #endif
 
+  // (after the GEMMs, whose operands its stores would push out of the cache)
+  if (a.dx) {
+#ifdef CP4_BWF_HALF
+    constexpr int kDtype = CP4_DTYPE_F16;
+#elif defined(CP4_BWF_IO16)
+    constexpr int kDtype = CP4_DTYPE_BF16;
+#else
+    constexpr int kDtype = CP4_DTYPE_F32;
+#endif
+    e = rank_expand_launch(a.FC, G1, a.dx, kDtype, N, a.C, HW, R, st);
+    if (e != hipSuccess) return e;
+  }
+
   ReduceArgs r{};
   const float* parts[4] = {pK, pC, pH, pW};
   float* outs[4] = {a.dFK, a.dFC, a.taps2d ? a.dtaps2d : a.dFH, a.dFW};
@@ -1898,6 +1911,10 @@ hipError_t bwd_filter_mfma_strided_launch(const BwdFilterArgs& a, const Geometry
   if (e != hipSuccess) return e;
   e = grad_one(a.x, G1, pC, a.C, N, R, l.pf, HW, ws, st);
   if (e != hipSuccess) return e;
+  if (a.dx) {
+    e = rank_expand_launch(a.FC, G1, a.dx, CP4_DTYPE_F32, N, a.C, HW, R, st);
+    if (e != hipSuccess) return e;
+  }
   ReduceArgs r{};
   const float* parts[4] = {pK, pC, pH, pW};
   float* outs[4] = {a.dFK, a.dFC, a.dFH, a.dFW};

@@ -1101,13 +1101,15 @@ cp4_status cp4_conv2d_backward_filter(const cp4_shape* shape, const float* x,
                                             workspace, workspace_bytes, -1, stream);
 }
 
-cp4_status cp4_conv2d_backward_filter_variant(const cp4_shape* shape, const float* x,
-                                              const float* dy, const float* FK,
-                                              const float* FC, const float* FH,
-                                              const float* FW, float* dFK, float* dFC,
-                                              float* dFH, float* dFW, void* workspace,
-                                              size_t workspace_bytes, int variant,
-                                              cp4_stream stream) {
+}  // extern "C"
+namespace {
+// (dx not null: the input gradient as well where the matrix-core variant runs on the layer as
+// it is, *dx_done)
+cp4_status backward_filter_f32(const cp4_shape* shape, const float* x, const float* dy,
+                               const float* FK, const float* FC, const float* FH, const float* FW,
+                               float* dFK, float* dFC, float* dFH, float* dFW, void* workspace,
+                               size_t workspace_bytes, int variant, void* dx, bool* dx_done,
+                               cp4_stream stream) {
   cp4_status rc = check_shape(shape);
   if (rc != CP4_OK) return rc;
   if (!FK || !FC || !FH || !FW || !dFK || !dFC || !dFH || !dFW)
@@ -1169,9 +1171,9 @@ cp4_status cp4_conv2d_backward_filter_variant(const cp4_shape* shape, const floa
       }
       CP4_HIP(cp4::pad_rows_launch(FC, w + l.fc, 1, s.C, t.C, s.Rank, st));
       CP4_HIP(cp4::pad_rows_launch(FK, w + l.fk, 1, s.T, t.T, s.Rank, st));
-      rc = cp4_conv2d_backward_filter_variant(&t, xp, dyp, w + l.fk, w + l.fc, FH, FW, w + l.gfk,
-                                              w + l.gfc, dFH, dFW, w + l.head,
-                                              workspace_bytes - l.head * sizeof(float), -1, stream);
+      rc = backward_filter_f32(&t, xp, dyp, w + l.fk, w + l.fc, FH, FW, w + l.gfk, w + l.gfc, dFH,
+                               dFW, w + l.head, workspace_bytes - l.head * sizeof(float), -1,
+                               t.C == s.C ? dx : nullptr, dx_done, stream);
       if (rc != CP4_OK) return rc;
       CP4_HIP(cp4::copy_f32_launch(dFC, w + l.gfc, (size_t)s.C * s.Rank, st));
       CP4_HIP(cp4::copy_f32_launch(dFK, w + l.gfk, (size_t)s.T * s.Rank, st));
@@ -1210,10 +1212,27 @@ cp4_status cp4_conv2d_backward_filter_variant(const cp4_shape* shape, const floa
     }
     return CP4_OK;
   }
+  if (variant == 1 && dx && s.Y == s.X && 2 * s.pad + 1 == s.Y) {
+    a.dx = dx;
+    *dx_done = true;
+  }
   if (variant == 2) CP4_HIP(cp4::bwd_filter_fused_launch(a, st));
   else if (variant == 1) CP4_HIP(cp4::bwd_filter_mfma_launch(a, st));
   else CP4_HIP(cp4::bwd_filter_launch(a, st));
   return CP4_OK;
+}
+}  // namespace
+extern "C" {
+
+cp4_status cp4_conv2d_backward_filter_variant(const cp4_shape* shape, const float* x,
+                                              const float* dy, const float* FK,
+                                              const float* FC, const float* FH,
+                                              const float* FW, float* dFK, float* dFC,
+                                              float* dFH, float* dFW, void* workspace,
+                                              size_t workspace_bytes, int variant,
+                                              cp4_stream stream) {
+  return backward_filter_f32(shape, x, dy, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
+                             workspace_bytes, variant, nullptr, nullptr, stream);
 }
 
 size_t cp4_noalloc_scratch_bytes(void) { return kScratchBytes; }
@@ -1252,7 +1271,7 @@ namespace {
 cp4_status backward_filter_16(const cp4_shape* shape, const void* x16, const void* dy16,
                               const float* FK, const float* FC, const float* FH, const float* FW,
                               float* dFK, float* dFC, float* dFH, float* dFW, void* workspace,
-                              size_t workspace_bytes, bool half, cp4_stream stream) {
+                              size_t workspace_bytes, bool half, void* dx, cp4_stream stream) {
   cp4_status rc = check_shape(shape);
   if (rc != CP4_OK) return rc;
   if (!FK || !FC || !FH || !FW || !dFK || !dFC || !dFH || !dFW)
@@ -1283,6 +1302,7 @@ cp4_status backward_filter_16(const cp4_shape* shape, const void* x16, const voi
   a.dFK = dFK; a.dFC = dFC; a.dFH = dFH; a.dFW = dFW; a.workspace = workspace;
   a.N = s.N; a.C = s.C; a.T = s.T; a.H = s.H; a.W = s.W; a.pad = s.pad;
   a.Y = s.Y; a.X = s.X; a.R = s.Rank;
+  a.dx = dx;
   if (half) CP4_HIP(cp4::bwd_filter_mfma_iof16_launch(a, st));
   else CP4_HIP(cp4::bwd_filter_mfma_io16_launch(a, st));
   return CP4_OK;
@@ -1296,7 +1316,7 @@ cp4_status cp4_conv2d_backward_filter_bf16(const cp4_shape* shape, const void* x
                                            float* dFH, float* dFW, void* workspace,
                                            size_t workspace_bytes, cp4_stream stream) {
   return backward_filter_16(shape, x_bf16, dy_bf16, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
-                            workspace_bytes, false, stream);
+                            workspace_bytes, false, nullptr, stream);
 }
 
 cp4_status cp4_conv2d_backward_filter_f16(const cp4_shape* shape, const void* x_f16,
@@ -1306,7 +1326,7 @@ cp4_status cp4_conv2d_backward_filter_f16(const cp4_shape* shape, const void* x_
                                           float* dFH, float* dFW, void* workspace,
                                           size_t workspace_bytes, cp4_stream stream) {
   return backward_filter_16(shape, x_f16, dy_f16, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
-                            workspace_bytes, true, stream);
+                            workspace_bytes, true, nullptr, stream);
 }
 
 cp4_status cp4_conv2d_backward_filter_full(const cp4_shape* shape,
@@ -1579,12 +1599,13 @@ cp4_status cp4_conv2d_backward_data_ex(const cp4_shape* shape, const cp4_geometr
   return run_geometry(a, st);
 }
 
-cp4_status cp4_conv2d_backward_filter_ex(const cp4_shape* shape, const cp4_geometry* g,
-                                         const float* x, const float* dy, const float* FK,
-                                         const float* FC, const float* FH, const float* FW,
-                                         float* dFK, float* dFC, float* dFH, float* dFW,
-                                         void* workspace, size_t workspace_bytes,
-                                         cp4_stream stream) {
+}  // extern "C"
+namespace {
+cp4_status backward_filter_geometry(const cp4_shape* shape, const cp4_geometry* g, const float* x,
+                                    const float* dy, const float* FK, const float* FC,
+                                    const float* FH, const float* FW, float* dFK, float* dFC,
+                                    float* dFH, float* dFW, void* workspace, size_t workspace_bytes,
+                                    void* dx, bool* dx_done, cp4_stream stream) {
   cp4_status rc = check_geometry(shape, g);
   if (rc != CP4_OK) return rc;
   const cp4_shape& s = *shape;
@@ -1614,6 +1635,8 @@ cp4_status cp4_conv2d_backward_filter_ex(const cp4_shape* shape, const cp4_geome
       b.workspace = workspace;
       b.N = (int)s.N; b.C = (int)s.C; b.T = (int)s.T; b.H = (int)s.H; b.W = (int)s.W; b.pad = 0;
       b.Y = (int)s.Y; b.X = (int)s.X; b.R = (int)s.Rank;
+      b.dx = dx;
+      if (dx) *dx_done = true;
       CP4_HIP(cp4::bwd_filter_mfma_strided_launch(b, gg, st));
       return CP4_OK;
     }
@@ -1636,6 +1659,39 @@ cp4_status cp4_conv2d_backward_filter_ex(const cp4_shape* shape, const cp4_geome
   const size_t used = (size_t)(w - static_cast<unsigned char*>(workspace));
   return cp4_conv2d_backward_filter(&sc, xc, dyc, FK, FC, FH, FW, dFK, dFC, dFH, dFW, w,
                                     workspace_bytes - used, stream);
+}
+}  // namespace
+
+namespace cp4 {
+cp4_status layer_backward_filter(const cp4_shape* s, const cp4_geometry* g, int dtype, const void* x,
+                                 const void* dy, const float* FK, const float* FC, const float* FH,
+                                 const float* FW, float* dFK, float* dFC, float* dFH, float* dFW,
+                                 void* workspace, size_t workspace_bytes, void* dx, bool* dx_done,
+                                 cp4_stream stream) {
+  *dx_done = false;
+  const float *xf = static_cast<const float*>(x), *dyf = static_cast<const float*>(dy);
+  if (g)
+    return backward_filter_geometry(s, g, xf, dyf, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
+                                    workspace_bytes, dx, dx_done, stream);
+  if (dtype == CP4_DTYPE_F32)
+    return backward_filter_f32(s, xf, dyf, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
+                               workspace_bytes, -1, dx, dx_done, stream);
+  if (s->Y != s->X || 2 * s->pad + 1 != s->Y) dx = nullptr;
+  *dx_done = dx != nullptr;
+  return backward_filter_16(s, x, dy, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
+                            workspace_bytes, dtype == CP4_DTYPE_F16, dx, stream);
+}
+}  // namespace cp4
+extern "C" {
+
+cp4_status cp4_conv2d_backward_filter_ex(const cp4_shape* shape, const cp4_geometry* g,
+                                         const float* x, const float* dy, const float* FK,
+                                         const float* FC, const float* FH, const float* FW,
+                                         float* dFK, float* dFC, float* dFH, float* dFW,
+                                         void* workspace, size_t workspace_bytes,
+                                         cp4_stream stream) {
+  return backward_filter_geometry(shape, g, x, dy, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
+                                  workspace_bytes, nullptr, nullptr, stream);
 }
 
 cp4_status cp4_time_forward(const cp4_shape* shape, const float* x,

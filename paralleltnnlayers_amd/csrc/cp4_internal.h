@@ -82,6 +82,15 @@ cp4_status check_layer_geometry(const cp4_shape*, const cp4_geometry*);
 cp4_status fail_with(cp4_status, const char* what);
 cp4_status fail_hip(hipError_t, const char* where);
 
+// The backward-filter entry points with the input gradient beside the factors' where the
+// variant that runs has it at hand (`dx` may be null; *dx_done says whether it was written).
+// dtype: a cp4_dtype, the type of x, dy and dx; `geometry` as in the _ex entry points.
+cp4_status layer_backward_filter(const cp4_shape*, const cp4_geometry*, int dtype, const void* x,
+                                 const void* dy, const float* FK, const float* FC, const float* FH,
+                                 const float* FW, float* dFK, float* dFC, float* dFH, float* dFW,
+                                 void* workspace, size_t workspace_bytes, void* dx, bool* dx_done,
+                                 cp4_stream);
+
 // Compute units of the current device (256 when no device can be asked).
 int num_compute_units();
 
@@ -162,6 +171,11 @@ hipError_t act_grad_launch(const void* y, const void* dy, void* out, int dtype, 
 hipError_t convert_launch(const void* src, int src_dtype, void* dst, int dst_dtype, size_t n,
                           hipStream_t);
 
+// dst[n,c,p] = sum_r F[c,r] Z[n,r,p] (ranks up to 64), dst of a cp4_dtype.
+bool rank_expand_supported(int N, int C, int HW, int R);
+hipError_t rank_expand_launch(const float* F, const float* Z, void* dst, int dtype, int N, int C,
+                              int HW, int R, hipStream_t);
+
 // Backward-filter (factor gradients).
 struct BwdFilterArgs {
   const float *x, *dy, *FK, *FC, *FH, *FW;
@@ -172,6 +186,9 @@ struct BwdFilterArgs {
   // of FH x FW and its gradient (FH, FW, dFH, dFW unused then).
   const float* taps2d;
   float* dtaps2d;
+  // Matrix-core variant only: not null, the input gradient too, dx = FC G1 (in the type of
+  // x; the forward's adjoint only where 2 * pad = Y - 1 = X - 1 or with a geometry).
+  void* dx;
 };
 // general (VALU, any shape) and matrix-core variants
 size_t bwd_filter_workspace_bytes(const cp4_shape&);

@@ -1,0 +1,228 @@
+// Rank -> channel expansion of planes in memory, dst[n,c,p] = sum_r F[c,r] Z[n,r,p]: the input
+// gradient of a layer whose backward pass has G1 (the adjoint taps of FK^T dy) at hand, as the
+// factor gradients do.  dx = FC G1 then reads R planes an image instead of contracting T
+// channels of dy again.
+//
+// Bound by the stores of dst: C channels out against R ranks in.  A wave takes 32 * PX
+// consecutive pixels (across images) and a slice of the channels; the lane that is column l of a
+// matrix block holds PX neighbouring pixels, one in each of PX blocks, so that every store
+// of a channel row is 16 bytes a lane, 512 contiguous bytes (PX = 4).  Z's pieces are loaded and
+// split once per wave (exact products from three bf16 parts, like every contraction here), F's
+// come from the cache and are split per block of 32 channels: no LDS, no barrier.  Waves of a
+// workgroup share the pixels and differ in the channel slice where there are slices, and
+// workgroups of one die (blockIdx & 7) take a contiguous range of the pixels, so that cache
+// lines that two blocks share meet in one L2.
+// N32 C256 56x56 R32 fp32 (103 MB written, 13 MB read): 24 us with streaming stores, 29 without; the backward-data pass from
+// dy takes 56.
+#include <cstdint>
+
+#include "cp4_internal.h"
+#include "split_bf16.h"
+
+namespace cp4 {
+namespace {
+
+using split::f32x16;
+using split::u32x4;
+
+constexpr int kThreads = 256;
+
+struct ExpandArgs {
+  const float *F, *Z;          // [C][R], [N][R][HW]
+  void* dst;                   // [N][C][HW]
+  int C, R, HW;
+  int cblocks;                 // blocks of 32 channels a wave takes
+  int slices;                  // waves a block of pixels is shared by
+  bool stream;                 // stores that leave the caches alone
+  long pixels, blocks, items;  // N * HW; blocks of pixels; blocks * slices
+};
+
+struct ToF32 {
+  using raw = float;
+  static __device__ __forceinline__ raw down(float v) { return v; }
+};
+struct ToBF16 {
+  using raw = unsigned short;
+  static __device__ __forceinline__ raw down(float v) {
+    return __builtin_bit_cast(raw, static_cast<__bf16>(v));
+  }
+};
+struct ToF16 {
+  using raw = unsigned short;
+  static __device__ __forceinline__ raw down(float v) {
+    return __builtin_bit_cast(raw, static_cast<_Float16>(v));
+  }
+};
+
+// KC chunks of 16 ranks.  VEC: HW a multiple of PX and dst on a PX-element boundary, a lane's PX
+// pixels are neighbours and move in one access; else they are 32 apart and move one by one
+// (planes start at any address then, and a wider access off its own boundary is the slower:
+// N16 C128 55x55 R32 28 us against 10.7).
+template <class Out, int KC, int PX, bool VEC>
+__global__ __launch_bounds__(kThreads, 2) void rank_expand_kernel(ExpandArgs a) {
+  using raw = typename Out::raw;
+  typedef float ZV __attribute__((ext_vector_type(PX)));
+  typedef raw OV __attribute__((ext_vector_type(PX)));
+  typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+  constexpr int NP = VEC ? 1 : PX;                           // accesses a row takes
+  const int lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5;
+  // workgroups of a die: consecutive ones
+  const unsigned die = blockIdx.x & 7, per = gridDim.x >> 3, rest = gridDim.x & 7;
+  const unsigned wg = die * per + (die < rest ? die : rest) + (blockIdx.x >> 3);
+  const long item = (long)wg * (kThreads / 64) + (threadIdx.x >> 6);
+  if (item >= a.items) return;
+  const int slice = (int)(item % a.slices);
+  const long g = item / a.slices * (32 * PX) + (VEC ? PX : 1) * l32;   // this lane's first pixel
+  const int HW = a.HW, R = a.R, C = a.C;
+  // (lanes past the last pixel keep a valid one for their loads and store nothing)
+  bool live[NP];
+  size_t zat[NP], oat[NP];
+  {
+    long n = (g < a.pixels ? g : a.pixels - 1) / HW;
+    long p = (g < a.pixels ? g : a.pixels - 1) - n * HW;
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+      live[q] = g + 32 * q < a.pixels;
+      if (live[q])
+        while (p >= HW) {
+          p -= HW;
+          ++n;
+        }
+      else {
+        n = (a.pixels - 1) / HW;
+        p = HW - (VEC ? PX : 1);
+      }
+      zat[q] = (size_t)n * R * HW + p;
+      oat[q] = (size_t)n * C * HW + p;
+      p += 32;
+    }
+  }
+  // ---- this lane's pixels, split: B operands [chunk][pixel][part] ----
+  u32x4 bh[KC][PX], bm[KC][PX], bl[KC][PX];
+#pragma unroll
+  for (int ch = 0; ch < KC; ++ch) {
+    float v[PX][8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int r = 16 * ch + 8 * hi + e;
+      const float* z = a.Z + (size_t)(r < R ? r : R - 1) * HW;
+      if constexpr (VEC) {
+        const ZV t = *reinterpret_cast<const ZV*>(z + zat[0]);
+#pragma unroll
+        for (int q = 0; q < PX; ++q) v[q][e] = t[q];
+      } else {
+#pragma unroll
+        for (int q = 0; q < PX; ++q) v[q][e] = z[zat[q]];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < PX; ++q) split::split8(v[q], bh[ch][q], bm[ch][q], bl[ch][q]);
+  }
+  // ---- channel blocks: F's rows are the A operand (zero past the last rank) ----
+  auto load_f = [&](float (&f)[KC][8], int c0) {
+    const int c = c0 + l32 < C ? c0 + l32 : C - 1;
+    const float* fp = a.F + (size_t)c * R;
+#pragma unroll
+    for (int ch = 0; ch < KC; ++ch) {
+      const int r0 = 16 * ch + 8 * hi;
+      if (r0 + 8 <= R) {
+        const f32x4u t0 = *reinterpret_cast<const f32x4u*>(fp + r0);
+        const f32x4u t1 = *reinterpret_cast<const f32x4u*>(fp + r0 + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { f[ch][e] = t0[e]; f[ch][4 + e] = t1[e]; }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[ch][e] = r0 + e < R ? fp[r0 + e] : 0.f;
+      }
+    }
+  };
+  const int first = slice * a.cblocks * 32;
+  const int last = first + a.cblocks * 32 < C ? first + a.cblocks * 32 : C;
+  if (first >= last) return;
+  raw* dst = static_cast<raw*>(a.dst);
+  float f[KC][8];
+  load_f(f, first);
+  for (int c0 = first; c0 < last; c0 += 32) {
+    f32x16 acc[PX];
+#pragma unroll
+    for (int q = 0; q < PX; ++q) acc[q] = (f32x16)(0.f);
+    u32x4 ah[KC], am[KC], al[KC];
+#pragma unroll
+    for (int ch = 0; ch < KC; ++ch) split::split8(f[ch], ah[ch], am[ch], al[ch]);
+    load_f(f, c0 + 32 < last ? c0 + 32 : c0);
+#pragma unroll
+    for (int ch = 0; ch < KC; ++ch)
+#pragma unroll
+      for (int q = 0; q < PX; ++q)
+        acc[q] = split::mfma_split(ah[ch], am[ch], al[ch], bh[ch][q], bm[ch][q], bl[ch][q], acc[q]);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int c = c0 + 8 * (v >> 2) + 4 * hi + (v & 3);
+      if (c >= C) continue;
+      if constexpr (VEC) {
+        OV o;
+#pragma unroll
+        for (int q = 0; q < PX; ++q) o[q] = Out::down(acc[q][v]);
+        OV* to = reinterpret_cast<OV*>(dst + oat[0] + (size_t)c * HW);
+        if (live[0] && a.stream) __builtin_nontemporal_store(o, to);
+        else if (live[0]) *to = o;
+      } else {
+#pragma unroll
+        for (int q = 0; q < PX; ++q)
+          if (live[q]) dst[oat[q] + (size_t)c * HW] = Out::down(acc[q][v]);
+      }
+    }
+  }
+}
+
+template <class Out>
+hipError_t launch(ExpandArgs a, hipStream_t st) {
+  // four pixels a lane while the parts of its ranks leave room for four accumulators
+  const int px = a.R <= 32 ? 4 : 2;
+  const long blocks = (a.pixels + 32 * px - 1) / (32 * px);
+  const int all = (a.C + 31) / 32;
+  // channel slices until there are about eight waves per compute unit
+  a.cblocks = all;
+  while (a.cblocks > 1 && blocks * ((all + a.cblocks - 1) / a.cblocks) < 8l * num_compute_units())
+    a.cblocks = (a.cblocks + 1) / 2;
+  a.slices = (all + a.cblocks - 1) / a.cblocks;
+  a.blocks = blocks;
+  a.items = blocks * a.slices;
+  const unsigned grid = (unsigned)((a.items + kThreads / 64 - 1) / (kThreads / 64));
+  // A result that fills a good part of the 256 MB memory-side cache is streamed past it: it would
+  // only push out x and dy, which the gradient GEMMs read again (N32 C256 56x56 R32: 29 -> 24
+  // us for this kernel).
+  a.stream = (size_t)a.pixels * a.C * sizeof(typename Out::raw) > ((size_t)48 << 20);
+  const bool vec = a.HW % px == 0 && reinterpret_cast<uintptr_t>(a.Z) % (4 * px) == 0 &&
+                   reinterpret_cast<uintptr_t>(a.dst) % (sizeof(typename Out::raw) * px) == 0;
+#define CP4_EXPAND(KC_, PX_)                                                             \
+  {                                                                                      \
+    if (vec) rank_expand_kernel<Out, KC_, PX_, true><<<grid, kThreads, 0, st>>>(a);      \
+    else rank_expand_kernel<Out, KC_, PX_, false><<<grid, kThreads, 0, st>>>(a);         \
+  }
+  if (a.R <= 16) CP4_EXPAND(1, 4)
+  else if (a.R <= 32) CP4_EXPAND(2, 4)
+  else if (a.R <= 48) CP4_EXPAND(3, 2)
+  else CP4_EXPAND(4, 2)
+#undef CP4_EXPAND
+  return hipGetLastError();
+}
+
+}  // namespace
+
+bool rank_expand_supported(int N, int C, int HW, int R) {
+  return R >= 1 && R <= 64 && C >= 1 && N >= 1 && HW >= 1;
+}
+
+hipError_t rank_expand_launch(const float* F, const float* Z, void* dst, int dtype, int N, int C,
+                              int HW, int R, hipStream_t st) {
+  ExpandArgs a{};
+  a.F = F; a.Z = Z; a.dst = dst;
+  a.C = C; a.R = R; a.HW = HW;
+  a.pixels = (long)N * HW;
+  if (dtype == CP4_DTYPE_BF16) return launch<ToBF16>(a, st);
+  if (dtype == CP4_DTYPE_F16) return launch<ToF16>(a, st);
+  return launch<ToF32>(a, st);
+}
+
+}  // namespace cp4

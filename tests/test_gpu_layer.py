@@ -65,7 +65,13 @@ def test_parts_on_their_own(capi):
     only_dx = capi.layer_backward(s, None, x, y, dy, *fac, "relu", True, False, False)
     only_f = capi.layer_backward(s, None, x, y, dy, *fac, "relu", False, True, False)
     only_b = capi.layer_backward(s, None, x, y, dy, *fac, "relu", False, False, True)
-    assert torch.equal(only_dx[0], dx) and only_dx[2] is None and only_dx[1][0] is None
+    # dx alone contracts dy itself, dx beside the factor gradients takes their G1: the same fp32
+    # sums (24 channels, 9 taps, 8 ranks) in another order, each rounded to 2^-24 of its terms
+    terms = torch.nn.functional.conv_transpose2d(
+        torch.where(y > 0, dy, torch.zeros_like(dy)).abs(),
+        torch.einsum("tr,cr,yr,xr->tcyx", *[f.abs() for f in fac]), padding=1)
+    assert ((only_dx[0] - dx).abs() <= 2 * (24 + 9 + 8) * 2.0 ** -24 * terms + 1e-30).all()
+    assert only_dx[2] is None and only_dx[1][0] is None
     assert all(torch.equal(a, b) for a, b in zip(only_f[1], grads)) and only_f[0] is None
     assert torch.equal(only_b[2], db)
 
@@ -84,3 +90,48 @@ def test_non_finite_gradient_behind_a_clipped_output_is_seen(capi, dtype):
     dy[n, t, h, w] = float("inf")
     dbias = capi.layer_backward(s, None, x, y, dy, *fac, "relu", False, False, True)[2]
     assert torch.isnan(dbias[t]) and int(torch.isfinite(dbias).sum()) == 11
+
+
+# The input gradient beside the factor gradients (dx = FC G1): pixels that no piece divides, blocks
+# over image boundaries, one channel block and several, every chunk count of ranks, a stride.
+@pytest.mark.parametrize("case", [(1, 16, 4, 4, 16, 3, 1, 1), (2, 16, 5, 7, 32, 3, 16, 1),
+                                  (9, 48, 7, 7, 16, 3, 17, 1), (3, 80, 14, 14, 32, 1, 32, 1),
+                                  (2, 32, 15, 30, 48, 5, 33, 1), (3, 272, 20, 20, 16, 3, 64, 1),
+                                  (2, 48, 55, 55, 32, 3, 32, 2), (2, 16, 56, 60, 16, 3, 48, 2)],
+                         ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16],
+                         ids=["f32", "bf16", "f16"])
+def test_input_gradient_beside_the_factors(capi, case, dtype):
+    N, C, H, W, T, k, R, stride = case
+    if stride > 1 and dtype != torch.float32:
+        pytest.skip("layers with a stride take fp32")
+    gen = torch.Generator(device="cuda").manual_seed(N + C + H + W + R)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x = mk(N, C, H, W).to(dtype)
+    fac = [mk(d, R) for d in (T, C, k, k)]
+    s = capi.shape_for(x.shape, *fac, k // 2)
+    g = capi.geometry(s, stride, "same") if stride > 1 else None
+    y = capi.layer_forward(s, g, x, *fac, mk(T), "relu")
+    dy = mk(*y.shape).to(dtype)
+    dx, _, _ = capi.layer_backward(s, g, x, y, dy, *fac, "relu")
+    masked = torch.where(y > 0, dy, torch.zeros_like(dy)).double().cpu()
+    K = torch.einsum("tr,cr,yr,xr->tcyx", *[f.double().cpu() for f in fac])
+    if g is None:
+        g = capi.geometry(s, 1, "same")
+    pads = (g.pad_left, (g.out_w - 1) * stride + k - W - g.pad_left,
+            g.pad_top, (g.out_h - 1) * stride + k - H - g.pad_top)
+
+    def adjoint(d, f):
+        z = torch.zeros(N, C, H, W, dtype=torch.float64, requires_grad=True)
+        out = torch.nn.functional.conv2d(torch.nn.functional.pad(z, pads), f, stride=stride)
+        return torch.autograd.grad(out, z, d)[0]
+
+    want = adjoint(masked, K)
+    # three fp32 contractions: 2^-24 a step of the sum of the terms' magnitudes (as a random walk,
+    # with a factor of four to spare), and the rounding of the stored result
+    terms = adjoint(masked.abs(), torch.einsum("tr,cr,yr,xr->tcyx", *[f.double().cpu().abs() for f in fac]))
+    eps = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    bound = 4 * (T + 2 * k + R) ** 0.5 * 2.0 ** -24 * terms + eps * want.abs() + 1e-30
+    if dtype == torch.float16:
+        bound = bound + 2.0 ** -24          # subnormal results
+    assert ((dx.double().cpu() - want).abs() <= bound).all()
