@@ -329,6 +329,7 @@ __global__ __launch_bounds__(kThreads) void dense_tiles_kernel(BwdFilterArgs a, 
 constexpr int kMThreads = 512, kMWaves = kMThreads / 64;
 constexpr int kMaxAcc = 6;                   // 32 x 32 blocks a wave holds
 constexpr int kMaxAcc16 = 8;                 // 16 x 16 blocks (up to 32 output channels, 16 waves)
+constexpr int kMaxAccMask = 4;               // ... in the masked build
 constexpr int kMaxOuts = 16384;              // T * C * Y * X up to here
 constexpr size_t kMLds = 160 * 1024;
 constexpr int kSlots = 6;                    // groups of four cells a thread stages per tile
@@ -392,12 +393,20 @@ __device__ __forceinline__ void split4(const float (&v)[4], u32x2& h, u32x2& m, 
   }
 }
 
-template <int FS, int MB, bool M16>
+//
+// MASK (16 x 16 blocks only): a layer's backward pass in which nothing else reads dy behind the
+// activation, as in a network's first layer: dy is masked by y on its way to the LDS and its
+// sums per channel, the bias gradient, leave with the partial sets.  A thread's slots belong to
+// fixed channels, so a sum is one register a slot.  y's cells wait in registers beside dy's: the
+// build holds half the accumulators, and stays within 128 registers.  (N16 C3 K64 224x224, dy
+// and y 411 MB: @@MASK@@ us against 119 for a pass that writes the masked dy and 64 for this
+// kernel on it.)
+template <int FS, int MB, bool M16, bool MASK>
 __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kernel(BwdFilterArgs a, MfmaPlan pl,
                                                                   float* partial) {
   // blocks of BW x BW entries of dK, steps of 2^SPLG pixels, NV accumulator registers a block
   constexpr int BW = M16 ? 16 : 32, LGBW = M16 ? 4 : 5, SPLG = M16 ? 5 : 4, NV = M16 ? 4 : 16;
-  constexpr int OWN = (M16 ? kMaxAcc16 : kMaxAcc) / MB;
+  constexpr int OWN = (MASK ? kMaxAccMask : M16 ? kMaxAcc16 : kMaxAcc) / MB;
   // threads: 16 waves where the accumulators are small (four waves per SIMD), else 8
   constexpr int THREADS = M16 ? 1024 : 512, SLOTS = kSlots * kMThreads / THREADS;
   typedef typename AccOf<M16>::type Acc;
@@ -462,7 +471,11 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
 
   const int tiles_per_image = pl.tilesX * pl.tilesY;
   const int lgcw = pl.lgTW - SPLG, nsteps = (pl.TH * pl.TW) >> SPLG;
-  float4 held[SLOTS];
+  float4 held[SLOTS], act[MASK ? SLOTS : 1];
+  float bsum[MASK ? SLOTS : 1];
+  if constexpr (MASK)
+#pragma unroll
+    for (int q = 0; q < SLOTS; ++q) bsum[q] = 0.f;
   // Tile t's cells into this thread's registers (zeros outside the image).
   auto fetch = [&](int t) {
     const int n = t / tiles_per_image, rem = t - n * tiles_per_image;
@@ -471,6 +484,7 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
     const int hd = ty * pl.TH, wd = tx * pl.TW;                      // dy's
     const float* xn = a.x + (size_t)n * a.C * HW;
     const float* dn = a.dy + (size_t)n * a.T * HW;
+    const float* yn = MASK && a.act_y ? a.act_y + (size_t)n * a.T * HW : nullptr;
 #pragma unroll
     for (int q = 0; q < SLOTS; ++q) {
       const int g = tid + THREADS * q;
@@ -481,6 +495,20 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
       const bool row_in = rc[q] >= 0 && (unsigned)h < (unsigned)H;
       const long at = (long)rel[q] + (long)h0 * W + w0;
       float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+      if constexpr (MASK) {
+        float4 yv = make_float4(1.f, 1.f, 1.f, 1.f);
+        if (yn && !isx && row_in) {
+          if (pl.vec) {
+            if ((unsigned)w < (unsigned)W) yv = *reinterpret_cast<const float4*>(yn + at);
+          } else {
+            if ((unsigned)w < (unsigned)W) yv.x = yn[at];
+            if ((unsigned)(w + 1) < (unsigned)W) yv.y = yn[at + 1];
+            if ((unsigned)(w + 2) < (unsigned)W) yv.z = yn[at + 2];
+            if ((unsigned)(w + 3) < (unsigned)W) yv.w = yn[at + 3];
+          }
+        }
+        act[q] = yv;
+      }
       if (pl.vec) {
         // rows start at multiples of four columns and W % 4 == 0: four cells are inside
         // the image together or not at all
@@ -505,7 +533,16 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
         const int e = isx ? 4 * g : 4 * (g - xgroups);
         const int plane = isx ? pl.xplane : pl.dplane;
         char* base = buf + (isx ? 0 : 6 * pl.xplane) + 2 * e;
-        const float v[4] = {held[q].x, held[q].y, held[q].z, held[q].w};
+        float v[4] = {held[q].x, held[q].y, held[q].z, held[q].w};
+        if constexpr (MASK) {
+          // (a product, as dy * (y > 0): a non-finite dy at a clipped output stays visible)
+          const float yv[4] = {act[q].x, act[q].y, act[q].z, act[q].w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            v[i] *= yv[i] > 0.f ? 1.f : 0.f;
+            bsum[q] += v[i];
+          }
+        }
         u32x2 h, m, l;
         split4(v, h, m, l);
         *reinterpret_cast<u32x2*>(base) = h;
@@ -591,6 +628,24 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
     if (more) deposit(bufs + (size_t)((it + 1) & 1) * pl.bufbytes);
     __syncthreads();
   }
+  if constexpr (MASK) {
+    // ---- the bias gradient's part: the slots of a channel, in order ----
+    if (a.dbias) {
+#pragma unroll
+      for (int q = 0; q < SLOTS; ++q) {
+        const int g = tid + THREADS * q;
+        if (g >= xgroups && g < groups) lds[g - xgroups] = bsum[q];
+      }
+      __syncthreads();
+      const int per = pl.DS >> 2;
+      if (tid < a.T) {
+        float s = 0.f;
+        for (int i = 0; i < per; ++i) s += lds[tid * per + i];
+        a.bias_part[(size_t)blockIdx.x * a.T + tid] = s;
+      }
+      __syncthreads();
+    }
+  }
   // ---- the waves that shared column blocks, added in order through LDS ----
   float* red = lds;                                  // [own block][row block][b][element][lane]
   for (int s2 = 1; s2 < pl.slices; ++s2) {
@@ -646,9 +701,19 @@ constexpr int kRedOuts = 32;
 template <int LANES>
 __global__ __launch_bounds__(kRedOuts * LANES) void dense_reduce_kernel(const float* partial,
                                                                         float* dK, int outs,
-                                                                        int sets) {
+                                                                        int sets,
+                                                                        const float* bias_part,
+                                                                        float* dbias, int T) {
   __shared__ float part[LANES][kRedOuts];
-  const int o = blockIdx.x * kRedOuts + threadIdx.x, y = threadIdx.y;
+  int block = blockIdx.x;
+  const int dk_blocks = (outs + kRedOuts - 1) / kRedOuts;
+  if (block >= dk_blocks) {            // the bias gradient's sets, behind those of dK
+    block -= dk_blocks;
+    partial = bias_part;
+    dK = dbias;
+    outs = T;
+  }
+  const int o = block * kRedOuts + threadIdx.x, y = threadIdx.y;
   float s = 0.f;
   if (o < outs) {
     int w = y;
@@ -922,7 +987,7 @@ int read_conflicts(int XR, int XS, int FS, int NC, int shift, bool m16) {
   return total;
 }
 
-bool mfma_plan_blocks(const cp4_shape& s, bool aligned16, int m16, MfmaPlan* best) {
+bool mfma_plan_blocks(const cp4_shape& s, bool aligned16, int m16, bool masked, MfmaPlan* best) {
   const int vec = aligned16 && s.W % 4 == 0 ? 1 : 0, xlead = vec ? 4 : (int)s.pad;
   const int FS = (int)s.Y, T = (int)s.T, C = (int)s.C;
   const int BW = m16 ? 16 : 32, step = m16 ? 32 : 16;
@@ -931,7 +996,7 @@ bool mfma_plan_blocks(const cp4_shape& s, bool aligned16, int m16, MfmaPlan* bes
   //  channels go over two groups of waves)
   const int rgroups = MBall > 2 ? 2 : 1, MB = MBall > 2 ? 2 : MBall;
   if (MBall > 2 * rgroups || (!m16 && rgroups > 1) || (long)T * NC > kMaxOuts) return false;
-  const int most_own = (m16 ? kMaxAcc16 : kMaxAcc) / MB;
+  const int most_acc = masked ? kMaxAccMask : m16 ? kMaxAcc16 : kMaxAcc, most_own = most_acc / MB;
   const int waves = (m16 ? 16 : kMWaves) / rgroups;   // per row group
   const int cus = num_compute_units();
   bool found = false;
@@ -942,7 +1007,7 @@ bool mfma_plan_blocks(const cp4_shape& s, bool aligned16, int m16, MfmaPlan* bes
   for (int nbw = 1; nbw <= waves; nbw *= 2) {
     if ((NB + nbw - 1) / nbw > most_own) continue;
     const int slices = waves / nbw, own = (NB + nbw - 1) / nbw;
-    const size_t red = (size_t)rgroups * (m16 ? kMaxAcc16 : kMaxAcc) * nbw * (m16 ? 256 : 1024) * sizeof(float);
+    const size_t red = (size_t)rgroups * most_acc * nbw * (m16 ? 256 : 1024) * sizeof(float);
   for (int TW = step; TW <= 128; TW *= 2)
     for (int TH = 1; TH <= 32; TH *= 2) {
       if (TH * TW / step < slices) continue;
@@ -1015,7 +1080,7 @@ bool mfma_plan_blocks(const cp4_shape& s, bool aligned16, int m16, MfmaPlan* bes
   pl.xplane = (pl.nx + 8 + 7) / 8 * 8;
   pl.bufbytes = 6 * (pl.xplane + pl.dplane);
   pl.lds_bytes = 2 * (size_t)pl.bufbytes;
-  const size_t red = (size_t)rgroups * (m16 ? kMaxAcc16 : kMaxAcc) * pl.nbw * (m16 ? 256 : 1024) * sizeof(float);
+  const size_t red = (size_t)rgroups * most_acc * pl.nbw * (m16 ? 256 : 1024) * sizeof(float);
   if (pl.slices > 1 && red > pl.lds_bytes) pl.lds_bytes = red;
   pl.chmagic = (unsigned)((0x100000000ull + (unsigned)pl.XR - 1) / (unsigned)pl.XR);
   return true;
@@ -1024,26 +1089,28 @@ bool mfma_plan_blocks(const cp4_shape& s, bool aligned16, int m16, MfmaPlan* bes
 // 16 x 16 blocks (all rows in use with up to 16 channels) on 16 waves, whose accumulators are
 // small enough for four waves per SIMD (N16 C16 K16 512x512: 330 -> 204 us); where no tile of
 // those fits, 32 x 32 blocks on 8 waves.
-bool mfma_plan_uncached(const cp4_shape& s, bool aligned16, MfmaPlan* best) {
-  if (mfma_plan_blocks(s, aligned16, 1, best)) return true;
-  return mfma_plan_blocks(s, aligned16, 0, best);
+bool mfma_plan_uncached(const cp4_shape& s, bool aligned16, bool masked, MfmaPlan* best) {
+  if (mfma_plan_blocks(s, aligned16, 1, masked, best)) return true;
+  return !masked && mfma_plan_blocks(s, aligned16, 0, false, best);
 }
 
 // (the search above is tens of thousands of operations: the last few answers are kept per
 //  thread; a layer's queries alternate between the two alignments and, with odd channel
 //  counts, the layer's zero-padded shape)
-bool mfma_plan(const cp4_shape& s, bool aligned16, MfmaPlan* best) {
+bool mfma_plan(const cp4_shape& s, bool aligned16, MfmaPlan* best, bool masked = false) {
   struct Entry {
-    bool valid = false, aligned16 = false, found = false;
+    bool valid = false, aligned16 = false, masked = false, found = false;
+    int cus = 0;
     cp4_shape shape;
     MfmaPlan plan;
   };
   constexpr int kEntries = 32;
   thread_local Entry cache[kEntries];
   thread_local int next = 0;
+  const int cus = num_compute_units();
   for (int i = 0; i < kEntries; ++i) {
     const Entry& e = cache[i];
-    if (e.valid && e.aligned16 == aligned16 && e.shape.N == s.N && e.shape.C == s.C &&
+    if (e.valid && e.aligned16 == aligned16 && e.masked == masked && e.cus == cus && e.shape.N == s.N && e.shape.C == s.C &&
         e.shape.T == s.T && e.shape.H == s.H && e.shape.W == s.W && e.shape.pad == s.pad &&
         e.shape.Y == s.Y && e.shape.X == s.X && e.shape.Rank == s.Rank) {
       if (e.found) *best = e.plan;
@@ -1052,7 +1119,9 @@ bool mfma_plan(const cp4_shape& s, bool aligned16, MfmaPlan* best) {
   }
   Entry& e = cache[next];
   next = (next + 1) % kEntries;
-  e.found = mfma_plan_uncached(s, aligned16, &e.plan);
+  e.found = mfma_plan_uncached(s, aligned16, masked, &e.plan);
+  e.masked = masked;
+  e.cus = cus;
   e.shape = s;
   e.aligned16 = aligned16;
   e.valid = true;
@@ -1062,11 +1131,13 @@ bool mfma_plan(const cp4_shape& s, bool aligned16, MfmaPlan* best) {
 
 template <int FS>
 hipError_t launch_mfma_fs(const BwdFilterArgs& a, const MfmaPlan& pl, float* partial, hipStream_t st) {
-  auto k0 = dense_mfma_kernel<FS, 1, true>;
-  auto k02 = dense_mfma_kernel<FS, 2, true>;
-  auto k1 = dense_mfma_kernel<FS, 1, false>;
-  auto k2 = dense_mfma_kernel<FS, 2, false>;
+  auto k0 = dense_mfma_kernel<FS, 1, true, false>;
+  auto k02 = dense_mfma_kernel<FS, 2, true, false>;
+  auto k1 = dense_mfma_kernel<FS, 1, false, false>;
+  auto k2 = dense_mfma_kernel<FS, 2, false, false>;
   auto k = pl.m16 ? (pl.MB == 2 ? k02 : k0) : (pl.MB == 2 ? k2 : k1);
+  if (a.act_y || a.dbias)
+    k = pl.MB == 2 ? dense_mfma_kernel<FS, 2, true, true> : dense_mfma_kernel<FS, 1, true, true>;
   if (pl.lds_bytes > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds_bytes);
@@ -1131,6 +1202,11 @@ bool use_mfma(const cp4_shape& s) {
 }  // namespace
 
 bool bwd_filter_dense_tiles_supported(const cp4_shape& s) { return valu_ok(s) || mfma_ok(s); }
+
+bool bwd_filter_dense_tiles_masks(const cp4_shape& s) {
+  MfmaPlan pl;
+  return use_mfma(s) && mfma_plan(s, false, &pl, true);
+}
 
 void bwd_filter_dense_tiles_force_kernel(int which) {
   g_forced_tile_kernel.store(which == 0 || which == 1 ? which : -1);
@@ -1202,10 +1278,23 @@ hipError_t bwd_filter_dense_tiles_launch(const BwdFilterArgs& a, hipStream_t st)
   hipError_t e;
   int sets;
   // (the partial sets are `outs` apart; the padded stride is only what the size allows for)
-  const bool aligned16 = ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.dy)) & 15) == 0;
-  if (use_mfma(s)) {
+  const bool aligned16 = ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.dy) |
+                           reinterpret_cast<uintptr_t>(a.act_y)) & 15) == 0;
+  const bool masked = a.act_y || a.dbias;
+  if (masked || use_mfma(s)) {
     MfmaPlan pl;
-    if (!mfma_plan(s, aligned16, &pl) && !mfma_plan(s, false, &pl)) return hipErrorInvalidValue;
+    if (!mfma_plan(s, aligned16, &pl, masked) && !mfma_plan(s, false, &pl, masked))
+      return hipErrorInvalidValue;
+    if (masked) {
+      // the workspace has room for the partial sets of the plain build's plans; smaller tiles
+      // could give this one more workgroups
+      MfmaPlan plain;
+      int most = 0;
+      for (const bool al : {false, true})
+        if (mfma_plan(s, al, &plain) && plain.grid > most) most = plain.grid;
+      if (pl.grid > most) pl.grid = most;
+      if (pl.grid < 1) return hipErrorInvalidValue;
+    }
     sets = pl.grid;
     switch (a.Y) {
       case 1: e = launch_mfma_fs<1>(a, pl, partial, st); break;
@@ -1223,12 +1312,14 @@ hipError_t bwd_filter_dense_tiles_launch(const BwdFilterArgs& a, hipStream_t st)
     }
   }
   if (e != hipSuccess) return e;
+  const int rblocks = (outs + kRedOuts - 1) / kRedOuts +
+                      (a.dbias ? (a.T + kRedOuts - 1) / kRedOuts : 0);
   if (outs <= 512)
-    dense_reduce_kernel<32><<<(outs + kRedOuts - 1) / kRedOuts, dim3(kRedOuts, 32), 0, st>>>(
-        partial, dK, outs, sets);
+    dense_reduce_kernel<32><<<rblocks, dim3(kRedOuts, 32), 0, st>>>(partial, dK, outs, sets,
+                                                                    a.bias_part, a.dbias, a.T);
   else
-    dense_reduce_kernel<8><<<(outs + kRedOuts - 1) / kRedOuts, dim3(kRedOuts, 8), 0, st>>>(
-        partial, dK, outs, sets);
+    dense_reduce_kernel<8><<<rblocks, dim3(kRedOuts, 8), 0, st>>>(partial, dK, outs, sets,
+                                                                  a.bias_part, a.dbias, a.T);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   const size_t fold_lds = fold_lds_bytes(s);

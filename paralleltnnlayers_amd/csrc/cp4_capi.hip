@@ -1681,6 +1681,35 @@ cp4_status layer_backward_filter(const cp4_shape* s, const cp4_geometry* g, int 
   return backward_filter_16(s, x, dy, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
                             workspace_bytes, dtype == CP4_DTYPE_F16, dx, stream);
 }
+
+bool layer_filter_masks(const cp4_shape& s, const float* x, const float* dy, const void* workspace) {
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy) |
+                         reinterpret_cast<uintptr_t>(workspace);
+  const FilterRoutes routes = filter_routes(s, (bits & 7) == 0, (bits & 15) == 0,
+                                            (reinterpret_cast<uintptr_t>(workspace) & 255) == 0);
+  return default_filter_variant(s, routes) == 3 && bwd_filter_dense_tiles_masks(s);
+}
+
+cp4_status layer_backward_filter_masked(const cp4_shape* shape, const float* x, const float* act_y,
+                                        const float* dy, const float* FK, const float* FC,
+                                        const float* FH, const float* FW, float* dFK, float* dFC,
+                                        float* dFH, float* dFW, float* dbias, float* bias_part,
+                                        void* workspace, size_t workspace_bytes, cp4_stream stream) {
+  if (!FK || !FC || !FH || !FW || !dFK || !dFC || !dFH || !dFW)
+    return fail(CP4_ERR_NULL_POINTER, "a factor or gradient pointer is NULL");
+  const cp4_shape& s = *shape;
+  if (!workspace || workspace_bytes < filter_workspace(s))
+    return fail(CP4_ERR_WORKSPACE,
+                "workspace smaller than cp4_conv2d_backward_filter_workspace_bytes");
+  BwdFilterArgs a{};
+  a.x = x; a.dy = dy; a.FK = FK; a.FC = FC; a.FH = FH; a.FW = FW;
+  a.dFK = dFK; a.dFC = dFC; a.dFH = dFH; a.dFW = dFW; a.workspace = workspace;
+  a.N = s.N; a.C = s.C; a.T = s.T; a.H = s.H; a.W = s.W; a.pad = s.pad;
+  a.Y = s.Y; a.X = s.X; a.R = s.Rank;
+  a.act_y = act_y; a.dbias = dbias; a.bias_part = bias_part;
+  CP4_HIP(bwd_filter_dense_tiles_launch(a, as_stream(stream)));
+  return CP4_OK;
+}
 }  // namespace cp4
 extern "C" {
 

@@ -90,6 +90,15 @@ cp4_status layer_backward_filter(const cp4_shape*, const cp4_geometry*, int dtyp
                                  const float* FW, float* dFK, float* dFC, float* dFH, float* dFW,
                                  void* workspace, size_t workspace_bytes, void* dx, bool* dx_done,
                                  cp4_stream);
+cp4_status layer_backward_filter_masked(const cp4_shape*, const float* x, const float* act_y,
+                                        const float* dy, const float* FK, const float* FC,
+                                        const float* FH, const float* FW, float* dFK, float* dFC,
+                                        float* dFH, float* dFW, float* dbias, float* bias_part,
+                                        void* workspace, size_t workspace_bytes, cp4_stream);
+
+// The factor gradients of an fp32 layer without an input gradient run the dense-gradient
+// route with the mask and the bias gradient in it (x and dy of these addresses).
+bool layer_filter_masks(const cp4_shape&, const float* x, const float* dy, const void* workspace);
 
 // Compute units of the current device (256 when no device can be asked).
 int num_compute_units();
@@ -189,6 +198,11 @@ struct BwdFilterArgs {
   // Matrix-core variant only: not null, the input gradient too, dx = FC G1 (in the type of
   // x; the forward's adjoint only where 2 * pad = Y - 1 = X - 1 or with a geometry).
   void* dx;
+  // Dense-gradient variant with bwd_filter_dense_tiles_masks only: dy counts where act_y > 0
+  // (null: everywhere) and dbias[t], its sum over images and pixels, comes along through
+  // bias_part (T floats per compute unit of scratch); all null: neither.
+  const float* act_y;
+  float *dbias, *bias_part;
 };
 // general (VALU, any shape) and matrix-core variants
 size_t bwd_filter_workspace_bytes(const cp4_shape&);
@@ -214,6 +228,8 @@ bool bwd_filter_dense_tiles_supported(const cp4_shape&);
 bool bwd_filter_dense_tiles_preferred(const cp4_shape&);
 size_t bwd_filter_dense_tiles_workspace_bytes(const cp4_shape&);
 hipError_t bwd_filter_dense_tiles_launch(const BwdFilterArgs&, hipStream_t);
+// The route takes the layer's activation mask and bias gradient with it (BwdFilterArgs::act_y).
+bool bwd_filter_dense_tiles_masks(const cp4_shape&);
 // 0: the plain multiply-add tile kernel, 1: the matrix-core one, wherever both can run the
 // shape; anything else: the route's own choice.
 void bwd_filter_dense_tiles_force_kernel(int which);

@@ -1,5 +1,6 @@
 // C ABI of a whole layer, y = act(conv + bias): which passes a call needs, on which element
 // type each runs, and where their intermediates lie in the caller's workspace.
+#include <algorithm>
 #include <array>
 #include <map>
 #include <mutex>
@@ -15,6 +16,7 @@ size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 struct BackwardPlan {
   bool dx16, filter16;       // dx / the factor gradients on the 16-bit activations (16-bit layers only)
   bool act16, act32;         // dy behind the activation is written in the layer's type / as fp32
+  bool may_mask;             // the factor gradients may take the mask and the bias gradient along
   size_t act16_at, act32_at; // ... here
   size_t x32_at, dx32_at;    // widened x, fp32 dx before it is rounded
   size_t bias_at, pass_at;   // partial bias sums, the passes' own workspace
@@ -53,7 +55,9 @@ BackwardPlan make_backward_plan(const cp4_shape& s, const cp4_geometry* g, int d
   p.x32_at = take(filter32, nx * 4);
   p.dx32_at = take(dx32, nx * 4);
   const int seg = cp4::act_grad_segments((int)s.N, (int)s.T, ny / ((size_t)s.N * s.T), dtype);
-  p.bias_at = take((wanted & CP4_WANT_BIAS) && seg > 1, (size_t)s.T * seg * 4);
+  p.may_mask = !g && !half && filter && !dx && (act != CP4_ACT_NONE || (wanted & CP4_WANT_BIAS));
+  const size_t parts = p.may_mask ? std::max(seg, cp4::num_compute_units()) : seg > 1 ? seg : 0;
+  p.bias_at = take((wanted & CP4_WANT_BIAS) && parts, s.T * parts * 4);
   p.pass_at = at;
   if (g) p.pass_bytes = dx || filter ? cp4_conv2d_backward_ex_workspace_bytes(&s, g) : 0;
   else p.pass_bytes = filter ? cp4_conv2d_backward_filter_workspace_bytes(&s) : 0;
@@ -186,6 +190,13 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* g, int
   const void* dya = dy;                                     // in the layer's type
   const float* dy32 = reinterpret_cast<const float*>(ws + p.act32_at);
   float* parts = reinterpret_cast<float*>(ws + p.bias_at);
+  if (p.may_mask && cp4::layer_filter_masks(s, static_cast<const float*>(x),
+                                            static_cast<const float*>(dy), ws + p.pass_at))
+    // a first layer: nothing but the factor gradients reads dy, masked on its way
+    return cp4::layer_backward_filter_masked(
+        shape, static_cast<const float*>(x), static_cast<const float*>(ym),
+        static_cast<const float*>(dy), FK, FC, FH, FW, dFK, dFC, dFH, dFW, dbias, parts,
+        ws + p.pass_at, p.pass_bytes, stream);
   if (p.act16) {
     CP4_LAUNCH(cp4::act_grad_launch(ym, dy, ws + p.act16_at, dtype, false, dbias, parts, N, T, plane, st));
     dya = ws + p.act16_at;

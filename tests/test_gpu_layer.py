@@ -72,7 +72,17 @@ def test_parts_on_their_own(capi):
         torch.einsum("tr,cr,yr,xr->tcyx", *[f.abs() for f in fac]), padding=1)
     assert ((only_dx[0] - dx).abs() <= 2 * (24 + 9 + 8) * 2.0 ** -24 * terms + 1e-30).all()
     assert only_dx[2] is None and only_dx[1][0] is None
-    assert all(torch.equal(a, b) for a, b in zip(only_f[1], grads)) and only_f[0] is None
+    # the factor gradients alone may take the mask with them on tiles of their own: the same fp32
+    # sums (2 * 9 * 11 pixels, then 24 * 9, 16 * 9 or 24 * 16 * 3 entries of dK) in another order
+    dK = torch.nn.grad.conv2d_weight(x.abs(), (24, 16, 3, 3), dy.abs(), padding=1)
+    f = [t.abs() for t in fac]
+    sums = [torch.einsum("tcyx,cr,yr,xr->tr", dK, f[1], f[2], f[3]),
+            torch.einsum("tcyx,tr,yr,xr->cr", dK, f[0], f[2], f[3]),
+            torch.einsum("tcyx,tr,cr,xr->yr", dK, f[0], f[1], f[3]),
+            torch.einsum("tcyx,tr,cr,yr->xr", dK, f[0], f[1], f[2])]
+    for a, b, t, n in zip(only_f[1], grads, sums, (16 * 9, 24 * 9, 24 * 16 * 3, 24 * 16 * 3)):
+        assert ((a - b).abs() <= 2 * (198 + n) ** 0.5 * 2.0 ** -24 * t).all()
+    assert only_f[0] is None
     assert torch.equal(only_b[2], db)
 
 
@@ -135,3 +145,48 @@ def test_input_gradient_beside_the_factors(capi, case, dtype):
     if dtype == torch.float16:
         bound = bound + 2.0 ** -24          # subnormal results
     assert ((dx.double().cpu() - want).abs() <= bound).all()
+
+
+# A first layer (no input gradient): mask and bias gradient inside the dense-gradient kernel.
+# Both counts of row blocks and groups, planes smaller than a tile, widths no piece divides,
+# several tiles a workgroup, operands off a 16-byte boundary.
+@pytest.mark.parametrize("case", [(1, 3, 1, 1, 1, 1, 1, 0), (2, 3, 7, 9, 16, 3, 4, 0),
+                                  (3, 1, 33, 20, 17, 5, 8, 0), (2, 3, 30, 31, 33, 3, 16, 0),
+                                  (2, 4, 16, 64, 64, 1, 16, 1), (16, 3, 90, 112, 64, 3, 16, 0),
+                                  (4, 3, 112, 112, 40, 3, 16, 1)],
+                         ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("relu", [True, False], ids=["relu", "linear"])
+def test_first_layer_without_an_input_gradient(capi, case, relu):
+    N, C, H, W, T, k, R, shift = case
+    gen = torch.Generator(device="cuda").manual_seed(N * H + W + T)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+
+    def placed(t):                      # the same values `shift` floats off the allocation
+        flat = torch.empty(t.numel() + shift, device="cuda")[shift:]
+        return flat.copy_(t.flatten()).view(t.shape)
+
+    x, dy = placed(mk(N, C, H, W)), placed(mk(N, T, H, W))
+    fac = [mk(d, R) for d in (T, C, k, k)]
+    s = capi.shape_for(x.shape, *fac, k // 2)
+    act = "relu" if relu else None
+    y = placed(capi.layer_forward(s, None, x, *fac, mk(T), act))
+    _, grads, dbias = capi.layer_backward(s, None, x, y, dy, *fac, act, False, True, True)
+    alone = capi.layer_backward(s, None, x, y, dy, *fac, act, False, True, False)[1]
+    assert all(torch.equal(a, b) for a, b in zip(grads, alone))
+    masked = (torch.where(y > 0, dy, torch.zeros_like(dy)) if relu else dy).double().cpu()
+    # fp32 sums: 2^-24 a step, as a random walk over the terms (a factor of four to spare)
+    n = N * H * W
+    want = masked.sum(dim=(0, 2, 3))
+    tol = 4 * 2.0 ** -24 * ((masked ** 2).sum(dim=(0, 2, 3)) * n).sqrt()
+    assert ((dbias.double().cpu() - want).abs() <= tol + 1e-30).all()
+    xd = x.double().cpu()
+    K = torch.zeros(T, C, k, k, dtype=torch.float64, requires_grad=True)
+    dK, = torch.autograd.grad(torch.nn.functional.conv2d(xd, K, padding=k // 2), K, masked)
+    f = [t.double().cpu() for t in fac]
+    wants = [torch.einsum("tcyx,cr,yr,xr->tr", dK, f[1], f[2], f[3]),
+             torch.einsum("tcyx,tr,yr,xr->cr", dK, f[0], f[2], f[3]),
+             torch.einsum("tcyx,tr,cr,xr->yr", dK, f[0], f[1], f[3]),
+             torch.einsum("tcyx,tr,cr,yr->xr", dK, f[0], f[1], f[2])]
+    # the repository's bar for factor gradients
+    for g, w in zip(grads, wants):
+        assert (g.double().cpu() - w).abs().max() <= 1e-3 * w.abs().max() + 1e-30
