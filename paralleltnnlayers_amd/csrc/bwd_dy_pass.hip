@@ -1,0 +1,239 @@
+// One pass over a layer's output gradient for everything in its backward that reads it: with
+// dya = dy where y > 0 (a layer behind a ReLU; dy itself without one) and Cc = the filtered
+// rank planes of x,
+//   G3[n,r,p] = sum_t FK[t,r] dya[n,t,p]     dFK[t,r] = sum_{n,p} dya[n,t,p] Cc[n,r,p]
+//   dbias[t]  = sum_{n,p} dya[n,t,p]
+// so dya never goes to memory.  (As passes of their own: the mask and the bias gradient read dy and y and
+// write dya, the contraction and the gradient GEMM read it once each - five times the plane
+// where this kernel moves two.)
+//
+// Bound by reading dy and y.  A workgroup takes chunks of 64 pixels of one image and all T channels
+// (up to 256), a wave per 32 channels; about eight waves a compute unit, each with a whole chunk's
+// dy and y (64 registers) in flight while it works on the chunk before.  Rows move as 16 bytes a
+// lane, 256 contiguous bytes a channel.  A wave's 32 x 64 tile of dya lies in LDS, its own: read
+// by rows (channel x 8 pixels) it is the A operand of the dFK product, read by columns (pixel
+// x 8 channels) the B operand of the contraction; exact fp32 products from three bf16 parts.  The
+// contraction's partial sums over a wave's channels go over its tile, which nothing reads any
+// more, and are added over the waves in order; Cc's fragments are split once a workgroup.  Two
+// barriers a chunk.  dFK and the bias sums stay in registers over a workgroup's contiguous
+// range of chunks: one partial set per workgroup, added in order by the caller's reduction.
+// N32 T256 56x56 R32 (206 MB): @@DYPASS@@.
+#include <algorithm>
+#include <cstdint>
+
+#include "cp4_internal.h"
+#include "split_bf16.h"
+
+namespace cp4 {
+namespace {
+
+using split::f32x16;
+using split::u32x4;
+
+constexpr int kPix = 64;                 // pixels of a chunk
+constexpr int kRow = kPix + 4;           // LDS row stride: 16-byte rows, four banks apart
+constexpr int kTile = 32 * kRow;         // floats of a wave's tile
+constexpr int kFrag = 4 * 3 * 2 * 32;    // 16-byte fragments of a chunk of Cc: [step][part][half][rank]
+
+struct DyPassArgs {
+  const float *dy, *y, *FK, *Cc;
+  float *G3, *partK, *partB;             // partB null: no bias gradient
+  int T, R, HW, cpi, chunks;             // chunks per image and in all
+};
+
+// KZ: (rank, octet) pairs of Cc a thread loads and splits (256 of them a chunk).
+template <bool MASK, int KZ>
+__global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  const int T = a.T, R = a.R, HW = a.HW, c0 = 32 * wave;
+  float* tile = lds + wave * kTile;
+  u32x4* Zf = reinterpret_cast<u32x4*>(lds + waves * kTile);
+  // workgroups of a die (blockIdx & 7): consecutive ranges
+  const unsigned die = blockIdx.x & 7, per = gridDim.x >> 3, rest = gridDim.x & 7;
+  const unsigned wg = die * per + (die < rest ? die : rest) + (blockIdx.x >> 3);
+  const int i0 = (int)((long)a.chunks * wg / gridDim.x), i1 = (int)((long)a.chunks * (wg + 1) / gridDim.x);
+
+  // this wave's rows of FK, split: the contraction's A operand (zero past the last rank)
+  u32x4 fh[2], fm[2], fl[2];
+#pragma unroll
+  for (int ch = 0; ch < 2; ++ch) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      v[e] = l32 < R ? a.FK[(size_t)(c0 + 16 * ch + 8 * hi + e) * R + l32] : 0.f;
+    split::split8(v, fh[ch], fm[ch], fl[ch]);
+  }
+
+  // ---- loads: row 4 j + lane / 16 of the wave's channels, four pixels a lane ----
+  const int lrow = lane >> 4, lcol = 4 * (lane & 15);
+  float4 dv[8], yv[MASK ? 8 : 1], zv[KZ][2];
+  auto load = [&](int i) {
+    const int n = i / a.cpi;
+    const int p0 = (i - n * a.cpi) * kPix;
+    const int p = p0 + lcol;
+    const size_t at = ((size_t)n * T + c0 + lrow) * HW + (p < HW ? p : 0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      dv[j] = *reinterpret_cast<const float4*>(a.dy + at + (size_t)(4 * j) * HW);
+      if constexpr (MASK) yv[j] = *reinterpret_cast<const float4*>(a.y + at + (size_t)(4 * j) * HW);
+    }
+#pragma unroll
+    for (int k = 0; k < KZ; ++k) {
+      const int it = threadIdx.x + k * blockDim.x, zr = it >> 3, pz = p0 + 8 * (it & 7);
+      const bool in = it < 256 && zr < R;
+      const float* z = a.Cc + ((size_t)n * R + (in ? zr : 0)) * HW;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        zv[k][h] = in && pz + 4 * h < HW ? *reinterpret_cast<const float4*>(z + pz + 4 * h)
+                                         : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  };
+  auto deposit_z = [&] {
+#pragma unroll
+    for (int k = 0; k < KZ; ++k) {
+      const int it = threadIdx.x + k * blockDim.x, zr = it >> 3, zo = it & 7;
+      if (it < 256) {
+        const float v[8] = {zv[k][0].x, zv[k][0].y, zv[k][0].z, zv[k][0].w,
+                            zv[k][1].x, zv[k][1].y, zv[k][1].z, zv[k][1].w};
+        u32x4 h, m, l;
+        split::split8(v, h, m, l);
+        u32x4* dst = Zf + ((zo >> 1) * 6 + (zo & 1)) * 32 + zr;
+        dst[0] = h;
+        dst[64] = m;
+        dst[128] = l;
+      }
+    }
+  };
+  f32x16 accK = (f32x16)(0.f);
+  float bs[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) bs[j] = 0.f;
+  if (i0 < i1) {
+    load(i0);
+    deposit_z();
+  }
+  __syncthreads();
+  for (int i = i0; i < i1; ++i) {
+    const int n = i / a.cpi;
+    const int p0 = (i - n * a.cpi) * kPix;
+    // ---- the held rows behind the activation, into the tile ----
+    const bool in = p0 + lcol < HW;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float4 m = in ? dv[j] : make_float4(0.f, 0.f, 0.f, 0.f);
+      if constexpr (MASK) {
+        // (a product, as dy * (y > 0): a non-finite dy at a clipped output stays visible)
+        m.x *= yv[j].x > 0.f ? 1.f : 0.f;
+        m.y *= yv[j].y > 0.f ? 1.f : 0.f;
+        m.z *= yv[j].z > 0.f ? 1.f : 0.f;
+        m.w *= yv[j].w > 0.f ? 1.f : 0.f;
+      }
+      bs[j] += (m.x + m.y) + (m.z + m.w);
+      *reinterpret_cast<float4*>(tile + (4 * j + lrow) * kRow + lcol) = m;
+    }
+    if (i + 1 < i1) load(i + 1);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // ---- dFK: rows of the tile against Cc ----
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+      const float* ap = tile + l32 * kRow + 16 * st + 8 * hi;
+      const float4 a0 = *reinterpret_cast<const float4*>(ap);
+      const float4 a1 = *reinterpret_cast<const float4*>(ap + 4);
+      const float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+      u32x4 ah, am, al;
+      split::split8(v, ah, am, al);
+      const u32x4* zp = Zf + (st * 6 + hi) * 32 + l32;
+      accK = split::mfma_split(ah, am, al, zp[0], zp[64], zp[128], accK);
+    }
+    // ---- G3: FK against columns of the tile ----
+    f32x16 accG[2];
+#pragma unroll
+    for (int pb = 0; pb < 2; ++pb) {
+      accG[pb] = (f32x16)(0.f);
+#pragma unroll
+      for (int ch = 0; ch < 2; ++ch) {
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = tile[(16 * ch + 8 * hi + e) * kRow + 32 * pb + l32];
+        u32x4 bh, bm, bl;
+        split::split8(v, bh, bm, bl);
+        accG[pb] = split::mfma_split(fh[ch], fm[ch], fl[ch], bh, bm, bl, accG[pb]);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int pb = 0; pb < 2; ++pb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) tile[(16 * pb + v) * 64 + lane] = accG[pb][v];
+    __syncthreads();              // partial sums complete; Cc's fragments read by every wave
+    for (int k = wave; k < 32; k += waves) {
+      float s = 0.f;
+      for (int w = 0; w < waves; ++w) s += lds[w * kTile + k * 64 + lane];
+      const int v = k & 15, r = 8 * (v >> 2) + 4 * hi + (v & 3);
+      const int p = p0 + 32 * (k >> 4) + l32;
+      if (r < R && p < HW) a.G3[((size_t)n * R + r) * HW + p] = s;
+    }
+    if (i + 1 < i1) deposit_z();
+    __syncthreads();              // tiles free, the next chunk's fragments complete
+  }
+  // ---- one partial set per workgroup ----
+  float* pk = a.partK + ((size_t)wg * T + c0) * R;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int d = 8 * (v >> 2) + 4 * hi + (v & 3);
+    if (l32 < R) pk[(size_t)d * R + l32] = accK[v];
+  }
+  if (a.partB) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float s = bs[j];
+#pragma unroll
+      for (int off = 8; off > 0; off >>= 1) s += __shfl_down(s, off, 16);
+      if ((lane & 15) == 0) a.partB[(size_t)wg * T + c0 + 4 * j + lrow] = s;
+    }
+  }
+}
+
+int grid_of(int N, int T, int HW) {
+  const long chunks = (long)N * ((HW + kPix - 1) / kPix);
+  const long wgs = (long)num_compute_units() * std::max(1, 8 / (T / 32));
+  return (int)std::min(chunks, wgs);
+}
+
+}  // namespace
+
+// 64 to 256 output channels in whole blocks of 32, ranks up to 32, rows that move as 16 bytes; at least
+// two chunks a workgroup (a workgroup reads all of FK and leaves a partial set whatever it does).
+bool bwd_dy_pass_supported(int N, int T, int R, int HW) {
+  if (T % 32 != 0 || T < 64 || T > 256 || R < 1 || R > 32 || HW % 4 != 0) return false;
+  const long chunks = (long)N * ((HW + kPix - 1) / kPix);
+  return chunks >= 2l * num_compute_units() * std::max(1, 8 / (T / 32));
+}
+int bwd_dy_pass_sets(int N, int T, int HW) { return grid_of(N, T, HW); }
+
+hipError_t bwd_dy_pass_launch(const float* dy, const float* y, const float* FK, const float* Cc,
+                              float* G3, float* partK, float* partB, int N, int T, int R, int HW,
+                              hipStream_t st) {
+  DyPassArgs a{};
+  a.dy = dy; a.y = y; a.FK = FK; a.Cc = Cc; a.G3 = G3; a.partK = partK; a.partB = partB;
+  a.T = T; a.R = R; a.HW = HW;
+  a.cpi = (HW + kPix - 1) / kPix;
+  a.chunks = N * a.cpi;
+  const int waves = T / 32;
+  const size_t lds = (size_t)waves * kTile * sizeof(float) + kFrag * 16;
+  auto k = waves >= 4 ? (y ? dy_pass_kernel<true, 1> : dy_pass_kernel<false, 1>)
+                      : (y ? dy_pass_kernel<true, 2> : dy_pass_kernel<false, 2>);
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  k<<<grid_of(N, T, HW), 64 * waves, lds, st>>>(a);
+  return hipGetLastError();
+}
+
+}  // namespace cp4

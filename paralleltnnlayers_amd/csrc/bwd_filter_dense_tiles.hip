@@ -399,7 +399,7 @@ __device__ __forceinline__ void split4(const float (&v)[4], u32x2& h, u32x2& m, 
 // sums per channel, the bias gradient, leave with the partial sets.  A thread's slots belong to
 // fixed channels, so a sum is one register a slot.  y's cells wait in registers beside dy's: the
 // build holds half the accumulators, and stays within 128 registers.  (N16 C3 K64 224x224, dy
-// and y 411 MB: @@MASK@@ us against 119 for a pass that writes the masked dy and 64 for this
+// and y 411 MB: 94 us against 119 for a pass that writes the masked dy and 64 for this
 // kernel on it.)
 template <int FS, int MB, bool M16, bool MASK>
 __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kernel(BwdFilterArgs a, MfmaPlan pl,

@@ -17,7 +17,7 @@
 //      split over images (and pixel ranges) across workgroups, the Z tile split once
 //      per 32-pixel chunk into double-buffered B fragments in LDS.  grad_gemm_kernel
 //      (fp32 MFMA) where rows cannot move as 16-byte vectors.
-//   4. reduce4_kernel: fixed-order sum of the per-workgroup partials (bit-reproducible).
+//   4. reduce_sets_kernel: fixed-order sum of the per-workgroup partials (bit-reproducible).
 // The library's choice for large problems and for shapes the three-launch variant
 // (bwd_filter_fused.hip) does not take; also the strided layer's pass and the
 // 3-factor op's (depthwise-filter tap step).
@@ -756,8 +756,10 @@ hipError_t launch_taps_wave(const float* A, const float* G3, const BwdFilterArgs
 // barrier.  Row t of A and G3 is requested kRowsAhead steps before it is used.
 // Step t completes B and Cc on row t-(FS-1-P), G2 on row t, G1 on row t-P and
 // the tap-gradient terms of row t-(FS-1-P).  Needs P <= FS-1.
+// Part of the work (kTaps...): Cc alone, from A alone, or everything but Cc.
+enum { kTapsAll, kTapsCc, kTapsRest };
 constexpr int kRowsAhead = 8;
-template <int FS>
+template <int FS, int PART>
 __global__ __launch_bounds__(256) void taps_column_kernel(
     const float* __restrict__ A, const float* __restrict__ G3, const float* __restrict__ FH,
     const float* __restrict__ FW, float* __restrict__ Cc, float* __restrict__ G1,
@@ -811,7 +813,7 @@ __global__ __launch_bounds__(256) void taps_column_kernel(
   auto request = [&](int slot, int row) {          // rows past the plane count as zero
     const int rc = row < H ? row : H - 1;
     ar[slot] = A[base + (size_t)rc * W + wc];
-    gr[slot] = G3[base + (size_t)rc * W + wc];
+    if constexpr (PART != kTapsCc) gr[slot] = G3[base + (size_t)rc * W + wc];
   };
 #pragma unroll
   for (int u = 0; u < kRowsAhead; ++u) request(u, tstart + u);
@@ -822,15 +824,16 @@ __global__ __launch_bounds__(256) void taps_column_kernel(
       const int t = t0 + u;
       if (t < r1 + tail) {
         const bool live = col && t < H;
-        const float a_t = live ? ar[u] : 0.f, g_t = live ? gr[u] : 0.f;
+        const float a_t = live ? ar[u] : 0.f, g_t = PART != kTapsCc && live ? gr[u] : 0.f;
         request(u, t + kRowsAhead);
         // G2 row t: horizontal adjoint taps of G3 row t
         float g2_t = 0.f;
+        if constexpr (PART != kTapsCc)
 #pragma unroll
-        for (int j = 0; j < FS; ++j) {
-          const float v = __shfl(g_t, srcb[j], 64);
-          g2_t += okb[j] ? fw[j] * v : 0.f;
-        }
+          for (int j = 0; j < FS; ++j) {
+            const float v = __shfl(g_t, srcb[j], 64);
+            g2_t += okb[j] ? fw[j] * v : 0.f;
+          }
 #pragma unroll
         for (int i = 0; i + 1 < FS; ++i) {
           aw[i] = aw[i + 1];
@@ -857,7 +860,7 @@ __global__ __launch_bounds__(256) void taps_column_kernel(
 #pragma unroll
           for (int i = 0; i < FS; ++i)
             accH[i] += mine ? g2w[P] * aw[i] : 0.f;   // G2[hb][w] * A[hb+i-P][w]
-          if (mine) Cc[base + (size_t)hb * W + gc] = cc;
+          if (PART != kTapsRest && mine) Cc[base + (size_t)hb * W + gc] = cc;
         }
         // G1 row hg: vertical adjoint taps of the G2 window
         const int hg = t - P;
@@ -865,11 +868,12 @@ __global__ __launch_bounds__(256) void taps_column_kernel(
           float g1 = 0.f;
 #pragma unroll
           for (int i = 0; i < FS; ++i) g1 += fh[i] * g2w[FS - 1 - i];
-          if (mine) G1[base + (size_t)hg * W + gc] = g1;
+          if (PART != kTapsCc && mine) G1[base + (size_t)hg * W + gc] = g1;
         }
       }
     }
   }
+  if constexpr (PART == kTapsCc) return;
 #pragma unroll
   for (int i = 0; i < FS; ++i) {
 #pragma unroll
@@ -907,7 +911,7 @@ int column_row_segments(int N, int R, int H, int W, int FS, int P) {
   return (H + RH - 1) / RH;
 }
 
-template <int FS>
+template <int FS, int PART = kTapsAll>
 hipError_t launch_taps_column(const float* A, const float* G3, const BwdFilterArgs& a, float* Cc,
                               float* G1, float* pH, float* pW, hipStream_t st) {
   const int nplanes = a.N * a.R, segs = column_segments(a.W, FS, a.pad);
@@ -915,7 +919,7 @@ hipError_t launch_taps_column(const float* A, const float* G3, const BwdFilterAr
   const int RH = column_row_height(a.N, a.R, a.H, a.W, FS, a.pad);
   const int rsegs = (a.H + RH - 1) / RH;
   const long units = (long)nplanes * segs * rsegs;
-  taps_column_kernel<FS><<<(unsigned)((units + 3) / 4), 256, 0, st>>>(
+  taps_column_kernel<FS, PART><<<(unsigned)((units + 3) / 4), 256, 0, st>>>(
       A, G3, a.FH, a.FW, Cc, G1, pH, pW, a.R, a.H, a.W, a.pad, nplanes, segs, Q, rsegs, RH);
   return hipGetLastError();
 }
@@ -1209,16 +1213,16 @@ __global__ __launch_bounds__(256) void tap_grad_kernel(const float* __restrict__
   }
 }
 
-// ---- 4. out[i] = sum_s partial[s][i], four segments in one launch -----------
+// ---- 4. out[i] = sum_s partial[s][i], up to five segments in one launch ------
 struct ReduceArgs {
-  const float* part[4];
-  float* out[4];
-  int count[4], S[4];
+  const float* part[5];
+  float* out[5];
+  int count[5], S[5];
 };
 // A workgroup owns 64 consecutive outputs; its four waves each sum a quarter of
 // the S partials in index order (eight loads in flight), then the four quarter
 // sums are added in wave order: the result does not depend on timing.
-__global__ __launch_bounds__(256) void reduce4_kernel(ReduceArgs a) {
+__global__ __launch_bounds__(256) void reduce_sets_kernel(ReduceArgs a) {
   __shared__ float quarter[4][64];
   const int seg = blockIdx.y;
   const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
@@ -1505,7 +1509,7 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs& a, hipStream_t st) {
     r.part[i] = parts[i]; r.out[i] = outs[i]; r.count[i] = counts[i]; r.S[i] = Ss[i];
     if (counts[i] > maxc) maxc = counts[i];
   }
-  reduce4_kernel<<<dim3((maxc + 63) / 64, 4), 256, 0, st>>>(r);
+  reduce_sets_kernel<<<dim3((maxc + 63) / 64, 4), 256, 0, st>>>(r);
   return hipGetLastError();
 }
 
@@ -1830,6 +1834,68 @@ hipError_t grad_one(const float* act, const float* Z, float* part, int D, int N,
   return hipGetLastError();
 }
 
+}  // namespace
+
+// ---- The pass for a whole layer behind an activation: mask and bias gradient in it ----
+// Where the taps run by columns, Cc can be formed from A alone before anything of dy is
+// read; one pass over dy and y then does all that needs dy (bwd_dy_pass.hip).  The partial sets of
+// that pass lie in mask_ws, the room the masked dy would take.
+bool bwd_filter_mfma_masks(const cp4_shape& s) {
+  if (!bwd_filter_mfma_supported(s) || s.C % 16 != 0 || (size_t)s.C * 192 > 160 * 1024) return false;
+  const int HW = (int)(s.H * s.W);
+  if (!bwd_dy_pass_supported((int)s.N, (int)s.T, (int)s.Rank, HW)) return false;
+  const Plan p = make_plan(s.N, s.C, s.T, s.H, s.W, s.Y, s.X, s.Rank, s.pad);
+  const size_t sets = bwd_dy_pass_sets((int)s.N, (int)s.T, HW);
+  return p.column_taps && sets * (s.Rank + 1) <= (size_t)s.N * HW;
+}
+
+hipError_t bwd_filter_mfma_masked_launch(const BwdFilterArgs& a, hipStream_t st) {
+  const int HW = a.H * a.W, R = a.R, N = a.N;
+  const Plan p = make_plan(N, a.C, a.T, a.H, a.W, a.Y, a.X, R, a.pad);
+  float* ws = static_cast<float*>(a.workspace);
+  float *A = ws, *Cc = ws + 2 * p.plane, *G3 = ws + 3 * p.plane, *G1 = ws + 5 * p.plane,
+        *pC = ws + 6 * p.plane;
+  float* pH = pC + (size_t)p.S * a.C * R;
+  float* pW = pH + (size_t)p.St * a.Y * R;
+  const int sets = bwd_dy_pass_sets(N, a.T, HW);
+  float *pK = a.mask_ws, *pB = pK + (size_t)sets * a.T * R;
+  hipError_t e = contract_one(a.x, a.FC, A, a.C, N, R, p.RP, HW, st);
+  if (e != hipSuccess) return e;
+#define CP4_TAPS(PART_)                                                                   \
+  switch (a.Y) {                                                                          \
+    case 1: e = launch_taps_column<1, PART_>(A, G3, a, Cc, G1, pH, pW, st); break;        \
+    case 3: e = launch_taps_column<3, PART_>(A, G3, a, Cc, G1, pH, pW, st); break;        \
+    case 5: e = launch_taps_column<5, PART_>(A, G3, a, Cc, G1, pH, pW, st); break;        \
+    default: e = launch_taps_column<7, PART_>(A, G3, a, Cc, G1, pH, pW, st); break;       \
+  }                                                                                       \
+  if (e != hipSuccess) return e;
+  CP4_TAPS(kTapsCc)
+  e = bwd_dy_pass_launch(a.dy, a.act_y, a.FK, Cc, G3, pK, a.dbias ? pB : nullptr, N, a.T, R, HW, st);
+  if (e != hipSuccess) return e;
+  CP4_TAPS(kTapsRest)
+#undef CP4_TAPS
+  e = grad_one(a.x, G1, pC, a.C, N, R, p, HW, ws, st);
+  if (e != hipSuccess) return e;
+  if (a.dx) {
+    e = rank_expand_launch(a.FC, G1, a.dx, CP4_DTYPE_F32, N, a.C, HW, R, st);
+    if (e != hipSuccess) return e;
+  }
+  ReduceArgs r{};
+  const float* parts[5] = {pK, pC, pH, pW, pB};
+  float* outs[5] = {a.dFK, a.dFC, a.dFH, a.dFW, a.dbias};
+  const int counts[5] = {a.T * R, a.C * R, a.Y * R, a.X * R, a.dbias ? a.T : 0};
+  const int Ss[5] = {sets, p.S, p.St, p.St, sets};
+  int maxc = 0;
+  for (int i = 0; i < 5; ++i) {
+    r.part[i] = parts[i]; r.out[i] = outs[i]; r.count[i] = counts[i]; r.S[i] = Ss[i];
+    if (counts[i] > maxc) maxc = counts[i];
+  }
+  reduce_sets_kernel<<<dim3((maxc + 63) / 64, 5), 256, 0, st>>>(r);
+  return hipGetLastError();
+}
+
+namespace {
+
 struct StridedLayout {
   Plan pf, ps;                                    // plans on the input's and on the output's grid
   size_t A, G1, G3, Cc, pK, pC, pH, pW, total;    // float offsets into the workspace
@@ -1925,7 +1991,7 @@ hipError_t bwd_filter_mfma_strided_launch(const BwdFilterArgs& a, const Geometry
     r.part[i] = parts[i]; r.out[i] = outs[i]; r.count[i] = counts[i]; r.S[i] = Ss[i];
     if (counts[i] > maxc) maxc = counts[i];
   }
-  reduce4_kernel<<<dim3((maxc + 63) / 64, 4), 256, 0, st>>>(r);
+  reduce_sets_kernel<<<dim3((maxc + 63) / 64, 4), 256, 0, st>>>(r);
   return hipGetLastError();
 }
 #endif  // !CP4_BWF_IO16

@@ -1682,19 +1682,24 @@ cp4_status layer_backward_filter(const cp4_shape* s, const cp4_geometry* g, int 
                             workspace_bytes, dtype == CP4_DTYPE_F16, dx, stream);
 }
 
-bool layer_filter_masks(const cp4_shape& s, const float* x, const float* dy, const void* workspace) {
+int layer_filter_masks(const cp4_shape& s, const float* x, const float* y, const float* dy,
+                       const void* workspace, const float* mask_ws, bool want_dx) {
   const uintptr_t bits = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy) |
                          reinterpret_cast<uintptr_t>(workspace);
   const FilterRoutes routes = filter_routes(s, (bits & 7) == 0, (bits & 15) == 0,
                                             (reinterpret_cast<uintptr_t>(workspace) & 255) == 0);
-  return default_filter_variant(s, routes) == 3 && bwd_filter_dense_tiles_masks(s);
+  const int variant = default_filter_variant(s, routes);
+  if (variant == 3) return !want_dx && bwd_filter_dense_tiles_masks(s) ? 3 : 0;
+  return variant == 1 && mask_ws && s.Y == s.X && 2 * s.pad + 1 == s.Y &&
+         ((bits | reinterpret_cast<uintptr_t>(y)) & 15) == 0 && bwd_filter_mfma_masks(s) ? 1 : 0;
 }
 
-cp4_status layer_backward_filter_masked(const cp4_shape* shape, const float* x, const float* act_y,
-                                        const float* dy, const float* FK, const float* FC,
+cp4_status layer_backward_filter_masked(int variant, const cp4_shape* shape, const float* x,
+                                        const float* act_y, const float* dy, const float* FK, const float* FC,
                                         const float* FH, const float* FW, float* dFK, float* dFC,
-                                        float* dFH, float* dFW, float* dbias, float* bias_part,
-                                        void* workspace, size_t workspace_bytes, cp4_stream stream) {
+                                        float* dFH, float* dFW, float* dx, float* dbias,
+                                        float* bias_part, float* mask_ws, void* workspace,
+                                        size_t workspace_bytes, cp4_stream stream) {
   if (!FK || !FC || !FH || !FW || !dFK || !dFC || !dFH || !dFW)
     return fail(CP4_ERR_NULL_POINTER, "a factor or gradient pointer is NULL");
   const cp4_shape& s = *shape;
@@ -1706,8 +1711,10 @@ cp4_status layer_backward_filter_masked(const cp4_shape* shape, const float* x, 
   a.dFK = dFK; a.dFC = dFC; a.dFH = dFH; a.dFW = dFW; a.workspace = workspace;
   a.N = s.N; a.C = s.C; a.T = s.T; a.H = s.H; a.W = s.W; a.pad = s.pad;
   a.Y = s.Y; a.X = s.X; a.R = s.Rank;
-  a.act_y = act_y; a.dbias = dbias; a.bias_part = bias_part;
-  CP4_HIP(bwd_filter_dense_tiles_launch(a, as_stream(stream)));
+  a.dx = dx;
+  a.act_y = act_y; a.dbias = dbias; a.bias_part = bias_part; a.mask_ws = mask_ws;
+  if (variant == 3) CP4_HIP(bwd_filter_dense_tiles_launch(a, as_stream(stream)));
+  else CP4_HIP(bwd_filter_mfma_masked_launch(a, as_stream(stream)));
   return CP4_OK;
 }
 }  // namespace cp4

@@ -90,15 +90,18 @@ cp4_status layer_backward_filter(const cp4_shape*, const cp4_geometry*, int dtyp
                                  const float* FW, float* dFK, float* dFC, float* dFH, float* dFW,
                                  void* workspace, size_t workspace_bytes, void* dx, bool* dx_done,
                                  cp4_stream);
-cp4_status layer_backward_filter_masked(const cp4_shape*, const float* x, const float* act_y,
+cp4_status layer_backward_filter_masked(int variant, const cp4_shape*, const float* x, const float* act_y,
                                         const float* dy, const float* FK, const float* FC,
                                         const float* FH, const float* FW, float* dFK, float* dFC,
-                                        float* dFH, float* dFW, float* dbias, float* bias_part,
-                                        void* workspace, size_t workspace_bytes, cp4_stream);
+                                        float* dFH, float* dFW, float* dx, float* dbias,
+                                        float* bias_part, float* mask_ws, void* workspace,
+                                        size_t workspace_bytes, cp4_stream);
 
-// The factor gradients of an fp32 layer without an input gradient run the dense-gradient
-// route with the mask and the bias gradient in it (x and dy of these addresses).
-bool layer_filter_masks(const cp4_shape&, const float* x, const float* dy, const void* workspace);
+// The backward-filter variant that an fp32 layer's factor gradients (and, want_dx, its input
+// gradient) run with the mask and the bias gradient in it, with operands of these addresses; 0:
+// none does.  mask_ws null: no room for the matrix-core variant's partial sets.
+int layer_filter_masks(const cp4_shape&, const float* x, const float* y, const float* dy,
+                       const void* workspace, const float* mask_ws, bool want_dx);
 
 // Compute units of the current device (256 when no device can be asked).
 int num_compute_units();
@@ -198,11 +201,12 @@ struct BwdFilterArgs {
   // Matrix-core variant only: not null, the input gradient too, dx = FC G1 (in the type of
   // x; the forward's adjoint only where 2 * pad = Y - 1 = X - 1 or with a geometry).
   void* dx;
-  // Dense-gradient variant with bwd_filter_dense_tiles_masks only: dy counts where act_y > 0
-  // (null: everywhere) and dbias[t], its sum over images and pixels, comes along through
-  // bias_part (T floats per compute unit of scratch); all null: neither.
+  // Dense-gradient variant with bwd_filter_dense_tiles_masks and the matrix-core variant's
+  // masked launch only: dy counts where act_y > 0 (null: everywhere) and dbias[t], its sum over
+  // images and pixels, comes along; all null: neither.  Scratch: bias_part, T floats per
+  // compute unit (dense gradient), mask_ws, N * T * H * W floats (matrix cores).
   const float* act_y;
-  float *dbias, *bias_part;
+  float *dbias, *bias_part, *mask_ws;
 };
 // general (VALU, any shape) and matrix-core variants
 size_t bwd_filter_workspace_bytes(const cp4_shape&);
@@ -211,6 +215,16 @@ bool bwd_filter_mfma_supported(const cp4_shape&);
 size_t bwd_filter_mfma_workspace_bytes(const cp4_shape&);
 bool bwd_filter_mfma_taps2d_supported(const cp4_shape&);   // with BwdFilterArgs::taps2d
 hipError_t bwd_filter_mfma_launch(const BwdFilterArgs&, hipStream_t);
+// The same with the layer's activation mask and bias gradient in it (BwdFilterArgs::act_y,
+// dbias, mask_ws); operands on 16-byte boundaries.
+bool bwd_filter_mfma_masks(const cp4_shape&);
+hipError_t bwd_filter_mfma_masked_launch(const BwdFilterArgs&, hipStream_t);
+// One pass over dy: G3, `sets` partial sets [set][T][R] of dFK and [set][T] of dbias.
+bool bwd_dy_pass_supported(int N, int T, int R, int HW);
+int bwd_dy_pass_sets(int N, int T, int HW);
+hipError_t bwd_dy_pass_launch(const float* dy, const float* y, const float* FK, const float* Cc,
+                              float* G3, float* partK, float* partB, int N, int T, int R, int HW,
+                              hipStream_t);
 // Matrix-core variant with the tap step inside the gradient GEMMs (three launches;
 // square odd filters up to 5 with 2 * pad == Y - 1, channel counts multiples of 16,
 // H * W a multiple of 4, x / dy / workspace 16-byte aligned).

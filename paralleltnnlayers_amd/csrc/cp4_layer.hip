@@ -55,8 +55,8 @@ BackwardPlan make_backward_plan(const cp4_shape& s, const cp4_geometry* g, int d
   p.x32_at = take(filter32, nx * 4);
   p.dx32_at = take(dx32, nx * 4);
   const int seg = cp4::act_grad_segments((int)s.N, (int)s.T, ny / ((size_t)s.N * s.T), dtype);
-  p.may_mask = !g && !half && filter && !dx && (act != CP4_ACT_NONE || (wanted & CP4_WANT_BIAS));
-  const size_t parts = p.may_mask ? std::max(seg, cp4::num_compute_units()) : seg > 1 ? seg : 0;
+  p.may_mask = !g && !half && filter && (act != CP4_ACT_NONE || (wanted & CP4_WANT_BIAS));
+  const size_t parts = p.may_mask && !dx ? std::max(seg, cp4::num_compute_units()) : seg > 1 ? seg : 0;
   p.bias_at = take((wanted & CP4_WANT_BIAS) && parts, s.T * parts * 4);
   p.pass_at = at;
   if (g) p.pass_bytes = dx || filter ? cp4_conv2d_backward_ex_workspace_bytes(&s, g) : 0;
@@ -190,13 +190,17 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* g, int
   const void* dya = dy;                                     // in the layer's type
   const float* dy32 = reinterpret_cast<const float*>(ws + p.act32_at);
   float* parts = reinterpret_cast<float*>(ws + p.bias_at);
-  if (p.may_mask && cp4::layer_filter_masks(s, static_cast<const float*>(x),
-                                            static_cast<const float*>(dy), ws + p.pass_at))
-    // a first layer: nothing but the factor gradients reads dy, masked on its way
-    return cp4::layer_backward_filter_masked(
-        shape, static_cast<const float*>(x), static_cast<const float*>(ym),
-        static_cast<const float*>(dy), FK, FC, FH, FW, dFK, dFC, dFH, dFW, dbias, parts,
-        ws + p.pass_at, p.pass_bytes, stream);
+  if (p.may_mask) {
+    // a route that masks dy as it reads it: dy behind the activation never goes to memory
+    const float *xf = static_cast<const float*>(x), *yf = static_cast<const float*>(ym),
+                *dyf = static_cast<const float*>(dy);
+    float* mask_ws = p.act16 ? reinterpret_cast<float*>(ws + p.act16_at) : nullptr;
+    const int variant = cp4::layer_filter_masks(s, xf, yf, dyf, ws + p.pass_at, mask_ws, dx != nullptr);
+    if (variant)
+      return cp4::layer_backward_filter_masked(variant, shape, xf, yf, dyf, FK, FC, FH, FW, dFK, dFC,
+                                               dFH, dFW, static_cast<float*>(dx), dbias, parts, mask_ws,
+                                               ws + p.pass_at, p.pass_bytes, stream);
+  }
   if (p.act16) {
     CP4_LAUNCH(cp4::act_grad_launch(ym, dy, ws + p.act16_at, dtype, false, dbias, parts, N, T, plane, st));
     dya = ws + p.act16_at;

@@ -190,3 +190,34 @@ def test_first_layer_without_an_input_gradient(capi, case, relu):
     # the repository's bar for factor gradients
     for g, w in zip(grads, wants):
         assert (g.double().cpu() - w).abs().max() <= 1e-3 * w.abs().max() + 1e-30
+
+
+# The one pass over dy of large layers: 3, 4 and 8 waves, planes that no chunk of 64 pixels
+# divides, ranks that fill a tile and not, every filter size of the column taps.
+@pytest.mark.parametrize("case", [(33, 32, 46, 54, 96, 5, 32), (24, 16, 64, 64, 128, 3, 16),
+                                  (70, 48, 32, 36, 256, 1, 7), (22, 16, 60, 68, 224, 3, 31),
+                                  (40, 16, 66, 66, 64, 7, 5)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_large_layer_behind_relu(capi, case):
+    N, C, H, W, T, k, R = case
+    gen = torch.Generator(device="cuda").manual_seed(N * H + W + T)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, dy = mk(N, C, H, W), mk(N, T, H, W)
+    fac = [mk(d, R) for d in (T, C, k, k)]
+    s = capi.shape_for(x.shape, *fac, k // 2)
+    y = capi.layer_forward(s, None, x, *fac, mk(T), "relu")
+    dx, grads, dbias = capi.layer_backward(s, None, x, y, dy, *fac, "relu")
+    masked = dy * (y > 0)
+    # against the passes on their own (each checked against float64 elsewhere): fp32 sums in
+    # another order, 2^-24 a step of the sum of the terms' magnitudes as a random walk over the
+    # terms (a factor of four to spare)
+    md = masked.double()
+    tol = 4 * 2.0 ** -24 * ((md ** 2).sum(dim=(0, 2, 3)) * N * H * W).sqrt()
+    assert ((dbias.double() - md.sum(dim=(0, 2, 3))).abs() <= tol).all()
+    want_dx = capi.conv2d_backward_data(masked, *fac, pad=k // 2)
+    terms = capi.conv2d_backward_data(masked.abs(), *[f.abs() for f in fac], pad=k // 2)
+    assert ((dx - want_dx).abs() <= 4 * (T + 2 * k + R) ** 0.5 * 2.0 ** -24 * terms).all()
+    want = capi.conv2d_backward_filter(x, masked, *fac, pad=k // 2)
+    terms = capi.conv2d_backward_filter(x.abs(), masked.abs(), *[f.abs() for f in fac], pad=k // 2)
+    for g, w, t in zip(grads, want, terms):
+        assert ((g - w).abs() <= 4 * 2.0 ** -24 * (N * H * W) ** 0.5 * t).all()
