@@ -17,7 +17,7 @@
 // more, and are added over the waves in order; Cc's fragments are split once a workgroup.  Two
 // barriers a chunk.  dFK and the bias sums stay in registers over a workgroup's contiguous
 // range of chunks: one partial set per workgroup, added in order by the caller's reduction.
-// N32 T256 56x56 R32 (206 MB): @@DYPASS@@.
+// N32 T256 56x56 R32 (206 MB): 60 us on rotating buffers, 3.4 TB/s of rows in 256-byte pieces (64 with the partial sums read one after the other).
 #include <algorithm>
 #include <cstdint>
 
@@ -33,6 +33,7 @@ using split::u32x4;
 constexpr int kPix = 64;                 // pixels of a chunk
 constexpr int kRow = kPix + 4;           // LDS row stride: 16-byte rows, four banks apart
 constexpr int kTile = 32 * kRow;         // floats of a wave's tile
+constexpr int kMaxWaves = 8;           // 256 channels
 constexpr int kFrag = 4 * 3 * 2 * 32;    // 16-byte fragments of a chunk of Cc: [step][part][half][rank]
 
 struct DyPassArgs {
@@ -55,23 +56,38 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
   const unsigned wg = die * per + (die < rest ? die : rest) + (blockIdx.x >> 3);
   const int i0 = (int)((long)a.chunks * wg / gridDim.x), i1 = (int)((long)a.chunks * (wg + 1) / gridDim.x);
 
-  // this wave's rows of FK, split: the contraction's A operand (zero past the last rank)
+  // This wave's rows of FK, split: the contraction's A operand (zero past the last rank).  Every
+  // other wave takes them with the sign reversed and its partial sums are subtracted: the matrix
+  // cores' sums come out low by a few hundredths of a unit in the last place whatever their sign, which
+  // a sum over all pixels into the nearly cancelling factor gradients brings to the front
+  // (N32 T256 56x56 R32: G3's mean error 1.9e-8 of its deviation, 4e-11 with the signs
+  // reversed, 6.9e-9 in the contraction kernel; dFC 3.8e-6 of its norm off, 4.7e-7 with them, 1.6e-6).
+  const float sign = wave & 1 ? -1.f : 1.f;
   u32x4 fh[2], fm[2], fl[2];
 #pragma unroll
   for (int ch = 0; ch < 2; ++ch) {
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e)
-      v[e] = l32 < R ? a.FK[(size_t)(c0 + 16 * ch + 8 * hi + e) * R + l32] : 0.f;
+      v[e] = l32 < R ? sign * a.FK[(size_t)(c0 + 16 * ch + 8 * hi + e) * R + l32] : 0.f;
     split::split8(v, fh[ch], fm[ch], fl[ch]);
   }
 
   // ---- loads: row 4 j + lane / 16 of the wave's channels, four pixels a lane ----
   const int lrow = lane >> 4, lcol = 4 * (lane & 15);
   float4 dv[8], yv[MASK ? 8 : 1], zv[KZ][2];
+  // (clamped, not branched; values outside are dropped where they are used.  Cc's first: its
+  // fragments are made before the rows are waited for)
   auto load = [&](int i) {
     const int n = i / a.cpi;
     const int p0 = (i - n * a.cpi) * kPix;
+#pragma unroll
+    for (int k = 0; k < KZ; ++k) {
+      const int it = (threadIdx.x + k * blockDim.x) & 255, zr = it >> 3, pz = p0 + 8 * (it & 7);
+      const float* z = a.Cc + ((size_t)n * R + (zr < R ? zr : 0)) * HW;
+      zv[k][0] = *reinterpret_cast<const float4*>(z + (pz < HW ? pz : 0));
+      zv[k][1] = *reinterpret_cast<const float4*>(z + (pz + 4 < HW ? pz + 4 : 0));
+    }
     const int p = p0 + lcol;
     const size_t at = ((size_t)n * T + c0 + lrow) * HW + (p < HW ? p : 0);
 #pragma unroll
@@ -79,24 +95,17 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
       dv[j] = *reinterpret_cast<const float4*>(a.dy + at + (size_t)(4 * j) * HW);
       if constexpr (MASK) yv[j] = *reinterpret_cast<const float4*>(a.y + at + (size_t)(4 * j) * HW);
     }
-#pragma unroll
-    for (int k = 0; k < KZ; ++k) {
-      const int it = threadIdx.x + k * blockDim.x, zr = it >> 3, pz = p0 + 8 * (it & 7);
-      const bool in = it < 256 && zr < R;
-      const float* z = a.Cc + ((size_t)n * R + (in ? zr : 0)) * HW;
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        zv[k][h] = in && pz + 4 * h < HW ? *reinterpret_cast<const float4*>(z + pz + 4 * h)
-                                         : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
   };
-  auto deposit_z = [&] {
+  auto deposit_z = [&](int i) {
 #pragma unroll
     for (int k = 0; k < KZ; ++k) {
-      const int it = threadIdx.x + k * blockDim.x, zr = it >> 3, zo = it & 7;
+      const int it = threadIdx.x + k * blockDim.x, zr = (it >> 3) & 31, zo = it & 7;
+      const int pz = (i % a.cpi) * kPix + 8 * zo;
+      const bool in0 = zr < R && pz < HW, in1 = zr < R && pz + 4 < HW;
+      const float v[8] = {in0 ? zv[k][0].x : 0.f, in0 ? zv[k][0].y : 0.f, in0 ? zv[k][0].z : 0.f,
+                          in0 ? zv[k][0].w : 0.f, in1 ? zv[k][1].x : 0.f, in1 ? zv[k][1].y : 0.f,
+                          in1 ? zv[k][1].z : 0.f, in1 ? zv[k][1].w : 0.f};
       if (it < 256) {
-        const float v[8] = {zv[k][0].x, zv[k][0].y, zv[k][0].z, zv[k][0].w,
-                            zv[k][1].x, zv[k][1].y, zv[k][1].z, zv[k][1].w};
         u32x4 h, m, l;
         split::split8(v, h, m, l);
         u32x4* dst = Zf + ((zo >> 1) * 6 + (zo & 1)) * 32 + zr;
@@ -112,7 +121,7 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
   for (int j = 0; j < 8; ++j) bs[j] = 0.f;
   if (i0 < i1) {
     load(i0);
-    deposit_z();
+    deposit_z(i0);
   }
   __syncthreads();
   for (int i = i0; i < i1; ++i) {
@@ -152,16 +161,25 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
     f32x16 accG[2];
 #pragma unroll
     for (int pb = 0; pb < 2; ++pb) {
-      accG[pb] = (f32x16)(0.f);
+      // (the small partial products of both channel chunks before the large ones, so that most
+      //  of the chain's roundings are small)
+      f32x16 g = (f32x16)(0.f);
+      u32x4 bh[2];
 #pragma unroll
       for (int ch = 0; ch < 2; ++ch) {
         float v[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = tile[(16 * ch + 8 * hi + e) * kRow + 32 * pb + l32];
-        u32x4 bh, bm, bl;
-        split::split8(v, bh, bm, bl);
-        accG[pb] = split::mfma_split(fh[ch], fm[ch], fl[ch], bh, bm, bl, accG[pb]);
+        u32x4 bm, bl;
+        split::split8(v, bh[ch], bm, bl);
+        g = split::mfma16(fl[ch], bh[ch], g);
+        g = split::mfma16(fm[ch], bm, g);
+        g = split::mfma16(fh[ch], bl, g);
+        g = split::mfma16(fm[ch], bh[ch], g);
+        g = split::mfma16(fh[ch], bm, g);
       }
+      g = split::mfma16(fh[0], bh[0], g);
+      accG[pb] = split::mfma16(fh[1], bh[1], g);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -171,13 +189,18 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
       for (int v = 0; v < 16; ++v) tile[(16 * pb + v) * 64 + lane] = accG[pb][v];
     __syncthreads();              // partial sums complete; Cc's fragments read by every wave
     for (int k = wave; k < 32; k += waves) {
-      float s = 0.f;
-      for (int w = 0; w < waves; ++w) s += lds[w * kTile + k * 64 + lane];
+      // (all of an entry's reads together: one after the other they were 6 us of the kernel)
+      float t[kMaxWaves], s = 0.f;
+#pragma unroll
+      for (int w = 0; w < kMaxWaves; ++w) t[w] = lds[(w < waves ? w : 0) * kTile + k * 64 + lane];
+#pragma unroll
+      for (int w = 0; w < kMaxWaves; ++w)
+        if (w < waves) s = w & 1 ? s - t[w] : s + t[w];
       const int v = k & 15, r = 8 * (v >> 2) + 4 * hi + (v & 3);
       const int p = p0 + 32 * (k >> 4) + l32;
       if (r < R && p < HW) a.G3[((size_t)n * R + r) * HW + p] = s;
     }
-    if (i + 1 < i1) deposit_z();
+    if (i + 1 < i1) deposit_z(i + 1);
     __syncthreads();              // tiles free, the next chunk's fragments complete
   }
   // ---- one partial set per workgroup ----

@@ -1220,7 +1220,7 @@ struct ReduceArgs {
   int count[5], S[5];
 };
 // A workgroup owns 64 consecutive outputs; its four waves each sum a quarter of
-// the S partials in index order (eight loads in flight), then the four quarter
+// the S partials in index order (eight loads in flight, added as a tree), then the four quarter
 // sums are added in wave order: the result does not depend on timing.
 __global__ __launch_bounds__(256) void reduce_sets_kernel(ReduceArgs a) {
   __shared__ float quarter[4][64];
@@ -1240,7 +1240,8 @@ __global__ __launch_bounds__(256) void reduce_sets_kernel(ReduceArgs a) {
 #pragma unroll
       for (int u = 0; u < 8; ++u) v[u] = p[(size_t)(k + u) * stride];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) s += v[u];
+      for (int u = 0; u < 4; ++u) v[u] += v[u + 4];
+      s += (v[0] + v[2]) + (v[1] + v[3]);
     }
     for (; k < k1; ++k) s += p[(size_t)k * stride];
   }
