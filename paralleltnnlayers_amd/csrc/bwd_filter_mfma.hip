@@ -757,9 +757,12 @@ hipError_t launch_taps_wave(const float* A, const float* G3, const BwdFilterArgs
 // Step t completes B and Cc on row t-(FS-1-P), G2 on row t, G1 on row t-P and
 // the tap-gradient terms of row t-(FS-1-P).  Needs P <= FS-1.
 // Part of the work (kTaps...): Cc alone, from A alone, or everything but Cc.
+// CENTRED (P = (FS - 1) / 2, "same" padding): the neighbours come by lane shifts on the vector
+// ALU instead of shuffles through the LDS unit, whose latency twice a row was most of the walk
+// (N32 56x56 R32, everything but Cc: 15.2 -> 14.1 us; N32 28x28 R16, all of it: 7.8 -> 7.2).
 enum { kTapsAll, kTapsCc, kTapsRest };
 constexpr int kRowsAhead = 8;
-template <int FS, int PART>
+template <int FS, int PART, bool CENTRED>
 __global__ __launch_bounds__(256) void taps_column_kernel(
     const float* __restrict__ A, const float* __restrict__ G3, const float* __restrict__ FH,
     const float* __restrict__ FW, float* __restrict__ Cc, float* __restrict__ G1,
@@ -803,6 +806,25 @@ __global__ __launch_bounds__(256) void taps_column_kernel(
     srcf[j] = okf[j] ? wf : 0;
     srcb[j] = okb[j] ? wb : 0;
   }
+  // out[j] = lane + j - P's value of v (lane - j + P's with `adjoint`); callers mask what falls
+  // outside
+  auto neighbours = [&](float v, float (&out)[FS], bool adjoint) {
+    if constexpr (CENTRED) {
+      constexpr int M = (FS - 1) / 2;
+      float left = v, right = v;                   // k lanes below / above
+      out[M] = v;
+#pragma unroll
+      for (int k = 1; k <= M; ++k) {
+        left = dpp_move<0x138, 0xf, true>(left);     // wave_shr:1
+        right = dpp_move<0x130, 0xf, true>(right);   // wave_shl:1
+        out[adjoint ? M + k : M - k] = left;
+        out[adjoint ? M - k : M + k] = right;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < FS; ++j) out[j] = __shfl(v, adjoint ? srcb[j] : srcf[j], 64);
+    }
+  };
   float aw[FS], gw[FS], g2w[FS];                   // rows t-FS+1 .. t of A, G3, G2
 #pragma unroll
   for (int i = 0; i < FS; ++i) aw[i] = gw[i] = g2w[i] = 0.f;
@@ -828,12 +850,12 @@ __global__ __launch_bounds__(256) void taps_column_kernel(
         request(u, t + kRowsAhead);
         // G2 row t: horizontal adjoint taps of G3 row t
         float g2_t = 0.f;
-        if constexpr (PART != kTapsCc)
+        if constexpr (PART != kTapsCc) {
+          float v[FS];
+          neighbours(g_t, v, true);
 #pragma unroll
-          for (int j = 0; j < FS; ++j) {
-            const float v = __shfl(g_t, srcb[j], 64);
-            g2_t += okb[j] ? fw[j] * v : 0.f;
-          }
+          for (int j = 0; j < FS; ++j) g2_t += okb[j] ? fw[j] * v[j] : 0.f;
+        }
 #pragma unroll
         for (int i = 0; i + 1 < FS; ++i) {
           aw[i] = aw[i + 1];
@@ -849,11 +871,11 @@ __global__ __launch_bounds__(256) void taps_column_kernel(
           float b = 0.f;
 #pragma unroll
           for (int i = 0; i < FS; ++i) b += fh[i] * aw[i];
-          float cc = 0.f;
+          float cc = 0.f, v[FS];
+          neighbours(b, v, false);
 #pragma unroll
           for (int j = 0; j < FS; ++j) {
-            const float v = __shfl(b, srcf[j], 64);
-            const float bj = okf[j] ? v : 0.f;
+            const float bj = okf[j] ? v[j] : 0.f;
             cc += fw[j] * bj;
             accW[j] += mine ? gw[P] * bj : 0.f;     // G3[hb][w] * B[hb][w+j-P]
           }
@@ -876,13 +898,10 @@ __global__ __launch_bounds__(256) void taps_column_kernel(
   if constexpr (PART == kTapsCc) return;
 #pragma unroll
   for (int i = 0; i < FS; ++i) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      accH[i] += __shfl_down(accH[i], off, 64);
-      accW[i] += __shfl_down(accW[i], off, 64);
-    }
+    accH[i] = wave_sum_to_lane63(accH[i]);
+    accW[i] = wave_sum_to_lane63(accW[i]);
   }
-  if (lane == 0) {
+  if (lane == 63) {
 #pragma unroll
     for (int i = 0; i < FS; ++i) {
       partH[((((size_t)n * segs + seg) * rsegs + rseg) * FS + i) * R + r] = accH[i];
@@ -919,8 +938,9 @@ hipError_t launch_taps_column(const float* A, const float* G3, const BwdFilterAr
   const int RH = column_row_height(a.N, a.R, a.H, a.W, FS, a.pad);
   const int rsegs = (a.H + RH - 1) / RH;
   const long units = (long)nplanes * segs * rsegs;
-  taps_column_kernel<FS, PART><<<(unsigned)((units + 3) / 4), 256, 0, st>>>(
-      A, G3, a.FH, a.FW, Cc, G1, pH, pW, a.R, a.H, a.W, a.pad, nplanes, segs, Q, rsegs, RH);
+  auto k = 2 * a.pad == FS - 1 ? taps_column_kernel<FS, PART, true> : taps_column_kernel<FS, PART, false>;
+  k<<<(unsigned)((units + 3) / 4), 256, 0, st>>>(A, G3, a.FH, a.FW, Cc, G1, pH, pW, a.R, a.H, a.W,
+                                                 a.pad, nplanes, segs, Q, rsegs, RH);
   return hipGetLastError();
 }
 
@@ -1649,7 +1669,15 @@ __global__ __launch_bounds__(256) void taps_strided_fast_kernel(
 #pragma unroll 4
       for (int k = threadIdx.x; k < (n >> 2); k += 256) d4[k] = s4[k];
     } else {
-      for (int k = threadIdx.x; k < n; k += 256) dst[k] = src[k];
+      // (eight loads in flight a thread: one by one a plane of 55 x 55 waited twelve times: N16 C128 K256 R32 stride 2 17.5 -> 15.8 us)
+      for (int k0 = threadIdx.x; k0 < n; k0 += 8 * 256) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = src[k0 + 256 * u < n ? k0 + 256 * u : n - 1];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (k0 + 256 * u < n) dst[k0 + 256 * u] = v[u];
+      }
     }
   };
   stage(sA, A + basef, HW);
