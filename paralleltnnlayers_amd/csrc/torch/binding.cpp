@@ -313,6 +313,16 @@ int activation_of(PyObject* o) {
   throw python_error();
 }
 
+// Python's o == 1.
+bool equals_one(PyObject* o) {
+  if (PyLong_Check(o)) return integer(o) == 1;
+  PyObject* one = PyLong_FromLong(1);
+  const int eq = one ? PyObject_RichCompareBool(o, one, Py_EQ) : -1;
+  Py_XDECREF(one);
+  if (eq < 0) throw python_error();
+  return eq != 0;
+}
+
 // An int or a pair of ints.
 void int_pair(PyObject* o, long* h, long* w) {
   if (PyLong_Check(o)) {
@@ -342,18 +352,18 @@ PyObject* layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   PyObject* padding = a[9] == Py_None ? a[5] : a[9];
   const bool same = PyUnicode_Check(padding) && PyUnicode_CompareWithASCIIString(padding, "same") == 0;
   const bool valid = PyUnicode_Check(padding) && PyUnicode_CompareWithASCIIString(padding, "valid") == 0;
-  long sh, sw;
-  int_pair(a[8], &sh, &sw);
   l.shape = shape_for(x_in, f, 0);
   const long Y = l.shape.Y, X = l.shape.X;
-  // the reference's own layer runs its three passes as they are
-  bool plain = PyLong_Check(a[8]) && sh == 1 && Y == X;
+  // the reference's own layer runs its three passes as they are (whatever number says stride 1)
+  bool plain = equals_one(a[8]) && Y == X;
   if (plain && PyLong_Check(padding)) plain = 2 * integer(padding) + 1 == Y;
   else plain = plain && same && Y % 2 == 1;
   if (plain) {
     l.shape.pad = (unsigned)(Y / 2);
   } else {
     l.has_geometry = true;
+    long sh, sw;
+    int_pair(a[8], &sh, &sw);
     if (same) {
       check(cp4_geometry_same(&l.shape, (unsigned)sh, (unsigned)sw, &l.geometry));
     } else if (valid) {
