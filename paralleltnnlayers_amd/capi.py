@@ -483,6 +483,13 @@ def _ptr_any(t):
     return ctypes.c_void_p(t.data_ptr())
 
 
+def _check_layer(s, x, FK, FC, FH, FW):
+    """x and the factors of a layer hold what the kernels read for shape s."""
+    assert tuple(x.shape) == (s.N, s.C, s.H, s.W)
+    assert all(f.numel() >= rows * s.Rank
+               for f, rows in ((FK, s.T), (FC, s.C), (FH, s.Y), (FW, s.X)))
+
+
 def _scratch(nbytes, device):
     """`nbytes` of device memory (the allocator's blocks start on 512-byte boundaries)."""
     return torch.empty(nbytes, device=device, dtype=torch.uint8) if nbytes else None
@@ -491,6 +498,8 @@ def _scratch(nbytes, device):
 def layer_forward(s, g, x, FK, FC, FH, FW, bias=None, activation=None, stream=None):
     """y = act(conv(x) + bias) in x's element type; g: a Geometry or None."""
     dtype = _DTYPES[x.dtype]
+    _check_layer(s, x, FK, FC, FH, FW)
+    assert bias is None or bias.numel() >= s.T
     gp = ctypes.byref(g) if g is not None else None
     oh, ow = (g.out_h, g.out_w) if g is not None else (s.H, s.W)
     y = torch.empty((s.N, s.T, oh, ow), device=x.device, dtype=x.dtype)
@@ -506,6 +515,10 @@ def layer_backward(s, g, x, y, dy, FK, FC, FH, FW, activation=None, want_dx=True
                    want_factors=True, want_bias=True, stream=None):
     """(dx, (dFK, dFC, dFH, dFW), dbias) of layer_forward, None where not wanted."""
     dtype, act = _DTYPES[x.dtype], ACTIVATIONS[activation]
+    _check_layer(s, x, FK, FC, FH, FW)
+    out = (s.N, s.T) + ((g.out_h, g.out_w) if g is not None else (s.H, s.W))
+    assert dy.dtype == x.dtype and tuple(dy.shape) == out
+    assert act == 0 or y is None or (y.dtype == x.dtype and tuple(y.shape) == out)
     gp = ctypes.byref(g) if g is not None else None
     dx = torch.empty_like(x) if want_dx else None
     grads = [torch.empty_like(f) if want_factors else None for f in (FK, FC, FH, FW)]

@@ -25,3 +25,60 @@ def test_stride_forms_that_are_taken(stride):
 def test_stride_forms_that_are_refused(stride, padding):
     with pytest.raises((TypeError, ValueError)):
         _layer(stride, padding)
+
+
+class _OnDevice(torch.Tensor):
+    """A host tensor that says it is on the device."""
+    is_cuda = True
+
+
+class _Reached(Exception):
+    pass
+
+
+@pytest.fixture()
+def layer_calls(monkeypatch):
+    """capi's layer functions down to the library call, which raises _Reached."""
+    from paralleltnnlayers_amd import capi
+
+    class Lib:
+        def __getattr__(self, name):
+            def call(*args):
+                if name.endswith("workspace_bytes"):
+                    return 0
+                raise _Reached(name)
+            return call
+
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: empty(*a, **k).as_subclass(_OnDevice))
+    monkeypatch.setattr(capi, "lib", lambda: Lib())
+    monkeypatch.setattr(capi, "_stream", lambda stream: None)
+    return capi
+
+
+def _on_device(*shape, dtype=torch.float32):
+    return torch.zeros(*shape, dtype=dtype).as_subclass(_OnDevice)
+
+
+@pytest.mark.parametrize("fault", [None, "dy type", "dy shape", "y type", "y shape", "x shape", "FH",
+                                   "bias"])
+def test_layer_calls_check_types_and_sizes(layer_calls, fault):
+    """An operand of another type or size than the layer's never reaches the library, whose
+    kernels would read past its end."""
+    capi = layer_calls
+    f32, bf16 = torch.float32, torch.bfloat16
+    x = _on_device(2, 4, 5, 7)
+    y = _on_device(2, 6, 5, 7 if fault != "y shape" else 6, dtype=bf16 if fault == "y type" else f32)
+    dy = _on_device(2, 6, 5, 7 if fault != "dy shape" else 6, dtype=bf16 if fault == "dy type" else f32)
+    fac = [_on_device(6, 3), _on_device(4, 3), _on_device(3, 2 if fault == "FH" else 3), _on_device(3, 3)]
+    s = capi.shape_for(x.shape, *fac, 1)
+    if fault == "x shape":
+        x = _on_device(2, 3, 5, 7)
+    backward = lambda: capi.layer_backward(s, None, x, y, dy, *fac, "relu", want_bias=False)
+    with pytest.raises(_Reached if fault in (None, "bias") else AssertionError):
+        backward()
+    if fault in ("dy type", "dy shape", "y type", "y shape"):
+        return
+    bias = _on_device(6 if fault != "bias" else 5)
+    with pytest.raises(_Reached if fault is None else AssertionError):
+        capi.layer_forward(s, None, x, *fac, bias, "relu")
