@@ -2,9 +2,12 @@
 
 Device memory and streams come from PyTorch (ROCm): every tensor argument must
 be a contiguous float32 CUDA(-HIP) tensor; its ``data_ptr()`` is what crosses
-the C ABI.  Launches go on torch's current stream unless ``stream`` is given.
+the C ABI.  Launches go on torch's current stream unless ``stream`` is given;
+what such a call allocates then belongs to ``stream``.
 """
 import ctypes
+import functools
+import inspect
 import os
 
 import torch
@@ -231,6 +234,42 @@ def _stream(stream):
     return ctypes.c_void_p(stream.cuda_stream)
 
 
+def _ordered(stream, fn, /, *args, **kw):
+    """fn(...), which allocates and launches on ``stream``, with ``stream`` current: what it
+    allocates comes from that stream's memory, so nothing queued on another stream still
+    uses it, and its scratch is not reused before the launch on ``stream`` is through.  The
+    tensors it returns may be used and dropped on the caller's current stream too."""
+    if not isinstance(stream, torch.cuda.Stream):
+        stream = torch.cuda.ExternalStream(stream.cuda_stream)
+    callers = torch.cuda.current_stream(stream.device)
+    if stream == callers:
+        return fn(*args, **kw)
+    with torch.cuda.stream(stream):
+        result = fn(*args, **kw)
+    todo = [result]
+    while todo:
+        t = todo.pop()
+        if isinstance(t, torch.Tensor):
+            t.record_stream(callers)
+        elif isinstance(t, (tuple, list)):
+            todo.extend(t)
+    return result
+
+
+def _stream_ordered(fn):
+    """A function that allocates and takes a ``stream``: see _ordered."""
+    at = list(inspect.signature(fn).parameters).index("stream")
+
+    @functools.wraps(fn)
+    def call(*args, **kw):
+        stream = args[at] if len(args) > at else kw.get("stream")
+        if stream is None:
+            return fn(*args, **kw)
+        return _ordered(stream, fn, *args, **kw)
+
+    return call
+
+
 def shape_for(x_or_dy_shape, FK, FC, FH, FW, pad):
     """tensor_shape as CP::Conv2dForward / Conv2dBackwardData derive it
     (Cuda_kernels/cp4Conv2d.cu:21-30, 55-64): N,H,W from the activation, T and
@@ -241,12 +280,15 @@ def shape_for(x_or_dy_shape, FK, FC, FH, FW, pad):
 
 
 def conv2d_forward(x, FK, FC, FH, FW, pad=1, out=None, variant=-1, stream=None):
-    return _native.forward(x, FK, FC, FH, FW, pad, out, variant, stream)
+    if stream is None or out is not None:              # (allocates y only)
+        return _native.forward(x, FK, FC, FH, FW, pad, out, variant, stream)
+    return _ordered(stream, _native.forward, x, FK, FC, FH, FW, pad, out, variant, stream)
 
 
 ACTIVATIONS = {None: 0, "none": 0, "relu": 1}
 
 
+@_stream_ordered
 def conv2d_forward_bias_act(x, FK, FC, FH, FW, bias=None, activation=None, pad=1, out=None,
                             stream=None):
     """y = act(conv(x) + bias[t]) with the epilogue fused into the stores."""
@@ -278,6 +320,7 @@ def geometry(s, stride=1, padding="same"):
     return g
 
 
+@_stream_ordered
 def conv2d_forward_ex(x, FK, FC, FH, FW, g, bias=None, activation=None, out=None, stream=None):
     """Forward with a stride / explicit padding / an output plane of its own."""
     s = shape_for(x.shape, FK, FC, FH, FW, 0)
@@ -304,6 +347,7 @@ def _ex_workspace(s, g, device, workspace):
     return workspace, workspace.numel() * workspace.element_size()
 
 
+@_stream_ordered
 def conv2d_backward_data_ex(dy, x_hw, FK, FC, FH, FW, g, out=None, workspace=None, stream=None):
     """dx [N,C,H,W] of the layer with geometry g for dy [N,T,out_h,out_w]; x_hw = (H, W)."""
     N, T = dy.shape[:2]
@@ -319,6 +363,7 @@ def conv2d_backward_data_ex(dy, x_hw, FK, FC, FH, FW, g, out=None, workspace=Non
     return dx
 
 
+@_stream_ordered
 def conv2d_backward_filter_ex(x, dy, FK, FC, FH, FW, g, workspace=None, stream=None):
     """(dFK, dFC, dFH, dFW) of the layer with geometry g."""
     s = shape_for(x.shape, FK, FC, FH, FW, 0)
@@ -336,6 +381,7 @@ def _ptr16(t, dtype=torch.bfloat16):
     return ctypes.c_void_p(t.data_ptr())
 
 
+@_stream_ordered
 def conv2d_forward_f16(x, FK, FC, FH, FW, bias=None, activation=None, pad=1, out=None,
                        stream=None):
     """float16 x -> float16 y = act(conv(x) + bias); fp32 factors, bias and arithmetic."""
@@ -350,6 +396,7 @@ def conv2d_forward_f16(x, FK, FC, FH, FW, bias=None, activation=None, pad=1, out
     return y
 
 
+@_stream_ordered
 def conv2d_backward_data_f16(dy, FK, FC, FH, FW, pad=1, out=None, stream=None):
     """float16 dy -> float16 dx; fp32 factors and arithmetic."""
     s = shape_for(dy.shape, FK, FC, FH, FW, pad)
@@ -376,6 +423,7 @@ def _rcp_workspace(s, d, device):
     return torch.empty(n + 256, device=device, dtype=torch.uint8), n + 256
 
 
+@_stream_ordered
 def rcp_conv2d_forward(x, K0, K1, KC, pad=1, out=None, stream=None):
     """Reshaped-CP op: x [N,S0*S1,H,W], K0 [S0,T0,R], K1 [S1,T1,R], KC [Y,X,R] -> [N,T0*T1,H,W]."""
     s, d = _rcp_shape(x.shape, K0, K1, KC, pad)
@@ -389,6 +437,7 @@ def rcp_conv2d_forward(x, K0, K1, KC, pad=1, out=None, stream=None):
     return y
 
 
+@_stream_ordered
 def rcp_conv2d_backward_data(dy, K0, K1, KC, pad=1, out=None, stream=None):
     s, d = _rcp_shape(dy.shape, K0, K1, KC, pad)
     assert dy.shape[1] == s.T
@@ -401,6 +450,7 @@ def rcp_conv2d_backward_data(dy, K0, K1, KC, pad=1, out=None, stream=None):
     return dx
 
 
+@_stream_ordered
 def rcp_conv2d_backward_filter(x, dy, K0, K1, KC, pad=1, stream=None):
     """(dK0, dK1, dKC)."""
     s, d = _rcp_shape(x.shape, K0, K1, KC, pad)
@@ -421,6 +471,7 @@ def bf16_backward_filter_supported(s):
     return bool(lib().cp4_bf16_backward_filter_supported(ctypes.byref(s)))
 
 
+@_stream_ordered
 def conv2d_forward_bf16(x, FK, FC, FH, FW, bias=None, activation=None, pad=1, out=None,
                         stream=None):
     """bfloat16 x -> bfloat16 y = act(conv(x) + bias); fp32 factors, bias and arithmetic."""
@@ -436,6 +487,7 @@ def conv2d_forward_bf16(x, FK, FC, FH, FW, bias=None, activation=None, pad=1, ou
     return y
 
 
+@_stream_ordered
 def conv2d_backward_data_bf16(dy, FK, FC, FH, FW, pad=1, out=None, stream=None):
     """bfloat16 dy -> bfloat16 dx; fp32 factors and arithmetic."""
     s = shape_for(dy.shape, FK, FC, FH, FW, pad)
@@ -447,6 +499,7 @@ def conv2d_backward_data_bf16(dy, FK, FC, FH, FW, pad=1, out=None, stream=None):
     return dx
 
 
+@_stream_ordered
 def conv2d_backward_filter_bf16(x, dy, FK, FC, FH, FW, pad=1, workspace=None, stream=None):
     """bfloat16 x, dy -> fp32 (dFK, dFC, dFH, dFW); fp32 factors and arithmetic."""
     s = shape_for(x.shape, FK, FC, FH, FW, pad)
@@ -459,6 +512,7 @@ def conv2d_backward_filter_bf16(x, dy, FK, FC, FH, FW, pad=1, workspace=None, st
     return tuple(outs)
 
 
+@_stream_ordered
 def conv2d_backward_filter_f16(x, dy, FK, FC, FH, FW, pad=1, workspace=None, stream=None):
     """float16 x, dy -> fp32 (dFK, dFC, dFH, dFW); fp32 factors and arithmetic."""
     s = shape_for(x.shape, FK, FC, FH, FW, pad)
@@ -495,6 +549,7 @@ def _scratch(nbytes, device):
     return torch.empty(nbytes, device=device, dtype=torch.uint8) if nbytes else None
 
 
+@_stream_ordered
 def layer_forward(s, g, x, FK, FC, FH, FW, bias=None, activation=None, stream=None):
     """y = act(conv(x) + bias) in x's element type; g: a Geometry or None."""
     dtype = _DTYPES[x.dtype]
@@ -511,6 +566,7 @@ def layer_forward(s, g, x, FK, FC, FH, FW, bias=None, activation=None, stream=No
     return y
 
 
+@_stream_ordered
 def layer_backward(s, g, x, y, dy, FK, FC, FH, FW, activation=None, want_dx=True,
                    want_factors=True, want_bias=True, stream=None):
     """(dx, (dFK, dFC, dFH, dFW), dbias) of layer_forward, None where not wanted."""
@@ -535,7 +591,9 @@ def layer_backward(s, g, x, y, dy, FK, FC, FH, FW, activation=None, want_dx=True
 
 
 def conv2d_backward_data(dy, FK, FC, FH, FW, pad=1, out=None, stream=None):
-    return _native.backward_data(dy, FK, FC, FH, FW, pad, out, stream)
+    if stream is None or out is not None:              # (allocates dx only)
+        return _native.backward_data(dy, FK, FC, FH, FW, pad, out, stream)
+    return _ordered(stream, _native.backward_data, dy, FK, FC, FH, FW, pad, out, stream)
 
 
 def backward_filter_workspace_bytes(s):
@@ -555,7 +613,10 @@ def _workspace(s, device, workspace):
 def conv2d_backward_filter(x, dy, FK, FC, FH, FW, pad=1, workspace=None, stream=None,
                            variant=-1):
     """Returns (dFK, dFC, dFH, dFW)."""
-    return _native.backward_filter(x, dy, FK, FC, FH, FW, pad, workspace, stream, variant)
+    if stream is None:
+        return _native.backward_filter(x, dy, FK, FC, FH, FW, pad, workspace, stream, variant)
+    return _ordered(stream, _native.backward_filter, x, dy, FK, FC, FH, FW, pad, workspace, stream,
+                    variant)
 
 
 def conv2d_backward_filter_noalloc(x, dy, FK, FC, FH, FW, outs, pad=1, stream=None):
@@ -569,6 +630,7 @@ def conv2d_backward_filter_noalloc(x, dy, FK, FC, FH, FW, outs, pad=1, stream=No
     return tuple(outs)
 
 
+@_stream_ordered
 def conv2d_backward_filter_full(x, dy, Y, X, pad=1, out=None, stream=None):
     N, C, H, W = x.shape
     s = Shape(N=N, H=H, W=W, pad=pad, T=dy.shape[1], C=C, Y=Y, X=X, Rank=0)
@@ -614,6 +676,7 @@ def time_backward_data(dy, FK, FC, FH, FW, dx, pad, warmup=1, profcount=47, stre
     return us.value
 
 
+@_stream_ordered
 def time_backward_filter(x, dy, FK, FC, FH, FW, pad, warmup=1, profcount=47,
                          workspace=None, stream=None):
     s = shape_for(x.shape, FK, FC, FH, FW, pad)
@@ -663,6 +726,7 @@ def tune_backward_data(dy, FK, FC, FH, FW, dx, pad, warmup=1, profcount=10, stre
     return best.value, us.value
 
 
+@_stream_ordered
 def tune_backward_filter(x, dy, FK, FC, FH, FW, pad, warmup=1, profcount=10, workspace=None,
                          stream=None):
     """(best variant: 0 general / 1 matrix cores in four launches / 2 with the tap step
@@ -813,6 +877,7 @@ def set_backward_filter_tile_kernel(which):
     lib().cp4_set_backward_filter_tile_kernel(int(which))
 
 
+@_stream_ordered
 def recompose(FK, FC, FH, FW, stream=None):
     s = Shape(T=FK.shape[0], C=FC.shape[0], Y=FH.shape[0], X=FW.shape[0], Rank=FK.shape[1])
     K = torch.empty((s.T, s.C, s.Y, s.X), device=FK.device, dtype=torch.float32)
@@ -830,6 +895,7 @@ def cp3_shape_for(x_shape, K0, K1, K2, pad):
                  X=K1.shape[1], Rank=K0.shape[1])
 
 
+@_stream_ordered
 def cp3_expand_factors(K0, K1, K2, stream=None):
     """The CP4 factors (FK, FC, FH, FW) of rank Y*R that compute the same convolution."""
     s = cp3_shape_for((0, 0, 1, 1), K0, K1, K2, 0)
@@ -841,6 +907,7 @@ def cp3_expand_factors(K0, K1, K2, stream=None):
     return tuple(out)
 
 
+@_stream_ordered
 def cp3_fold_gradients(dFK, dFC, dFW, Y, stream=None):
     """(dK0, dK1, dK2) from the gradients of the expanded CP4 factors."""
     Q = dFK.shape[1]
@@ -864,6 +931,7 @@ def _cp3_pass(fn, s, src, K0, K1, K2, dst, workspace, stream):
     return dst
 
 
+@_stream_ordered
 def cp3_conv2d_forward(x, K0, K1, K2, pad=1, out=None, workspace=None, stream=None):
     s = cp3_shape_for(x.shape, K0, K1, K2, pad)
     assert x.shape[1] == s.C
@@ -872,6 +940,7 @@ def cp3_conv2d_forward(x, K0, K1, K2, pad=1, out=None, workspace=None, stream=No
     return _cp3_pass(lib().cp3_conv2d_forward, s, x, K0, K1, K2, y, workspace, stream)
 
 
+@_stream_ordered
 def cp3_conv2d_backward_data(dy, K0, K1, K2, pad=1, out=None, workspace=None, stream=None):
     s = cp3_shape_for(dy.shape, K0, K1, K2, pad)
     assert dy.shape[1] == s.T
@@ -880,6 +949,7 @@ def cp3_conv2d_backward_data(dy, K0, K1, K2, pad=1, out=None, workspace=None, st
     return _cp3_pass(lib().cp3_conv2d_backward_data, s, dy, K0, K1, K2, dx, workspace, stream)
 
 
+@_stream_ordered
 def cp3_conv2d_backward_filter(x, dy, K0, K1, K2, pad=1, stream=None):
     """(dK0 [C,R], dK1 [Y,X,R], dK2 [R,T]) of the 3-factor CP op."""
     s = cp3_shape_for(x.shape, K0, K1, K2, pad)
@@ -902,6 +972,7 @@ def count_exceeding(a, b, tol, stream=None):
     return n.value
 
 
+@_stream_ordered
 def random_uniform(shape, seed, device="cuda", stream=None):
     t = torch.empty(shape, device=device, dtype=torch.float32)
     check(lib().cp4_random_uniform(_ptr(t), t.numel(), seed, _stream(stream)))

@@ -129,6 +129,8 @@ cp4_shape shape_for(const Tensor& act, const Factors& f, long pad) {
 }
 
 // ---- the three passes (capi.conv2d_forward, _backward_data, _backward_filter) --------
+// (Outputs and scratch come from the current stream's memory: a caller that names another
+// stream makes it current around the call, as capi.py does.)
 
 // (x, FK, FC, FH, FW, pad, out, variant, stream) -> y
 PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
