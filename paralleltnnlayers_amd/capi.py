@@ -554,7 +554,8 @@ def layer_forward(s, g, x, FK, FC, FH, FW, bias=None, activation=None, stream=No
     """y = act(conv(x) + bias) in x's element type; g: a Geometry or None."""
     dtype = _DTYPES[x.dtype]
     _check_layer(s, x, FK, FC, FH, FW)
-    assert bias is None or bias.numel() >= s.T
+    assert bias is None or tuple(bias.shape) == (s.T,) or (
+        (g is not None or x.dtype == torch.float16) and bias.numel() >= s.T)
     gp = ctypes.byref(g) if g is not None else None
     oh, ow = (g.out_h, g.out_w) if g is not None else (s.H, s.W)
     y = torch.empty((s.N, s.T, oh, ow), device=x.device, dtype=x.dtype)

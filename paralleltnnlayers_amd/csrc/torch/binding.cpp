@@ -119,12 +119,14 @@ struct Factors {
 };
 // tensor_shape as CP::Conv2dForward / Conv2dBackwardData derive it (Cuda_kernels/cp4Conv2d.cu:21-30)
 cp4_shape shape_for(const Tensor& act, const Factors& f, long pad) {
-  require(act.dim() == 4 && f.FK.dim() == 2 && f.FC.dim() == 2 && f.FH.dim() == 2 && f.FW.dim() == 2);
+  require(act.dim() == 4 && f.FK.dim() >= 2 && f.FC.dim() >= 1 && f.FH.dim() >= 1 && f.FW.dim() >= 1,
+          "expected an activation [N, C, H, W] and factors [rows, rank]");
   cp4_shape s;
   s.N = (unsigned)act.size(0); s.H = (unsigned)act.size(2); s.W = (unsigned)act.size(3);
   s.pad = (unsigned)pad;
   s.T = (unsigned)f.FK.size(0); s.C = (unsigned)f.FC.size(0); s.Y = (unsigned)f.FH.size(0);
   s.X = (unsigned)f.FW.size(0); s.Rank = (unsigned)f.FK.size(1);
+  // (rows and rank count, not the form: at rank 1 a vector holds a factor as well)
   return s;
 }
 
@@ -139,7 +141,8 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Tensor& x = tensor(a[0]);
   const Factors f{tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4])};
   const cp4_shape s = shape_for(x, f, integer(a[5]));
-  require(x.size(1) == s.C && f.FC.size(1) == s.Rank);
+  require(x.size(1) == s.C && f.FC.dim() >= 2 && f.FC.size(1) == s.Rank,
+          "x or FC does not match the factors");
   const int variant = (int)integer(a[7]);
   void* st = stream_of(a[8]);
   Tensor y = a[6] != Py_None ? tensor(a[6]) : Tensor();
@@ -381,12 +384,16 @@ PyObject* layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const bool half = plain && (t == at::kBFloat16 || t == at::kHalf);
   l.dtype = !half ? CP4_DTYPE_F32 : t == at::kBFloat16 ? CP4_DTYPE_BF16 : CP4_DTYPE_F16;
   const Tensor x = half ? x_in.contiguous() : as_f32(x_in);
-  require(x.is_cuda() && x.size(1) == l.shape.C && f.FC.size(1) == l.shape.Rank,
+  require(x.is_cuda() && x.size(1) == l.shape.C && f.FC.dim() >= 2 && f.FC.size(1) == l.shape.Rank,
           "expected a device tensor [N, C, H, W] that matches the factors");
   std::optional<Tensor> bias;
   if (a[6] != Py_None) {
     bias = tensor(a[6]);
-    require(bias->dim() == 1 && bias->size(0) == l.shape.T);
+    // (a layer with a geometry and a float16 one take any form that holds T entries)
+    require(l.has_geometry || l.dtype == CP4_DTYPE_F16
+                ? bias->numel() >= l.shape.T
+                : bias->dim() == 1 && bias->size(0) == l.shape.T,
+            "bias does not match the layer's output channels");
     l.has_bias = true;
   }
   const c10::DeviceGuard guard(x.device());

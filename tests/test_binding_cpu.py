@@ -27,6 +27,37 @@ def test_stride_forms_that_are_refused(stride, padding):
         _layer(stride, padding)
 
 
+def _pass(name, *fac):
+    from paralleltnnlayers_amd import capi
+    x, dy = torch.zeros(1, 4, 5, 5), torch.zeros(1, 6, 5, 5)
+
+    class Stream:               # (without a device there is no current one to ask for)
+        cuda_stream = 0
+
+    if name == "conv2d_forward":
+        return capi._native.forward(x, *fac, 1, None, -1, Stream)
+    if name == "conv2d_backward_data":
+        return capi._native.backward_data(dy, *fac, 1, None, Stream)
+    if name == "conv2d_backward_filter":
+        return capi._native.backward_filter(x, dy, *fac, 1, None, Stream, -1)
+    return torch_ops.cp4_conv2d(x, *fac, 1)
+
+
+PASSES = ["conv2d_forward", "conv2d_backward_data", "conv2d_backward_filter", "layer"]
+
+
+@pytest.mark.parametrize("forms", [((6, 2), (4, 2), (3, 2), (3, 2)), ((6, 1), (4, 1), (3,), (3,)),
+                                   ((6, 2, 1), (4, 2), (3, 2, 1), (3, 1, 2)), ((6, 1), (4,), (3,), (3, 1))],
+                         ids=repr)
+@pytest.mark.parametrize("name", PASSES)
+def test_factor_forms_that_are_taken(name, forms):
+    """Rows and rank count; FC names its channels by its second dimension only in the backward
+    passes."""
+    refused = len(forms[1]) == 1 and name in ("conv2d_forward", "layer")
+    with pytest.raises(AssertionError, match="match" if refused else "device tensor"):
+        _pass(name, *[torch.zeros(*f) for f in forms])
+
+
 class _OnDevice(torch.Tensor):
     """A host tensor that says it is on the device."""
     is_cuda = True

@@ -194,3 +194,34 @@ def test_bias_gradient_under_create_graph(ops):
     assert torch.allclose(db, (dy * (y > 0)).sum(dim=(0, 2, 3)), rtol=1e-4, atol=1e-4)
     (gg,) = torch.autograd.grad(db.sum(), dy)
     assert torch.equal(gg, (y > 0).float())
+
+
+def test_vector_factors_at_rank_one(ops):
+    """A tap factor of rank 1 as a vector computes what the one-column matrix does."""
+    import paralleltnnlayers_amd as cp4
+    x, dy = torch.randn(2, 8, 9, 10, device="cuda"), torch.randn(2, 12, 9, 10, device="cuda")
+    cols = [torch.randn(d, 1, device="cuda") for d in (12, 8, 3, 3)]
+    vecs = cols[:2] + [f.flatten() for f in cols[2:]]
+    assert torch.equal(cp4.conv2d_forward(x, *vecs), cp4.conv2d_forward(x, *cols))
+    assert torch.equal(cp4.conv2d_backward_data(dy, *vecs), cp4.conv2d_backward_data(dy, *cols))
+    for a, v, c in zip(vecs, cp4.conv2d_backward_filter(x, dy, *vecs),
+                       cp4.conv2d_backward_filter(x, dy, *cols)):
+        assert v.shape == a.shape and torch.equal(v.flatten(), c.flatten())
+    leaves = [[f.clone().requires_grad_() for f in fac] for fac in (vecs, cols)]
+    ys = [ops.cp4_conv2d(x, *fac, 1) for fac in leaves]
+    assert torch.equal(*ys)
+    for y in ys:
+        y.backward(dy)
+    assert all(torch.equal(a.grad.flatten(), b.grad.flatten()) for a, b in zip(*leaves))
+
+
+@pytest.mark.parametrize("kw", [{"dtype": torch.float16}, {"stride": 2}], ids=["f16", "stride"])
+def test_bias_forms(ops, kw):
+    """Half-precision layers and layers with a geometry take a bias of any form."""
+    x = torch.randn(2, 16, 9, 10, device="cuda", dtype=kw.get("dtype", torch.float32))
+    fac = [torch.randn(d, 4, device="cuda") for d in (16, 16, 3, 3)]
+    bias = torch.randn(16, device="cuda")
+    run = lambda b: ops.cp4_conv2d(x, *fac, 1, bias=b, stride=kw.get("stride", 1))
+    assert torch.equal(run(bias.view(1, 16, 1, 1)), run(bias))
+    with pytest.raises(AssertionError):
+        run(bias[:15].contiguous())
