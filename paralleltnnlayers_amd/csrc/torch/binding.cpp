@@ -127,6 +127,8 @@ cp4_shape shape_for(const Tensor& act, const Factors& f, long pad) {
   s.T = (unsigned)f.FK.size(0); s.C = (unsigned)f.FC.size(0); s.Y = (unsigned)f.FH.size(0);
   s.X = (unsigned)f.FW.size(0); s.Rank = (unsigned)f.FK.size(1);
   // (rows and rank count, not the form: at rank 1 a vector holds a factor as well)
+  for (const Tensor* t : {&f.FK, &f.FC, &f.FH, &f.FW})
+    require(t->numel() >= t->size(0) * (int64_t)s.Rank, "a factor holds fewer than rows * rank entries");
   return s;
 }
 
@@ -150,6 +152,7 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     NoGil unlocked;
     const float *px = f32(x), *pK = f32(f.FK), *pC = f32(f.FC), *pH = f32(f.FH), *pW = f32(f.FW);
     if (!y.defined()) y = empty({s.N, s.T, s.H, s.W}, at::kFloat, x);
+    require(y.numel() >= (int64_t)s.N * s.T * s.H * s.W, "out is smaller than the result");
     check(cp4_conv2d_forward_variant(&s, px, pK, pC, pH, pW, f32(y), variant, st));
   }
   return THPVariable_Wrap(std::move(y));
@@ -170,6 +173,7 @@ PyObject* backward_data(PyObject*, PyObject* const* a, Py_ssize_t n) {
     NoGil unlocked;
     const float *pdy = f32(dy), *pK = f32(f.FK), *pC = f32(f.FC), *pH = f32(f.FH), *pW = f32(f.FW);
     if (!dx.defined()) dx = empty({s.N, s.C, s.H, s.W}, at::kFloat, dy);
+    require(dx.numel() >= (int64_t)s.N * s.C * s.H * s.W, "out is smaller than the result");
     check(cp4_conv2d_backward_data(&s, pdy, pK, pC, pH, pW, f32(dx), st));
   }
   return THPVariable_Wrap(std::move(dx));

@@ -58,6 +58,16 @@ def test_factor_forms_that_are_taken(name, forms):
         _pass(name, *[torch.zeros(*f) for f in forms])
 
 
+@pytest.mark.parametrize("short", [1, 2, 3])
+@pytest.mark.parametrize("name", PASSES)
+def test_factors_with_too_few_entries_are_refused(name, short):
+    """The kernels would read past their end."""
+    fac = [torch.zeros(d, 2) for d in (6, 4, 3, 3)]
+    fac[short] = fac[short][:, :1].contiguous()
+    with pytest.raises(AssertionError, match="fewer"):
+        _pass(name, *fac)
+
+
 class _OnDevice(torch.Tensor):
     """A host tensor that says it is on the device."""
     is_cuda = True

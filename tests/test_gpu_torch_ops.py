@@ -225,3 +225,14 @@ def test_bias_forms(ops, kw):
     assert torch.equal(run(bias.view(1, 16, 1, 1)), run(bias))
     with pytest.raises(AssertionError):
         run(bias[:15].contiguous())
+
+
+def test_out_smaller_than_the_result_is_refused(ops):
+    import paralleltnnlayers_amd as cp4
+    x = torch.randn(2, 8, 9, 10, device="cuda")
+    fac = [torch.randn(d, 4, device="cuda") for d in (8, 8, 3, 3)]
+    for run in (cp4.conv2d_forward, cp4.conv2d_backward_data):
+        with pytest.raises(AssertionError, match="smaller"):
+            run(x, *fac, out=torch.empty(2, 8, 9, 9, device="cuda"))
+        out = torch.empty(2 * 8 * 9 * 10, device="cuda")
+        assert torch.equal(run(x, *fac, out=out).view(2, 8, 9, 10), run(x, *fac))
