@@ -61,7 +61,9 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
   // cores' sums come out low by a few hundredths of a unit in the last place whatever their sign, which
   // a sum over all pixels into the nearly cancelling factor gradients brings to the front
   // (N32 T256 56x56 R32: G3's mean error 1.9e-8 of its deviation, 4e-11 with the signs
-  // reversed, 6.9e-9 in the contraction kernel; dFC 3.8e-6 of its norm off, 4.7e-7 with them, 1.6e-6).
+  // reversed, 6.9e-9 in the contraction kernel; dFC 4.0e-6 of its norm off, 5.4e-7 with them, 1.3e-6.
+  // With 3, 5 or 7 waves one wave's share of the drift is left: dFC at N53 C128 T96 56x56 R32 1.2e-6, T224
+  // 4.9e-7; 1.6e-6 and 1.2e-6 with the contraction kernel).
   const float sign = wave & 1 ? -1.f : 1.f;
   u32x4 fh[2], fm[2], fl[2];
 #pragma unroll
@@ -105,9 +107,13 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
       const float v[8] = {in0 ? zv[k][0].x : 0.f, in0 ? zv[k][0].y : 0.f, in0 ? zv[k][0].z : 0.f,
                           in0 ? zv[k][0].w : 0.f, in1 ? zv[k][1].x : 0.f, in1 ? zv[k][1].y : 0.f,
                           in1 ? zv[k][1].z : 0.f, in1 ? zv[k][1].w : 0.f};
+      const unsigned flip = (i - i0) & 1 ? 0x80000000u : 0u;      // the chunk's sign, see accK
+      float sv[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sv[e] = __uint_as_float(__float_as_uint(v[e]) ^ flip);
       if (it < 256) {
         u32x4 h, m, l;
-        split::split8(v, h, m, l);
+        split::split8(sv, h, m, l);
         u32x4* dst = Zf + ((zo >> 1) * 6 + (zo & 1)) * 32 + zr;
         dst[0] = h;
         dst[64] = m;
@@ -115,6 +121,10 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
       }
     }
   };
+  // dFK, with the opposite sign after every other chunk (those chunks' Cc has it reversed), for
+  // the same reason as above: a workgroup's chunks are one chain of sums.  (dFK of N27 C128 T256 56x56
+  // R32: 4.1e-7 of its norm off without, 3.3e-7 with, 3.8e-7 in the gradient GEMM; N105 T64: 5.8e-7,
+  // 3.4e-7, 7.4e-7.  No time: 57 shapes within 0.3 % of each other on the mean.)
   f32x16 accK = (f32x16)(0.f);
   float bs[8];
 #pragma unroll
@@ -146,6 +156,7 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     // ---- dFK: rows of the tile against Cc ----
+    accK = -accK;
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
       const float* ap = tile + l32 * kRow + 16 * st + 8 * hi;
@@ -204,6 +215,7 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
     __syncthreads();              // tiles free, the next chunk's fragments complete
   }
   // ---- one partial set per workgroup ----
+  if ((i1 - i0 - 1) & 1) accK = -accK;
   float* pk = a.partK + ((size_t)wg * T + c0) * R;
 #pragma unroll
   for (int v = 0; v < 16; ++v) {

@@ -221,3 +221,40 @@ def test_large_layer_behind_relu(capi, case):
     terms = capi.conv2d_backward_filter(x.abs(), masked.abs(), *[f.abs() for f in fac], pad=k // 2)
     for g, w, t in zip(grads, want, terms):
         assert ((g - w).abs() <= 4 * 2.0 ** -24 * (N * H * W) ** 0.5 * t).all()
+
+
+def _float64_factor_gradients(x, dy, fac, k):
+    """(dFK, dFC, dFH, dFW) of the layer without an epilogue, factor by factor in float64."""
+    (N, C, H, W), P = x.shape, k // 2
+    FK, FC, FH, FW = leaves = [f.double().requires_grad_() for f in fac]
+    R = FK.shape[1]
+    A = torch.matmul(FC.t(), x.double().flatten(2)).view(N, R, H, W)
+    A = torch.nn.functional.pad(A, (P, P, P, P))
+    B = sum(FH[i].view(1, R, 1, 1) * A[:, :, i:i + H] for i in range(k))
+    Z = sum(FW[j].view(1, R, 1, 1) * B[..., j:j + W] for j in range(k))
+    y = torch.matmul(FK, Z.flatten(2))
+    return torch.autograd.grad(y, leaves, dy.double().flatten(2))
+
+
+# Sums over all pixels that nearly cancel: the matrix cores' accumulation comes out low by a
+# little whatever its sign, which the pass over dy cancels by alternating signs (over the waves
+# in G3, hence in dFC; over a workgroup's chunks in dFK).  Errors in the 2-norm with the
+# alternation and without it: T64 dFK 3.5e-7 and 6.8e-7, dFC 8.4e-7 and 3.0e-6; T256 dFK 3.6e-7
+# and 4.6e-7, dFC 5.4e-7 and 4.0e-6.  The bounds lie between.
+@pytest.mark.parametrize("case,bounds", [
+    ((128, 128, 56, 56, 64, 3, 32), (4.8e-7, 1.6e-6)),
+    ((32, 256, 56, 56, 256, 3, 32), (4.05e-7, 1.5e-6)),
+], ids=["T64", "T256"])
+def test_large_layer_factor_gradients_do_not_drift(capi, case, bounds):
+    N, C, H, W, T, k, R = case
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x = mk(N, C, H, W).clamp_(min=0)
+    fac = [mk(d, R) * (2.0 / (C * k * k * R)) ** 0.125 for d in (T, C, k, k)]
+    s = capi.shape_for(x.shape, *fac, k // 2)
+    y = capi.layer_forward(s, None, x, *fac, 0.1 * mk(T), "relu")
+    dy = mk(*y.shape)
+    _, grads, _ = capi.layer_backward(s, None, x, y, dy, *fac, "relu")
+    want = _float64_factor_gradients(x, dy * (y > 0), fac, k)
+    for g, w, bound in zip(grads, want, bounds):          # dFK, dFC
+        assert float((g.double() - w).norm() / w.norm()) <= bound
