@@ -465,6 +465,14 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* geomet
                               void* dx, float* dFK, float* dFC, float* dFH, float* dFW,
                               float* dbias, void* workspace, size_t workspace_bytes,
                               cp4_stream stream);
+/* What the calling thread's last cp4_layer_backward launched beside the passes on their own, as
+ * a sum of CP4_ROUTE_*; 0: nothing. */
+enum {
+  CP4_ROUTE_MASKED_TILES = 1, /* mask and bias gradient inside the dense-gradient tile kernel */
+  CP4_ROUTE_DY_PASS = 2,      /* one pass over dy for mask, bias gradient, G3 and dFK */
+  CP4_ROUTE_DX_FROM_G1 = 4    /* the input gradient from the factor gradients' G1 plane */
+};
+int cp4_layer_last_backward_route(void);
 
 /* ---- 3-factor CP sibling op ------------------------------------------------
  * Stands where the reference registers its TensorFlow op Conv2dCpFusedNchw

@@ -591,6 +591,15 @@ def layer_backward(s, g, x, y, dy, FK, FC, FH, FW, activation=None, want_dx=True
     return dx, tuple(grads), dbias
 
 
+ROUTE_MASKED_TILES, ROUTE_DY_PASS, ROUTE_DX_FROM_G1 = 1, 2, 4       # CP4_ROUTE_*
+
+
+def layer_last_backward_route():
+    """What this thread's last layer_backward launched beside the passes on their own
+    (a sum of ROUTE_*)."""
+    return lib().cp4_layer_last_backward_route()
+
+
 def conv2d_backward_data(dy, FK, FC, FH, FW, pad=1, out=None, stream=None):
     if stream is None or out is not None:              # (allocates dx only)
         return _native.backward_data(dy, FK, FC, FH, FW, pad, out, stream)

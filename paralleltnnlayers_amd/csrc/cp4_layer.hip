@@ -85,6 +85,8 @@ BackwardPlan backward_plan(const cp4_shape& s, const cp4_geometry* g, int dtype,
   return plans[key] = make_backward_plan(s, g, dtype, act, wanted);
 }
 
+thread_local int g_route = 0;      // of this thread's last cp4_layer_backward
+
 cp4_status check_layer(const cp4_shape* s, const cp4_geometry* g, int dtype, int act) {
   cp4_status rc = g ? cp4::check_layer_geometry(s, g) : cp4::check_layer_shape(s);
   if (rc != CP4_OK) return rc;
@@ -159,6 +161,7 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* g, int
                               void* dx, float* dFK, float* dFC, float* dFH, float* dFW,
                               float* dbias, void* workspace, size_t workspace_bytes,
                               cp4_stream stream) {
+  g_route = 0;
   CP4_TRY(check_layer(shape, g, dtype, activation));
   const cp4_shape& s = *shape;
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -196,10 +199,12 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* g, int
                 *dyf = static_cast<const float*>(dy);
     float* mask_ws = p.act16 ? reinterpret_cast<float*>(ws + p.act16_at) : nullptr;
     const int variant = cp4::layer_filter_masks(s, xf, yf, dyf, ws + p.pass_at, mask_ws, dx != nullptr);
-    if (variant)
+    if (variant) {
+      g_route = variant == 3 ? CP4_ROUTE_MASKED_TILES : CP4_ROUTE_DY_PASS | (dx ? CP4_ROUTE_DX_FROM_G1 : 0);
       return cp4::layer_backward_filter_masked(variant, shape, xf, yf, dyf, FK, FC, FH, FW, dFK, dFC,
                                                dFH, dFW, static_cast<float*>(dx), dbias, parts, mask_ws,
                                                ws + p.pass_at, p.pass_bytes, stream);
+    }
   }
   if (p.act16) {
     CP4_LAUNCH(cp4::act_grad_launch(ym, dy, ws + p.act16_at, dtype, false, dbias, parts, N, T, plane, st));
@@ -218,6 +223,7 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* g, int
   if (filter && (!half || p.filter16)) {
     CP4_TRY(cp4::layer_backward_filter(shape, g, dtype, x, dya, FK, FC, FH, FW, dFK, dFC, dFH, dFW,
                                        pass_ws, p.pass_bytes, dx, &dx_done, stream));
+    if (dx && dx_done) g_route |= CP4_ROUTE_DX_FROM_G1;
     dx_done = dx_done || !dx;
   } else if (filter) {
     float* x32 = reinterpret_cast<float*>(ws + p.x32_at);
@@ -241,5 +247,7 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* g, int
   CP4_LAUNCH(cp4::convert_launch(dx32, CP4_DTYPE_F32, dx, dtype, elements(s, s.C), st));
   return CP4_OK;
 }
+
+int cp4_layer_last_backward_route(void) { return g_route; }
 
 }  // extern "C"
