@@ -241,12 +241,22 @@ int grid_of(int N, int T, int HW) {
 
 }  // namespace
 
-// 64 to 256 output channels in whole blocks of 32, ranks up to 32, rows that move as 16 bytes; at least
-// two chunks a workgroup (a workgroup reads all of FK and leaves a partial set whatever it does).
+// 64 to 256 output channels in whole blocks of 32, ranks up to 32, rows that move as 16 bytes, and
+// gain over the passes on their own: it saves the masked dy's way to memory and back, and pays for a
+// second pass over the rank planes (Cc before the others), a launch, FK and a partial set per
+// workgroup, and workgroups that sit out the last round of chunks.  The line, in us, fits
+// 450 layers (T 64-256, R 1-32, filters 1-7, C 16-512, 17x17 to 240x240) timed both ways from two
+// chunks a workgroup on; the choice is 0.2 % off the better one on the mean, 6.5 % at worst,
+// the pass everywhere 1.5 and 19 % (N21 C64 T96 56x56 R16, two chunks a workgroup: 78 us, 70 apart;
+// N63, six: 139, 155).
 bool bwd_dy_pass_supported(int N, int T, int R, int HW) {
   if (T % 32 != 0 || T < 64 || T > 256 || R < 1 || R > 32 || HW % 4 != 0) return false;
   const long chunks = (long)N * ((HW + kPix - 1) / kPix);
-  return chunks >= 2l * num_compute_units() * std::max(1, 8 / (T / 32));
+  const long wgs = (long)num_compute_units() * std::max(1, 8 / (T / 32));
+  if (chunks < 2 * wgs) return false;
+  const double pixels = 1e-6 * N * HW;
+  const double idle = 1e-6 * ((chunks + wgs - 1) / wgs * wgs - chunks) * kPix;
+  return T * (1.7 * pixels - 0.75 * idle) - 2.1 * R * pixels > 11.6;
 }
 int bwd_dy_pass_sets(int N, int T, int HW) { return grid_of(N, T, HW); }
 

@@ -198,13 +198,17 @@ def test_first_layer_without_an_input_gradient(capi, case, relu):
         assert (g.double().cpu() - w).abs().max() <= 1e-3 * w.abs().max() + 1e-30
 
 
-# The one pass over dy of large layers: 3, 4 and 8 waves, planes that no chunk of 64 pixels
-# divides, ranks that fill a tile and not, every filter size of the column taps.
-@pytest.mark.parametrize("case", [(33, 32, 46, 54, 96, 5, 32), (24, 16, 64, 64, 128, 3, 16),
-                                  (70, 48, 32, 36, 256, 1, 7), (22, 16, 60, 68, 224, 3, 31),
-                                  (40, 16, 66, 66, 64, 7, 5)],
-                         ids=lambda c: "x".join(map(str, c)))
-def test_large_layer_behind_relu(capi, case):
+# The one pass over dy of large layers: 2, 3, 4, 5, 7 and 8 waves, planes that no chunk of 64 pixels
+# divides, ranks that fill a tile and not, every filter size of the column taps; and layers on the
+# other side of the line, where the passes on their own are the quicker.
+@pytest.mark.parametrize("case,one_pass", [
+    ((33, 32, 46, 54, 96, 5, 32), False), ((24, 16, 64, 64, 128, 3, 16), True),
+    ((70, 48, 32, 36, 256, 1, 7), True), ((22, 16, 60, 68, 224, 3, 31), True),
+    ((40, 16, 66, 66, 64, 7, 5), True), ((70, 32, 46, 54, 96, 5, 32), True),
+    ((48, 32, 40, 44, 160, 3, 32), True), ((96, 64, 56, 60, 64, 3, 16), True),
+    ((21, 64, 56, 56, 96, 3, 16), False), ((11, 16, 56, 56, 160, 3, 32), False)],
+    ids=lambda c: "x".join(map(str, c)) if isinstance(c, tuple) else ("apart", "one")[c])
+def test_large_layer_behind_relu(capi, case, one_pass):
     N, C, H, W, T, k, R = case
     gen = torch.Generator(device="cuda").manual_seed(N * H + W + T)
     mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)
@@ -213,7 +217,8 @@ def test_large_layer_behind_relu(capi, case):
     s = capi.shape_for(x.shape, *fac, k // 2)
     y = capi.layer_forward(s, None, x, *fac, mk(T), "relu")
     dx, grads, dbias = capi.layer_backward(s, None, x, y, dy, *fac, "relu")
-    assert capi.layer_last_backward_route() == capi.ROUTE_DY_PASS | capi.ROUTE_DX_FROM_G1
+    assert capi.layer_last_backward_route() == (capi.ROUTE_DX_FROM_G1 |
+                                                (capi.ROUTE_DY_PASS if one_pass else 0))
     masked = dy * (y > 0)
     # against the passes on their own (each checked against float64 elsewhere): fp32 sums in
     # another order, 2^-24 a step of the sum of the terms' magnitudes as a random walk over the
