@@ -12,8 +12,13 @@
 // workgroup share the pixels and differ in the channel slice where there are slices, and
 // workgroups of one die (blockIdx & 7) take a contiguous range of the pixels, so that cache
 // lines that two blocks share meet in one L2.
-// N32 C256 56x56 R32 fp32 (103 MB written, 13 MB read): 24 us with streaming stores, 29 without; the backward-data pass from
-// dy takes 56.
+// N32 C256 56x56 R32 fp32 (103 MB written, 13 MB read): 29 us; the backward-data pass from dy takes 56.
+// (Stores that leave the caches alone take 24 us here and as much more in what runs beside them: 26
+// layers of 48 to 270 MB, no backward call more than 0.7 % apart on the best of five.)
+// The factor gradients' four-launch variant and its strided and 16-bit siblings bring dx along
+// wherever they run: 100 layers (fp32 and bf16, C and T 16-256, R 8-64 also beyond C and T, filters
+// 1-5, stride 1 and 2) took 0.99 to 1.82 times as long with the pass of its own (C = T = 16, R 64,
+// N16 160x160 bf16: 539 us against 316).
 #include <cstdint>
 
 #include "cp4_internal.h"
@@ -33,7 +38,6 @@ struct ExpandArgs {
   int C, R, HW;
   int cblocks;                 // blocks of 32 channels a wave takes
   int slices;                  // waves a block of pixels is shared by
-  bool stream;                 // stores that leave the caches alone
   long pixels, blocks, items;  // N * HW; blocks of pixels; blocks * slices
 };
 
@@ -163,9 +167,7 @@ __global__ __launch_bounds__(kThreads, 2) void rank_expand_kernel(ExpandArgs a) 
         OV o;
 #pragma unroll
         for (int q = 0; q < PX; ++q) o[q] = Out::down(acc[q][v]);
-        OV* to = reinterpret_cast<OV*>(dst + oat[0] + (size_t)c * HW);
-        if (live[0] && a.stream) __builtin_nontemporal_store(o, to);
-        else if (live[0]) *to = o;
+        if (live[0]) *reinterpret_cast<OV*>(dst + oat[0] + (size_t)c * HW) = o;
       } else {
 #pragma unroll
         for (int q = 0; q < PX; ++q)
@@ -189,10 +191,6 @@ hipError_t launch(ExpandArgs a, hipStream_t st) {
   a.blocks = blocks;
   a.items = blocks * a.slices;
   const unsigned grid = (unsigned)((a.items + kThreads / 64 - 1) / (kThreads / 64));
-  // A result that fills a good part of the 256 MB memory-side cache is streamed past it: it would
-  // only push out x and dy, which the gradient GEMMs read again (N32 C256 56x56 R32: 29 -> 24
-  // us for this kernel).
-  a.stream = (size_t)a.pixels * a.C * sizeof(typename Out::raw) > ((size_t)48 << 20);
   const bool vec = a.HW % px == 0 && reinterpret_cast<uintptr_t>(a.Z) % (4 * px) == 0 &&
                    reinterpret_cast<uintptr_t>(a.dst) % (sizeof(typename Out::raw) * px) == 0;
 #define CP4_EXPAND(KC_, PX_)                                                             \
