@@ -1,23 +1,26 @@
-// One pass over a layer's output gradient for everything in its backward that reads it: with
-// dya = dy where y > 0 (a layer behind a ReLU; dy itself without one) and Cc = the filtered
-// rank planes of x,
+// One pass over the output gradient of a layer behind a ReLU for everything in its backward that
+// reads it: with dya = dy where y > 0 and Cc = the filtered rank planes of x,
 //   G3[n,r,p] = sum_t FK[t,r] dya[n,t,p]     dFK[t,r] = sum_{n,p} dya[n,t,p] Cc[n,r,p]
 //   dbias[t]  = sum_{n,p} dya[n,t,p]
 // so dya never goes to memory.  (As passes of their own: the mask and the bias gradient read dy and y and
 // write dya, the contraction and the gradient GEMM read it once each - five times the plane
 // where this kernel moves two.)
 //
-// Bound by reading dy and y.  A workgroup takes chunks of 64 pixels of one image and all T channels
-// (up to 256), a wave per 32 channels; about eight waves a compute unit, each with a whole chunk's
-// dy and y (64 registers) in flight while it works on the chunk before.  Rows move as 16 bytes a
-// lane, 256 contiguous bytes a channel.  A wave's 32 x 64 tile of dya lies in LDS, its own: read
-// by rows (channel x 8 pixels) it is the A operand of the dFK product, read by columns (pixel
-// x 8 channels) the B operand of the contraction; exact fp32 products from three bf16 parts.  The
+// Bound by reading dy and y.  A workgroup takes chunks of 64 pixels of one image and all T
+// channels (up to 256), a wave per 32 channels; eight waves a compute unit where the channel
+// count allows (5 at 160 channels, 6 at 96 and 192, 7 at 224), each with a whole chunk's dy and y
+// (64 registers) in flight while it works on the chunk before.  Rows move as 16 bytes a lane, 256
+// contiguous bytes a channel.  A wave's 32 x 64 tile of dya lies in LDS, its own: read by rows
+// (channel x 8 pixels) it is the A operand of the dFK product, read by columns (pixel x 8
+// channels) the B operand of the contraction; exact fp32 products from three bf16 parts.  The
 // contraction's partial sums over a wave's channels go over its tile, which nothing reads any
 // more, and are added over the waves in order; Cc's fragments are split once a workgroup.  Two
 // barriers a chunk.  dFK and the bias sums stay in registers over a workgroup's contiguous
 // range of chunks: one partial set per workgroup, added in order by the caller's reduction.
-// N32 T256 56x56 R32 (206 MB): 60 us on rotating buffers, 3.4 TB/s of rows in 256-byte pieces (64 with the partial sums read one after the other).
+// 248 registers with four waves and more; with two or three (64 and 96 channels), where a thread
+// also holds two pieces of Cc, 256 and six of them in scratch memory.
+// N32 T256 56x56 R32 (206 MB): 60 us on rotating buffers, 3.4 TB/s of rows in 256-byte pieces (64
+// with the partial sums read one after the other).
 #include <algorithm>
 #include <cstdint>
 
@@ -43,7 +46,7 @@ struct DyPassArgs {
 };
 
 // KZ: (rank, octet) pairs of Cc a thread loads and splits (256 of them a chunk).
-template <bool MASK, int KZ>
+template <int KZ>
 __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5;
@@ -77,7 +80,7 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
 
   // ---- loads: row 4 j + lane / 16 of the wave's channels, four pixels a lane ----
   const int lrow = lane >> 4, lcol = 4 * (lane & 15);
-  float4 dv[8], yv[MASK ? 8 : 1], zv[KZ][2];
+  float4 dv[8], yv[8], zv[KZ][2];
   // (clamped, not branched; values outside are dropped where they are used.  Cc's first: its
   // fragments are made before the rows are waited for)
   auto load = [&](int i) {
@@ -95,7 +98,7 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       dv[j] = *reinterpret_cast<const float4*>(a.dy + at + (size_t)(4 * j) * HW);
-      if constexpr (MASK) yv[j] = *reinterpret_cast<const float4*>(a.y + at + (size_t)(4 * j) * HW);
+      yv[j] = *reinterpret_cast<const float4*>(a.y + at + (size_t)(4 * j) * HW);
     }
   };
   auto deposit_z = [&](int i) {
@@ -142,13 +145,11 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       float4 m = in ? dv[j] : make_float4(0.f, 0.f, 0.f, 0.f);
-      if constexpr (MASK) {
-        // (a product, as dy * (y > 0): a non-finite dy at a clipped output stays visible)
-        m.x *= yv[j].x > 0.f ? 1.f : 0.f;
-        m.y *= yv[j].y > 0.f ? 1.f : 0.f;
-        m.z *= yv[j].z > 0.f ? 1.f : 0.f;
-        m.w *= yv[j].w > 0.f ? 1.f : 0.f;
-      }
+      // (a product, as dy * (y > 0): a non-finite dy at a clipped output stays visible)
+      m.x *= yv[j].x > 0.f ? 1.f : 0.f;
+      m.y *= yv[j].y > 0.f ? 1.f : 0.f;
+      m.z *= yv[j].z > 0.f ? 1.f : 0.f;
+      m.w *= yv[j].w > 0.f ? 1.f : 0.f;
       bs[j] += (m.x + m.y) + (m.z + m.w);
       *reinterpret_cast<float4*>(tile + (4 * j + lrow) * kRow + lcol) = m;
     }
@@ -263,6 +264,7 @@ int bwd_dy_pass_sets(int N, int T, int HW) { return grid_of(N, T, HW); }
 hipError_t bwd_dy_pass_launch(const float* dy, const float* y, const float* FK, const float* Cc,
                               float* G3, float* partK, float* partB, int N, int T, int R, int HW,
                               hipStream_t st) {
+  if (!y) return hipErrorInvalidValue;
   DyPassArgs a{};
   a.dy = dy; a.y = y; a.FK = FK; a.Cc = Cc; a.G3 = G3; a.partK = partK; a.partB = partB;
   a.T = T; a.R = R; a.HW = HW;
@@ -270,8 +272,7 @@ hipError_t bwd_dy_pass_launch(const float* dy, const float* y, const float* FK, 
   a.chunks = N * a.cpi;
   const int waves = T / 32;
   const size_t lds = (size_t)waves * kTile * sizeof(float) + kFrag * 16;
-  auto k = waves >= 4 ? (y ? dy_pass_kernel<true, 1> : dy_pass_kernel<false, 1>)
-                      : (y ? dy_pass_kernel<true, 2> : dy_pass_kernel<false, 2>);
+  auto k = waves >= 4 ? dy_pass_kernel<1> : dy_pass_kernel<2>;
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

@@ -184,7 +184,6 @@ hipError_t convert_launch(const void* src, int src_dtype, void* dst, int dst_dty
                           hipStream_t);
 
 // dst[n,c,p] = sum_r F[c,r] Z[n,r,p] (ranks up to 64), dst of a cp4_dtype.
-bool rank_expand_supported(int N, int C, int HW, int R);
 hipError_t rank_expand_launch(const float* F, const float* Z, void* dst, int dtype, int N, int C,
                               int HW, int R, hipStream_t);
 
@@ -219,7 +218,7 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs&, hipStream_t);
 // dbias, mask_ws); operands on 16-byte boundaries.
 bool bwd_filter_mfma_masks(const cp4_shape&);
 hipError_t bwd_filter_mfma_masked_launch(const BwdFilterArgs&, hipStream_t);
-// One pass over dy: G3, `sets` partial sets [set][T][R] of dFK and [set][T] of dbias.
+// One pass over dy behind a ReLU (y, its output): G3, `sets` partial sets [set][T][R] of dFK and [set][T] of dbias.
 bool bwd_dy_pass_supported(int N, int T, int R, int HW);
 int bwd_dy_pass_sets(int N, int T, int HW);
 hipError_t bwd_dy_pass_launch(const float* dy, const float* y, const float* FK, const float* Cc,

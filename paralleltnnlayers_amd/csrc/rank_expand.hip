@@ -38,7 +38,7 @@ struct ExpandArgs {
   int C, R, HW;
   int cblocks;                 // blocks of 32 channels a wave takes
   int slices;                  // waves a block of pixels is shared by
-  long pixels, blocks, items;  // N * HW; blocks of pixels; blocks * slices
+  long pixels, items;          // N * HW; blocks of pixels * slices
 };
 
 struct ToF32 {
@@ -188,7 +188,6 @@ hipError_t launch(ExpandArgs a, hipStream_t st) {
   while (a.cblocks > 1 && blocks * ((all + a.cblocks - 1) / a.cblocks) < 8l * num_compute_units())
     a.cblocks = (a.cblocks + 1) / 2;
   a.slices = (all + a.cblocks - 1) / a.cblocks;
-  a.blocks = blocks;
   a.items = blocks * a.slices;
   const unsigned grid = (unsigned)((a.items + kThreads / 64 - 1) / (kThreads / 64));
   const bool vec = a.HW % px == 0 && reinterpret_cast<uintptr_t>(a.Z) % (4 * px) == 0 &&
@@ -208,12 +207,9 @@ hipError_t launch(ExpandArgs a, hipStream_t st) {
 
 }  // namespace
 
-bool rank_expand_supported(int N, int C, int HW, int R) {
-  return R >= 1 && R <= 64 && C >= 1 && N >= 1 && HW >= 1;
-}
-
 hipError_t rank_expand_launch(const float* F, const float* Z, void* dst, int dtype, int N, int C,
                               int HW, int R, hipStream_t st) {
+  if (R > 64) return hipErrorInvalidValue;         // (four chunks of ranks)
   ExpandArgs a{};
   a.F = F; a.Z = Z; a.dst = dst;
   a.C = C; a.R = R; a.HW = HW;
