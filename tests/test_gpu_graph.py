@@ -124,3 +124,43 @@ def test_cp3_passes_replay(cp4, dims):
         torch.cuda.synchronize()
         for name, a, b in zip(("y", "dx"), got, (y, dx)):
             assert (a - b).abs().max().item() <= 1e-6 * b.abs().max().item(), (replay, name)
+
+
+# (N, C, H, W, T, k, R, dtype, stride, dx): dx from G1 / the passes on their own / the one pass
+# over dy / the masked tiles of a first layer / 16-bit activations, also on widened copies / a stride
+LAYERS = [(2, 64, 28, 30, 64, 3, 16, "float32", 1, True), (3, 5, 9, 9, 7, 3, 3, "float32", 1, True),
+          (24, 16, 64, 64, 128, 3, 16, "float32", 1, True), (4, 3, 56, 60, 32, 3, 16, "float32", 1, False),
+          (2, 64, 28, 28, 64, 3, 16, "bfloat16", 1, True), (2, 5, 9, 10, 7, 3, 3, "float16", 1, True),
+          (2, 48, 27, 27, 32, 3, 16, "float32", 2, True)]
+
+
+@pytest.mark.parametrize("case", LAYERS, ids=lambda c: "x".join(map(str, c)))
+def test_layer_replays_match_eager(cp4, case):
+    N, C, H, W, T, k, R, dtype, stride, want_dx = case
+    capi, dtype = cp4.capi, getattr(torch, dtype)
+    gen = torch.Generator(device="cuda").manual_seed(N + C + H)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, fac, bias = mk(N, C, H, W).to(dtype), [mk(d, R) for d in (T, C, k, k)], mk(T)
+    s = capi.shape_for(x.shape, *fac, k // 2)
+    g = capi.geometry(s, stride, "same") if stride > 1 else None
+
+    def step():
+        y = capi.layer_forward(s, g, x, *fac, bias, "relu")
+        dx, grads, dbias = capi.layer_backward(s, g, x, y, dy, *fac, "relu", want_dx=want_dx)
+        return [y, dbias, *grads] + ([dx] if want_dx else [])
+
+    dy = mk(*capi.layer_forward(s, g, x, *fac, bias, "relu").shape).to(dtype)
+    step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        held = step()
+    for _ in range(3):
+        for t in (x, dy, bias, *fac):
+            t.copy_(mk(*t.shape))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in held]
+        want = step()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))

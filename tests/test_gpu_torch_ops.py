@@ -236,3 +236,75 @@ def test_out_smaller_than_the_result_is_refused(ops):
             run(x, *fac, out=torch.empty(2, 8, 9, 9, device="cuda"))
         out = torch.empty(2 * 8 * 9 * 10, device="cuda")
         assert torch.equal(run(x, *fac, out=out).view(2, 8, 9, 10), run(x, *fac))
+
+
+@pytest.mark.parametrize("kw", [{}, {"stride": 2, "padding": "same"}], ids=["plain", "stride"])
+def test_saved_tensor_hooks_see_what_the_layer_saves(ops, kw):
+    """Offloading the saved tensors changes nothing; x, the factors and y are what is saved."""
+    layer, x = _small_layer(ops, **kw)
+    dy = torch.randn_like(layer(x))
+
+    def grads(run):
+        xi = x.clone().requires_grad_()
+        layer.zero_grad(set_to_none=True)
+        run(xi).backward(dy)
+        return [xi.grad] + [p.grad for p in layer.parameters()]
+
+    def offloaded(xi):
+        with torch.autograd.graph.save_on_cpu():
+            return layer(xi)
+
+    want = grads(layer)
+    assert all(torch.equal(a, b) for a, b in zip(grads(offloaded), want))
+    shapes = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (shapes.append(tuple(t.shape)), t)[1],
+                                                  lambda t: t):
+        y = layer(x.clone().requires_grad_())
+    assert sorted(shapes) == sorted([tuple(x.shape), tuple(y.shape)] +
+                                    [tuple(f.shape) for f in (layer.FK, layer.FC, layer.FH, layer.FW)])
+
+
+def test_functional_transforms_are_refused(ops):
+    """The library sees memory, not batched or wrapped tensors: an error, never a result."""
+    import paralleltnnlayers_amd as cp4
+    layer, x = _small_layer(ops)
+    fac = [f.detach() for f in (layer.FK, layer.FC, layer.FH, layer.FW)]
+    dy = torch.randn_like(layer(x)).detach()
+    xs = torch.stack([x, x])
+    batched = lambda t: torch.stack([t, t])
+    with torch.no_grad():
+        calls = [lambda: torch.vmap(layer)(xs),
+                 lambda: torch.vmap(lambda f: ops.cp4_conv2d(x, f, *fac[1:], 1))(batched(fac[0])),
+                 lambda: torch.vmap(lambda b: ops.cp4_conv2d(x, *fac, 1, bias=b))(batched(layer.bias)),
+                 lambda: torch.vmap(lambda t: cp4.conv2d_forward(t, *fac))(xs),
+                 lambda: torch.vmap(lambda t: cp4.conv2d_backward_data(t, *fac))(batched(dy)),
+                 lambda: torch.vmap(lambda t: cp4.conv2d_backward_filter(x, t, *fac)[0])(batched(dy))]
+    calls += [lambda: torch.func.grad(lambda t: layer(t).sum())(x),
+              lambda: torch.func.jvp(layer, (x,), (x,))]
+    xi = x.clone().requires_grad_()
+    y = layer(xi)
+    calls += [lambda: torch.autograd.grad(y, xi, torch.stack([dy, dy]), is_grads_batched=True)]
+    for call in calls:
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            call()
+
+
+def test_layer_on_a_side_stream(ops):
+    """Forward and backward run on the stream that is current at the forward call."""
+    layer, x = _small_layer(ops)
+    x = x.repeat(4, 1, 8, 8).requires_grad_()
+    dy = torch.randn_like(layer(x))
+    layer(x).backward(dy)
+    want = [x.grad] + [p.grad for p in layer.parameters()]
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    for _ in range(3):
+        x.grad = None
+        layer.zero_grad(set_to_none=True)
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            y = layer(x * 1)                      # (work of its own in front of it)
+            y.backward(dy)
+        torch.cuda.current_stream().wait_stream(side)
+        got = [x.grad] + [p.grad for p in layer.parameters()]
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
