@@ -63,10 +63,9 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
   // other wave takes them with the sign reversed and its partial sums are subtracted: the matrix
   // cores' sums come out low by a few hundredths of a unit in the last place whatever their sign, which
   // a sum over all pixels into the nearly cancelling factor gradients brings to the front
-  // (N32 T256 56x56 R32: G3's mean error 1.9e-8 of its deviation, 4e-11 with the signs
-  // reversed, 6.9e-9 in the contraction kernel; dFC 4.0e-6 of its norm off, 5.4e-7 with them, 1.3e-6.
-  // With 3, 5 or 7 waves one wave's share of the drift is left: dFC at N53 C128 T96 56x56 R32 1.2e-6, T224
-  // 4.9e-7; 1.6e-6 and 1.2e-6 with the contraction kernel).
+  // (N32 C256 T256 56x56 R32: G3's mean error 1.9e-8 of its deviation, 4e-11 with the signs reversed;
+  // dFC 4.0e-6 of its norm off, 5.4e-7 with them).  With 3, 5 or 7 waves one wave's share of the drift is
+  // left: dFC at N53 C128 T96 56x56 R32 1.2e-6, T224 4.9e-7.
   const float sign = wave & 1 ? -1.f : 1.f;
   u32x4 fh[2], fm[2], fl[2];
 #pragma unroll

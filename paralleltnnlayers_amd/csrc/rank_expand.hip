@@ -154,11 +154,22 @@ __global__ __launch_bounds__(kThreads, 2) void rank_expand_kernel(ExpandArgs a) 
 #pragma unroll
     for (int ch = 0; ch < KC; ++ch) split::split8(f[ch], ah[ch], am[ch], al[ch]);
     load_f(f, c0 + 32 < last ? c0 + 32 : c0);
+    // (the small partial products of all ranks before the large ones, so that most of the chain's
+    //  roundings are small)
 #pragma unroll
     for (int ch = 0; ch < KC; ++ch)
 #pragma unroll
-      for (int q = 0; q < PX; ++q)
-        acc[q] = split::mfma_split(ah[ch], am[ch], al[ch], bh[ch][q], bm[ch][q], bl[ch][q], acc[q]);
+      for (int q = 0; q < PX; ++q) {
+        acc[q] = split::mfma16(al[ch], bh[ch][q], acc[q]);
+        acc[q] = split::mfma16(am[ch], bm[ch][q], acc[q]);
+        acc[q] = split::mfma16(ah[ch], bl[ch][q], acc[q]);
+        acc[q] = split::mfma16(am[ch], bh[ch][q], acc[q]);
+        acc[q] = split::mfma16(ah[ch], bm[ch][q], acc[q]);
+      }
+#pragma unroll
+    for (int ch = 0; ch < KC; ++ch)
+#pragma unroll
+      for (int q = 0; q < PX; ++q) acc[q] = split::mfma16(ah[ch], bh[ch][q], acc[q]);
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const int c = c0 + 8 * (v >> 2) + 4 * hi + (v & 3);

@@ -235,12 +235,12 @@ def test_large_layer_behind_relu(capi, case, one_pass):
         assert ((g - w).abs() <= 4 * 2.0 ** -24 * (N * H * W) ** 0.5 * t).all()
 
 
-def _float64_factor_gradients(x, dy, fac, k):
-    """(dFK, dFC, dFH, dFW) of the layer without an epilogue, factor by factor in float64."""
+def _float64_gradients(x, dy, fac, k):
+    """(dFK, dFC, dFH, dFW, dx) of the layer without an epilogue, factor by factor in float64."""
     (N, C, H, W), P = x.shape, k // 2
-    FK, FC, FH, FW = leaves = [f.double().requires_grad_() for f in fac]
+    FK, FC, FH, FW, xd = leaves = [f.double().requires_grad_() for f in (*fac, x)]
     R = FK.shape[1]
-    A = torch.matmul(FC.t(), x.double().flatten(2)).view(N, R, H, W)
+    A = torch.matmul(FC.t(), xd.flatten(2)).view(N, R, H, W)
     A = torch.nn.functional.pad(A, (P, P, P, P))
     B = sum(FH[i].view(1, R, 1, 1) * A[:, :, i:i + H] for i in range(k))
     Z = sum(FW[j].view(1, R, 1, 1) * B[..., j:j + W] for j in range(k))
@@ -268,6 +268,31 @@ def test_large_layer_factor_gradients_do_not_drift(capi, case, bounds):
     dy = mk(*y.shape)
     _, grads, _ = capi.layer_backward(s, None, x, y, dy, *fac, "relu")
     assert capi.layer_last_backward_route() == capi.ROUTE_DY_PASS | capi.ROUTE_DX_FROM_G1
-    want = _float64_factor_gradients(x, dy * (y > 0), fac, k)
+    want = _float64_gradients(x, dy * (y > 0), fac, k)
     for g, w, bound in zip(grads, want, bounds):          # dFK, dFC
         assert float((g.double() - w).norm() / w.norm()) <= bound
+
+
+# The passes on their own, dx from their G1 (the gradients before the products of the high parts
+# had accumulators of their own: dx 2.3e-7 and dFC 7.4e-7 at T256, dx 1.8e-7 and dFC 1.1e-6 at T64; the
+# pass of dx from dy 1.8e-7 and 1.7e-7).  The bounds lie between those and what is measured now:
+# dx 1.5e-7 and 1.3e-7, dFC 2.8e-7 and 3.3e-7.
+@pytest.mark.parametrize("case,bounds", [
+    ((16, 256, 40, 40, 256, 3, 64), {4: 1.7e-7, 1: 5e-7}),
+    ((16, 64, 80, 80, 64, 3, 64), {4: 1.5e-7, 1: 5e-7}),
+], ids=["T256", "T64"])
+def test_gradients_of_the_passes_apart_do_not_drift(capi, case, bounds):
+    N, C, H, W, T, k, R = case
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x = mk(N, C, H, W).clamp_(min=0)
+    fac = [mk(d, R) * (2.0 / (C * k * k * R)) ** 0.125 for d in (T, C, k, k)]
+    s = capi.shape_for(x.shape, *fac, k // 2)
+    y = capi.layer_forward(s, None, x, *fac, 0.1 * mk(T), "relu")
+    dy = mk(*y.shape)
+    dx, grads, _ = capi.layer_backward(s, None, x, y, dy, *fac, "relu")
+    assert capi.layer_last_backward_route() == capi.ROUTE_DX_FROM_G1
+    want = _float64_gradients(x, dy * (y > 0), fac, k)
+    for i, bound in bounds.items():
+        got = (*grads, dx)[i]
+        assert float((got.double() - want[i]).norm() / want[i].norm()) <= bound
