@@ -275,13 +275,16 @@ __global__ __launch_bounds__(kSW) void contract_split_kernel(ContractArgs a) {
   __syncthreads();
   BSTAMP(a.dbg, 0, dwg, 8, 2)
   const u32x4* fbase = reinterpret_cast<const u32x4*>(Fb + hi * 512 + l32 * 16);
-  // Software pipeline: while the six MFMAs of chunk c run, the vector ALU splits chunk c+1.
-  // (fp32: the products of the high parts have an accumulator of their own and the small ones
-  // the other, so a chunk rounds once at the sum's magnitude; with three there and three here
-  // dx = FC G1 was up to 23 % further from float64 than the pass from dy, and dFC, dFH and dFW, where
-  // the rounding's bias adds up over the pixels, 3 to 5 times as far off as now: N16 C256 T256 40x40
-  // R64: dx 2.3e-7 of its norm, now 1.5e-7, the pass 1.8e-7; dFH 8.6e-7, now 1.9e-7.)
+  // Software pipeline: while the six MFMAs of chunk c run (accumulators in turn, so that they
+  // do not wait for each other), the vector ALU splits chunk c+1.
+  // (fp32: acc1 takes the products of the high parts alone, so a chunk rounds once at the sum's
+  // magnitude; with three roundings there dx = FC G1 was up to 23 % further from float64 than the
+  // pass from dy, and dFC, dFH and dFW, where the rounding's bias adds up over the pixels, 3 to 5
+  // times as far off as now: N16 C256 T256 40x40 R64: dx 2.3e-7 of its norm, now 1.5e-7, the pass
+  // 1.8e-7; dFH 8.6e-7, now 1.9e-7.  Two accumulators, the small products in a row: N64 C256 14x14
+  // R64 34.25 us for the whole pass, 34.1 with three, 33.95 before.)
   f32x16 acc0 = (f32x16)(0.f), acc1 = (f32x16)(0.f);
+  [[maybe_unused]] f32x16 acc2 = (f32x16)(0.f);
   u32x4 xh, xm, xl;
 #ifdef CP4_BWF_HALF
   // half-precision activations: widened, then two bf16 parts
@@ -341,17 +344,17 @@ __global__ __launch_bounds__(kSW) void contract_split_kernel(ContractArgs a) {
         acc0 = mfma16(fl, xh, acc0);
         piece(0);
         __builtin_amdgcn_sched_barrier(0);
-        acc0 = mfma16(fm, xm, acc0);
+        acc2 = mfma16(fm, xm, acc2);
         piece(1);
         __builtin_amdgcn_sched_barrier(0);
         acc0 = mfma16(fh, xl, acc0);
         piece(2);
         __builtin_amdgcn_sched_barrier(0);
-        acc1 = mfma16(fh, xh, acc1);
+        acc2 = mfma16(fm, xh, acc2);
         piece(3);
         __builtin_amdgcn_sched_barrier(0);
-        acc0 = mfma16(fm, xh, acc0);
         acc0 = mfma16(fh, xm, acc0);
+        acc1 = mfma16(fh, xh, acc1);
         ld_chunk(nx, c + 1 + kSplitRing);             // refill the slot just split
 #endif
       }
@@ -361,7 +364,11 @@ __global__ __launch_bounds__(kSW) void contract_split_kernel(ContractArgs a) {
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+#ifdef CP4_BWF_IO16
   f32x16 acc = acc0 + acc1;
+#else
+  f32x16 acc = (acc0 + acc2) + acc1;
+#endif
   BSTAMP(a.dbg, 0, dwg, 8, 3)
   float* zn = a.Z[which] + (size_t)n * R * HW + p;
   if (ks == 1) {
