@@ -64,8 +64,8 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
   // cores' sums come out low by a few hundredths of a unit in the last place whatever their sign, which
   // a sum over all pixels into the nearly cancelling factor gradients brings to the front
   // (N32 C256 T256 56x56 R32: G3's mean error 1.9e-8 of its deviation, 4e-11 with the signs reversed;
-  // dFC 4.0e-6 of its norm off, 5.4e-7 with them).  With 3, 5 or 7 waves one wave's share of the drift is
-  // left: dFC at N53 C128 T96 56x56 R32 1.2e-6, T224 4.9e-7.
+  // dFC 4.2e-6 of its norm off, 2.9e-7 with them).  With 3, 5 or 7 waves one wave's share of the drift is
+  // left: dFC at N53 C128 T96 56x56 R32 1.0e-6, at N27 T224 4.0e-7.
   const float sign = wave & 1 ? -1.f : 1.f;
   u32x4 fh[2], fm[2], fl[2];
 #pragma unroll
@@ -124,9 +124,9 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
     }
   };
   // dFK, with the opposite sign after every other chunk (those chunks' Cc has it reversed), for
-  // the same reason as above: a workgroup's chunks are one chain of sums.  (dFK of N27 C128 T256 56x56
-  // R32: 4.1e-7 of its norm off without, 3.3e-7 with, 3.8e-7 in the gradient GEMM; N105 T64: 5.8e-7,
-  // 3.4e-7, 7.4e-7.  No time: 57 shapes within 0.3 % of each other on the mean.)
+  // the same reason as above: a workgroup's chunks are one chain of sums.  (dFK of N32 C256 T256 56x56
+  // R32: 4.3e-7 of its norm off without, 3.2e-7 with; N128 C128 T64: 6.8e-7, 3.4e-7.  No time: 57
+  // shapes within 0.3 % of each other on the mean.)
   f32x16 accK = (f32x16)(0.f);
   float bs[8];
 #pragma unroll

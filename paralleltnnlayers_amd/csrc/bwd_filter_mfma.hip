@@ -1190,6 +1190,14 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
   f32x16 acc[RB];
 #pragma unroll
   for (int mb = 0; mb < RB; ++mb) acc[mb] = (f32x16)(0.f);
+#ifndef CP4_BWF_IO16
+  // the partial products below the high parts': one rounding a step at the sum's magnitude, not
+  // six (N105 C128 T64 56x56 R32: dFK 7.2e-7 of its norm off float64, now 2.1e-7; the backward
+  // calls of 62 fp32 layers 0.3 % longer on the mean)
+  f32x16 small[RB];
+#pragma unroll
+  for (int mb = 0; mb < RB; ++mb) small[mb] = (f32x16)(0.f);
+#endif
   if (ch0 < ch1) load_tiles(ch0);
   for (int ch = ch0; ch < ch1; ++ch) {
     const int buf = (ch - ch0) & 1;
@@ -1234,12 +1242,21 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
 #pragma unroll
       for (int mb = 0; mb < RB; ++mb) {
         const u32x4* zp = &Zf[buf][((mb * 2 + st) * 3 * 2 + hi) * 32 + l32];
-        acc[mb] = mfma_split(ah, am, al, zp[0], zp[64], zp[128], acc[mb]);
+        small[mb] = mfma16(al, zp[0], small[mb]);
+        small[mb] = mfma16(am, zp[64], small[mb]);
+        small[mb] = mfma16(ah, zp[128], small[mb]);
+        acc[mb] = mfma16(ah, zp[0], acc[mb]);
+        small[mb] = mfma16(am, zp[0], small[mb]);
+        small[mb] = mfma16(ah, zp[64], small[mb]);
       }
 #endif
     }
   }
   BSTAMP(a.dbg, 1, dwg, 4, 4)
+#ifndef CP4_BWF_IO16
+#pragma unroll
+  for (int mb = 0; mb < RB; ++mb) acc[mb] += small[mb];
+#endif
   float* out = a.part[which] + (size_t)s * D * R;
 #pragma unroll
   for (int mb = 0; mb < RB; ++mb)
