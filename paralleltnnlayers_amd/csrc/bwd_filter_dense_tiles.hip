@@ -400,8 +400,17 @@ __device__ __forceinline__ void split4(const float (&v)[4], u32x2& h, u32x2& m, 
 // fixed channels, so a sum is one register a slot.  y's cells wait in registers beside dy's: the
 // build holds half the accumulators, and stays within 128 registers.  (N16 C3 K64 224x224, dy
 // and y 411 MB: 94 us against 119 for a pass that writes the masked dy and 64 for this
-// kernel on it.)
-template <int FS, int MB, bool M16, bool MASK>
+// kernel on it.  The layer's backward pass against the one with the mask apart, 61 layers of T 1-64,
+// C 1-16, filters 1-5, 28x28 to 224x224 with odd planes: 1.07 to 1.87 times as fast on each.)
+//
+// BALANCE (masked builds): half the accumulators can mean that fewer waves share the pixels,
+// whose chains of sums are longer then.  The matrix cores' sums come out low by a little whatever
+// their sign, and round six times a step.  Here dy's second half of a tile has the sign reversed (the
+// first one of the next tile, too), and the accumulators with it; a step's products are
+// added up apart and go to the accumulators in one correctly rounded addition.  N16 C16 K48 112x112 3x3
+// R16, distance from float64 in the 2-norm: dFK 5.8e-7 without, 2.2e-7 with, 4.3e-7 in the plain
+// build; dFH 9.4e-7, 2.6e-7, 6.7e-7; 4 to 6 % of the pass's time.
+template <int FS, int MB, bool M16, bool MASK, bool BALANCE>
 __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kernel(BwdFilterArgs a, MfmaPlan pl,
                                                                   float* partial) {
   // blocks of BW x BW entries of dK, steps of 2^SPLG pixels, NV accumulator registers a block
@@ -523,8 +532,9 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
       held[q] = v;
     }
   };
-  // The registers, split, into buffer `buf`.
-  auto deposit = [&](char* buf) {
+  // The registers, split, into buffer `buf` (BALANCE: dy of the tile's second half, or in a tile of
+  // odd index of its first, with the sign reversed).
+  auto deposit = [&](char* buf, [[maybe_unused]] int index) {
 #pragma unroll
     for (int q = 0; q < SLOTS; ++q) {
       const int g = tid + THREADS * q;
@@ -537,10 +547,15 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
         if constexpr (MASK) {
           // (a product, as dy * (y > 0): a non-finite dy at a clipped output stays visible)
           const float yv[4] = {act[q].x, act[q].y, act[q].z, act[q].w};
+          float one = 1.f;
+          if constexpr (BALANCE) {
+            const int st = ((rc[q] >> 16) << lgcw) + ((rc[q] & 0xffff) >> SPLG);
+            if (!isx && (st >= nsteps / 2) != (index & 1)) one = -1.f;
+          }
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            v[i] *= yv[i] > 0.f ? 1.f : 0.f;
-            bsum[q] += v[i];
+            v[i] *= yv[i] > 0.f ? one : 0.f;
+            bsum[q] += one * v[i];
           }
         }
         u32x2 h, m, l;
@@ -556,9 +571,17 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
   const TileRange tr = tiles_of_workgroup(pl.ntiles);
   if (tr.first < tr.end) {
     fetch(tr.first);
-    deposit(bufs);
+    deposit(bufs, 0);
   }
   __syncthreads();
+  [[maybe_unused]] auto negate = [&] {
+#pragma unroll
+    for (int o = 0; o < OWN; ++o)
+#pragma unroll
+      for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) acc[o][m][v] = -acc[o][m][v];
+  };
   int it = 0;
   for (int t = tr.first; t < tr.end; t += tr.step, ++it) {
     const bool more = t + tr.step < tr.end;
@@ -568,7 +591,14 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
     const char* dp = cur + 6 * pl.xplane;
     const int xw = pl.xplane >> 1;                     // a plane of x in dwords
     // ---- this wave's steps ----
+    [[maybe_unused]] bool first_half = true;
     for (int st = sl; st < nsteps; st += pl.slices) {
+      if constexpr (BALANCE) {
+        if (first_half && st >= nsteps / 2) {
+          negate();
+          first_half = false;
+        }
+      }
       const int row = st >> lgcw, col0 = (st & ((1 << lgcw) - 1)) << SPLG;
       u32x4 ah[MB], am[MB], al[MB];
 #pragma unroll
@@ -619,15 +649,23 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
             const unsigned shift = (unsigned)(boff[o] & 1) * 16u;
             const u32x4 bh = funnel(dh, shift), bm = funnel(dm, shift), bl = funnel(dl, shift);
 #pragma unroll
-            for (int m = 0; m < MB; ++m)
-              acc[o][m] = mfma_split_any(ah[m], am[m], al[m], bh, bm, bl, acc[o][m]);
+            for (int m = 0; m < MB; ++m) {
+              if constexpr (BALANCE)
+                acc[o][m] += mfma_split_any(ah[m], am[m], al[m], bh, bm, bl, Acc{});
+              else
+                acc[o][m] = mfma_split_any(ah[m], am[m], al[m], bh, bm, bl, acc[o][m]);
+            }
           }
         }
       }
     }
-    if (more) deposit(bufs + (size_t)((it + 1) & 1) * pl.bufbytes);
+    if constexpr (BALANCE)
+      if (first_half) negate();
+    if (more) deposit(bufs + (size_t)((it + 1) & 1) * pl.bufbytes, it + 1);
     __syncthreads();
   }
+  if constexpr (BALANCE)
+    if (it & 1) negate();
   if constexpr (MASK) {
     // ---- the bias gradient's part: the slots of a channel, in order ----
     if (a.dbias) {
@@ -1130,14 +1168,17 @@ bool mfma_plan(const cp4_shape& s, bool aligned16, MfmaPlan* best, bool masked =
 }
 
 template <int FS>
-hipError_t launch_mfma_fs(const BwdFilterArgs& a, const MfmaPlan& pl, float* partial, hipStream_t st) {
-  auto k0 = dense_mfma_kernel<FS, 1, true, false>;
-  auto k02 = dense_mfma_kernel<FS, 2, true, false>;
-  auto k1 = dense_mfma_kernel<FS, 1, false, false>;
-  auto k2 = dense_mfma_kernel<FS, 2, false, false>;
+hipError_t launch_mfma_fs(const BwdFilterArgs& a, const MfmaPlan& pl, bool balance, float* partial,
+                          hipStream_t st) {
+  auto k0 = dense_mfma_kernel<FS, 1, true, false, false>;
+  auto k02 = dense_mfma_kernel<FS, 2, true, false, false>;
+  auto k1 = dense_mfma_kernel<FS, 1, false, false, false>;
+  auto k2 = dense_mfma_kernel<FS, 2, false, false, false>;
   auto k = pl.m16 ? (pl.MB == 2 ? k02 : k0) : (pl.MB == 2 ? k2 : k1);
-  if (a.act_y || a.dbias)
-    k = pl.MB == 2 ? dense_mfma_kernel<FS, 2, true, true> : dense_mfma_kernel<FS, 1, true, true>;
+  if ((a.act_y || a.dbias) && balance)
+    k = pl.MB == 2 ? dense_mfma_kernel<FS, 2, true, true, true> : dense_mfma_kernel<FS, 1, true, true, true>;
+  else if (a.act_y || a.dbias)
+    k = pl.MB == 2 ? dense_mfma_kernel<FS, 2, true, true, false> : dense_mfma_kernel<FS, 1, true, true, false>;
   if (pl.lds_bytes > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds_bytes);
@@ -1285,21 +1326,26 @@ hipError_t bwd_filter_dense_tiles_launch(const BwdFilterArgs& a, hipStream_t st)
     MfmaPlan pl;
     if (!mfma_plan(s, aligned16, &pl, masked) && !mfma_plan(s, false, &pl, masked))
       return hipErrorInvalidValue;
+    bool balance = false;
     if (masked) {
       // the workspace has room for the partial sets of the plain build's plans; smaller tiles
       // could give this one more workgroups
       MfmaPlan plain;
-      int most = 0;
+      int most = 0, chains = 0;                        // (waves that share an entry's pixels)
       for (const bool al : {false, true})
-        if (mfma_plan(s, al, &plain) && plain.grid > most) most = plain.grid;
+        if (mfma_plan(s, al, &plain)) {
+          most = std::max(most, plain.grid);
+          chains = std::max(chains, plain.grid * plain.slices);
+        }
       if (pl.grid > most) pl.grid = most;
       if (pl.grid < 1) return hipErrorInvalidValue;
+      balance = pl.grid * pl.slices < chains;
     }
     sets = pl.grid;
     switch (a.Y) {
-      case 1: e = launch_mfma_fs<1>(a, pl, partial, st); break;
-      case 3: e = launch_mfma_fs<3>(a, pl, partial, st); break;
-      default: e = launch_mfma_fs<5>(a, pl, partial, st); break;
+      case 1: e = launch_mfma_fs<1>(a, pl, balance, partial, st); break;
+      case 3: e = launch_mfma_fs<3>(a, pl, balance, partial, st); break;
+      default: e = launch_mfma_fs<5>(a, pl, balance, partial, st); break;
     }
   } else {
     DensePlan pl;
