@@ -553,10 +553,8 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
             if (!isx && (st >= nsteps / 2) != (index & 1)) one = -1.f;
           }
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            v[i] *= yv[i] > 0.f ? one : 0.f;
-            bsum[q] += one * v[i];
-          }
+          for (int i = 0; i < 4; ++i) v[i] *= yv[i] > 0.f ? one : 0.f;
+          bsum[q] += one * ((v[0] + v[1]) + (v[2] + v[3]));
         }
         u32x2 h, m, l;
         split4(v, h, m, l);
@@ -677,9 +675,14 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
       __syncthreads();
       const int per = pl.DS >> 2;
       if (tid < a.T) {
-        float s = 0.f;
-        for (int i = 0; i < per; ++i) s += lds[tid * per + i];
-        a.bias_part[(size_t)blockIdx.x * a.T + tid] = s;
+        float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        int i = 0;
+        for (; i + 8 <= per; i += 8)
+#pragma unroll
+          for (int u = 0; u < 8; ++u) s[u] += lds[tid * per + i + u];
+        for (; i < per; ++i) s[0] += lds[tid * per + i];
+        a.bias_part[(size_t)blockIdx.x * a.T + tid] =
+            ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
       }
       __syncthreads();
     }
