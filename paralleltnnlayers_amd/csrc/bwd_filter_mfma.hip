@@ -16,7 +16,8 @@
 //   3. grad_split_kernel: dF[d,r] = sum_{n,p} act[n,d,p] Z[n,r,p] as split products,
 //      split over images (and pixel ranges) across workgroups, the Z tile split once
 //      per 32-pixel chunk into double-buffered B fragments in LDS.  grad_gemm_kernel
-//      (fp32 MFMA) where rows cannot move as 16-byte vectors.
+//      (fp32 MFMA) on planes of an even number of pixels that is no multiple of four, or
+//      with operands off a 16-byte boundary.
 //   4. reduce_sets_kernel: fixed-order sum of the per-workgroup partials (bit-reproducible).
 // The library's choice for large problems and for shapes the three-launch variant
 // (bwd_filter_fused.hip) does not take; also the strided layer's pass and the
@@ -1116,8 +1117,8 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
     return v;
   };
 #endif
-  // VEC: H*W is a multiple of 4 and the operands are 16-byte aligned, rows move
-  // as float4; otherwise element by element with per-pixel bounds.
+  // kRowsVec: a float4; kRowsAny: four floats at any element, moved back to end with the row
+  // (settle() puts them where they belong); kRowsEach: one by one with per-pixel bounds.
   auto load4 = [&](const float* row, int p) {
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (ROWS == kRowsAny) {

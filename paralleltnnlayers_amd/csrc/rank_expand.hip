@@ -12,9 +12,9 @@
 // workgroup share the pixels and differ in the channel slice where there are slices, and
 // workgroups of one die (blockIdx & 7) take a contiguous range of the pixels, so that cache
 // lines that two blocks share meet in one L2.
-// N32 C256 56x56 R32 fp32 (103 MB written, 13 MB read): 29 us; the backward-data pass from dy takes 56.
-// (Stores that leave the caches alone take 24 us here and as much more in what runs beside them: 26
-// layers of 48 to 270 MB, no backward call more than 0.7 % apart on the best of five.)
+// N32 C256 56x56 R32 fp32 (103 MB written, 13 MB read): 26 us in a training step; the backward-data
+// pass from dy takes 56.  (Stores that leave the caches alone make no difference to a backward
+// call: 26 layers of 48 to 270 MB, none more than 1 % apart on the best of five.)
 // The factor gradients' four-launch variant and its strided and 16-bit siblings bring dx along
 // wherever they run: 100 layers (fp32 and bf16, C and T 16-256, R 8-64 also beyond C and T, filters
 // 1-5, stride 1 and 2) took 0.99 to 1.82 times as long with the pass of its own (C = T = 16, R 64,
