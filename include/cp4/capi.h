@@ -473,6 +473,9 @@ enum {
   CP4_ROUTE_DX_FROM_G1 = 4    /* the input gradient from the factor gradients' G1 plane */
 };
 int cp4_layer_last_backward_route(void);
+/* 1 if its mask and bias gradient ran inside the contraction and the gradient GEMM of the factor
+ * gradients' passes on their own, without a pass of theirs; else 0. */
+int cp4_layer_last_backward_mask_inside(void);
 
 /* ---- 3-factor CP sibling op ------------------------------------------------
  * Stands where the reference registers its TensorFlow op Conv2dCpFusedNchw

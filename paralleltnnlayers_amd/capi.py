@@ -600,6 +600,11 @@ def layer_last_backward_route():
     return lib().cp4_layer_last_backward_route()
 
 
+def layer_last_backward_mask_inside():
+    """Whether its mask and bias gradient ran inside the factor gradients' passes on their own."""
+    return bool(lib().cp4_layer_last_backward_mask_inside())
+
+
 def conv2d_backward_data(dy, FK, FC, FH, FW, pad=1, out=None, stream=None):
     if stream is None or out is not None:              # (allocates dx only)
         return _native.backward_data(dy, FK, FC, FH, FW, pad, out, stream)

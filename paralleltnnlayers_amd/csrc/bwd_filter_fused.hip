@@ -45,16 +45,17 @@ struct ContractAllArgs {
   int Cin0, Cin1;
   int R, HW, npb, items;   // items per operand = N * npb (32-pixel blocks)
   int vecfill;             // both factors 16-byte aligned and R a multiple of 4
+  const float* y;          // masked build: dy counts where y > 0 ...
+  float* masked;           // ... and is written so to here
 };
 
 // x / dy and the factor are read through buffer descriptors: an address is
 // (descriptor base) + (32-bit lane offset) + (scalar offset), so the walk over
 // channels runs on the scalar unit and a load costs no vector instruction.
-template <int RB, int KS, int RING>
-__global__ __launch_bounds__(512) void contract_all_kernel(ContractAllArgs a) {
+template <int RB, int KS, int RING, bool MASK>
+__device__ __forceinline__ void contract_all(const ContractAllArgs& a, const int which) {
   extern __shared__ float Fs[];
   unsigned char* Fb = reinterpret_cast<unsigned char*>(Fs);
-  const int which = blockIdx.y;
   const int Cin = which ? a.Cin1 : a.Cin0, R = a.R, HW = a.HW;
   const float* src = which ? a.src1 : a.src0;
   const float* F = which ? a.F1 : a.F0;
@@ -73,24 +74,45 @@ __global__ __launch_bounds__(512) void contract_all_kernel(ContractAllArgs a) {
   const int nch = (Cin >> 4) / KS, c0 = part * nch;   // this wave's chunks c0 .. c0 + nch - 1
   const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(src + (size_t)n * Cin * HW), 0, Cin * HW * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t yrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>((MASK ? a.y : src) + (size_t)n * Cin * HW), 0, Cin * HW * 4, 0x00020000);
   const unsigned voff = (unsigned)(8 * hi * HW + pc) * 4u;   // lane's channel 16*chunk + 8*hi + e
   const unsigned sbase = (unsigned)(16 * c0) * (unsigned)HW * 4u;
   float xb[RING][8];
+  [[maybe_unused]] float yb[MASK ? RING : 1][8];             // y's, of the same chunks
   // (Every load of the sweep is issued on every path - chunks past the wave's last are
   // clamped to it - so that the count of loads in flight at each wait is a constant the
   // compiler can put into the wait instruction; a load skipped on some path makes it
   // wait for the youngest load instead of the one it needs.)
-  auto ld_chunk = [&](float (&dst)[8], int ch) {
+  auto ld_chunk = [&](int slot, int ch) {
     ch = ch < nch ? ch : nch - 1;
     const unsigned soff = sbase + (unsigned)(16 * ch) * (unsigned)HW * 4u;
 #pragma unroll
     for (int e = 0; e < 8; ++e)
-      dst[e] = __builtin_bit_cast(
+      xb[slot][e] = __builtin_bit_cast(
           float, __builtin_amdgcn_raw_buffer_load_b32(xrs, voff, soff + (unsigned)e * HW * 4u, 0));
+    if constexpr (MASK)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        yb[slot][e] = __builtin_bit_cast(
+            float, __builtin_amdgcn_raw_buffer_load_b32(yrs, voff, soff + (unsigned)e * HW * 4u, 0));
+  };
+  // the chunk of a ring slot behind the activation, and that into memory.  (A product, as dy *
+  // (y > 0): a non-finite dy at a clipped output stays visible.)
+  auto mask_chunk = [&](int slot, int ch) {
+    if constexpr (MASK) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xb[slot][e] *= yb[slot][e] > 0.f ? 1.f : 0.f;
+      if (ch < nch && valid) {
+        float* out = a.masked + ((size_t)n * Cin + 16 * (c0 + ch) + 8 * hi) * HW + p;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) out[(size_t)e * HW] = xb[slot][e];
+      }
+    }
   };
   // the first activation chunks are requested before the factor tile is built
 #pragma unroll
-  for (int u = 0; u < RING; ++u) ld_chunk(xb[u], u);
+  for (int u = 0; u < RING; ++u) ld_chunk(u, u);
   // factor tile: fragment entry (channel octet o, rank rr) = the three bf16 parts of
   // F[8o .. 8o+7][rr], 16 bytes each
   {
@@ -171,8 +193,9 @@ __global__ __launch_bounds__(512) void contract_all_kernel(ContractAllArgs a) {
     const u32x4* fbase = reinterpret_cast<const u32x4*>(Fb + hi * 512 + l32 * 16);
     const int zero_chunk = Cin >> 4;                   // an all-zero fragment block behind the tile
     u32x4 xh, xm, xl;
+    mask_chunk(0, 0);
     split8(xb[0], xh, xm, xl);
-    ld_chunk(xb[0], RING);
+    ld_chunk(0, RING);
     // rounds of RING chunks; chunks past the last multiply the zero block
     for (int ch = 0; ch < nch; ch += RING) {
 #pragma unroll
@@ -180,6 +203,7 @@ __global__ __launch_bounds__(512) void contract_all_kernel(ContractAllArgs a) {
         const int c = ch + u;                          // chunk whose parts are in xh / xm / xl
         const u32x4* fp = fbase + (size_t)(c < nch ? c0 + c : zero_chunk) * RB * (kFragBytes / 16);
         float (&nx)[8] = xb[(u + 1) % RING];
+        mask_chunk((u + 1) % RING, c + 1);
         u32x4 nh, nm, nl;
         auto piece = [&](int d) {                      // a quarter of the next chunk's split
           const float x0 = nx[2 * d], x1 = nx[2 * d + 1];
@@ -229,7 +253,7 @@ __global__ __launch_bounds__(512) void contract_all_kernel(ContractAllArgs a) {
           acc[0] = mfma16(fh0, xh, acc[0]);
           acc[1] = mfma16(fh1, xh, acc[1]);
         }
-        ld_chunk(nx, c + 1 + RING);                    // refill the slot just split
+        ld_chunk((u + 1) % RING, c + 1 + RING);        // refill the slot just split
         xh = nh;
         xm = nm;
         xl = nl;
@@ -276,6 +300,12 @@ __global__ __launch_bounds__(512) void contract_all_kernel(ContractAllArgs a) {
     }
 }
 
+template <int RB, int KS, int RING, bool MASK>
+__global__ __launch_bounds__(512) void contract_all_kernel(ContractAllArgs a) {
+  if (MASK && blockIdx.y) contract_all<RB, KS, RING / 2, true>(a, 1);     // (as many loads in flight)
+  else contract_all<RB, KS, RING, false>(a, blockIdx.y);
+}
+
 // ---- 2. taps in LDS + gradient GEMMs + tap gradients --------------------------------
 struct FusedArgs {
   const float *act0, *act1;     // dy, x            (gradient 0: dFK, 1: dFC)
@@ -284,6 +314,7 @@ struct FusedArgs {
   const float *FH, *FW;
   float *part0, *part1;         // [S][D][R]
   float *partH, *partW;         // [S * TG][FS][R]
+  float* partB;                 // [S][D0] sums of dy's rows, the layer's bias gradient; may be null
   int D0, D1;
   int N, R, H, W, P, HW;
   int TG;                     // channel groups of dFK that share the tap gradients (1 or 2)
@@ -338,6 +369,8 @@ __global__ __launch_bounds__(512) void grad_fused_kernel(FusedArgs a) {
   f32x16 acc[RB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) acc[rb] = (f32x16)(0.f);
+  const bool sums = which == 0 && a.partB;
+  float bs = 0.f;                      // this lane's share of the sum of row d
   const float* Zs = which ? a.Zsrc1 : a.Zsrc0;
   const float* act = which ? a.act1 : a.act0;
 
@@ -545,6 +578,11 @@ __global__ __launch_bounds__(512) void grad_fused_kernel(FusedArgs a) {
         float4 rv[2] = {ring[u][0], ring[u][1]};
         issue(ring[u], s + kRing * KH);
         gemm_step(rv, s);
+        if (sums) {                    // (pixels of this strip: the others are a clamped load's)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            if (q0 + 16 * s + 8 * hi + 4 * j < q1) bs += (rv[j].x + rv[j].y) + (rv[j].z + rv[j].w);
+        }
         // keep the steps in program order: the refill above must stay behind the loads
         // of the following steps, or their waits would cover it too
         __builtin_amdgcn_sched_barrier(0);
@@ -593,6 +631,19 @@ __global__ __launch_bounds__(512) void grad_fused_kernel(FusedArgs a) {
         }
     }
   }
+  if (sums) {
+    // the two halves of a row's lanes, then the KH waves of its channel tile in order
+    bs += __shfl_down(bs, 32, 64);
+    __syncthreads();
+    if (hi == 0) red[wave * 32 + l32] = bs;
+    __syncthreads();
+    if (kh == 0 && hi == 0 && drow) {
+      float t = bs;
+      for (int k2 = 1; k2 < KH; ++k2) t += red[(wave + k2) * 32 + l32];
+      a.partB[(size_t)sidx * D + d] = t;
+    }
+    __syncthreads();
+  }
   if (tapgroup) {
     // thread t holds sums of rank t % RP: fixed-order sum over the 512 / RP threads of a rank
 #pragma unroll
@@ -613,11 +664,11 @@ __global__ __launch_bounds__(512) void grad_fused_kernel(FusedArgs a) {
   }
 }
 
-// ---- 3. out[i] = sum_s partial[s][i], four segments in one launch -------------------
+// ---- 3. out[i] = sum_s partial[s][i], up to five segments in one launch -------------------
 struct ReduceFusedArgs {
-  const float* part[4];
-  float* out[4];
-  int count[4], S[4];
+  const float* part[5];
+  float* out[5];
+  int count[5], S[5];
 };
 // A workgroup owns 64 consecutive outputs; its four waves each sum a quarter of the
 // S partials in index order, then the quarter sums are added in wave order.
@@ -763,6 +814,8 @@ size_t bwd_filter_fused_workspace_bytes(const cp4_shape& s) {
   return (2 * p.plane + p.part_elems) * sizeof(float);
 }
 
+int bwd_filter_fused_bias_sets(const cp4_shape& s) { return make_fused_plan(s).S; }
+
 hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
   cp4_shape s{};
   s.N = a.N; s.C = a.C; s.T = a.T; s.H = a.H; s.W = a.W; s.pad = a.pad; s.Y = a.Y; s.X = a.X;
@@ -781,16 +834,19 @@ hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
   c.src0 = a.x; c.F0 = a.FC; c.Z0 = A; c.Cin0 = a.C;
   c.src1 = a.dy; c.F1 = a.FK; c.Z1 = G3; c.Cin1 = a.T;
   c.R = R; c.HW = HW; c.npb = (HW + 31) / 32; c.items = N * c.npb;
+  c.y = a.act_y; c.masked = a.mask_ws;
   c.vecfill = (R & 3) == 0 && ((reinterpret_cast<uintptr_t>(a.FC) | reinterpret_cast<uintptr_t>(a.FK)) & 15) == 0;
   const long slots = (long)c.items * p.ks;
   const dim3 cgrid((unsigned)((slots + p.nw - 1) / p.nw), 2);
   hipError_t e;
 #define CP4_CONTRACT(RB_, KS_, RING_)                                                          \
   {                                                                                            \
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(contract_all_kernel<RB_, KS_, RING_>), \
+    auto k = c.y ? contract_all_kernel<RB_, KS_, RING_, true>                                  \
+                 : contract_all_kernel<RB_, KS_, RING_, false>;                                \
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),                                  \
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds_contract);  \
     if (e != hipSuccess) return e;                                                             \
-    contract_all_kernel<RB_, KS_, RING_><<<cgrid, p.nw * 64, p.lds_contract, st>>>(c);         \
+    k<<<cgrid, p.nw * 64, p.lds_contract, st>>>(c);                                            \
   }
 #define CP4_CONTRACT_KS(RB_, RING_)                                                            \
   {                                                                                            \
@@ -807,9 +863,10 @@ hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
 #undef CP4_CONTRACT
 
   FusedArgs g{};
-  g.act0 = a.dy; g.Zsrc0 = A; g.part0 = pK; g.D0 = a.T;
+  g.act0 = a.act_y ? a.mask_ws : a.dy; g.Zsrc0 = A; g.part0 = pK; g.D0 = a.T;
   g.act1 = a.x; g.Zsrc1 = G3; g.part1 = pC; g.D1 = a.C;
   g.FH = a.FH; g.FW = a.FW; g.partH = pH; g.partW = pW;
+  g.partB = a.dbias ? a.bias_part : nullptr;
   g.N = N; g.R = R; g.H = a.H; g.W = a.W; g.P = a.pad; g.HW = HW;
   g.TG = p.TG; g.TH = p.TH; g.NS = p.NS; g.items = p.items; g.S = p.S; g.MT = p.MT;
   g.Wp = p.Wp; g.PSt = p.PSt; g.KSmax = p.KSmax;
@@ -835,16 +892,16 @@ hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
 #undef CP4_FUSED
 
   ReduceFusedArgs r{};
-  const float* parts[4] = {pK, pC, pH, pW};
-  float* outs[4] = {a.dFK, a.dFC, a.dFH, a.dFW};
-  const int counts[4] = {a.T * R, a.C * R, FS * R, FS * R};
+  const float* parts[5] = {pK, pC, pH, pW, a.bias_part};
+  float* outs[5] = {a.dFK, a.dFC, a.dFH, a.dFW, a.dbias};
+  const int counts[5] = {a.T * R, a.C * R, FS * R, FS * R, a.dbias ? a.T : 0};
+  const int Ss[5] = {p.S, p.S, p.S * p.TG, p.S * p.TG, p.S};
   int maxc = 0;
-  for (int i = 0; i < 4; ++i) {
-    r.part[i] = parts[i]; r.out[i] = outs[i]; r.count[i] = counts[i];
-    r.S[i] = i < 2 ? p.S : p.S * p.TG;
+  for (int i = 0; i < 5; ++i) {
+    r.part[i] = parts[i]; r.out[i] = outs[i]; r.count[i] = counts[i]; r.S[i] = Ss[i];
     if (counts[i] > maxc) maxc = counts[i];
   }
-  reduce_fused_kernel<<<dim3((maxc + 63) / 64, 4), 256, 0, st>>>(r);
+  reduce_fused_kernel<<<dim3((maxc + 63) / 64, a.dbias ? 5 : 4), 256, 0, st>>>(r);
   return hipGetLastError();
 }
 

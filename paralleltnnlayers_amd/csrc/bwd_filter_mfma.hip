@@ -22,8 +22,10 @@
 // The library's choice for large problems and for shapes the three-launch variant
 // (bwd_filter_fused.hip) does not take; also the strided layer's pass and the
 // 3-factor op's (depthwise-filter tap step).
+#include <algorithm>
 #include <cstdint>
 #include <cstdlib>
+#include <type_traits>
 
 #include "cp4_internal.h"
 #ifdef CP4_DEBUG_PHASES
@@ -77,6 +79,25 @@ using act_t = float;
 [[maybe_unused]] __device__ __forceinline__ float act_to_f32(act_t v) { return v; }
 #endif
 
+// dy behind a ReLU, as dy * (y > 0): a non-finite dy at a clipped output stays visible.
+#ifdef CP4_BWF_HALF
+[[maybe_unused]] __device__ __forceinline__ unsigned masked_act(unsigned d, unsigned y) {
+  const _Float16 m = __builtin_bit_cast(_Float16, (act_t)d) *
+                     (__builtin_bit_cast(_Float16, (act_t)y) > (_Float16)0 ? (_Float16)1 : (_Float16)0);
+  return __builtin_bit_cast(act_t, m);
+}
+#elif defined(CP4_BWF_IO16)
+// (the product with 0 or 1 is a bfloat16 value: its high half is all of it)
+[[maybe_unused]] __device__ __forceinline__ unsigned masked_act(unsigned d, unsigned y) {
+  const float m = __uint_as_float(d << 16) * (__uint_as_float(y << 16) > 0.f ? 1.f : 0.f);
+  return __float_as_uint(m) >> 16;
+}
+#else
+[[maybe_unused]] __device__ __forceinline__ float masked_act(float d, float y) {
+  return d * (y > 0.f ? 1.f : 0.f);
+}
+#endif
+
 using split::f32x16;
 
 [[maybe_unused]] __device__ __forceinline__ f32x16 mfma32(float a, float b, f32x16 c) {
@@ -104,8 +125,12 @@ struct ContractArgs {
   float* Z[2];           // A, G3
   int Cin[2];
   int ldc[2];            // split kernel: channels of an image in memory when Cin is a slice of them (0: Cin)
-  int N, R, RP, HW, npb, items;   // items per contraction and rank tile = N * npb
-  int ks;   // split kernel: waves per item, each contracting 1/ks of the channels (1, 2 or 4)
+  int HW[2], npb[2], items[2];    // items per contraction and rank tile = N * npb
+  int N, R, RP;
+  int ks[2];   // split kernel: waves per item, each contracting 1/ks of the channels (1, 2 or 4)
+  // split kernel's masked build: operand 1 counts where y > 0 and is written so to `masked`
+  const act_t* y;
+  act_t* masked;
   long long* dbg;
 };
 
@@ -113,14 +138,14 @@ struct ContractArgs {
 __global__ __launch_bounds__(kCW) void contract_mfma_kernel(ContractArgs a) {
   extern __shared__ float Fs[];   // [slice of Cin][32]: the 32-rank tile mb of F, zero-padded
   const int which = blockIdx.y, mb = blockIdx.z;
-  const int Cin = a.Cin[which], R = a.R, HW = a.HW;
+  const int Cin = a.Cin[which], R = a.R, HW = a.HW[which], npb = a.npb[which];
   constexpr int RP = 32;
   const float* F = a.F[which];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hi = lane >> 5;
   const int item = blockIdx.x * (kCW / 64) + wave;   // (image, 64-pixel block)
-  const bool active = item < a.items;                 // (idle waves still meet the barriers)
-  const int pb = active ? item % a.npb : 0, n = active ? item / a.npb : 0;
+  const bool active = item < a.items[which];          // (idle waves still meet the barriers)
+  const int pb = active ? item % npb : 0, n = active ? item / npb : 0;
   const int p = pb * 64 + 2 * l32;
   const bool valid = active && p < HW;
   const int pc = valid ? p : HW - 2;
@@ -203,90 +228,144 @@ __global__ __launch_bounds__(kCW) void contract_mfma_kernel(ContractArgs a) {
 // waves share an item, each contracting 1/ks of the channels - shorter dependent
 // load chains and ks times the waves - and add their partial sums through LDS
 // in fixed order.
+// Bound by the latency of the activations' loads: no load or store sits in a branch, so that the
+// number in flight at each wait is a constant and a wait covers the chunk it needs, not the whole ring
+// (N64 C256 14x14 R64, x and dy: 13.5 us with a branch over the chunks past the last, 12.1 without; both
+// rank tiles in a wave, x and dy read once but half the waves: 14.8).
 constexpr int kSplitRing = 4;
-constexpr long kKsWaves = 1024;   // channel splits only while the grid stays below this many waves
-constexpr int kSW = 512;    // 8 waves share one factor tile: one fill per workgroup
-__global__ __launch_bounds__(kSW) void contract_split_kernel(ContractArgs a) {
+constexpr long kKsWaves = 512;   // channel splits only while an operand's waves stay below this many
+constexpr int kSW = 512;    // 8 waves share the factor tile: one fill per workgroup
+constexpr int kFragChunk = 6 * 32;   // 16-byte fragments of a chunk: [part][half][rank]
+
+template <bool MASK>
+__device__ __forceinline__ void contract_split(const ContractArgs& a, const int which) {
   using namespace split;
+  constexpr int kRing = MASK ? kSplitRing / 2 : kSplitRing;     // (as many loads in flight)
   extern __shared__ float Fs[];
-  unsigned char* Fb = reinterpret_cast<unsigned char*>(Fs);
-  const int which = blockIdx.y, mb = blockIdx.z;
-  const int Cin = a.Cin[which], R = a.R, HW = a.HW;
+  u32x4* Fb = reinterpret_cast<u32x4*>(Fs);
+  const int mb = blockIdx.z;
+  const int Cin = a.Cin[which], R = a.R, HW = a.HW[which], npb = a.npb[which], items = a.items[which];
   const float* F = a.F[which];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hi = lane >> 5;
   // This wave's item; waves past the end keep a valid (clamped) item for their
   // loads and skip the store, so that every wave reaches the barrier.
-  const int ks = a.ks;
+  const int ks = a.ks[which];
+  if ((int)blockIdx.x * (kSW / 64) >= items * ks) return;         // whole workgroup
   [[maybe_unused]] const int dwg = (blockIdx.z * 2 + blockIdx.y) * gridDim.x + blockIdx.x;
   BSTAMP(a.dbg, 0, dwg, 8, 0)
   const int slot = blockIdx.x * (kSW / 64) + wave;        // (item, channel split)
   const int item_raw = slot / ks, part = slot - item_raw * ks;   // item = (image, 32-pixel block)
-  const bool has_item = item_raw < a.items;
-  const int item = has_item ? item_raw : a.items - 1;
-  const int pb = item % a.npb, n = item / a.npb;
+  const bool has_item = item_raw < items;
+  const int item = has_item ? item_raw : items - 1;
+  const int n = item / npb, pb = item - n * npb;
   const int p = pb * 32 + l32;
   const bool valid = has_item && p < HW;
   const int pc = p < HW ? p : HW - 1;
-  // lane's channel 16*chunk + 8*hi + e
+  // factor entries (channel octet, rank) of a thread: two a round, their loads issued together
+  // (entries past the last are that one again: no branch)
+  const int nfill = (Cin >> 3) * 32;
+  auto fill_load = [&](float (&v)[2][8], int it) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int i = min(it + t * kSW, nfill - 1), o = i >> 5, r = 32 * mb + (i & 31);
+      const float* f = F + (size_t)(8 * o) * R + (r < R ? r : 0);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[t][e] = f[(size_t)e * R];
+    }
+  };
+  auto fill_store = [&](const float (&v)[2][8], int it) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int i = min(it + t * kSW, nfill - 1), o = i >> 5, rr = i & 31;
+      float w[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) w[e] = 32 * mb + rr < R ? v[t][e] : 0.f;
+      u32x4 h, m, l;
+      split8(w, h, m, l);
+      u32x4* dst = Fb + (size_t)(o >> 1) * kFragChunk + (o & 1) * 32 + rr;
+      dst[0] = h;          // part stride: 2 halves x 32 ranks
+      dst[64] = m;
+      dst[128] = l;
+    }
+  };
+  float fv[2][8];
+  fill_load(fv, tid);
+  // lane's channel 16*chunk + 8*hi + e; the walk over the channels is scalar
   const int nch = (Cin >> 4) / ks, c0 = part * nch;     // this wave's chunks c0 .. c0 + nch - 1
-  const act_t* xp = a.src[which] +
-                    ((size_t)n * (a.ldc[which] ? a.ldc[which] : Cin) + 16 * c0 + 8 * hi) * HW + pc;
+  const size_t at = ((size_t)n * (a.ldc[which] ? a.ldc[which] : Cin) + 16 * c0) * HW;
+  constexpr unsigned kEl = sizeof(act_t);
+  const unsigned voff = (unsigned)(8 * hi * HW + pc) * kEl;
+  auto chunk_of = [&](const act_t* base, int ch) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<act_t*>(base + at + (size_t)(16 * ch) * HW), 0,
+                                             16 * HW * (int)kEl, 0x00020000);
+  };
 #ifdef CP4_BWF_IO16
   using ring_t = unsigned;     // raw 16-bit values, zero-extended
+  auto load1 = [&](__amdgpu_buffer_rsrc_t rs, int e) -> ring_t {
+    return __builtin_amdgcn_raw_buffer_load_b16(rs, voff, (unsigned)(e * HW) * kEl, 0);
+  };
 #else
   using ring_t = float;
+  auto load1 = [&](__amdgpu_buffer_rsrc_t rs, int e) -> ring_t {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff, (unsigned)(e * HW) * kEl, 0));
+  };
 #endif
-  ring_t xb[kSplitRing][8];
-  auto ld_chunk = [&](ring_t (&dst)[8], int ch) {
+  ring_t xb[kRing][8];
+  [[maybe_unused]] ring_t yb[MASK ? kRing : 1][8];      // y's, of the same chunks
+  auto ld_chunk = [&](int slot, int ch) {
     ch = ch < nch ? ch : nch - 1;                     // clamped, not branched
-    const act_t* base = xp + (size_t)(16 * ch) * HW;
+    const __amdgpu_buffer_rsrc_t rs = chunk_of(a.src[which], ch);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) dst[e] = base[(size_t)e * HW];
+    for (int e = 0; e < 8; ++e) xb[slot][e] = load1(rs, e);
+    if constexpr (MASK) {
+      const __amdgpu_buffer_rsrc_t ry = chunk_of(a.y, ch);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) yb[slot][e] = load1(ry, e);
+    }
+  };
+  // the chunk of a ring slot behind the activation, and that into memory.  (Lanes and waves past
+  // the end hold the last pixel's or item's values and store those once more, and so do the waves
+  // of further rank tiles.)
+  auto mask_chunk = [&](int slot, int ch) {
+    if constexpr (MASK) {
+      const __amdgpu_buffer_rsrc_t ro = chunk_of(a.masked, ch);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        xb[slot][e] = masked_act(xb[slot][e], yb[slot][e]);
+#ifdef CP4_BWF_IO16
+        __builtin_amdgcn_raw_buffer_store_b16((act_t)xb[slot][e], ro, voff, (unsigned)(e * HW) * kEl, 0);
+#else
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(xb[slot][e]), ro, voff, (unsigned)(e * HW) * kEl, 0);
+#endif
+      }
+    }
   };
   // the first activation chunks are requested before the factor tile is built,
   // so their HBM latency runs under the fill
 #pragma unroll
-  for (int u = 0; u < kSplitRing; ++u) ld_chunk(xb[u], u);
-  // two (channel octet, rank) entries per thread and round, their sixteen factor
-  // loads issued together
-  const int nfill = (Cin >> 3) * 32, fr = 32 * mb + (tid & 31);
-  for (int it = tid; it < nfill; it += 2 * kSW) {
-    float v[2][8];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int o = min(it + t * kSW, nfill - 1) >> 5;       // channel octet (clamped)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[t][e] = fr < R ? F[(size_t)(8 * o + e) * R + fr] : 0.f;
-    }
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      if (it + t * kSW >= nfill) break;
-      const int o = (it + t * kSW) >> 5;
-      u32x4 h, m, l;
-      split8(v[t], h, m, l);
-      u32x4* dst =
-          reinterpret_cast<u32x4*>(Fb + ((size_t)(o >> 1) * 6 + (o & 1)) * 512 + (tid & 31) * 16);
-      dst[0] = h;          // part stride: 2 planes of 512 B
-      dst[64] = m;
-      dst[128] = l;
-    }
+  for (int u = 0; u < kRing; ++u) ld_chunk(u, u);
+  fill_store(fv, tid);
+  for (int it = tid + 2 * kSW; it < nfill; it += 2 * kSW) {
+    fill_load(fv, it);
+    fill_store(fv, it);
   }
   BSTAMP(a.dbg, 0, dwg, 8, 1)
   __syncthreads();
   BSTAMP(a.dbg, 0, dwg, 8, 2)
-  const u32x4* fbase = reinterpret_cast<const u32x4*>(Fb + hi * 512 + l32 * 16);
-  // Software pipeline: while the six MFMAs of chunk c run (accumulators in turn, so that they
+  const u32x4* fbase = Fb + (size_t)c0 * kFragChunk + hi * 32 + l32;
+  // Software pipeline: while the MFMAs of chunk c run (accumulators in turn, so that they
   // do not wait for each other), the vector ALU splits chunk c+1.
   // (fp32: acc1 takes the products of the high parts alone, so a chunk rounds once at the sum's
   // magnitude; with three roundings there dx = FC G1 was up to 23 % further from float64 than the
   // pass from dy, and dFC, dFH and dFW, where the rounding's bias adds up over the pixels, 3 to 5
   // times as far off as now: N16 C256 T256 40x40 R64: dx 2.3e-7 of its norm, now 1.5e-7, the pass
-  // 1.8e-7; dFH 8.6e-7, now 1.9e-7.  Two accumulators, the small products in a row: N64 C256 14x14
-  // R64 34.25 us for the whole pass, 34.1 with three, 33.95 before.)
+  // 1.8e-7; dFH 8.6e-7, now 1.9e-7.)
   f32x16 acc0 = (f32x16)(0.f), acc1 = (f32x16)(0.f);
   [[maybe_unused]] f32x16 acc2 = (f32x16)(0.f);
   u32x4 xh, xm, xl;
+  mask_chunk(0, 0);
 #ifdef CP4_BWF_HALF
   // half-precision activations: widened, then two bf16 parts
   auto pack8 = [](const ring_t (&v)[8], u32x4& h, u32x4& m) {
@@ -309,62 +388,68 @@ __global__ __launch_bounds__(kSW) void contract_split_kernel(ContractArgs a) {
   split8(xb[0], xh, xm, xl);
 #endif
   BSTAMP(a.dbg, 0, dwg, 8, 5)
-  ld_chunk(xb[0], kSplitRing);
-  for (int ch = 0; ch < nch; ch += kSplitRing) {
+  ld_chunk(0, kRing);
+  // A round is kRing chunks; the last one requests nothing and ends with the wave's last chunk.
+  auto round = [&](int ch, auto more) {
+    constexpr bool MORE = decltype(more)::value;
 #pragma unroll
-    for (int u = 0; u < kSplitRing; ++u) {
+    for (int u = 0; u < kRing; ++u) {
       const int c = ch + u;                           // chunk whose parts are in xh/xm/xl
+      const int s1 = (u + 1) % kRing;
+      if (!MORE && c >= nch) break;
+      const bool next = MORE || u + 1 < kRing;        // (compile time; past the last chunk: unused)
       u32x4 nh = xh, nm = xm, nl = xl;
-      if (c < nch) {
-        const u32x4* fp = fbase + (size_t)(c0 + c) * (6 * 32);
-        const u32x4 fh = fp[0], fm = fp[64], fl = fp[128];
-        // one MFMA, then a quarter of the next chunk's split, pinned in this order
-        ring_t (&nx)[8] = xb[(u + 1) % kSplitRing];
+      const u32x4* fp = fbase + (size_t)c * kFragChunk;
+      const u32x4 fh = fp[0], fm = fp[64], fl = fp[128];
+      // one MFMA, then a quarter of the next chunk's split, pinned in this order
+      ring_t (&nx)[8] = xb[s1];
+      if (MORE || (next && c + 1 < nch)) mask_chunk(s1, c + 1);
 #ifdef CP4_BWF_HALF
-        acc0 = mfma16(fl, xh, acc0);
-        acc1 = mfma16(fm, xm, acc1);
-        acc0 = mfma16(fm, xh, acc0);
-        acc1 = mfma16(fh, xm, acc1);
-        acc0 = mfma16(fh, xh, acc0);
-        pack8(nx, nh, nm);
-        ld_chunk(nx, c + 1 + kSplitRing);             // refill the slot just split
+      acc0 = mfma16(fl, xh, acc0);
+      acc1 = mfma16(fm, xm, acc1);
+      acc0 = mfma16(fm, xh, acc0);
+      acc1 = mfma16(fh, xm, acc1);
+      acc0 = mfma16(fh, xh, acc0);
+      if (next) pack8(nx, nh, nm);
 #elif defined(CP4_BWF_IO16)
-        acc0 = mfma16(fl, xh, acc0);
-        acc1 = mfma16(fm, xh, acc1);
-        acc0 = mfma16(fh, xh, acc0);
-        pack8(nx, nh, nm);
-        ld_chunk(nx, c + 1 + kSplitRing);             // refill the slot just packed
+      acc0 = mfma16(fl, xh, acc0);
+      acc1 = mfma16(fm, xh, acc1);
+      acc0 = mfma16(fh, xh, acc0);
+      if (next) pack8(nx, nh, nm);
 #else
-        auto piece = [&](int d) {
-          const float x0 = nx[2 * d], x1 = nx[2 * d + 1];
-          nh[d] = pack_hi16(x0, x1);
-          const float r0 = x0 - trunc_bf16(x0), r1 = x1 - trunc_bf16(x1);
-          nm[d] = pack_hi16(r0, r1);
-          nl[d] = pack_hi16(r0 - trunc_bf16(r0), r1 - trunc_bf16(r1));
-        };
-        acc0 = mfma16(fl, xh, acc0);
-        piece(0);
-        __builtin_amdgcn_sched_barrier(0);
-        acc2 = mfma16(fm, xm, acc2);
-        piece(1);
-        __builtin_amdgcn_sched_barrier(0);
-        acc0 = mfma16(fh, xl, acc0);
-        piece(2);
-        __builtin_amdgcn_sched_barrier(0);
-        acc2 = mfma16(fm, xh, acc2);
-        piece(3);
-        __builtin_amdgcn_sched_barrier(0);
-        acc0 = mfma16(fh, xm, acc0);
-        acc1 = mfma16(fh, xh, acc1);
-        ld_chunk(nx, c + 1 + kSplitRing);             // refill the slot just split
+      auto piece = [&](int d) {
+        if (!next) return;
+        const float x0 = nx[2 * d], x1 = nx[2 * d + 1];
+        nh[d] = pack_hi16(x0, x1);
+        const float r0 = x0 - trunc_bf16(x0), r1 = x1 - trunc_bf16(x1);
+        nm[d] = pack_hi16(r0, r1);
+        nl[d] = pack_hi16(r0 - trunc_bf16(r0), r1 - trunc_bf16(r1));
+      };
+      acc0 = mfma16(fl, xh, acc0);
+      piece(0);
+      __builtin_amdgcn_sched_barrier(0);
+      acc2 = mfma16(fm, xm, acc2);
+      piece(1);
+      __builtin_amdgcn_sched_barrier(0);
+      acc0 = mfma16(fh, xl, acc0);
+      piece(2);
+      __builtin_amdgcn_sched_barrier(0);
+      acc2 = mfma16(fm, xh, acc2);
+      piece(3);
+      __builtin_amdgcn_sched_barrier(0);
+      acc0 = mfma16(fh, xm, acc0);
+      acc1 = mfma16(fh, xh, acc1);
 #endif
-      }
+      if (MORE) ld_chunk(s1, c + 1 + kRing);          // refill the slot just split
       xh = nh;
       xm = nm;
       xl = nl;
       __builtin_amdgcn_sched_barrier(0);
     }
-  }
+  };
+  int ch = 0;
+  for (; ch + kRing < nch; ch += kRing) round(ch, std::true_type{});
+  round(ch, std::false_type{});
 #ifdef CP4_BWF_IO16
   f32x16 acc = acc0 + acc1;
 #else
@@ -400,6 +485,18 @@ __global__ __launch_bounds__(kSW) void contract_split_kernel(ContractArgs a) {
     const int r = 32 * mb + 8 * (v >> 2) + 4 * hi + (v & 3);
     if (valid && r < R) zn[(size_t)r * HW] = sum;
   }
+}
+
+// (up to 128 registers: two workgroups a compute unit)
+__global__ __launch_bounds__(kSW, 4) void contract_split_kernel(ContractArgs a) {
+  contract_split<false>(a, blockIdx.y);
+}
+// ... with operand 1 behind the layer's activation.  Against a pass of its own over dy and y and
+// one over its partial bias sums: N16 C128 T256 55x55 R32 stride 2 37.5 us (with the two contractions one
+// after the other) and now 16.8, N32 C128 28x28 R16 bf16 19.2 and 11.3.
+__global__ __launch_bounds__(kSW, 4) void contract_split_masked_kernel(ContractArgs a) {
+  if (blockIdx.y) contract_split<true>(a, 1);
+  else contract_split<false>(a, 0);
 }
 
 // ---- 2. taps: B, Cc from A; G2, G1 from G3 ----------------------------------
@@ -962,7 +1059,9 @@ struct GradArgs {
   const float* Z[2];     // Cc, G1
   float* part[2];        // [S][D][R]
   int D[2];
-  int N, R, RP, HW, PS, cps;   // PS pixel splits per image, cps 32-pixel chunks per split
+  int HW[2], S[2], PS[2], cps[2];   // S = N * PS; PS pixel splits per image, cps 32-pixel chunks per split
+  int N, R, RP;
+  float* partB;          // grad_split_kernel with SUMS: [S][D] sums of operand 0 over the split's pixels
   long long* dbg;
 };
 
@@ -974,14 +1073,14 @@ __global__ __launch_bounds__(kCT) void grad_gemm_kernel(GradArgs a) {
   __shared__ float Zs[32 * RB * kLd];
   __shared__ float As[kCT / 64][32 * kLd];
   const int which = blockIdx.z;
-  const int D = a.D[which], R = a.R, HW = a.HW;
+  const int D = a.D[which], R = a.R, HW = a.HW[which], PS = a.PS[which], cps = a.cps[which];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hi = lane >> 5;
   const int d0 = blockIdx.y * 128 + wave * 32;
-  if ((int)blockIdx.y * 128 >= D) return;
-  const int s = blockIdx.x, n = s / a.PS, ps = s - n * a.PS;
+  if ((int)blockIdx.y * 128 >= D || (int)blockIdx.x >= a.S[which]) return;
+  const int s = blockIdx.x, n = s / PS, ps = s - n * PS;
   const int nch_total = (HW + 31) >> 5;
-  const int ch0 = ps * a.cps, ch1 = min(nch_total, ch0 + a.cps);
+  const int ch0 = ps * cps, ch1 = min(nch_total, ch0 + cps);
   const float* actn = a.act[which] + (size_t)n * D * HW;
   const float* zn = a.Z[which] + (size_t)n * R * HW;
   // tile loads: a lane moves float2; 16 lanes cover one 32-pixel row
@@ -1057,23 +1156,23 @@ constexpr int kLdS = 36;   // LDS row stride (floats) of the activation tile: 16
 // their own: N16 D128 55x55 R32 14.8 -> 11.6 us.
 enum { kRowsVec, kRowsAny, kRowsEach };
 
-template <int RB, int ROWS>
+template <int RB, int ROWS, bool SUMS>
 __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
   constexpr bool VEC = ROWS == kRowsVec;
   using namespace split;
   __shared__ __attribute__((aligned(16))) float As[kCT / 64][32 * kLdS];
   __shared__ u32x4 Zf[2][RB * 2 * 3 * 2 * 32];
   const int which = blockIdx.z;
-  const int D = a.D[which], R = a.R, HW = a.HW;
+  const int D = a.D[which], R = a.R, HW = a.HW[which], PS = a.PS[which], cps = a.cps[which];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hi = lane >> 5;
   const int d0 = blockIdx.y * 128 + wave * 32;
-  if ((int)blockIdx.y * 128 >= D) return;
-  const int s = blockIdx.x, n = s / a.PS, ps = s - n * a.PS;
+  if ((int)blockIdx.y * 128 >= D || (int)blockIdx.x >= a.S[which]) return;
+  const int s = blockIdx.x, n = s / PS, ps = s - n * PS;
   [[maybe_unused]] const int dwg = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
   BSTAMP(a.dbg, 1, dwg, 4, 0)
   const int nch_total = (HW + 31) >> 5;
-  const int ch0 = ps * a.cps, ch1 = min(nch_total, ch0 + a.cps);
+  const int ch0 = ps * cps, ch1 = min(nch_total, ch0 + cps);
   const act_t* actn = a.act[which] + (size_t)n * D * HW;
   const float* zn = a.Z[which] + (size_t)n * R * HW;
   // activation tile: lane moves float4; 8 lanes cover one 32-pixel row, 8 rows per load
@@ -1082,6 +1181,9 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
   const int zr = tid >> 2, zo = tid & 3;             // 64 rows x 4 octets = 256 threads
   const bool zmine = zr < 32 * RB;
   float4 av[4], zv[2];
+  // the layer's bias gradient: a lane's share of the sums of its four rows
+  const bool sums = SUMS && which == 0;
+  float bs[4] = {0.f, 0.f, 0.f, 0.f};
 #ifdef CP4_BWF_IO16
   // four 16-bit activations (one 8-byte load unless kRowsEach) widened to fp32
   auto load4_act = [&](const act_t* row, int p) {
@@ -1177,6 +1279,10 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       *reinterpret_cast<float4*>(&As[wave][(8 * j + arow) * kLdS + acol]) = av[j];
+    if (sums) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) bs[j] += (av[j].x + av[j].y) + (av[j].z + av[j].w);
+    }
     if (zmine) {
       const float v[8] = {zv[0].x, zv[0].y, zv[0].z, zv[0].w, zv[1].x, zv[1].y, zv[1].z, zv[1].w};
       u32x4 h, m, l;
@@ -1266,18 +1372,33 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
       const int d = d0 + 8 * (v >> 2) + 4 * hi + (v & 3), r = 32 * mb + l32;
       if (d < D && r < R) out[(size_t)d * R + r] = acc[mb][v];
     }
+  if (sums) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float t = bs[j];
+#pragma unroll
+      for (int off = 4; off > 0; off >>= 1) t += __shfl_down(t, off, 8);
+      const int d = d0 + 8 * j + arow;
+      if ((lane & 7) == 0 && d < D) a.partB[(size_t)s * D + d] = t;
+    }
+  }
   BSTAMP(a.dbg, 1, dwg, 4, 5)
 }
 
-// Any plane size and alignment.
-[[maybe_unused]] void launch_grad_any(int RP, dim3 grid, const GradArgs& g, hipStream_t st) {
-  if (g.HW < 4) {
-    if (RP == 32) grad_split_kernel<1, kRowsEach><<<grid, kCT, 0, st>>>(g);
-    else grad_split_kernel<2, kRowsEach><<<grid, kCT, 0, st>>>(g);
-  } else {
-    if (RP == 32) grad_split_kernel<1, kRowsAny><<<grid, kCT, 0, st>>>(g);
-    else grad_split_kernel<2, kRowsAny><<<grid, kCT, 0, st>>>(g);
+// vec: both operands kRowsVec; else any plane size and alignment.
+[[maybe_unused]] hipError_t launch_grad_split(bool vec, dim3 grid, const GradArgs& g, hipStream_t st) {
+  const bool each = !vec && (g.HW[0] < 4 || g.HW[1] < 4);
+#define CP4_GRAD(ROWS_)                                                                       \
+  {                                                                                           \
+    auto k = g.RP == 32 ? (g.partB ? grad_split_kernel<1, ROWS_, true> : grad_split_kernel<1, ROWS_, false>)  \
+                        : (g.partB ? grad_split_kernel<2, ROWS_, true> : grad_split_kernel<2, ROWS_, false>); \
+    k<<<grid, kCT, 0, st>>>(g);                                                               \
   }
+  if (vec) CP4_GRAD(kRowsVec)
+  else if (each) CP4_GRAD(kRowsEach)
+  else CP4_GRAD(kRowsAny)
+#undef CP4_GRAD
+  return hipGetLastError();
 }
 
 // ---- 3b. tap gradients: partial[s][t][r] over images of split s -------------
@@ -1388,6 +1509,54 @@ Plan make_plan(int N, int C, int T, int H, int W, int Y, int X, int R, int pad) 
   return p;
 }
 
+// The split contraction takes these channel counts with one factor tile in LDS.
+bool split_contraction(int C, int T) {
+  return (C & 15) == 0 && (T & 15) == 0 && (size_t)(C > T ? C : T) * 192 <= 160 * 1024;
+}
+
+// The split contractions of `operands` planes of HW[i] pixels in one launch (ContractArgs::npb,
+// items and ks are filled in here): 32-pixel blocks, fragments of 6 bytes per factor entry.
+hipError_t launch_contract_split(ContractArgs c, int operands, hipStream_t st) {
+  long most = 0;
+  size_t smem = 0;
+  for (int i = 0; i < operands; ++i) {
+    c.npb[i] = (c.HW[i] + 31) / 32;
+    c.items[i] = c.N * c.npb[i];
+    // few items: 2 or 4 waves per item, each on a slice of the channels, until
+    // there are about 512 waves (every workgroup builds the whole factor tile,
+    // so more splits than that cost more than they hide; a slice keeps >= 2 chunks),
+    // 1024 where a wave moves the mask's operands too (N16 T256 28x28 R32 beside C128 55x55: 18.9 -> 16.8
+    // us; in 16 bits 11.3 -> 12.0)
+    const long waves = i == 1 && c.y ? kKsWaves * (long)sizeof(act_t) / 2 : kKsWaves;
+    const int nch = c.Cin[i] >> 4;
+    int& ks = c.ks[i];
+    ks = 1;
+    while (ks < 4 && (long)c.items[i] * (c.RP / 32) * ks < waves && nch % (2 * ks) == 0 &&
+           nch / (2 * ks) >= 2)
+      ks *= 2;
+    most = std::max(most, (long)c.items[i] * ks);
+    smem = std::max(smem, std::max((size_t)c.Cin[i] * 192, ks > 1 ? (size_t)kSW * 16 * sizeof(float) : 0));
+  }
+  auto k = c.y ? contract_split_masked_kernel : contract_split_kernel;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+  if (e != hipSuccess) return e;
+  k<<<dim3((unsigned)((most + kSW / 64 - 1) / (kSW / 64)), operands, c.RP / 32), kSW, smem, st>>>(c);
+  return hipGetLastError();
+}
+
+hipError_t launch_reduce(const float* const (&parts)[5], float* const (&outs)[5],
+                         const int (&counts)[5], const int (&Ss)[5], hipStream_t st) {
+  ReduceArgs r{};
+  int most = 0;
+  for (int i = 0; i < 5; ++i) {
+    r.part[i] = parts[i]; r.out[i] = outs[i]; r.count[i] = counts[i]; r.S[i] = Ss[i];
+    if (counts[i] > most) most = counts[i];
+  }
+  reduce_sets_kernel<<<dim3((most + 63) / 64, counts[4] ? 5 : 4), 256, 0, st>>>(r);
+  return hipGetLastError();
+}
+
 }  // namespace
 
 bool bwd_filter_mfma_supported(const cp4_shape& s) {
@@ -1406,6 +1575,16 @@ bool bwd_filter_mfma_supported(const cp4_shape& s) {
 }
 
 #ifndef CP4_BWF_IO16
+// BwdFilterArgs::act_y and dbias: the mask sits in the split contraction, the bias sums in the split
+// gradient GEMM.
+bool bwd_filter_mfma_masks(const cp4_shape& s, bool aligned16) {
+  const size_t HW = (size_t)s.H * s.W;
+  return split_contraction((int)s.C, (int)s.T) && ((HW & 1) || ((HW & 3) == 0 && aligned16));
+}
+int bwd_filter_mfma_bias_sets(const cp4_shape& s) {
+  return make_plan(s.N, s.C, s.T, s.H, s.W, s.Y, s.X, s.Rank, s.pad).S;
+}
+
 // The depthwise-filter tap step keeps two planes and Y*X partial sums in LDS.
 bool bwd_filter_mfma_taps2d_supported(const cp4_shape& s) {
   return bwd_filter_mfma_supported(s) &&
@@ -1435,34 +1614,22 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs& a, hipStream_t st) {
   const act_t* ady = reinterpret_cast<const act_t*>(a.dy);
   c.src[0] = ax; c.F[0] = a.FC; c.Z[0] = A; c.Cin[0] = a.C;
   c.src[1] = ady; c.F[1] = a.FK; c.Z[1] = G3; c.Cin[1] = a.T;
-  c.N = N; c.R = R; c.RP = p.RP; c.HW = HW; c.npb = p.npb;
-  c.items = N * p.npb;
+  c.N = N; c.R = R; c.RP = p.RP;
+  c.HW[0] = c.HW[1] = HW;
+  c.npb[0] = c.npb[1] = p.npb;
+  c.items[0] = c.items[1] = N * p.npb;
 #ifdef CP4_DEBUG_PHASES
   c.dbg = debug_stamp_buffer();
 #endif
   const int cmax = a.C > a.T ? a.C : a.T;
   hipError_t e;
-  if ((a.C & 15) == 0 && (a.T & 15) == 0 && (size_t)cmax * 192 <= 160 * 1024) {
-    // exact split products: 32-pixel blocks, fragments of 6 bytes per factor entry
-    c.npb = (HW + 31) / 32;
-    c.items = N * c.npb;
-    // few items: 2 or 4 waves per item, each on a slice of the channels, until
-    // there are about 1024 waves (every workgroup builds the whole factor tile,
-    // so more splits than that cost more than they hide; a slice keeps >= 2 chunks)
-    c.ks = 1;
-    const int nch_min = (a.C < a.T ? a.C : a.T) >> 4;
-    while (c.ks < 4 && (long)c.items * 2 * (p.RP / 32) * c.ks < kKsWaves &&
-           ((a.C >> 4) % (2 * c.ks)) == 0 && ((a.T >> 4) % (2 * c.ks)) == 0 &&
-           nch_min / (2 * c.ks) >= 2)
-      c.ks *= 2;
-    size_t smem = (size_t)cmax * 192;
-    if (c.ks > 1 && smem < (size_t)kSW * 16 * sizeof(float)) smem = (size_t)kSW * 16 * sizeof(float);
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(contract_split_kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+  if (split_contraction(a.C, a.T)) {
+    c.y = reinterpret_cast<const act_t*>(a.act_y);
+    c.masked = reinterpret_cast<act_t*>(a.mask_ws);
+    e = launch_contract_split(c, 2, st);
     if (e != hipSuccess) return e;
-    const long slots = (long)c.items * c.ks;
-    contract_split_kernel<<<dim3((unsigned)((slots + kSW / 64 - 1) / (kSW / 64)), 2, p.RP / 32),
-                            kSW, smem, st>>>(c);
+    // (everything below reads dy behind the activation)
+    if (c.y) ady = c.masked;
 #ifndef CP4_BWF_IO16
   } else if ((a.C & 15) == 0 && (a.T & 15) == 0 && (HW & 1)) {
     // an odd plane (no float2 rows for the fp32 kernel below) with more channels than
@@ -1472,9 +1639,9 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs& a, hipStream_t st) {
     // so the extra pass over them is cheap; N8 C2048 K512 7x7: 90 us, general kernel
     // 1085).  Even planes: one launch of the fp32 kernel, which slices its own factor
     // tile, is the quicker (N4 C1024 K2048 14x14 R48: 108 against 121 us).
-    c.npb = (HW + 31) / 32;
-    c.items = N * c.npb;
-    c.ks = 1;
+    c.npb[0] = (HW + 31) / 32;
+    c.items[0] = N * c.npb[0];
+    c.ks[0] = 1;
     for (int which = 0; which < 2; ++which) {
       const int Cin = which ? a.T : a.C;
       const int nsl = (Cin + kSplitSlice - 1) / kSplitSlice;
@@ -1491,7 +1658,7 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs& a, hipStream_t st) {
         e = hipFuncSetAttribute(reinterpret_cast<const void*>(contract_split_kernel),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
         if (e != hipSuccess) return e;
-        contract_split_kernel<<<dim3((unsigned)((c.items + kSW / 64 - 1) / (kSW / 64)), 1,
+        contract_split_kernel<<<dim3((unsigned)((c.items[0] + kSW / 64 - 1) / (kSW / 64)), 1,
                                      p.RP / 32),
                                 kSW, smem, st>>>(d);
         if (c0) {
@@ -1509,7 +1676,7 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs& a, hipStream_t st) {
     e = hipFuncSetAttribute(reinterpret_cast<const void*>(contract_mfma_kernel),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (e != hipSuccess) return e;
-    contract_mfma_kernel<<<dim3((c.items + kCW / 64 - 1) / (kCW / 64), 2, p.RP / 32), kCW, smem,
+    contract_mfma_kernel<<<dim3((c.items[0] + kCW / 64 - 1) / (kCW / 64), 2, p.RP / 32), kCW, smem,
                            st>>>(c);
 #endif
   }
@@ -1555,7 +1722,14 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs& a, hipStream_t st) {
   GradArgs g{};
   g.act[0] = ady; g.Z[0] = Cc; g.part[0] = pK; g.D[0] = a.T;
   g.act[1] = ax; g.Z[1] = G1; g.part[1] = pC; g.D[1] = a.C;
-  g.N = N; g.R = R; g.RP = p.RP; g.HW = HW; g.PS = p.PS; g.cps = p.cps;
+  g.N = N; g.R = R; g.RP = p.RP;
+  for (int i = 0; i < 2; ++i) {
+    g.HW[i] = HW;
+    g.S[i] = p.S;
+    g.PS[i] = p.PS;
+    g.cps[i] = p.cps;
+  }
+  g.partB = a.dbias ? a.bias_part : nullptr;
 #ifdef CP4_DEBUG_PHASES
   g.dbg = debug_stamp_buffer();
 #endif
@@ -1564,24 +1738,20 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs& a, hipStream_t st) {
   // rows of four pixels as one load: 16 bytes of fp32, 8 bytes of bfloat16
   const bool grad_split =
       (HW & 3) == 0 && (reinterpret_cast<uintptr_t>(ws) & 15) == 0 &&
-      ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.dy)) &
+      ((reinterpret_cast<uintptr_t>(ax) | reinterpret_cast<uintptr_t>(ady)) &
        (4 * sizeof(act_t) - 1)) == 0;
-  if (grad_split) {
-    if (p.RP == 32) grad_split_kernel<1, kRowsVec><<<ggrid, kCT, 0, st>>>(g);
-    else grad_split_kernel<2, kRowsVec><<<ggrid, kCT, 0, st>>>(g);
 #ifdef CP4_BWF_IO16
-  } else {
-    launch_grad_any(p.RP, ggrid, g, st);
-  }
+  e = launch_grad_split(grad_split, ggrid, g, st);
 #else
-  } else if (HW & 1) {
-    // odd planes: the float2 staging of the fp32 kernel does not apply
-    launch_grad_any(p.RP, ggrid, g, st);
+  if (grad_split || (HW & 1)) {    // (odd planes: the float2 staging of the fp32 kernel does not apply)
+    e = launch_grad_split(grad_split, ggrid, g, st);
   } else {
     if (p.RP == 32) grad_gemm_kernel<1><<<ggrid, kCT, 0, st>>>(g);
     else grad_gemm_kernel<2><<<ggrid, kCT, 0, st>>>(g);
+    e = hipGetLastError();
   }
 #endif
+  if (e != hipSuccess) return e;
 
   // (after the GEMMs, whose operands its stores would push out of the cache)
   if (a.dx) {
@@ -1596,19 +1766,12 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs& a, hipStream_t st) {
     if (e != hipSuccess) return e;
   }
 
-  ReduceArgs r{};
-  const float* parts[4] = {pK, pC, pH, pW};
-  float* outs[4] = {a.dFK, a.dFC, a.taps2d ? a.dtaps2d : a.dFH, a.dFW};
-  const int counts[4] = {a.T * R, a.C * R, a.taps2d ? a.Y * a.X * R : a.Y * R,
-                         a.taps2d ? 0 : a.X * R};
-  const int Ss[4] = {p.S, p.S, a.taps2d ? N : p.St, p.St};
-  int maxc = 0;
-  for (int i = 0; i < 4; ++i) {
-    r.part[i] = parts[i]; r.out[i] = outs[i]; r.count[i] = counts[i]; r.S[i] = Ss[i];
-    if (counts[i] > maxc) maxc = counts[i];
-  }
-  reduce_sets_kernel<<<dim3((maxc + 63) / 64, 4), 256, 0, st>>>(r);
-  return hipGetLastError();
+  const float* parts[5] = {pK, pC, pH, pW, a.bias_part};
+  float* outs[5] = {a.dFK, a.dFC, a.taps2d ? a.dtaps2d : a.dFH, a.dFW, a.dbias};
+  const int counts[5] = {a.T * R, a.C * R, a.taps2d ? a.Y * a.X * R : a.Y * R,
+                         a.taps2d ? 0 : a.X * R, a.dbias ? a.T : 0};
+  const int Ss[5] = {p.S, p.S, a.taps2d ? N : p.St, p.St, p.S};
+  return launch_reduce(parts, outs, counts, Ss, st);
 }
 
 #ifndef CP4_BWF_IO16
@@ -1888,34 +2051,23 @@ hipError_t contract_one(const float* src, const float* F, float* Z, int Cin, int
                         int HW, hipStream_t st) {
   ContractArgs c{};
   c.src[0] = src; c.F[0] = F; c.Z[0] = Z; c.Cin[0] = Cin;
-  c.N = N; c.R = R; c.RP = RP; c.HW = HW;
-  hipError_t e;
-  if ((Cin & 15) == 0 && (size_t)Cin * 192 <= 160 * 1024) {
-    c.npb = (HW + 31) / 32;
-    c.items = N * c.npb;
-    c.ks = 1;
-    while (c.ks < 4 && (long)c.items * (RP / 32) * c.ks < kKsWaves / 2 &&
-           ((Cin >> 4) % (2 * c.ks)) == 0 && (Cin >> 4) / (2 * c.ks) >= 2)
-      c.ks *= 2;
-    size_t smem = (size_t)Cin * 192;
-    if (c.ks > 1 && smem < (size_t)kSW * 16 * sizeof(float)) smem = (size_t)kSW * 16 * sizeof(float);
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(contract_split_kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    if (e != hipSuccess) return e;
-    const long slots = (long)c.items * c.ks;
-    contract_split_kernel<<<dim3((unsigned)((slots + kSW / 64 - 1) / (kSW / 64)), 1, RP / 32), kSW,
-                            smem, st>>>(c);
-  } else {
-    c.npb = (HW + 63) / 64;
-    c.items = N * c.npb;
-    const size_t smem = (size_t)(Cin < kContractSlice ? Cin : kContractSlice) * 32 * sizeof(float);
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(contract_mfma_kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    if (e != hipSuccess) return e;
-    contract_mfma_kernel<<<dim3((c.items + kCW / 64 - 1) / (kCW / 64), 1, RP / 32), kCW, smem,
-                           st>>>(c);
-  }
+  c.N = N; c.R = R; c.RP = RP; c.HW[0] = HW;
+  if (split_contraction(Cin, Cin)) return launch_contract_split(c, 1, st);
+  c.npb[0] = (HW + 63) / 64;
+  c.items[0] = N * c.npb[0];
+  const size_t smem = (size_t)(Cin < kContractSlice ? Cin : kContractSlice) * 32 * sizeof(float);
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(contract_mfma_kernel),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+  if (e != hipSuccess) return e;
+  contract_mfma_kernel<<<dim3((c.items[0] + kCW / 64 - 1) / (kCW / 64), 1, RP / 32), kCW, smem,
+                         st>>>(c);
   return hipGetLastError();
+}
+
+// Rows of an operand of the gradient GEMM, and its rank planes in the workspace, move as 16 bytes.
+bool grad_rows_vec(int HW, const void* ws, const float* act) {
+  return (HW & 3) == 0 &&
+         ((reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(act)) & 15) == 0;
 }
 
 // One gradient GEMM part[s][d][r] = sum_{p in split s} act[n,d,p] Z[n,r,p] on planes of HW pixels.
@@ -1923,19 +2075,13 @@ hipError_t grad_one(const float* act, const float* Z, float* part, int D, int N,
                     const Plan& p, int HW, const void* ws, hipStream_t st) {
   GradArgs g{};
   g.act[0] = act; g.Z[0] = Z; g.part[0] = part; g.D[0] = D;
-  g.N = N; g.R = R; g.RP = p.RP; g.HW = HW; g.PS = p.PS; g.cps = p.cps;
+  g.N = N; g.R = R; g.RP = p.RP;
+  g.HW[0] = g.HW[1] = HW; g.S[0] = p.S; g.PS[0] = p.PS; g.cps[0] = p.cps;
   const dim3 ggrid(p.S, (D + 127) / 128, 1);
-  const bool vec = (HW & 3) == 0 && (reinterpret_cast<uintptr_t>(ws) & 15) == 0 &&
-                   (reinterpret_cast<uintptr_t>(act) & 15) == 0;
-  if (vec) {
-    if (p.RP == 32) grad_split_kernel<1, kRowsVec><<<ggrid, kCT, 0, st>>>(g);
-    else grad_split_kernel<2, kRowsVec><<<ggrid, kCT, 0, st>>>(g);
-  } else if (HW & 1) {
-    launch_grad_any(p.RP, ggrid, g, st);
-  } else {
-    if (p.RP == 32) grad_gemm_kernel<1><<<ggrid, kCT, 0, st>>>(g);
-    else grad_gemm_kernel<2><<<ggrid, kCT, 0, st>>>(g);
-  }
+  const bool vec = grad_rows_vec(HW, ws, act);
+  if (vec || (HW & 1)) return launch_grad_split(vec, ggrid, g, st);
+  if (p.RP == 32) grad_gemm_kernel<1><<<ggrid, kCT, 0, st>>>(g);
+  else grad_gemm_kernel<2><<<ggrid, kCT, 0, st>>>(g);
   return hipGetLastError();
 }
 
@@ -1945,7 +2091,7 @@ hipError_t grad_one(const float* act, const float* Z, float* part, int D, int N,
 // Where the taps run by columns, Cc can be formed from A alone before anything of dy is
 // read; one pass over dy and y then does all that needs dy (bwd_dy_pass.hip).  The partial sets of
 // that pass lie in mask_ws, the room the masked dy would take.
-bool bwd_filter_mfma_masks(const cp4_shape& s) {
+bool bwd_filter_mfma_dy_pass_masks(const cp4_shape& s) {
   if (!bwd_filter_mfma_supported(s) || s.C % 16 != 0 || (size_t)s.C * 192 > 160 * 1024) return false;
   const int HW = (int)(s.H * s.W);
   if (!bwd_dy_pass_supported((int)s.N, (int)s.T, (int)s.Rank, HW)) return false;
@@ -1985,18 +2131,11 @@ hipError_t bwd_filter_mfma_masked_launch(const BwdFilterArgs& a, hipStream_t st)
     e = rank_expand_launch(a.FC, G1, a.dx, CP4_DTYPE_F32, N, a.C, HW, R, st);
     if (e != hipSuccess) return e;
   }
-  ReduceArgs r{};
   const float* parts[5] = {pK, pC, pH, pW, pB};
   float* outs[5] = {a.dFK, a.dFC, a.dFH, a.dFW, a.dbias};
   const int counts[5] = {a.T * R, a.C * R, a.Y * R, a.X * R, a.dbias ? a.T : 0};
   const int Ss[5] = {sets, p.S, p.St, p.St, sets};
-  int maxc = 0;
-  for (int i = 0; i < 5; ++i) {
-    r.part[i] = parts[i]; r.out[i] = outs[i]; r.count[i] = counts[i]; r.S[i] = Ss[i];
-    if (counts[i] > maxc) maxc = counts[i];
-  }
-  reduce_sets_kernel<<<dim3((maxc + 63) / 64, 5), 256, 0, st>>>(r);
-  return hipGetLastError();
+  return launch_reduce(parts, outs, counts, Ss, st);
 }
 
 namespace {
@@ -2033,6 +2172,12 @@ bool bwd_filter_mfma_strided_supported(const cp4_shape& s, const Geometry& g) {
          strided_taps_lds(s.H, s.W, g.Ho, g.Wo, s.Y, s.X) <= 150 * 1024;
 }
 
+bool bwd_filter_mfma_strided_masks(const cp4_shape& s, const Geometry& g, bool aligned16) {
+  cp4_shape so = s;
+  so.H = g.Ho; so.W = g.Wo;
+  return bwd_filter_mfma_masks(s, aligned16) && bwd_filter_mfma_masks(so, aligned16);
+}
+
 size_t bwd_filter_mfma_strided_workspace_bytes(const cp4_shape& s, const Geometry& g) {
   return strided_layout(s, g).total * sizeof(float);
 }
@@ -2047,10 +2192,23 @@ hipError_t bwd_filter_mfma_strided_launch(const BwdFilterArgs& a, const Geometry
   float *A = ws + l.A, *G1 = ws + l.G1, *G3 = ws + l.G3, *Cc = ws + l.Cc, *pK = ws + l.pK,
         *pC = ws + l.pC, *pH = ws + l.pH, *pW = ws + l.pW;
   const int N = a.N, R = a.R, HW = a.H * a.W, HWo = g.Ho * g.Wo;
-  hipError_t e = contract_one(a.x, a.FC, A, a.C, N, R, l.pf.RP, HW, st);
-  if (e != hipSuccess) return e;
-  e = contract_one(a.dy, a.FK, G3, a.T, N, R, l.ps.RP, HWo, st);
-  if (e != hipSuccess) return e;
+  const float* dy = a.dy;
+  hipError_t e;
+  if (split_contraction(a.C, a.T)) {
+    ContractArgs c{};
+    c.src[0] = a.x; c.F[0] = a.FC; c.Z[0] = A; c.Cin[0] = a.C; c.HW[0] = HW;
+    c.src[1] = dy; c.F[1] = a.FK; c.Z[1] = G3; c.Cin[1] = a.T; c.HW[1] = HWo;
+    c.N = N; c.R = R; c.RP = l.pf.RP;
+    c.y = a.act_y; c.masked = a.mask_ws;
+    e = launch_contract_split(c, 2, st);
+    if (e != hipSuccess) return e;
+    if (c.y) dy = c.masked;
+  } else {
+    e = contract_one(a.x, a.FC, A, a.C, N, R, l.pf.RP, HW, st);
+    if (e != hipSuccess) return e;
+    e = contract_one(dy, a.FK, G3, a.T, N, R, l.ps.RP, HWo, st);
+    if (e != hipSuccess) return e;
+  }
   const size_t tsm = strided_taps_lds(a.H, a.W, g.Ho, g.Wo, a.Y, a.X);
   const bool fast = a.Y == a.X && (a.Y == 1 || a.Y == 3 || a.Y == 5 || a.Y == 7);
 #define CP4_STRIDED_TAPS(FS_)                                                                    \
@@ -2078,26 +2236,42 @@ hipError_t bwd_filter_mfma_strided_launch(const BwdFilterArgs& a, const Geometry
                                                        g.pl);
   }
 #undef CP4_STRIDED_TAPS
-  e = grad_one(a.dy, Cc, pK, a.T, N, R, l.ps, HWo, ws, st);
-  if (e != hipSuccess) return e;
-  e = grad_one(a.x, G1, pC, a.C, N, R, l.pf, HW, ws, st);
+  // the two gradient GEMMs side by side where both run as split products
+  GradArgs q{};
+  q.act[0] = dy; q.Z[0] = Cc; q.part[0] = pK; q.D[0] = a.T;
+  q.act[1] = a.x; q.Z[1] = G1; q.part[1] = pC; q.D[1] = a.C;
+  q.N = N; q.R = R; q.RP = l.pf.RP;
+  const Plan* plans[2] = {&l.ps, &l.pf};
+  const int planes[2] = {HWo, HW};
+  bool vec = true, split = true;
+  for (int i = 0; i < 2; ++i) {
+    q.HW[i] = planes[i];
+    q.S[i] = plans[i]->S;
+    q.PS[i] = plans[i]->PS;
+    q.cps[i] = plans[i]->cps;
+    const bool v = grad_rows_vec(planes[i], ws, q.act[i]);
+    vec = vec && v;
+    split = split && (v || (planes[i] & 1));
+  }
+  q.partB = a.dbias ? a.bias_part : nullptr;
+  if (split) {
+    const dim3 grid(l.ps.S > l.pf.S ? l.ps.S : l.pf.S, ((a.T > a.C ? a.T : a.C) + 127) / 128, 2);
+    e = launch_grad_split(vec, grid, q, st);
+  } else {
+    e = grad_one(dy, Cc, pK, a.T, N, R, l.ps, HWo, ws, st);
+    if (e != hipSuccess) return e;
+    e = grad_one(a.x, G1, pC, a.C, N, R, l.pf, HW, ws, st);
+  }
   if (e != hipSuccess) return e;
   if (a.dx) {
     e = rank_expand_launch(a.FC, G1, a.dx, CP4_DTYPE_F32, N, a.C, HW, R, st);
     if (e != hipSuccess) return e;
   }
-  ReduceArgs r{};
-  const float* parts[4] = {pK, pC, pH, pW};
-  float* outs[4] = {a.dFK, a.dFC, a.dFH, a.dFW};
-  const int counts[4] = {a.T * R, a.C * R, a.Y * R, a.X * R};
-  const int Ss[4] = {l.ps.S, l.pf.S, N, N};
-  int maxc = 0;
-  for (int i = 0; i < 4; ++i) {
-    r.part[i] = parts[i]; r.out[i] = outs[i]; r.count[i] = counts[i]; r.S[i] = Ss[i];
-    if (counts[i] > maxc) maxc = counts[i];
-  }
-  reduce_sets_kernel<<<dim3((maxc + 63) / 64, 4), 256, 0, st>>>(r);
-  return hipGetLastError();
+  const float* parts[5] = {pK, pC, pH, pW, a.bias_part};
+  float* outs[5] = {a.dFK, a.dFC, a.dFH, a.dFW, a.dbias};
+  const int counts[5] = {a.T * R, a.C * R, a.Y * R, a.X * R, a.dbias ? a.T : 0};
+  const int Ss[5] = {l.ps.S, l.pf.S, N, N, l.ps.S};
+  return launch_reduce(parts, outs, counts, Ss, st);
 }
 #endif  // !CP4_BWF_IO16
 

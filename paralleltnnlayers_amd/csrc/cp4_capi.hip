@@ -1103,13 +1103,20 @@ cp4_status cp4_conv2d_backward_filter(const cp4_shape* shape, const float* x,
 
 }  // extern "C"
 namespace {
+void set_mask(cp4::BwdFilterArgs& a, const cp4::LayerMask& m) {
+  a.act_y = static_cast<const float*>(m.y);
+  a.mask_ws = static_cast<float*>(m.masked);
+  a.dbias = m.dbias;
+  a.bias_part = m.bias_part;
+}
+
 // (dx not null: the input gradient as well where the matrix-core variant runs on the layer as
 // it is, *dx_done)
 cp4_status backward_filter_f32(const cp4_shape* shape, const float* x, const float* dy,
                                const float* FK, const float* FC, const float* FH, const float* FW,
                                float* dFK, float* dFC, float* dFH, float* dFW, void* workspace,
                                size_t workspace_bytes, int variant, void* dx, bool* dx_done,
-                               cp4_stream stream) {
+                               const cp4::LayerMask* mask, cp4_stream stream) {
   cp4_status rc = check_shape(shape);
   if (rc != CP4_OK) return rc;
   if (!FK || !FC || !FH || !FW || !dFK || !dFC || !dFH || !dFW)
@@ -1140,6 +1147,7 @@ cp4_status backward_filter_f32(const cp4_shape* shape, const float* x, const flo
   a.dFK = dFK; a.dFC = dFC; a.dFH = dFH; a.dFW = dFW; a.workspace = workspace;
   a.N = s.N; a.C = s.C; a.T = s.T; a.H = s.H; a.W = s.W; a.pad = s.pad;
   a.Y = s.Y; a.X = s.X; a.R = s.Rank;
+  if (mask) set_mask(a, *mask);
   // few channels on both sides: the dense-gradient route takes any channel count as it is
   if (variant < 0 && default_filter_variant(s, routes) == 3) variant = 3;
   if (variant == 3) {
@@ -1173,7 +1181,7 @@ cp4_status backward_filter_f32(const cp4_shape* shape, const float* x, const flo
       CP4_HIP(cp4::pad_rows_launch(FK, w + l.fk, 1, s.T, t.T, s.Rank, st));
       rc = backward_filter_f32(&t, xp, dyp, w + l.fk, w + l.fc, FH, FW, w + l.gfk, w + l.gfc, dFH,
                                dFW, w + l.head, workspace_bytes - l.head * sizeof(float), -1,
-                               t.C == s.C ? dx : nullptr, dx_done, stream);
+                               t.C == s.C ? dx : nullptr, dx_done, nullptr, stream);
       if (rc != CP4_OK) return rc;
       CP4_HIP(cp4::copy_f32_launch(dFC, w + l.gfc, (size_t)s.C * s.Rank, st));
       CP4_HIP(cp4::copy_f32_launch(dFK, w + l.gfk, (size_t)s.T * s.Rank, st));
@@ -1232,7 +1240,7 @@ cp4_status cp4_conv2d_backward_filter_variant(const cp4_shape* shape, const floa
                                               size_t workspace_bytes, int variant,
                                               cp4_stream stream) {
   return backward_filter_f32(shape, x, dy, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
-                             workspace_bytes, variant, nullptr, nullptr, stream);
+                             workspace_bytes, variant, nullptr, nullptr, nullptr, stream);
 }
 
 size_t cp4_noalloc_scratch_bytes(void) { return kScratchBytes; }
@@ -1271,7 +1279,8 @@ namespace {
 cp4_status backward_filter_16(const cp4_shape* shape, const void* x16, const void* dy16,
                               const float* FK, const float* FC, const float* FH, const float* FW,
                               float* dFK, float* dFC, float* dFH, float* dFW, void* workspace,
-                              size_t workspace_bytes, bool half, void* dx, cp4_stream stream) {
+                              size_t workspace_bytes, bool half, void* dx,
+                              const cp4::LayerMask* mask, cp4_stream stream) {
   cp4_status rc = check_shape(shape);
   if (rc != CP4_OK) return rc;
   if (!FK || !FC || !FH || !FW || !dFK || !dFC || !dFH || !dFW)
@@ -1303,6 +1312,7 @@ cp4_status backward_filter_16(const cp4_shape* shape, const void* x16, const voi
   a.N = s.N; a.C = s.C; a.T = s.T; a.H = s.H; a.W = s.W; a.pad = s.pad;
   a.Y = s.Y; a.X = s.X; a.R = s.Rank;
   a.dx = dx;
+  if (mask) set_mask(a, *mask);
   if (half) CP4_HIP(cp4::bwd_filter_mfma_iof16_launch(a, st));
   else CP4_HIP(cp4::bwd_filter_mfma_io16_launch(a, st));
   return CP4_OK;
@@ -1316,7 +1326,7 @@ cp4_status cp4_conv2d_backward_filter_bf16(const cp4_shape* shape, const void* x
                                            float* dFH, float* dFW, void* workspace,
                                            size_t workspace_bytes, cp4_stream stream) {
   return backward_filter_16(shape, x_bf16, dy_bf16, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
-                            workspace_bytes, false, nullptr, stream);
+                            workspace_bytes, false, nullptr, nullptr, stream);
 }
 
 cp4_status cp4_conv2d_backward_filter_f16(const cp4_shape* shape, const void* x_f16,
@@ -1326,7 +1336,7 @@ cp4_status cp4_conv2d_backward_filter_f16(const cp4_shape* shape, const void* x_
                                           float* dFH, float* dFW, void* workspace,
                                           size_t workspace_bytes, cp4_stream stream) {
   return backward_filter_16(shape, x_f16, dy_f16, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
-                            workspace_bytes, true, nullptr, stream);
+                            workspace_bytes, true, nullptr, nullptr, stream);
 }
 
 cp4_status cp4_conv2d_backward_filter_full(const cp4_shape* shape,
@@ -1605,7 +1615,8 @@ cp4_status backward_filter_geometry(const cp4_shape* shape, const cp4_geometry* 
                                     const float* dy, const float* FK, const float* FC,
                                     const float* FH, const float* FW, float* dFK, float* dFC,
                                     float* dFH, float* dFW, void* workspace, size_t workspace_bytes,
-                                    void* dx, bool* dx_done, cp4_stream stream) {
+                                    void* dx, bool* dx_done, const cp4::LayerMask* mask,
+                                    cp4_stream stream) {
   cp4_status rc = check_geometry(shape, g);
   if (rc != CP4_OK) return rc;
   const cp4_shape& s = *shape;
@@ -1636,6 +1647,7 @@ cp4_status backward_filter_geometry(const cp4_shape* shape, const cp4_geometry* 
       b.N = (int)s.N; b.C = (int)s.C; b.T = (int)s.T; b.H = (int)s.H; b.W = (int)s.W; b.pad = 0;
       b.Y = (int)s.Y; b.X = (int)s.X; b.R = (int)s.Rank;
       b.dx = dx;
+      if (mask) set_mask(b, *mask);
       if (dx) *dx_done = true;
       CP4_HIP(cp4::bwd_filter_mfma_strided_launch(b, gg, st));
       return CP4_OK;
@@ -1667,19 +1679,48 @@ cp4_status layer_backward_filter(const cp4_shape* s, const cp4_geometry* g, int 
                                  const void* dy, const float* FK, const float* FC, const float* FH,
                                  const float* FW, float* dFK, float* dFC, float* dFH, float* dFW,
                                  void* workspace, size_t workspace_bytes, void* dx, bool* dx_done,
-                                 cp4_stream stream) {
+                                 int variant, const LayerMask* mask, cp4_stream stream) {
   *dx_done = false;
   const float *xf = static_cast<const float*>(x), *dyf = static_cast<const float*>(dy);
   if (g)
     return backward_filter_geometry(s, g, xf, dyf, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
-                                    workspace_bytes, dx, dx_done, stream);
+                                    workspace_bytes, dx, dx_done, mask, stream);
   if (dtype == CP4_DTYPE_F32)
     return backward_filter_f32(s, xf, dyf, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
-                               workspace_bytes, -1, dx, dx_done, stream);
+                               workspace_bytes, variant, dx, dx_done, mask, stream);
   if (s->Y != s->X || 2 * s->pad + 1 != s->Y) dx = nullptr;
   *dx_done = dx != nullptr;
   return backward_filter_16(s, x, dy, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
-                            workspace_bytes, dtype == CP4_DTYPE_F16, dx, stream);
+                            workspace_bytes, dtype == CP4_DTYPE_F16, dx, mask, stream);
+}
+
+int layer_filter_takes_mask(const cp4_shape& s, const cp4_geometry* g, int dtype, const void* x,
+                            const void* dy, const void* workspace) {
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy) |
+                         reinterpret_cast<uintptr_t>(workspace);
+  const bool aligned16 = (bits & 15) == 0;
+  if (g) {
+    const Geometry gg{(int)g->stride_h, (int)g->stride_w, (int)g->pad_top, (int)g->pad_left,
+                      (int)g->out_h, (int)g->out_w};
+    return (gg.sh > 1 || gg.sw > 1) && bwd_filter_mfma_strided_supported(s, gg) &&
+           bwd_filter_mfma_strided_masks(s, gg, aligned16);
+  }
+  if (dtype != CP4_DTYPE_F32) return bwd_filter_mfma_io16_supported(s);
+  const FilterRoutes routes = filter_routes(s, (bits & 7) == 0, aligned16,
+                                            (reinterpret_cast<uintptr_t>(workspace) & 255) == 0);
+  if (routes.tiles_ok || filter_pad_route(s)) return 0;
+  const int variant = default_filter_variant(s, routes);
+  return variant == 2 || (variant == 1 && bwd_filter_mfma_masks(s, aligned16)) ? variant : 0;
+}
+
+size_t layer_bias_sets(const cp4_shape& s, const cp4_geometry* g) {
+  if (g) {
+    cp4_shape so = s;
+    so.H = g->out_h; so.W = g->out_w; so.pad = 0;
+    return (size_t)bwd_filter_mfma_bias_sets(so);
+  }
+  const size_t sets = (size_t)bwd_filter_mfma_bias_sets(s);
+  return bwd_filter_fused_supported(s) ? std::max(sets, (size_t)bwd_filter_fused_bias_sets(s)) : sets;
 }
 
 int layer_filter_masks(const cp4_shape& s, const float* x, const float* y, const float* dy,
@@ -1691,7 +1732,7 @@ int layer_filter_masks(const cp4_shape& s, const float* x, const float* y, const
   const int variant = default_filter_variant(s, routes);
   if (variant == 3) return !want_dx && bwd_filter_dense_tiles_masks(s) ? 3 : 0;
   return variant == 1 && mask_ws && s.Y == s.X && 2 * s.pad + 1 == s.Y &&
-         ((bits | reinterpret_cast<uintptr_t>(y)) & 15) == 0 && bwd_filter_mfma_masks(s) ? 1 : 0;
+         ((bits | reinterpret_cast<uintptr_t>(y)) & 15) == 0 && bwd_filter_mfma_dy_pass_masks(s) ? 1 : 0;
 }
 
 cp4_status layer_backward_filter_masked(int variant, const cp4_shape* shape, const float* x,
@@ -1727,7 +1768,7 @@ cp4_status cp4_conv2d_backward_filter_ex(const cp4_shape* shape, const cp4_geome
                                          void* workspace, size_t workspace_bytes,
                                          cp4_stream stream) {
   return backward_filter_geometry(shape, g, x, dy, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
-                                  workspace_bytes, nullptr, nullptr, stream);
+                                  workspace_bytes, nullptr, nullptr, nullptr, stream);
 }
 
 cp4_status cp4_time_forward(const cp4_shape* shape, const float* x,

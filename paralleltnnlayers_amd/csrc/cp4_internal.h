@@ -82,14 +82,32 @@ cp4_status check_layer_geometry(const cp4_shape*, const cp4_geometry*);
 cp4_status fail_with(cp4_status, const char* what);
 cp4_status fail_hip(hipError_t, const char* where);
 
+// A layer's mask and bias gradient inside the passes of its factor gradients: dy counts where
+// y > 0 and is written so, in its own type, to `masked` as the contraction reads it (y null: dy as
+// it is); dbias (may be null) is summed as the gradient GEMM reads that, in partial sets in
+// bias_part.
+struct LayerMask {
+  const void* y;
+  void* masked;
+  float *dbias, *bias_part;
+};
+
 // The backward-filter entry points with the input gradient beside the factors' where the
 // variant that runs has it at hand (`dx` may be null; *dx_done says whether it was written).
-// dtype: a cp4_dtype, the type of x, dy and dx; `geometry` as in the _ex entry points.
+// dtype: a cp4_dtype, the type of x, dy and dx; `geometry` as in the _ex entry points.  `mask`
+// (may be null): with the variant that layer_filter_takes_mask gave for these operands; `variant`
+// is -1 without it.
 cp4_status layer_backward_filter(const cp4_shape*, const cp4_geometry*, int dtype, const void* x,
                                  const void* dy, const float* FK, const float* FC, const float* FH,
                                  const float* FW, float* dFK, float* dFC, float* dFH, float* dFW,
                                  void* workspace, size_t workspace_bytes, void* dx, bool* dx_done,
-                                 cp4_stream);
+                                 int variant, const LayerMask* mask, cp4_stream);
+// The backward-filter variant (strided and 16-bit layers: any number above 0) that such a call
+// runs with the mask and the bias gradient in it; 0: none does.
+int layer_filter_takes_mask(const cp4_shape&, const cp4_geometry*, int dtype, const void* x,
+                            const void* dy, const void* workspace);
+// Most partial sets of T floats that any of those variants leaves of the bias gradient.
+size_t layer_bias_sets(const cp4_shape&, const cp4_geometry*);
 cp4_status layer_backward_filter_masked(int variant, const cp4_shape*, const float* x, const float* act_y,
                                         const float* dy, const float* FK, const float* FC,
                                         const float* FH, const float* FW, float* dFK, float* dFC,
@@ -200,10 +218,10 @@ struct BwdFilterArgs {
   // Matrix-core variant only: not null, the input gradient too, dx = FC G1 (in the type of
   // x; the forward's adjoint only where 2 * pad = Y - 1 = X - 1 or with a geometry).
   void* dx;
-  // Dense-gradient variant with bwd_filter_dense_tiles_masks and the matrix-core variant's
-  // masked launch only: dy counts where act_y > 0 (null: everywhere) and dbias[t], its sum over
-  // images and pixels, comes along; all null: neither.  Scratch: bias_part, T floats per
-  // compute unit (dense gradient), mask_ws, N * T * H * W floats (matrix cores).
+  // Where the variant's _masks function says so: dy counts where act_y > 0 (null: everywhere) and
+  // dbias[t], its sum over images and pixels, comes along; all null: neither.  Scratch:
+  // bias_part, T floats per compute unit (dense gradient) or partial set (_bias_sets), mask_ws, N * T * H * W
+  // elements (matrix cores: dy behind the activation or, in the masked launch, partial sets).
   const float* act_y;
   float *dbias, *bias_part, *mask_ws;
 };
@@ -214,9 +232,14 @@ bool bwd_filter_mfma_supported(const cp4_shape&);
 size_t bwd_filter_mfma_workspace_bytes(const cp4_shape&);
 bool bwd_filter_mfma_taps2d_supported(const cp4_shape&);   // with BwdFilterArgs::taps2d
 hipError_t bwd_filter_mfma_launch(const BwdFilterArgs&, hipStream_t);
+// That launch and the strided one take BwdFilterArgs::act_y and dbias (operands and workspace on
+// 16-byte boundaries or not), and the partial sets of the bias gradient they leave.
+bool bwd_filter_mfma_masks(const cp4_shape&, bool aligned16);
+bool bwd_filter_mfma_strided_masks(const cp4_shape&, const Geometry&, bool aligned16);
+int bwd_filter_mfma_bias_sets(const cp4_shape&);
 // The same with the layer's activation mask and bias gradient in it (BwdFilterArgs::act_y,
 // dbias, mask_ws); operands on 16-byte boundaries.
-bool bwd_filter_mfma_masks(const cp4_shape&);
+bool bwd_filter_mfma_dy_pass_masks(const cp4_shape&);
 hipError_t bwd_filter_mfma_masked_launch(const BwdFilterArgs&, hipStream_t);
 // One pass over dy behind a ReLU (y, its output): G3, `sets` partial sets [set][T][R] of dFK and [set][T] of dbias.
 bool bwd_dy_pass_supported(int N, int T, int R, int HW);
@@ -232,6 +255,7 @@ bool bwd_filter_fused_supported(const cp4_shape&);
 // time is launches and first-load latencies rather than bandwidth).
 bool bwd_filter_fused_preferred(const cp4_shape&);
 size_t bwd_filter_fused_workspace_bytes(const cp4_shape&);
+int bwd_filter_fused_bias_sets(const cp4_shape&);      // takes BwdFilterArgs::act_y and dbias throughout
 hipError_t bwd_filter_fused_launch(const BwdFilterArgs&, hipStream_t);
 // Few channels on both sides (square filters of 1, 3, 5 taps; T * C up to 256 with plain
 // multiply-adds, or up to 64 output channels and 16384 entries of the dense gradient on the

@@ -56,7 +56,8 @@ BackwardPlan make_backward_plan(const cp4_shape& s, const cp4_geometry* g, int d
   p.dx32_at = take(dx32, nx * 4);
   const int seg = cp4::act_grad_segments((int)s.N, (int)s.T, ny / ((size_t)s.N * s.T), dtype);
   p.may_mask = !g && !half && filter && (act != CP4_ACT_NONE || (wanted & CP4_WANT_BIAS));
-  const size_t parts = p.may_mask && !dx ? std::max(seg, cp4::num_compute_units()) : seg > 1 ? seg : 0;
+  size_t parts = p.may_mask && !dx ? std::max(seg, cp4::num_compute_units()) : seg > 1 ? seg : 0;
+  if (filter && !filter32) parts = std::max(parts, cp4::layer_bias_sets(s, g));
   p.bias_at = take((wanted & CP4_WANT_BIAS) && parts, s.T * parts * 4);
   p.pass_at = at;
   if (g) p.pass_bytes = dx || filter ? cp4_conv2d_backward_ex_workspace_bytes(&s, g) : 0;
@@ -86,6 +87,7 @@ BackwardPlan backward_plan(const cp4_shape& s, const cp4_geometry* g, int dtype,
 }
 
 thread_local int g_route = 0;      // of this thread's last cp4_layer_backward
+thread_local int g_mask_inside = 0;
 
 cp4_status check_layer(const cp4_shape* s, const cp4_geometry* g, int dtype, int act) {
   cp4_status rc = g ? cp4::check_layer_geometry(s, g) : cp4::check_layer_shape(s);
@@ -161,7 +163,7 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* g, int
                               void* dx, float* dFK, float* dFC, float* dFH, float* dFW,
                               float* dbias, void* workspace, size_t workspace_bytes,
                               cp4_stream stream) {
-  g_route = 0;
+  g_route = g_mask_inside = 0;
   CP4_TRY(check_layer(shape, g, dtype, activation));
   const cp4_shape& s = *shape;
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -206,14 +208,21 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* g, int
                                                ws + p.pass_at, p.pass_bytes, stream);
     }
   }
-  if (p.act16) {
+  // or one whose contraction masks dy as it reads it and leaves it in memory for the others
+  const cp4::LayerMask mask{ym, ws + p.act16_at, dbias, parts};
+  int inside = 0;
+  if (filter && !p.act32 && (!half || p.filter16) && (ym || dbias))
+    inside = cp4::layer_filter_takes_mask(s, g, dtype, x, dy, ws + p.pass_at);
+  if (inside && ym) dya = mask.masked;
+  g_mask_inside = inside != 0;
+  if (p.act16 && !inside) {
     CP4_LAUNCH(cp4::act_grad_launch(ym, dy, ws + p.act16_at, dtype, false, dbias, parts, N, T, plane, st));
     dya = ws + p.act16_at;
   }
   if (p.act32)
     CP4_LAUNCH(cp4::act_grad_launch(ym, dy, ws + p.act32_at, dtype, true, p.act16 ? nullptr : dbias,
                                     parts, N, T, plane, st));
-  if (!p.act16 && !p.act32 && dbias)
+  if (!p.act16 && !p.act32 && dbias && !inside)
     CP4_LAUNCH(cp4::act_grad_launch(ym, dy, nullptr, dtype, false, dbias, parts, N, T, plane, st));
   // 2. the factor gradients, and the input gradient with them where their pass has G1 at hand:
   // dx = FC G1 reads R planes an image, the pass of its own contracts the T channels of dy again
@@ -221,8 +230,10 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* g, int
   void* pass_ws = ws + p.pass_at;
   bool dx_done = !dx;
   if (filter && (!half || p.filter16)) {
-    CP4_TRY(cp4::layer_backward_filter(shape, g, dtype, x, dya, FK, FC, FH, FW, dFK, dFC, dFH, dFW,
-                                       pass_ws, p.pass_bytes, dx, &dx_done, stream));
+    CP4_TRY(cp4::layer_backward_filter(shape, g, dtype, x, inside ? dy : dya, FK, FC, FH, FW, dFK, dFC,
+                                       dFH, dFW, pass_ws, p.pass_bytes, dx, &dx_done,
+                                       inside && !half && !g ? inside : -1, inside ? &mask : nullptr,
+                                       stream));
     if (dx && dx_done) g_route |= CP4_ROUTE_DX_FROM_G1;
     dx_done = dx_done || !dx;
   } else if (filter) {
@@ -249,5 +260,6 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* g, int
 }
 
 int cp4_layer_last_backward_route(void) { return g_route; }
+int cp4_layer_last_backward_mask_inside(void) { return g_mask_inside; }
 
 }  // extern "C"

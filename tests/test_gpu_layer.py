@@ -152,6 +152,64 @@ def test_input_gradient_beside_the_factors(capi, case, dtype):
     assert ((dx.double().cpu() - want).abs() <= bound).all()
 
 
+# Mask and bias gradient inside the factor gradients' contraction and gradient GEMM: both variants,
+# every split of the channels over waves (1, 2, 4), one rank tile and two, planes that no block of 32
+# pixels or four divides, strides with planes of either kind, channel groups the last block does
+# not fill, every element type.
+INSIDE = [(1, 64, 8, 8, 64, 3, 8, 1), (3, 144, 9, 12, 80, 3, 33, 1), (16, 64, 32, 32, 64, 3, 16, 1),
+          (2, 32, 16, 20, 272, 5, 64, 1), (2, 32, 7, 9, 48, 3, 16, 1), (5, 256, 15, 15, 144, 1, 64, 1),
+          (24, 64, 40, 40, 64, 3, 64, 1), (2, 48, 55, 55, 32, 3, 32, 2), (3, 64, 56, 60, 176, 3, 48, 2),
+          (2, 16, 9, 9, 16, 1, 4, 2)]
+
+
+@pytest.mark.parametrize("relu", [True, False], ids=["relu", "linear"])
+@pytest.mark.parametrize("case,dtype", [
+    pytest.param(c, t, id="x".join(map(str, c)) + "-" + n) for c in INSIDE
+    for t, n in ((torch.float32, "f32"), (torch.bfloat16, "bf16"), (torch.float16, "f16"))
+    if c[-1] == 1 or t == torch.float32])
+def test_mask_and_bias_gradient_inside_the_passes(capi, case, dtype, relu):
+    N, C, H, W, T, k, R, stride = case
+    gen = torch.Generator(device="cuda").manual_seed(N + C + H + W + R)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x = mk(N, C, H, W).to(dtype)
+    fac = [mk(d, R) for d in (T, C, k, k)]
+    s = capi.shape_for(x.shape, *fac, k // 2)
+    g = capi.geometry(s, stride, "same") if stride > 1 else None
+    act = "relu" if relu else None
+    y = capi.layer_forward(s, g, x, *fac, mk(T), act)
+    dy = mk(*y.shape).to(dtype)
+    dx, grads, dbias = capi.layer_backward(s, g, x, y, dy, *fac, act)
+    assert capi.layer_last_backward_mask_inside()
+    masked = dy * (y > 0) if relu else dy
+    md = masked.double()
+    # fp32 sums: 2^-24 a step, as a random walk over the terms (a factor of four to spare)
+    n = N * md.shape[2] * md.shape[3]
+    tol = 4 * 2.0 ** -24 * ((md ** 2).sum(dim=(0, 2, 3)) * n).sqrt()
+    assert ((dbias.double() - md.sum(dim=(0, 2, 3))).abs() <= tol).all()
+    # the other gradients are bit for bit the same call's on the masked dy, which it does not mask
+    dx2, grads2, _ = capi.layer_backward(s, g, x, None, masked, *fac, None, True, True, False)
+    assert not capi.layer_last_backward_mask_inside()
+    assert torch.equal(dx, dx2) and all(torch.equal(a, b) for a, b in zip(grads, grads2))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16],
+                         ids=["f32", "bf16", "f16"])
+def test_non_finite_gradient_is_seen_inside_the_passes(capi, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, fac = mk(2, 64, 12, 12).to(dtype), [mk(d, 4) for d in (80, 64, 1, 1)]
+    s = capi.shape_for(x.shape, *fac, 0)
+    y = capi.layer_forward(s, None, x, *fac, mk(80), "relu")
+    n, t, h, w = (int(v) for v in (y == 0).nonzero()[-1])
+    dy = torch.zeros_like(y)
+    dy[n, t, h, w] = float("inf")
+    dx, grads, dbias = capi.layer_backward(s, None, x, y, dy, *fac, "relu")
+    assert capi.layer_last_backward_mask_inside()
+    assert torch.isnan(dbias[t]) and int(torch.isfinite(dbias).sum()) == 79
+    assert torch.isnan(grads[0][t]).all() and torch.isnan(dx[n, :, h, w]).all()
+    assert int(torch.isnan(dx).sum()) == 64          # (no other pixel)
+
+
 # A first layer (no input gradient): mask and bias gradient inside the dense-gradient kernel.
 # Both counts of row blocks and groups, planes smaller than a tile, widths no piece divides,
 # several tiles a workgroup, operands off a 16-byte boundary.
