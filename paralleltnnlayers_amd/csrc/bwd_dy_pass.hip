@@ -67,22 +67,19 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
   // dFC 4.2e-6 of its norm off, 2.9e-7 with them).  With 3, 5 or 7 waves one wave's share of the drift is
   // left: dFC at N53 C128 T96 56x56 R32 1.0e-6, at N27 T224 4.0e-7.
   const float sign = wave & 1 ? -1.f : 1.f;
-  u32x4 fh[2], fm[2], fl[2];
+  float fk[2][8];
 #pragma unroll
-  for (int ch = 0; ch < 2; ++ch) {
-    float v[8];
+  for (int ch = 0; ch < 2; ++ch)
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      v[e] = l32 < R ? sign * a.FK[(size_t)(c0 + 16 * ch + 8 * hi + e) * R + l32] : 0.f;
-    split::split8(v, fh[ch], fm[ch], fl[ch]);
-  }
+    for (int e = 0; e < 8; ++e)      // (clamped, not branched: sixteen branches waited for a load each)
+      fk[ch][e] = a.FK[(size_t)(c0 + 16 * ch + 8 * hi + e) * R + (l32 < R ? l32 : 0)];
 
   // ---- loads: row 4 j + lane / 16 of the wave's channels, four pixels a lane ----
   const int lrow = lane >> 4, lcol = 4 * (lane & 15);
   float4 dv[8], yv[8], zv[KZ][2];
   // (clamped, not branched; values outside are dropped where they are used.  Cc's first: its
   // fragments are made before the rows are waited for)
-  auto load = [&](int i) {
+  auto load_z = [&](int i) {
     const int n = i / a.cpi;
     const int p0 = (i - n * a.cpi) * kPix;
 #pragma unroll
@@ -92,13 +89,15 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
       zv[k][0] = *reinterpret_cast<const float4*>(z + (pz < HW ? pz : 0));
       zv[k][1] = *reinterpret_cast<const float4*>(z + (pz + 4 < HW ? pz + 4 : 0));
     }
-    const int p = p0 + lcol;
-    const size_t at = ((size_t)n * T + c0 + lrow) * HW + (p < HW ? p : 0);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      dv[j] = *reinterpret_cast<const float4*>(a.dy + at + (size_t)(4 * j) * HW);
-      yv[j] = *reinterpret_cast<const float4*>(a.y + at + (size_t)(4 * j) * HW);
-    }
+  };
+  auto row_at = [&](int i) {
+    const int n = i / a.cpi;
+    const int p = (i - n * a.cpi) * kPix + lcol;
+    return ((size_t)n * T + c0 + lrow) * HW + (p < HW ? p : 0);
+  };
+  auto load_row = [&](size_t at, int j) {
+    dv[j] = *reinterpret_cast<const float4*>(a.dy + at + (size_t)(4 * j) * HW);
+    yv[j] = *reinterpret_cast<const float4*>(a.y + at + (size_t)(4 * j) * HW);
   };
   auto deposit_z = [&](int i) {
 #pragma unroll
@@ -131,28 +130,46 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
   float bs[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) bs[j] = 0.f;
-  if (i0 < i1) {
-    load(i0);
-    deposit_z(i0);
+  {                                  // (every workgroup has a chunk)
+    load_z(i0);
+    const size_t at = row_at(i0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) load_row(at, j);
   }
+  u32x4 fh[2], fm[2], fl[2];
+#pragma unroll
+  for (int ch = 0; ch < 2; ++ch) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) fk[ch][e] = l32 < R ? sign * fk[ch][e] : 0.f;
+    split::split8(fk[ch], fh[ch], fm[ch], fl[ch]);
+  }
+  deposit_z(i0);
   __syncthreads();
   for (int i = i0; i < i1; ++i) {
     const int n = i / a.cpi;
     const int p0 = (i - n * a.cpi) * kPix;
     // ---- the held rows behind the activation, into the tile ----
+    // (the next chunk's row is requested as one goes to the tile; past the last, that one again)
     const bool in = p0 + lcol < HW;
+    const int inext = i + 1 < i1 ? i + 1 : i;
+    const size_t next = row_at(inext);
+    load_z(inext);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      float4 m = in ? dv[j] : make_float4(0.f, 0.f, 0.f, 0.f);
+      float4 m = dv[j];
       // (a product, as dy * (y > 0): a non-finite dy at a clipped output stays visible)
       m.x *= yv[j].x > 0.f ? 1.f : 0.f;
       m.y *= yv[j].y > 0.f ? 1.f : 0.f;
       m.z *= yv[j].z > 0.f ? 1.f : 0.f;
       m.w *= yv[j].w > 0.f ? 1.f : 0.f;
+      m.x = in ? m.x : 0.f;
+      m.y = in ? m.y : 0.f;
+      m.z = in ? m.z : 0.f;
+      m.w = in ? m.w : 0.f;
       bs[j] += (m.x + m.y) + (m.z + m.w);
       *reinterpret_cast<float4*>(tile + (4 * j + lrow) * kRow + lcol) = m;
+      load_row(next, j);
     }
-    if (i + 1 < i1) load(i + 1);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     // ---- dFK: rows of the tile against Cc ----
@@ -211,7 +228,7 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
       const int p = p0 + 32 * (k >> 4) + l32;
       if (r < R && p < HW) a.G3[((size_t)n * R + r) * HW + p] = s;
     }
-    if (i + 1 < i1) deposit_z(i + 1);
+    deposit_z(inext);
     __syncthreads();              // tiles free, the next chunk's fragments complete
   }
   // ---- one partial set per workgroup ----
