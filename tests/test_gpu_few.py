@@ -112,6 +112,33 @@ def test_few_with_bias_and_relu(cp4, oracle):
     cp4.device_status()
 
 
+# The bias from LDS and the factors staged around it: fewer and more channels than threads, one
+# chunk of input channels and four, ranks that fill a block and not, more than 64 KB of LDS.
+@pytest.mark.parametrize("dims", [(1, 1, 5, 7, 1, 1, 1), (2, 17, 9, 33, 33, 3, 5), (1, 64, 20, 24, 300, 3, 16),
+                                  (1, 3, 40, 70, 600, 1, 9)], ids=lambda d: "x".join(map(str, d)))
+def test_few_bias_of_any_number_of_channels(cp4, dims):
+    import torch
+    N, C, H, W, T, k, R = dims
+    gen = torch.Generator().manual_seed(sum(dims))
+    mk = lambda *s: torch.randn(*s, generator=gen)
+    x, fac, b = mk(N, C, H, W), [mk(d, R) for d in (T, C, k, k)], mk(T)
+    s = cp4.capi.shape_for(x.shape, *fac, k // 2)
+    cp4.tune_clear()
+    try:
+        cp4.set_tuned_choice(s, variant_index(cp4))
+        y = cp4.conv2d_forward_bias_act(x.cuda(), *[f.cuda() for f in fac], b.cuda(), "none", pad=k // 2)
+    finally:
+        cp4.tune_clear()
+    K, terms = (torch.einsum("tr,cr,yr,xr->tcyx", *fs)
+                for fs in ([f.double() for f in fac], [f.double().abs() for f in fac]))
+    want = torch.nn.functional.conv2d(x.double(), K, b.double(), padding=k // 2)
+    terms = torch.nn.functional.conv2d(x.abs().double(), terms, b.abs().double(), padding=k // 2)
+    # two fp32 contractions, the taps and the bias: 2^-24 a step of the sum of the terms' magnitudes, as
+    # a random walk (a factor of four to spare)
+    bound = 4 * (C + 2 * k + R + 1) ** 0.5 * 2.0 ** -24 * terms
+    assert ((y.cpu().double() - want).abs() <= bound).all()
+
+
 def test_few_is_the_default_on_large_planes_with_few_channels(cp4):
     def shape(N, C, H, W, T, R, Y=3):
         return cp4.capi.Shape(N=N, H=H, W=W, pad=Y // 2, T=T, C=C, Y=Y, X=Y, Rank=R)
