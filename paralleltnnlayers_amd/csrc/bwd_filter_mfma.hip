@@ -1147,6 +1147,10 @@ __global__ __launch_bounds__(kCT) void grad_gemm_kernel(GradArgs a) {
 // 16 B, double-buffered: one barrier per chunk); every wave stages its own 32
 // activation rows through a wave-private LDS tile (row-contiguous global reads)
 // and splits them as the A operand.
+// Bound by the latency of a chunk's loads: two chunks are in flight, their loads in no branch, so
+// that a wait covers one of them; all threads take a share of Z.  N32 C128 28x28 R16 bf16 17.0 ->
+// 8.9 us, N64 C256 14x14 R64 16.0 -> 14.9, one operand of N32 C256 56x56 R32 30.2 -> 26.2.  (Three
+// chunks in flight: 9.4, 15.0 and 27.9; more splits of the pixels move as much more in partial sets.)
 constexpr int kLdS = 36;   // LDS row stride (floats) of the activation tile: 16-byte aligned rows
 
 // How rows move: as 16 bytes (kRowsVec: H*W a multiple of 4, operands on 16-byte boundaries), as
@@ -1177,88 +1181,52 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
   const float* zn = a.Z[which] + (size_t)n * R * HW;
   // activation tile: lane moves float4; 8 lanes cover one 32-pixel row, 8 rows per load
   const int arow = lane >> 3, acol = 4 * (lane & 7);
-  // Z tile: thread t splits the 8 pixels (octet zo) of rank row zr
-  const int zr = tid >> 2, zo = tid & 3;             // 64 rows x 4 octets = 256 threads
-  const bool zmine = zr < 32 * RB;
-  float4 av[4], zv[2];
+  // Z tile: a thread splits NZ quads of pixels, from quad zq on, of rank row zr
+  constexpr int NZ = RB;                             // 32 RB rows x 8 quads over 256 threads
+  const int zr = tid / (8 / NZ), zq = NZ * (tid & (8 / NZ - 1));
+  // Two chunks in flight a lane: its four pieces of the activation rows, raw as in memory, and
+  // its NZ of Z.  Only kRowsEach has loads in branches.
+  typedef act_t act_vec __attribute__((ext_vector_type(4)));
+  typedef float z_vec __attribute__((ext_vector_type(4)));
+  act_vec av[2][4];
+  z_vec zv[2][NZ];
   // the layer's bias gradient: a lane's share of the sums of its four rows
   const bool sums = SUMS && which == 0;
   float bs[4] = {0.f, 0.f, 0.f, 0.f};
-#ifdef CP4_BWF_IO16
-  // four 16-bit activations (one 8-byte load unless kRowsEach) widened to fp32
-  auto load4_act = [&](const act_t* row, int p) {
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (ROWS == kRowsAny) {
-      typedef act_t vec __attribute__((ext_vector_type(4), aligned(sizeof(act_t))));
-      const vec t = *reinterpret_cast<const vec*>(row + min(p, HW - 4));
-      v.x = act_to_f32(t[0]);
-      v.y = act_to_f32(t[1]);
-      v.z = act_to_f32(t[2]);
-      v.w = act_to_f32(t[3]);
-    } else if (VEC) {
-      if (p < HW) {
-        const uint2 b = *reinterpret_cast<const uint2*>(row + p);
-#ifdef CP4_BWF_HALF
-        v.x = act_to_f32((act_t)(b.x & 0xffffu));
-        v.y = act_to_f32((act_t)(b.x >> 16));
-        v.z = act_to_f32((act_t)(b.y & 0xffffu));
-        v.w = act_to_f32((act_t)(b.y >> 16));
-#else
-        v.x = __uint_as_float(b.x << 16);
-        v.y = __uint_as_float(b.x & 0xffff0000u);
-        v.z = __uint_as_float(b.y << 16);
-        v.w = __uint_as_float(b.y & 0xffff0000u);
-#endif
+  // kRowsVec: 16 bytes (16-bit activations: 8); kRowsAny: the same off their boundaries; both moved
+  // back to end with the row (settle() puts them where they belong); kRowsEach: one by one
+  auto load4 = [&](auto& v, const auto* row, int p) {
+    using vec = std::remove_reference_t<decltype(v)>;
+    if constexpr (ROWS == kRowsEach) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] = 0;
+        if (p + e < HW) v[e] = row[p + e];
       }
+    } else if constexpr (VEC) {
+      v = *reinterpret_cast<const vec*>(row + min(p, HW - 4));
     } else {
-      if (p < HW) v.x = act_to_f32(row[p]);
-      if (p + 1 < HW) v.y = act_to_f32(row[p + 1]);
-      if (p + 2 < HW) v.z = act_to_f32(row[p + 2]);
-      if (p + 3 < HW) v.w = act_to_f32(row[p + 3]);
+      typedef float z_any __attribute__((ext_vector_type(4), aligned(4)));
+      typedef act_t act_any __attribute__((ext_vector_type(4), aligned(sizeof(act_t))));
+      if constexpr (std::is_same_v<vec, z_vec>) v = *reinterpret_cast<const z_any*>(row + min(p, HW - 4));
+      else v = *reinterpret_cast<const act_any*>(row + min(p, HW - 4));
     }
-    return v;
   };
-#endif
-  // kRowsVec: a float4; kRowsAny: four floats at any element, moved back to end with the row
-  // (settle() puts them where they belong); kRowsEach: one by one with per-pixel bounds.
-  auto load4 = [&](const float* row, int p) {
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (ROWS == kRowsAny) {
-      typedef float vec __attribute__((ext_vector_type(4), aligned(4)));
-      const vec t = *reinterpret_cast<const vec*>(row + min(p, HW - 4));
-      v = make_float4(t[0], t[1], t[2], t[3]);
-    } else if (VEC) {
-      if (p < HW) v = *reinterpret_cast<const float4*>(row + p);
-    } else {
-      if (p < HW) v.x = row[p];
-      if (p + 1 < HW) v.y = row[p + 1];
-      if (p + 2 < HW) v.z = row[p + 2];
-      if (p + 3 < HW) v.w = row[p + 3];
-    }
-    return v;
-  };
-  auto load_tiles = [&](int ch) {
+  // (rows past D: the last one again, which is not stored; ranks past R count as zero below)
+  auto load_tiles = [&](int slot, int ch) {
     const int p = ch * 32 + acol;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int d = d0 + 8 * j + arow;
-#ifdef CP4_BWF_IO16
-      av[j] = d < D ? load4_act(actn + (size_t)d * HW, p) : make_float4(0.f, 0.f, 0.f, 0.f);
-#else
-      av[j] = d < D ? load4(actn + (size_t)d * HW, p) : make_float4(0.f, 0.f, 0.f, 0.f);
-#endif
-    }
-    const int pz = ch * 32 + 8 * zo;
+    for (int j = 0; j < 4; ++j)
+      load4(av[slot][j], actn + (size_t)min(d0 + 8 * j + arow, D - 1) * HW, p);
+    const int pz = ch * 32 + 4 * zq;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-      zv[j] = (zmine && zr < R) ? load4(zn + (size_t)zr * HW, pz + 4 * j)
-                                : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int j = 0; j < NZ; ++j) load4(zv[slot][j], zn + (size_t)min(zr, R - 1) * HW, pz + 4 * j);
   };
-  // kRowsAny: a piece that was moved back to end with the row, shifted to where it belongs
-  // (pixels p .. p + 3; zeros past the row's end)
+  // A piece that was moved back to end with the row, shifted to where it belongs (pixels
+  // p .. p + 3; zeros past the row's end).
   auto settle = [&](float4 v, int p) {
     const int back = p - (HW - 4);
-    if (back <= 0) return v;
+    if (ROWS == kRowsEach || back <= 0) return v;
     const float e[4] = {v.x, v.y, v.z, v.w};
     float4 o;
     o.x = back == 1 ? e[1] : back == 2 ? e[2] : back == 3 ? e[3] : 0.f;
@@ -1267,31 +1235,43 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
     o.w = 0.f;
     return o;
   };
-  auto store_tiles = [&](int ch, int buf) {
-    if constexpr (ROWS == kRowsAny) {
-      if (ch * 32 + 32 > HW) {                          // the row's last chunk
+  auto store_tiles = [&](int slot, int ch, int buf) {
+    float4 ra[4], rz[NZ];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) av[j] = settle(av[j], ch * 32 + acol);
+    for (int j = 0; j < 4; ++j) {
+      const act_vec t = av[slot][j];
+      ra[j] = make_float4(act_to_f32(t[0]), act_to_f32(t[1]), act_to_f32(t[2]), act_to_f32(t[3]));
+    }
 #pragma unroll
-        for (int j = 0; j < 2; ++j) zv[j] = settle(zv[j], ch * 32 + 8 * zo + 4 * j);
-      }
+    for (int j = 0; j < NZ; ++j) {
+      const z_vec t = zv[slot][j];
+      rz[j] = zr < R ? make_float4(t[0], t[1], t[2], t[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    if (ch * 32 + 32 > HW) {                            // the row's last chunk
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ra[j] = settle(ra[j], ch * 32 + acol);
+#pragma unroll
+      for (int j = 0; j < NZ; ++j) rz[j] = settle(rz[j], ch * 32 + 4 * (zq + j));
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      *reinterpret_cast<float4*>(&As[wave][(8 * j + arow) * kLdS + acol]) = av[j];
+      *reinterpret_cast<float4*>(&As[wave][(8 * j + arow) * kLdS + acol]) = ra[j];
     if (sums) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) bs[j] += (av[j].x + av[j].y) + (av[j].z + av[j].w);
+      for (int j = 0; j < 4; ++j) bs[j] += (ra[j].x + ra[j].y) + (ra[j].z + ra[j].w);
     }
-    if (zmine) {
-      const float v[8] = {zv[0].x, zv[0].y, zv[0].z, zv[0].w, zv[1].x, zv[1].y, zv[1].z, zv[1].w};
-      u32x4 h, m, l;
-      split8(v, h, m, l);
-      // fragment (rank block zr/32, step zo/2, part, half zo&1, rank zr%32)
-      u32x4* dst = &Zf[buf][(((zr >> 5) * 2 + (zo >> 1)) * 3 * 2 + (zo & 1)) * 32 + (zr & 31)];
-      dst[0] = h;
-      dst[64] = m;          // part stride: 2 halves x 32 ranks
-      dst[128] = l;
+    // fragment (rank block zr/32, step zq/4, part, half (zq/2)&1, rank zr%32), four pixels a quad
+    u32x2* dst = reinterpret_cast<u32x2*>(
+                     &Zf[buf][(((zr >> 5) * 2 + (zq >> 2)) * 3 * 2 + ((zq >> 1) & 1)) * 32 + (zr & 31)]) +
+                 (zq & 1);
+#pragma unroll
+    for (int j = 0; j < NZ; ++j) {
+      const float v[4] = {rz[j].x, rz[j].y, rz[j].z, rz[j].w};
+      u32x2 h, m, l;
+      split4(v, h, m, l);
+      dst[j] = h;
+      dst[128 + j] = m;     // part stride: 2 halves x 32 ranks
+      dst[256 + j] = l;
     }
   };
   f32x16 acc[RB];
@@ -1305,13 +1285,13 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
 #pragma unroll
   for (int mb = 0; mb < RB; ++mb) small[mb] = (f32x16)(0.f);
 #endif
-  if (ch0 < ch1) load_tiles(ch0);
-  for (int ch = ch0; ch < ch1; ++ch) {
+  auto step = [&](int ch, int slot, bool more) {
     const int buf = (ch - ch0) & 1;
-    store_tiles(ch, buf);
+    store_tiles(slot, ch, buf);
     if (ch - ch0 < 3) { BSTAMP(a.dbg, 1, dwg, 4, 1 + (ch - ch0)) }
     __syncthreads();        // Z fragments of this chunk are complete; the other buffer is free
-    if (ch + 1 < ch1) load_tiles(ch + 1);   // in flight during the MFMAs
+    if (more) load_tiles(slot, RB == 1 ? ch + 2 : min(ch + 2, ch1 - 1));
+    __builtin_amdgcn_sched_barrier(0);      // (requested here, not behind the products)
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
       const float* ap = &As[wave][l32 * kLdS + 16 * st + 8 * hi];
@@ -1357,6 +1337,36 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
         small[mb] = mfma16(ah, zp[64], small[mb]);
       }
 #endif
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (ch0 < ch1) {
+    // Every wait with a known number of loads in flight.  With one rank block the last one to three
+    // chunks have steps of their own, of which only those that need it request; with two that
+    // costs registers, and chunks past the last are that one again.
+    load_tiles(0, ch0);
+    load_tiles(1, min(ch0 + 1, ch1 - 1));
+    int ch = ch0;
+    if constexpr (RB == 1) {
+      for (; ch + 4 <= ch1; ch += 2) {
+        step(ch, 0, true);
+        step(ch + 1, 1, true);
+      }
+      if (ch + 3 == ch1) {
+        step(ch, 0, true);
+        step(ch + 1, 1, false);
+        step(ch + 2, 0, false);
+      } else {
+        step(ch, 0, false);
+        if (ch + 1 < ch1) step(ch + 1, 1, false);
+      }
+    } else {
+      for (; ch + 2 < ch1; ch += 2) {
+        step(ch, 0, true);
+        step(ch + 1, 1, true);
+      }
+      step(ch, 0, false);
+      if (ch + 1 < ch1) step(ch + 1, 1, false);
     }
   }
   BSTAMP(a.dbg, 1, dwg, 4, 4)
@@ -1440,17 +1450,20 @@ struct ReduceArgs {
   float* out[5];
   int count[5], S[5];
 };
-// A workgroup owns 64 consecutive outputs; its four waves each sum a quarter of
-// the S partials in index order (eight loads in flight, added as a tree), then the four quarter
-// sums are added in wave order: the result does not depend on timing.
-__global__ __launch_bounds__(256) void reduce_sets_kernel(ReduceArgs a) {
-  __shared__ float quarter[4][64];
-  const int seg = blockIdx.y;
+// A workgroup owns 64 consecutive outputs; its waves (sixteen, four below 128 sets) each
+// sum a part of the S partials in index order (eight loads in flight, added as a tree), then the
+// parts are added in wave order: the result does not depend on timing.  Bound by the latency of
+// those loads: N16 C128 T256 55x55 R32 stride 2, 224 and 64 sets, 4.6 us with four waves, 3.9 with sixteen;
+// N64 C256 T256 14x14 R64, 64 sets, 3.95 and 4.7.
+constexpr int kReduceWaves = 16;
+__global__ __launch_bounds__(64 * kReduceWaves) void reduce_sets_kernel(ReduceArgs a) {
+  __shared__ float part[kReduceWaves][64];
+  const int seg = blockIdx.y, waves = blockDim.x >> 6;
   const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
   const int i = blockIdx.x * 64 + lane;
   const int count = a.count[seg], S = a.S[seg];
   if ((int)blockIdx.x * 64 >= count) return;               // whole workgroup
-  const int k0 = (int)((long)S * q / 4), k1 = (int)((long)S * (q + 1) / 4);
+  const int k0 = (int)((long)S * q / waves), k1 = (int)((long)S * (q + 1) / waves);
   float s = 0.f;
   if (i < count) {
     const float* p = a.part[seg] + i;
@@ -1464,12 +1477,20 @@ __global__ __launch_bounds__(256) void reduce_sets_kernel(ReduceArgs a) {
       for (int u = 0; u < 4; ++u) v[u] += v[u + 4];
       s += (v[0] + v[2]) + (v[1] + v[3]);
     }
-    for (; k < k1; ++k) s += p[(size_t)k * stride];
+    // (the rest together too, the last set in place of those past it)
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = p[(size_t)(k + u < k1 ? k + u : k1 - 1 > 0 ? k1 - 1 : 0) * stride];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += k + u < k1 ? v[u] : 0.f;
   }
-  quarter[q][lane] = s;
+  part[q][lane] = s;
   __syncthreads();
-  if (q == 0 && i < count)
-    a.out[seg][i] = ((quarter[0][lane] + quarter[1][lane]) + quarter[2][lane]) + quarter[3][lane];
+  if (q == 0 && i < count) {
+    float t = part[0][lane];
+    for (int w = 1; w < waves; ++w) t += part[w][lane];
+    a.out[seg][i] = t;
+  }
 }
 
 struct Plan {
@@ -1548,12 +1569,14 @@ hipError_t launch_contract_split(ContractArgs c, int operands, hipStream_t st) {
 hipError_t launch_reduce(const float* const (&parts)[5], float* const (&outs)[5],
                          const int (&counts)[5], const int (&Ss)[5], hipStream_t st) {
   ReduceArgs r{};
-  int most = 0;
+  int most = 0, sets = 0;
   for (int i = 0; i < 5; ++i) {
+    if (counts[i] > 0) sets = std::max(sets, Ss[i]);
     r.part[i] = parts[i]; r.out[i] = outs[i]; r.count[i] = counts[i]; r.S[i] = Ss[i];
     if (counts[i] > most) most = counts[i];
   }
-  reduce_sets_kernel<<<dim3((most + 63) / 64, counts[4] ? 5 : 4), 256, 0, st>>>(r);
+  reduce_sets_kernel<<<dim3((most + 63) / 64, counts[4] ? 5 : 4), sets >= 128 ? 64 * kReduceWaves : 256, 0,
+                       st>>>(r);
   return hipGetLastError();
 }
 

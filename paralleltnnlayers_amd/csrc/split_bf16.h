@@ -26,10 +26,11 @@ __device__ __forceinline__ unsigned pack_hi16(float a, float b) {
 __device__ __forceinline__ float trunc_bf16(float v) {
   return __uint_as_float(__float_as_uint(v) & 0xffff0000u);
 }
-// Exact split of 8 floats into bf16 parts h, m, l (x = h + m + l bit-exactly).
-__device__ __forceinline__ void split8(const float (&v)[8], u32x4& h, u32x4& m, u32x4& l) {
+// Exact split of 8 (4) floats into bf16 parts h, m, l (x = h + m + l bit-exactly).
+template <int D, class U>
+__device__ __forceinline__ void split_pairs(const float (&v)[2 * D], U& h, U& m, U& l) {
 #pragma unroll
-  for (int d = 0; d < 4; ++d) {
+  for (int d = 0; d < D; ++d) {
     const float a = v[2 * d], b = v[2 * d + 1];
     h[d] = pack_hi16(a, b);
     const float ra = a - trunc_bf16(a), rb = b - trunc_bf16(b);
@@ -37,6 +38,12 @@ __device__ __forceinline__ void split8(const float (&v)[8], u32x4& h, u32x4& m, 
     const float sa = ra - trunc_bf16(ra), sb = rb - trunc_bf16(rb);
     l[d] = pack_hi16(sa, sb);
   }
+}
+__device__ __forceinline__ void split8(const float (&v)[8], u32x4& h, u32x4& m, u32x4& l) {
+  split_pairs<4>(v, h, m, l);
+}
+__device__ __forceinline__ void split4(const float (&v)[4], u32x2& h, u32x2& m, u32x2& l) {
+  split_pairs<2>(v, h, m, l);
 }
 __device__ __forceinline__ f32x16 mfma_split(u32x4 ah, u32x4 am, u32x4 al, u32x4 bh, u32x4 bm,
                                              u32x4 bl, f32x16 acc) {
