@@ -1161,7 +1161,7 @@ constexpr int kLdS = 36;   // LDS row stride (floats) of the activation tile: 16
 enum { kRowsVec, kRowsAny, kRowsEach };
 
 template <int RB, int ROWS, bool SUMS>
-__global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
+__global__ __launch_bounds__(kCT, RB == 1 ? 3 : 2) void grad_split_kernel(GradArgs a) {
   constexpr bool VEC = ROWS == kRowsVec;
   using namespace split;
   __shared__ __attribute__((aligned(16))) float As[kCT / 64][32 * kLdS];
