@@ -26,6 +26,7 @@
 
 #include "cp4_internal.h"
 #include "split_bf16.h"
+#include "store_policy.h"
 
 namespace cp4 {
 namespace {
@@ -43,6 +44,7 @@ struct DyPassArgs {
   const float *dy, *y, *FK, *Cc;
   float *G3, *partK, *partB;             // partB null: no bias gradient
   int T, R, HW, cpi, chunks;             // chunks per image and in all
+  int lines;                             // G3's planes are whole cache lines
 };
 
 // KZ: (rank, octet) pairs of Cc a thread loads and splits (256 of them a chunk).
@@ -226,7 +228,11 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
         if (w < waves) s = w & 1 ? s - t[w] : s + t[w];
       const int v = k & 15, r = 8 * (v >> 2) + 4 * hi + (v & 3);
       const int p = p0 + 32 * (k >> 4) + l32;
-      if (r < R && p < HW) a.G3[((size_t)n * R + r) * HW + p] = s;
+      if (r < R && p < HW) {
+        float* g = a.G3 + ((size_t)n * R + r) * HW + p;
+        if (a.lines) store_through(g, s);
+        else *g = s;
+      }
     }
     deposit_z(inext);
     __syncthreads();              // tiles free, the next chunk's fragments complete
@@ -284,6 +290,7 @@ hipError_t bwd_dy_pass_launch(const float* dy, const float* y, const float* FK, 
   DyPassArgs a{};
   a.dy = dy; a.y = y; a.FK = FK; a.Cc = Cc; a.G3 = G3; a.partK = partK; a.partB = partB;
   a.T = T; a.R = R; a.HW = HW;
+  a.lines = store_policy(G3, HW * sizeof(float), (size_t)N * R * HW * sizeof(float), ~(size_t)0) == kStoreThrough;
   a.cpi = (HW + kPix - 1) / kPix;
   a.chunks = N * a.cpi;
   const int waves = T / 32;

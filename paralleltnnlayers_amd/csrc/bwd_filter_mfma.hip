@@ -32,6 +32,7 @@
 #include "cp4_debug.h"
 #endif
 #include "split_bf16.h"
+#include "store_policy.h"
 
 // Compiled twice more with CP4_BWF_IO16: x and dy are then 16-bit in memory (factors,
 // intermediates and gradients stay fp32).  Only the split-bf16 kernels exist in
@@ -131,6 +132,7 @@ struct ContractArgs {
   // split kernel's masked build: operand 1 counts where y > 0 and is written so to `masked`
   const act_t* y;
   act_t* masked;
+  int through[2];        // Z goes through the L2
   long long* dbg;
 };
 
@@ -459,11 +461,15 @@ __device__ __forceinline__ void contract_split(const ContractArgs& a, const int 
   float* zn = a.Z[which] + (size_t)n * R * HW + p;
   if (ks == 1) {
     if (valid) {
+      auto store = [&](auto policy) {
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int r = 32 * mb + 8 * (v >> 2) + 4 * hi + (v & 3);
-        if (r < R) zn[(size_t)r * HW] = acc[v];
-      }
+        for (int v = 0; v < 16; ++v) {
+          const int r = 32 * mb + 8 * (v >> 2) + 4 * hi + (v & 3);
+          if (r < R) store_as<decltype(policy)::value>(zn + (size_t)r * HW, (float)acc[v]);
+        }
+      };
+      if (a.through[which]) store(std::integral_constant<int, kStoreThrough>{});
+      else store(std::integral_constant<int, kStorePlain>{});
     }
     BSTAMP(a.dbg, 0, dwg, 8, 4)
     return;
@@ -1161,7 +1167,7 @@ constexpr int kLdS = 36;   // LDS row stride (floats) of the activation tile: 16
 enum { kRowsVec, kRowsAny, kRowsEach };
 
 template <int RB, int ROWS, bool SUMS>
-__global__ __launch_bounds__(kCT, RB == 1 ? 3 : 2) void grad_split_kernel(GradArgs a) {
+__global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
   constexpr bool VEC = ROWS == kRowsVec;
   using namespace split;
   __shared__ __attribute__((aligned(16))) float As[kCT / 64][32 * kLdS];
@@ -1380,7 +1386,7 @@ __global__ __launch_bounds__(kCT, RB == 1 ? 3 : 2) void grad_split_kernel(GradAr
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const int d = d0 + 8 * (v >> 2) + 4 * hi + (v & 3), r = 32 * mb + l32;
-      if (d < D && r < R) out[(size_t)d * R + r] = acc[mb][v];
+      if (d < D && r < R) store_through(out + (size_t)d * R + r, (float)acc[mb][v]);
     }
   if (sums) {
 #pragma unroll
@@ -1543,6 +1549,8 @@ hipError_t launch_contract_split(ContractArgs c, int operands, hipStream_t st) {
   for (int i = 0; i < operands; ++i) {
     c.npb[i] = (c.HW[i] + 31) / 32;
     c.items[i] = c.N * c.npb[i];
+    const size_t plane = (size_t)c.HW[i] * sizeof(float);
+    c.through[i] = store_policy(c.Z[i], plane, plane * c.N * c.R, ~(size_t)0) == kStoreThrough;
     // few items: 2 or 4 waves per item, each on a slice of the channels, until
     // there are about 512 waves (every workgroup builds the whole factor tile,
     // so more splits than that cost more than they hide; a slice keeps >= 2 chunks),

@@ -30,6 +30,7 @@
 
 #include "cp4_internal.h"
 #include "split_bf16.h"
+#include "store_policy.h"
 
 namespace cp4 {
 namespace {
@@ -64,8 +65,8 @@ struct FewPlan {
 
 // FS: filter size; NCH: 16-channel chunks of the input (1, 2 or 4); RING: chunk loads in
 // flight per lane, a multiple of NCH; OCC: waves per SIMD the register budget is set for.
-// BIAS: a branch on it per group cost layers without one 2 to 4 %.
-template <int FS, int NCH, int RING, int OCC, int NW, bool BIAS>
+// BIAS: a branch on it per group cost layers without one 2 to 4 %.  STORE: a StorePolicy for y.
+template <int FS, int NCH, int RING, int OCC, int NW, bool BIAS, int STORE>
 __global__ __launch_bounds__(64 * NW, OCC) void fwd_few_kernel(FwdArgs a, FewPlan pl) {
   constexpr int kWaves = NW;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
@@ -396,7 +397,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void fwd_few_kernel(FwdArgs a, FewPla
             const unsigned so = __builtin_amdgcn_readfirstlane((unsigned)kk * (unsigned)HW * 4u);
             if (pair_ok) {                                       // (W even: both pixels or neither)
               u32x2 o = {__float_as_uint(o0), __float_as_uint(o1)};
-              __builtin_amdgcn_raw_buffer_store_b64(o, yrs, vo0, so, 0);
+              __builtin_amdgcn_raw_buffer_store_b64(o, yrs, vo0, so, buffer_policy(STORE));
             } else {
               __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o0), yrs, vo0, so, 0);
               __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o1), yrs, vo1, so, 0);
@@ -522,7 +523,15 @@ bool plan_uncached(const FwdArgs& a, FewPlan* best) {
 
 template <int FS, int NCH, int RING, int OCC, int NW>
 hipError_t launch_as(const FwdArgs& a, const FewPlan& pl, hipStream_t st) {
-  auto k = a.bias ? fwd_few_kernel<FS, NCH, RING, OCC, NW, true> : fwd_few_kernel<FS, NCH, RING, OCC, NW, false>;
+  const size_t plane = (size_t)a.H * a.W * sizeof(float);
+  const int store = store_policy(a.y, plane, plane * a.N * a.Cout,
+                                 a.bias || a.act ? kStreamBytesLayer : kStreamBytes);
+#define CP4_FEW(BIAS_)                                                                        \
+  (store == kStoreStreamed  ? fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStoreStreamed>   \
+   : store == kStoreThrough ? fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStoreThrough>    \
+                            : fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStorePlain>)
+  auto k = a.bias ? CP4_FEW(true) : CP4_FEW(false);
+#undef CP4_FEW
   const size_t lds = pl.lds_bytes + (a.bias ? (size_t)pl.nkb * 32 * sizeof(float) : 0);
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),

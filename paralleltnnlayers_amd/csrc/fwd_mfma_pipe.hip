@@ -73,6 +73,7 @@
 #include "cp4_internal.h"
 #include "split_bf16.h"
 #include "pipe_wait.h"
+#include "store_policy.h"
 #ifdef CP4_DEBUG_PHASES
 #include "cp4_debug.h"
 #endif
@@ -156,7 +157,9 @@ struct PipePlan {
 // pixels as one dword, a wave's block is 64 pixels (128-byte pieces of every
 // channel row instead of 64-byte ones) and holds two accumulators, one per pixel
 // parity; the progress words stay per 32 pixels.
-template <int FS, int CPQ, int KR, int NQ = 4, bool PAIR = false>
+// STORE: how y goes to memory, a StorePolicy (builds of their own: two kinds of store in one cost ten
+// registers that there are not).
+template <int FS, int CPQ, int KR, int NQ = 4, bool PAIR = false, int STORE = kStorePlain>
 __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdArgs a, PipePlan pl) {
   extern __shared__ float lds[];
   // A plane: [rank quad][QA cells] of four fp32 each (the quad's ranks side by side:
@@ -1045,7 +1048,8 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdArgs a, PipePlan 
       // the lane's pixel pair as one store: float2, or two bfloat16 in a dword
       auto store_pair = [&](io_t* dst, float v0, float v1) {
 #ifdef CP4_PIPE_IO16
-        *reinterpret_cast<unsigned*>(dst) = (unsigned)to_io(v0) | ((unsigned)to_io(v1) << 16);
+        const unsigned o = (unsigned)to_io(v0) | ((unsigned)to_io(v1) << 16);
+        store_as<STORE>(reinterpret_cast<unsigned*>(dst), o);
 #else
         float2 o;
         o.x = v0;
@@ -1057,7 +1061,7 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdArgs a, PipePlan 
           o.y += old.y;
         }
 #endif
-        *reinterpret_cast<float2*>(dst) = o;
+        store_as<STORE>(reinterpret_cast<float2*>(dst), o);
 #endif
       };
       auto store_one = [&](io_t* dst, float v) {
@@ -1496,27 +1500,42 @@ bool plan(const FwdArgs& a, PipePlan* best) {
 }
 #endif
 
-template <int FS, int CPQ, int KR, int NQ = 4>
+template <int FS, int CPQ, int KR, int NQ, bool PAIR, int STORE>
+hipError_t launch_stored(const FwdArgs& a, const PipePlan& pl, hipStream_t st) {
+  auto k = fwd_pipe_kernel<FS, CPQ, KR, NQ, PAIR, STORE>;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds_bytes);
+  if (e != hipSuccess) return e;
+  k<<<dim3(8u * ((pl.nWG + 7) / 8), pl.kparts), kThreads, pl.lds_bytes, st>>>(a, pl);
+  return hipGetLastError();
+}
+
+template <int FS, int CPQ, int KR, int NQ = 4, bool PAIR = false>
 hipError_t launch_as(const FwdArgs& a, const PipePlan& pl, hipStream_t st) {
 #ifdef CP4_PIPE_IO16
   // even rows, activations on a 4-byte boundary: the producers load pixel pairs
-  if ((a.W & 1) == 0 && (reinterpret_cast<uintptr_t>(a.x) & 3) == 0) {
-    const void* fp = reinterpret_cast<const void*>(fwd_pipe_kernel<FS, CPQ, KR, NQ, true>);
-    hipError_t ep = hipFuncSetAttribute(fp, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        (int)pl.lds_bytes);
-    if (ep != hipSuccess) return ep;
-    fwd_pipe_kernel<FS, CPQ, KR, NQ, true>
-        <<<dim3(8u * ((pl.nWG + 7) / 8), pl.kparts), kThreads, pl.lds_bytes, st>>>(a, pl);
-    return hipGetLastError();
+  if constexpr (!PAIR)
+    if ((a.W & 1) == 0 && (reinterpret_cast<uintptr_t>(a.x) & 3) == 0)
+      return launch_as<FS, CPQ, KR, NQ, true>(a, pl, st);
+#endif
+  // (the 2-D-tap and rank-pass builds and 7x7 filters: plain stores only)
+#if !defined(CP4_PIPE_RANKPASS) && !defined(CP4_PIPE_TAPS2D)
+  if constexpr (FS <= 5) {
+    const Geometry g = geometry_of(a);
+    const size_t plane = (size_t)g.Ho * g.Wo * kIoBytes, bytes = plane * a.N * a.Cout;
+#ifdef CP4_PIPE_EPILOGUE
+    const int policy = store_policy(a.y, plane, bytes, kStreamBytesLayer);
+#else
+    const int policy = store_policy(a.y, plane, bytes, kStreamBytes);
+#endif
+#if !defined(CP4_PIPE_IO16) && !defined(CP4_PIPE_STRIDED)
+    if (policy == kStoreStreamed) return launch_stored<FS, CPQ, KR, NQ, PAIR, kStoreStreamed>(a, pl, st);
+#endif
+    if (policy != kStorePlain && !a.accumulate)
+      return launch_stored<FS, CPQ, KR, NQ, PAIR, kStoreThrough>(a, pl, st);
   }
 #endif
-  const void* fn = reinterpret_cast<const void*>(fwd_pipe_kernel<FS, CPQ, KR, NQ>);
-  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)pl.lds_bytes);
-  if (e != hipSuccess) return e;
-  const dim3 grid(8u * ((pl.nWG + 7) / 8), pl.kparts);
-  fwd_pipe_kernel<FS, CPQ, KR, NQ><<<grid, kThreads, pl.lds_bytes, st>>>(a, pl);
-  return hipGetLastError();
+  return launch_stored<FS, CPQ, KR, NQ, PAIR, kStorePlain>(a, pl, st);
 }
 
 template <int FS>

@@ -23,6 +23,7 @@
 
 #include "cp4_internal.h"
 #include "split_bf16.h"
+#include "store_policy.h"
 
 namespace cp4 {
 namespace {
@@ -62,7 +63,7 @@ struct ToF16 {
 // pixels are neighbours and move in one access; else they are 32 apart and move one by one
 // (planes start at any address then, and a wider access off its own boundary is the slower:
 // N16 C128 55x55 R32 28 us against 10.7).
-template <class Out, int KC, int PX, bool VEC>
+template <class Out, int KC, int PX, bool VEC, int STORE>
 __global__ __launch_bounds__(kThreads, 2) void rank_expand_kernel(ExpandArgs a) {
   using raw = typename Out::raw;
   typedef float ZV __attribute__((ext_vector_type(PX)));
@@ -144,6 +145,8 @@ __global__ __launch_bounds__(kThreads, 2) void rank_expand_kernel(ExpandArgs a) 
   const int last = first + a.cblocks * 32 < C ? first + a.cblocks * 32 : C;
   if (first >= last) return;
   raw* dst = static_cast<raw*>(a.dst);
+  const __amdgpu_buffer_rsrc_t drs = __builtin_amdgcn_make_buffer_rsrc(
+      a.dst, 0, STORE == kStoreThrough ? (int)(a.pixels * C * sizeof(raw)) : 0, 0x00020000);
   float f[KC][8];
   load_f(f, first);
   for (int c0 = first; c0 < last; c0 += 32) {
@@ -178,7 +181,20 @@ __global__ __launch_bounds__(kThreads, 2) void rank_expand_kernel(ExpandArgs a) 
         OV o;
 #pragma unroll
         for (int q = 0; q < PX; ++q) o[q] = Out::down(acc[q][v]);
-        if (live[0]) *reinterpret_cast<OV*>(dst + oat[0] + (size_t)c * HW) = o;
+        const size_t at = oat[0] + (size_t)c * HW;
+        if (!live[0]) continue;
+        if constexpr (STORE == kStoreThrough) {         // (below kStreamBytes: 32-bit offsets)
+          typedef unsigned words __attribute__((ext_vector_type(sizeof(OV) / 4)));
+          const words w = __builtin_bit_cast(words, o);
+          if constexpr (sizeof(OV) == 16)
+            __builtin_amdgcn_raw_buffer_store_b128(w, drs, (unsigned)at * sizeof(raw), 0, buffer_policy(STORE));
+          else
+            __builtin_amdgcn_raw_buffer_store_b64(w, drs, (unsigned)at * sizeof(raw), 0, buffer_policy(STORE));
+        } else if constexpr (STORE == kStoreStreamed) {
+          __builtin_nontemporal_store(o, reinterpret_cast<OV*>(dst + at));
+        } else {
+          *reinterpret_cast<OV*>(dst + at) = o;
+        }
       } else {
 #pragma unroll
         for (int q = 0; q < PX; ++q)
@@ -203,10 +219,18 @@ hipError_t launch(ExpandArgs a, hipStream_t st) {
   const unsigned grid = (unsigned)((a.items + kThreads / 64 - 1) / (kThreads / 64));
   const bool vec = a.HW % px == 0 && reinterpret_cast<uintptr_t>(a.Z) % (4 * px) == 0 &&
                    reinterpret_cast<uintptr_t>(a.dst) % (sizeof(typename Out::raw) * px) == 0;
+  const size_t plane = a.HW * sizeof(typename Out::raw);
+  // (two-pixel pieces of 16-bit elements are a dword: plain)
+  const int store = vec && px * sizeof(typename Out::raw) >= 8
+                        ? store_policy(a.dst, plane, plane * (a.pixels / a.HW) * a.C, kStreamBytes) : kStorePlain;
 #define CP4_EXPAND(KC_, PX_)                                                             \
   {                                                                                      \
-    if (vec) rank_expand_kernel<Out, KC_, PX_, true><<<grid, kThreads, 0, st>>>(a);      \
-    else rank_expand_kernel<Out, KC_, PX_, false><<<grid, kThreads, 0, st>>>(a);         \
+    constexpr bool wide = PX_ * sizeof(typename Out::raw) >= 8;                          \
+    auto k = !vec ? rank_expand_kernel<Out, KC_, PX_, false, kStorePlain>                \
+             : store == kStoreStreamed ? rank_expand_kernel<Out, KC_, PX_, true, wide ? kStoreStreamed : kStorePlain> \
+             : store == kStoreThrough ? rank_expand_kernel<Out, KC_, PX_, true, wide ? kStoreThrough : kStorePlain>   \
+                                      : rank_expand_kernel<Out, KC_, PX_, true, kStorePlain>;              \
+    k<<<grid, kThreads, 0, st>>>(a);                                                     \
   }
   if (a.R <= 16) CP4_EXPAND(1, 4)
   else if (a.R <= 32) CP4_EXPAND(2, 4)
