@@ -1917,7 +1917,7 @@ __global__ __launch_bounds__(256) void taps_strided_plane_kernel(
 // accumulated in registers while Cc is formed (one pass over the plane instead of
 // one per tap), and the adjoint taps are walked per block of sh x sw input pixels.
 template <int FS>
-__global__ __launch_bounds__(256) void taps_strided_fast_kernel(
+__global__ __launch_bounds__(FS <= 5 ? 1024 : 512) void taps_strided_fast_kernel(
     const float* __restrict__ A, const float* __restrict__ G3, const float* __restrict__ FH,
     const float* __restrict__ FW, float* __restrict__ Cc, float* __restrict__ G1,
     float* __restrict__ partH, float* __restrict__ partW, int R, int H, int W, int Ho, int Wo,
@@ -1926,8 +1926,9 @@ __global__ __launch_bounds__(256) void taps_strided_fast_kernel(
   extern __shared__ float pl[];
   const int HW = H * W, HWo = Ho * Wo;
   float *sA = pl, *sG = pl + HW;
-  float* red = sG + HWo;                          // [Y + X][4] wave partials
-  float* fh = red + 4 * (Y + X);                  // this rank's tap weights, read once
+  const int threads = blockDim.x, waves = threads >> 6;
+  float* red = sG + HWo;                          // [Y + X][waves] wave partials
+  float* fh = red + waves * (Y + X);                  // this rank's tap weights, read once
   float* fw = fh + Y;
   const int plane = blockIdx.x, r = plane % R, n = plane / R;
   const size_t basef = (size_t)plane * HW, bases = (size_t)plane * HWo;
@@ -1938,16 +1939,16 @@ __global__ __launch_bounds__(256) void taps_strided_fast_kernel(
       const float4* s4 = reinterpret_cast<const float4*>(src);
       float4* d4 = reinterpret_cast<float4*>(dst);
 #pragma unroll 4
-      for (int k = threadIdx.x; k < (n >> 2); k += 256) d4[k] = s4[k];
+      for (int k = threadIdx.x; k < (n >> 2); k += threads) d4[k] = s4[k];
     } else {
       // (eight loads in flight a thread: one by one a plane of 55 x 55 waited twelve times: N16 C128 K256 R32 stride 2 17.5 -> 15.8 us)
-      for (int k0 = threadIdx.x; k0 < n; k0 += 8 * 256) {
+      for (int k0 = threadIdx.x; k0 < n; k0 += 8 * threads) {
         float v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = src[k0 + 256 * u < n ? k0 + 256 * u : n - 1];
+        for (int u = 0; u < 8; ++u) v[u] = src[k0 + threads * u < n ? k0 + threads * u : n - 1];
 #pragma unroll
         for (int u = 0; u < 8; ++u)
-          if (k0 + 256 * u < n) dst[k0 + 256 * u] = v[u];
+          if (k0 + threads * u < n) dst[k0 + threads * u] = v[u];
       }
     }
   };
@@ -1962,7 +1963,7 @@ __global__ __launch_bounds__(256) void taps_strided_fast_kernel(
   float gh[FS], gw[FS];
 #pragma unroll
   for (int t = 0; t < FS; ++t) gh[t] = gw[t] = 0.f;
-  for (int q = threadIdx.x; q < HWo; q += 256) {
+  for (int q = threadIdx.x; q < HWo; q += threads) {
     const int ho = q / Wo, wo = q - ho * Wo;
     const float gv = sG[q];
     int ro[FS], co[FS];
@@ -2012,7 +2013,7 @@ __global__ __launch_bounds__(256) void taps_strided_fast_kernel(
     dw[i] = (bj[i] + pl_ - i) / sw;
   }
   const int nbw = (W + sw - 1) / sw, nbh = (H + sh - 1) / sh;
-  for (int blk = threadIdx.x; blk < nbh * nbw; blk += 256) {
+  for (int blk = threadIdx.x; blk < nbh * nbw; blk += threads) {
     const int bh = blk / nbw, bw = blk - bh * nbw;
     // the FS*FS values of G3 the block's pixels draw on (0 outside the plane), once
     float gv[FS][FS];
@@ -2050,7 +2051,7 @@ __global__ __launch_bounds__(256) void taps_strided_fast_kernel(
       }
     }
   }
-  // wave sums of the tap gradients to LDS, one barrier, fixed-order sum of the four
+  // wave sums of the tap gradients to LDS, one barrier, fixed-order sum of them
 #pragma unroll
   for (int t = 0; t < FS; ++t) {
     float a = gh[t], b = gw[t];
@@ -2060,14 +2061,15 @@ __global__ __launch_bounds__(256) void taps_strided_fast_kernel(
       b += __shfl_down(b, off, 64);
     }
     if ((threadIdx.x & 63) == 0) {
-      red[t * 4 + (threadIdx.x >> 6)] = a;
-      red[(Y + t) * 4 + (threadIdx.x >> 6)] = b;
+      red[t * waves + (threadIdx.x >> 6)] = a;
+      red[(Y + t) * waves + (threadIdx.x >> 6)] = b;
     }
   }
   __syncthreads();
   if ((int)threadIdx.x < Y + X) {
     const int t = threadIdx.x;
-    const float tot = red[t * 4] + red[t * 4 + 1] + red[t * 4 + 2] + red[t * 4 + 3];
+    float tot = red[t * waves];
+    for (int w = 1; w < waves; ++w) tot += red[t * waves + w];
     if (t < Y) partH[((size_t)n * Y + t) * R + r] = tot;
     else partW[((size_t)n * X + (t - Y)) * R + r] = tot;
   }
@@ -2240,14 +2242,19 @@ hipError_t bwd_filter_mfma_strided_launch(const BwdFilterArgs& a, const Geometry
     e = contract_one(dy, a.FK, G3, a.T, N, R, l.ps.RP, HWo, st);
     if (e != hipSuccess) return e;
   }
-  const size_t tsm = strided_taps_lds(a.H, a.W, g.Ho, g.Wo, a.Y, a.X);
+  // (room for the partial sums of sixteen waves, of which the limit on the planes counts four)
+  const size_t tsm = strided_taps_lds(a.H, a.W, g.Ho, g.Wo, a.Y, a.X) + 12 * (a.Y + a.X) * sizeof(float);
+  // a thread for some six pixels of the input's plane: threads that take one or two are mostly set-up
+  // (us with 256, 512 and 1024 threads: N64 14x14 R32 13.4, 20.5, 40.6; N32 28x28 R16 7.7, 8.1, 11.8;
+  // N16 55x55 R32 15.8, 13.6, 18.6; N4 112x112 R16 33.6, 20.5, 17.0; N8 150x150 R8 55, 32, 23.5)
+  const int tap_threads = HW <= 1536 ? 256 : HW <= 6144 || a.Y == 7 ? 512 : 1024;
   const bool fast = a.Y == a.X && (a.Y == 1 || a.Y == 3 || a.Y == 5 || a.Y == 7);
 #define CP4_STRIDED_TAPS(FS_)                                                                    \
   {                                                                                              \
     e = hipFuncSetAttribute(reinterpret_cast<const void*>(taps_strided_fast_kernel<FS_>),        \
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)tsm);               \
     if (e != hipSuccess) return e;                                                               \
-    taps_strided_fast_kernel<FS_><<<N * R, 256, tsm, st>>>(A, G3, a.FH, a.FW, Cc, G1, pH, pW, R, \
+    taps_strided_fast_kernel<FS_><<<N * R, tap_threads, tsm, st>>>(A, G3, a.FH, a.FW, Cc, G1, pH, pW, R, \
                                                            a.H, a.W, g.Ho, g.Wo, g.sh, g.sw,     \
                                                            g.pt, g.pl);                          \
   }

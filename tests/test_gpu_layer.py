@@ -159,7 +159,7 @@ def test_input_gradient_beside_the_factors(capi, case, dtype):
 INSIDE = [(1, 64, 8, 8, 64, 3, 8, 1), (3, 144, 9, 12, 80, 3, 33, 1), (16, 64, 32, 32, 64, 3, 16, 1),
           (2, 32, 16, 20, 272, 5, 64, 1), (2, 32, 7, 9, 48, 3, 16, 1), (5, 256, 15, 15, 144, 1, 64, 1),
           (24, 64, 40, 40, 64, 3, 64, 1), (2, 48, 55, 55, 32, 3, 32, 2), (3, 64, 56, 60, 176, 3, 48, 2),
-          (2, 16, 9, 9, 16, 1, 4, 2)]
+          (2, 16, 9, 9, 16, 1, 4, 2), (1, 16, 120, 121, 16, 3, 4, 2)]
 
 
 @pytest.mark.parametrize("relu", [True, False], ids=["relu", "linear"])
