@@ -24,6 +24,7 @@
 //       the bias / activation epilogue (FwdArgs::bias, act) applied on the way.
 #include "cp4_internal.h"
 #include "split_bf16.h"
+#include "store_policy.h"
 
 namespace cp4 {
 namespace {
@@ -47,7 +48,8 @@ struct LightPlan {
   size_t lds_bytes;
 };
 
-template <int FS, int NW>
+// STORE: a StorePolicy for y.
+template <int FS, int NW, int STORE>
 __global__ __launch_bounds__(64 * NW) void fwd_light_kernel(FwdArgs a, LightPlan pl) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   float4* As4 = reinterpret_cast<float4*>(lds_raw);                  // [quads][QA]
@@ -282,7 +284,7 @@ __global__ __launch_bounds__(64 * NW) void fwd_light_kernel(FwdArgs a, LightPlan
             o.x = o.x < 0.f ? 0.f : o.x;
             o.y = o.y < 0.f ? 0.f : o.y;
           }
-          *reinterpret_cast<float2*>(yn + (size_t)k * HW + p) = o;
+          store_as<STORE>(reinterpret_cast<float2*>(yn + (size_t)k * HW + p), o);
         }
       }
     }
@@ -339,11 +341,13 @@ bool plan(const FwdArgs& a, LightPlan* best) {
 
 template <int FS, int NW>
 hipError_t launch_nw(const FwdArgs& a, const LightPlan& pl, hipStream_t st) {
-  const void* fn = reinterpret_cast<const void*>(fwd_light_kernel<FS, NW>);
-  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)pl.lds_bytes);
+  const size_t plane = (size_t)a.H * a.W * sizeof(float);
+  auto k = store_policy(a.y, plane, plane * a.N * a.Cout, kStreamBytes) == kStoreThrough
+               ? fwd_light_kernel<FS, NW, kStoreThrough> : fwd_light_kernel<FS, NW, kStorePlain>;
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds_bytes);
   if (e != hipSuccess) return e;
-  fwd_light_kernel<FS, NW><<<pl.nWG, 64 * NW, pl.lds_bytes, st>>>(a, pl);
+  k<<<pl.nWG, 64 * NW, pl.lds_bytes, st>>>(a, pl);
   return hipGetLastError();
 }
 template <int FS>

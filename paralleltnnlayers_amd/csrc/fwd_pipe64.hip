@@ -42,6 +42,7 @@
 #include "cp4_internal.h"
 #include "split_bf16.h"
 #include "pipe_wait.h"
+#include "store_policy.h"
 
 namespace cp4 {
 namespace {
@@ -76,7 +77,8 @@ struct Plan64 {
 
 // FS: filter size; CPQ: 16-channel chunks per channel eighth (1: up to 128 input
 // channels, 2: up to 256); NCH: 16-rank chunks (3: up to 48 ranks, 4: up to 64).
-template <int FS, int CPQ, int NCH>
+// ACC: a later pass, y += (FwdArgs::accumulate); STORE: a StorePolicy for y.
+template <int FS, int CPQ, int NCH, bool ACC, int STORE>
 __global__ __launch_bounds__(kThreads) void fwd_pipe64_kernel(FwdArgs a, Plan64 pl) {
   extern __shared__ float lds[];
   // A plane: [rank quad][QA cells] of four fp32 each
@@ -322,7 +324,6 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe64_kernel(FwdArgs a, Plan64 
           fw[qi][rr][j] = r < R ? a.FW[tap * ldf + r] : 0.f;
         }
     float* yn = a.y + ((size_t)n * CoutAll + k0) * HW + (size_t)h0 * W;
-    const bool accumulate = a.accumulate != 0;
     const bool pair_stores =                       // one store per pixel pair is legal
         ((W | HW) & 1) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 7) == 0;
 
@@ -456,20 +457,32 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe64_kernel(FwdArgs a, Plan64 
         // W and H*W even, y aligned to a pair: p is even and the pair is one store
         if (pin0) {
           const unsigned lofs = (unsigned)(4 * hi * HW + p);
+          // (what a later pass adds to is read four rows at a time: row by row, each load waited for
+          // the stores before it.  Rows past the last: the first one's, not stored)
+          constexpr int kBatch = 4;
 #pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const int kk = 8 * (v >> 2) + (v & 3);         // + 4*hi is in lofs
-            if (32 * kb + kk + 4 * hi < Cout) {
-              float2* dst = reinterpret_cast<float2*>(rowbase + (size_t)kk * HW + lofs);
-              float2 o;
-              o.x = acc0[v];
-              o.y = acc1[v];
-              if (accumulate) {                      // a later pass: y += (wave-uniform)
-                const float2 old = *dst;
-                o.x += old.x;
-                o.y += old.y;
+          for (int v0 = 0; v0 < 16; v0 += kBatch) {
+            [[maybe_unused]] float2 old[kBatch];
+            if constexpr (ACC)
+#pragma unroll
+              for (int u = 0; u < kBatch; ++u) {
+                const int v = v0 + u, kk = 8 * (v >> 2) + (v & 3);
+                const bool in = 32 * kb + kk + 4 * hi < Cout;
+                old[u] = *reinterpret_cast<const float2*>(in ? rowbase + (size_t)kk * HW + lofs : yn + p);
               }
-              *dst = o;
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+              const int v = v0 + u, kk = 8 * (v >> 2) + (v & 3);         // + 4*hi is in lofs
+              if (32 * kb + kk + 4 * hi < Cout) {
+                float2 o;
+                o.x = acc0[v];
+                o.y = acc1[v];
+                if constexpr (ACC) {
+                  o.x += old[u].x;
+                  o.y += old[u].y;
+                }
+                store_as<STORE>(reinterpret_cast<float2*>(rowbase + (size_t)kk * HW + lofs), o);
+              }
             }
           }
         }
@@ -481,8 +494,8 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe64_kernel(FwdArgs a, Plan64 
           const int kk = 8 * (v >> 2) + (v & 3);
           if (32 * kb + kk + 4 * hi < Cout) {
             float* rp = rowbase + (size_t)kk * HW + lofs;
-            if (pin0) rp[0] = accumulate ? rp[0] + acc0[v] : acc0[v];
-            if (pin1) rp[1] = accumulate ? rp[1] + acc1[v] : acc1[v];
+            if (pin0) rp[0] = ACC ? rp[0] + acc0[v] : acc0[v];
+            if (pin1) rp[1] = ACC ? rp[1] + acc1[v] : acc1[v];
           }
         }
       }
@@ -597,12 +610,16 @@ bool plan(const FwdArgs& a, Plan64* best) {
 
 template <int FS, int CPQ, int NCH>
 hipError_t launch_as(const FwdArgs& a, const Plan64& pl, hipStream_t st) {
-  const void* fn = reinterpret_cast<const void*>(fwd_pipe64_kernel<FS, CPQ, NCH>);
-  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)pl.lds_bytes);
+  const size_t plane = (size_t)a.H * a.W * sizeof(float);
+  const int store = store_policy(a.y, plane, plane * a.N * a.Cout, kStreamBytes);
+  auto k = a.accumulate             ? fwd_pipe64_kernel<FS, CPQ, NCH, true, kStorePlain>
+           : store == kStoreStreamed ? fwd_pipe64_kernel<FS, CPQ, NCH, false, kStoreStreamed>
+           : store == kStoreThrough  ? fwd_pipe64_kernel<FS, CPQ, NCH, false, kStoreThrough>
+                                     : fwd_pipe64_kernel<FS, CPQ, NCH, false, kStorePlain>;
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds_bytes);
   if (e != hipSuccess) return e;
-  const dim3 grid(8u * ((pl.nWG + 7) / 8), pl.kparts);
-  fwd_pipe64_kernel<FS, CPQ, NCH><<<grid, kThreads, pl.lds_bytes, st>>>(a, pl);
+  k<<<dim3(8u * ((pl.nWG + 7) / 8), pl.kparts), kThreads, pl.lds_bytes, st>>>(a, pl);
   return hipGetLastError();
 }
 
