@@ -21,9 +21,11 @@
 //   3. reduce_fused_kernel: fixed-order sum of the partials (bit-reproducible; no
 //      floating-point atomics anywhere).
 #include <cstdint>
+#include <type_traits>
 
 #include "cp4_internal.h"
 #include "split_bf16.h"
+#include "store_policy.h"
 
 namespace cp4 {
 namespace {
@@ -47,6 +49,7 @@ struct ContractAllArgs {
   int vecfill;             // both factors 16-byte aligned and R a multiple of 4
   const float* y;          // masked build: dy counts where y > 0 ...
   float* masked;           // ... and is written so to here
+  int through;             // A and G3 go through the L2
 };
 
 // x / dy and the factor are read through buffer descriptors: an address is
@@ -265,13 +268,17 @@ __device__ __forceinline__ void contract_all(const ContractAllArgs& a, const int
   float* zn = Z + (size_t)n * R * HW + p;
   if (KS == 1) {
     if (valid) {
+      auto store = [&](auto policy) {
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
+        for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int r = 32 * rb + 8 * (v >> 2) + 4 * hi + (v & 3);
-          if (r < R) zn[(size_t)r * HW] = acc[rb][v];
-        }
+          for (int v = 0; v < 16; ++v) {
+            const int r = 32 * rb + 8 * (v >> 2) + 4 * hi + (v & 3);
+            if (r < R) store_as<decltype(policy)::value>(zn + (size_t)r * HW, (float)acc[rb][v]);
+          }
+      };
+      if (a.through) store(std::integral_constant<int, kStoreThrough>{});
+      else store(std::integral_constant<int, kStorePlain>{});
     }
     return;
   }
@@ -296,7 +303,10 @@ __device__ __forceinline__ void contract_all(const ContractAllArgs& a, const int
 #pragma unroll
       for (int q = 0; q < KS; ++q) sum += red[(((w0 + q) * RB + rb) * 16 + v) * 64 + lane];
       const int r = 32 * rb + 8 * (v >> 2) + 4 * hi + (v & 3);
-      if (valid && r < R) zn[(size_t)r * HW] = sum;
+      if (valid && r < R) {
+        if (a.through) store_through(zn + (size_t)r * HW, sum);
+        else zn[(size_t)r * HW] = sum;
+      }
     }
 }
 
@@ -627,7 +637,8 @@ __global__ __launch_bounds__(512) void grad_fused_kernel(FusedArgs a) {
         if (dbase + 16 * (v >> 3) < D) {                // wave-uniform
           const float val = acc[rb][v];
           __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(val), ors, vo,
-                                                (unsigned)((8 * (v >> 2) + (v & 3)) * R) * 4u, 0);
+                                                (unsigned)((8 * (v >> 2) + (v & 3)) * R) * 4u,
+                                                buffer_policy(kStoreThrough));
         }
     }
   }
@@ -835,6 +846,8 @@ hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
   c.src1 = a.dy; c.F1 = a.FK; c.Z1 = G3; c.Cin1 = a.T;
   c.R = R; c.HW = HW; c.npb = (HW + 31) / 32; c.items = N * c.npb;
   c.y = a.act_y; c.masked = a.mask_ws;
+  c.through = store_policy(A, HW * sizeof(float), (size_t)N * R * HW * sizeof(float), ~(size_t)0) == kStoreThrough &&
+              store_policy(G3, HW * sizeof(float), (size_t)N * R * HW * sizeof(float), ~(size_t)0) == kStoreThrough;
   c.vecfill = (R & 3) == 0 && ((reinterpret_cast<uintptr_t>(a.FC) | reinterpret_cast<uintptr_t>(a.FK)) & 15) == 0;
   const long slots = (long)c.items * p.ks;
   const dim3 cgrid((unsigned)((slots + p.nw - 1) / p.nw), 2);
