@@ -813,11 +813,21 @@ bool bwd_filter_fused_supported(const cp4_shape& s) {
 // 32.7 us, N8 C32 112x112: 63.9 against 44.9).  On planes of up to 256 pixels with more
 // than 32 ranks one partial set per image outweighs the planes from about 10 MB of
 // activations on (N64 C256 14x14 R64: 36.3 against 34.0 us).
+// Two lines lie lower, measured over 170 shapes with three sets of buffers in turn.  Under
+// a 5 x 5 filter the tap step, the longest part, fills the chip only in a launch of its
+// own: the three-launch variant is ahead up to 12,544 pixels (N16 C128 28x28 R32: 27.2
+// against 27.9 us, N26 C128 20x20 R32 at 10,400: 26.2 against 27.8) and behind from there
+// on (N24 C128 28x28 R32: 34.2 against 29.6, N7 C128 56x56 R32: 34.3 against 28.9, N64 C64
+// 28x28 R8: 42.8 against 31.4).  Under a 3 x 3 filter with up to 16 ranks the planes are
+// small beside the activations and saving them is worth least: behind from 39,000 pixels
+// on (N44 C128 T256 32x32 R16: 54.6 against 46.3, N50 C64 28x28 R4: 30.7 against 28.8).
 bool bwd_filter_fused_preferred(const cp4_shape& s) {
   if (!bwd_filter_fused_supported(s)) return false;
   const long plane = (long)s.H * s.W, pixels = plane * s.N;
   if (plane <= 256 && s.Rank > 32) return 4e-6 * s.N * ((double)s.C + s.T) * plane <= 10.;
-  return pixels <= 25088 || (plane <= 1024 && pixels <= 65536);
+  if (s.Y == 5) return pixels <= 12544;
+  const long most = s.Y == 3 && s.Rank <= 16 ? 39000 : 65536;
+  return pixels <= 25088 || (plane <= 1024 && pixels <= most);
 }
 
 size_t bwd_filter_fused_workspace_bytes(const cp4_shape& s) {
