@@ -1574,6 +1574,44 @@ hipError_t launch_contract_split(ContractArgs c, int operands, hipStream_t st) {
   return hipGetLastError();
 }
 
+#ifndef CP4_BWF_IO16
+// One channel -> rank contraction Z[n,r,p] = sum_c F[c,r] src[n,c,p] with more channels than
+// the split kernel's fragment tile holds (853), any plane size: the sum over channels runs a
+// slice of up to 768 at a time, each slice's contraction after the first into `slice` (as large
+// as Z) and added to Z in slice order (the planes have R rows against hundreds of channels, so
+// the extra pass over them is cheap; N8 C2048 K512 7x7: 90 us, general kernel 1085).  Even
+// planes: one launch of the fp32 kernel, which slices its own factor tile, is the quicker (N4
+// C1024 K2048 14x14 R48: 108 against 121 us).
+hipError_t contract_slices(const float* src, const float* F, float* Z, float* slice, int Cin, int N,
+                           int R, int RP, int HW, hipStream_t st) {
+  ContractArgs c{};
+  c.N = N; c.R = R; c.RP = RP; c.HW[0] = HW;
+  c.npb[0] = (HW + 31) / 32;
+  c.items[0] = N * c.npb[0];
+  c.ks[0] = 1;
+  c.ldc[0] = Cin;
+  const int nsl = (Cin + kSplitSlice - 1) / kSplitSlice;
+  const int cs = ((Cin + nsl - 1) / nsl + 15) / 16 * 16;
+  for (int c0 = 0; c0 < Cin; c0 += cs) {
+    c.src[0] = src + (size_t)c0 * HW;
+    c.F[0] = F + (size_t)c0 * R;
+    c.Z[0] = c0 ? slice : Z;
+    c.Cin[0] = Cin - c0 < cs ? Cin - c0 : cs;
+    const size_t smem = (size_t)c.Cin[0] * 192;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(contract_split_kernel),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) return e;
+    contract_split_kernel<<<dim3((unsigned)((c.items[0] + kSW / 64 - 1) / (kSW / 64)), 1, RP / 32), kSW,
+                            smem, st>>>(c);
+    if (c0) {
+      e = add_f32_launch(Z, slice, (size_t)N * R * HW, st);
+      if (e != hipSuccess) return e;
+    }
+  }
+  return hipGetLastError();
+}
+#endif
+
 hipError_t launch_reduce(const float* const (&parts)[5], float* const (&outs)[5],
                          const int (&counts)[5], const int (&Ss)[5], hipStream_t st) {
   ReduceArgs r{};
@@ -1652,7 +1690,6 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs& a, hipStream_t st) {
 #ifdef CP4_DEBUG_PHASES
   c.dbg = debug_stamp_buffer();
 #endif
-  const int cmax = a.C > a.T ? a.C : a.T;
   hipError_t e;
   if (split_contraction(a.C, a.T)) {
     c.y = reinterpret_cast<const act_t*>(a.act_y);
@@ -1663,46 +1700,17 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs& a, hipStream_t st) {
     if (c.y) ady = c.masked;
 #ifndef CP4_BWF_IO16
   } else if ((a.C & 15) == 0 && (a.T & 15) == 0 && (HW & 1)) {
-    // an odd plane (no float2 rows for the fp32 kernel below) with more channels than
-    // the split kernel's fragment tile holds (853): the sum over channels runs a slice
-    // of up to 768 at a time, each slice's contraction into the idle B plane and added
-    // to its plane in slice order (the planes have R rows against hundreds of channels,
-    // so the extra pass over them is cheap; N8 C2048 K512 7x7: 90 us, general kernel
-    // 1085).  Even planes: one launch of the fp32 kernel, which slices its own factor
-    // tile, is the quicker (N4 C1024 K2048 14x14 R48: 108 against 121 us).
-    c.npb[0] = (HW + 31) / 32;
-    c.items[0] = N * c.npb[0];
-    c.ks[0] = 1;
-    for (int which = 0; which < 2; ++which) {
-      const int Cin = which ? a.T : a.C;
-      const int nsl = (Cin + kSplitSlice - 1) / kSplitSlice;
-      const int cs = ((Cin + nsl - 1) / nsl + 15) / 16 * 16;
-      float* Z = which ? G3 : A;
-      for (int c0 = 0; c0 < Cin; c0 += cs) {
-        ContractArgs d = c;
-        d.src[0] = (which ? ady : ax) + (size_t)c0 * HW;
-        d.F[0] = (which ? a.FK : a.FC) + (size_t)c0 * R;
-        d.Z[0] = c0 ? B : Z;
-        d.Cin[0] = Cin - c0 < cs ? Cin - c0 : cs;
-        d.ldc[0] = Cin;
-        const size_t smem = (size_t)d.Cin[0] * 192;
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(contract_split_kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return e;
-        contract_split_kernel<<<dim3((unsigned)((c.items[0] + kSW / 64 - 1) / (kSW / 64)), 1,
-                                     p.RP / 32),
-                                kSW, smem, st>>>(d);
-        if (c0) {
-          e = add_f32_launch(Z, B, (size_t)N * R * HW, st);
-          if (e != hipSuccess) return e;
-        }
-      }
-    }
+    // an odd plane (no float2 rows for the fp32 kernel below), by way of the idle B plane
+    e = contract_slices(ax, a.FC, A, B, a.C, N, R, p.RP, HW, st);
+    if (e != hipSuccess) return e;
+    e = contract_slices(ady, a.FK, G3, B, a.T, N, R, p.RP, HW, st);
+    if (e != hipSuccess) return e;
 #endif
   } else {
 #ifdef CP4_BWF_IO16
     return hipErrorInvalidValue;      // excluded by bwd_filter_mfma_io16_supported
 #else
+    const int cmax = a.C > a.T ? a.C : a.T;
     const size_t smem = (size_t)(cmax < kContractSlice ? cmax : kContractSlice) * 32 * sizeof(float);
     e = hipFuncSetAttribute(reinterpret_cast<const void*>(contract_mfma_kernel),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
@@ -2079,13 +2087,16 @@ size_t strided_taps_lds(int H, int W, int Ho, int Wo, int Y, int X) {
   return ((size_t)H * W + (size_t)Ho * Wo + 5 * (size_t)(Y + X)) * sizeof(float);
 }
 
-// One channel -> rank contraction Z[n,r,p] = sum_c F[c,r] src[n,c,p] on planes of HW pixels.
-hipError_t contract_one(const float* src, const float* F, float* Z, int Cin, int N, int R, int RP,
-                        int HW, hipStream_t st) {
+// One channel -> rank contraction Z[n,r,p] = sum_c F[c,r] src[n,c,p] on planes of HW pixels
+// (`slice`: as large as Z, where the channels do not fit one factor tile and HW is odd).
+hipError_t contract_one(const float* src, const float* F, float* Z, float* slice, int Cin, int N, int R,
+                        int RP, int HW, hipStream_t st) {
   ContractArgs c{};
   c.src[0] = src; c.F[0] = F; c.Z[0] = Z; c.Cin[0] = Cin;
   c.N = N; c.R = R; c.RP = RP; c.HW[0] = HW;
   if (split_contraction(Cin, Cin)) return launch_contract_split(c, 1, st);
+  // (the kernel below moves pixels in pairs)
+  if (HW & 1) return contract_slices(src, F, Z, slice, Cin, N, R, RP, HW, st);
   c.npb[0] = (HW + 63) / 64;
   c.items[0] = N * c.npb[0];
   const size_t smem = (size_t)(Cin < kContractSlice ? Cin : kContractSlice) * 32 * sizeof(float);
@@ -2143,7 +2154,7 @@ hipError_t bwd_filter_mfma_masked_launch(const BwdFilterArgs& a, hipStream_t st)
   float* pW = pH + (size_t)p.St * a.Y * R;
   const int sets = bwd_dy_pass_sets(N, a.T, HW);
   float *pK = a.mask_ws, *pB = pK + (size_t)sets * a.T * R;
-  hipError_t e = contract_one(a.x, a.FC, A, a.C, N, R, p.RP, HW, st);
+  hipError_t e = contract_one(a.x, a.FC, A, G1, a.C, N, R, p.RP, HW, st);
   if (e != hipSuccess) return e;
 #define CP4_TAPS(PART_)                                                                   \
   switch (a.Y) {                                                                          \
@@ -2237,9 +2248,10 @@ hipError_t bwd_filter_mfma_strided_launch(const BwdFilterArgs& a, const Geometry
     if (e != hipSuccess) return e;
     if (c.y) dy = c.masked;
   } else {
-    e = contract_one(a.x, a.FC, A, a.C, N, R, l.pf.RP, HW, st);
+    // (G1 and Cc are written by the tap step only)
+    e = contract_one(a.x, a.FC, A, G1, a.C, N, R, l.pf.RP, HW, st);
     if (e != hipSuccess) return e;
-    e = contract_one(dy, a.FK, G3, a.T, N, R, l.ps.RP, HWo, st);
+    e = contract_one(dy, a.FK, G3, Cc, a.T, N, R, l.ps.RP, HWo, st);
     if (e != hipSuccess) return e;
   }
   // (room for the partial sums of sixteen waves, of which the limit on the planes counts four)

@@ -222,3 +222,27 @@ def test_same_padding_layer_matches_the_framework_rule(cp4):
                                [xd.grad] + [t.grad for t in fd] + [bd.grad]):
         tol = 1e-4 if name == "dx" else 1e-3
         assert (got.double() - want).abs().max() <= tol * want.abs().max(), name
+
+
+# N, C, H, W, T, Y, R: more channels than one factor tile of the contraction holds (853) on planes of an
+# odd number of pixels - of the output, of the input, of both
+@pytest.mark.parametrize("dims", [(2, 32, 14, 14, 1024, 3, 16), (2, 1024, 13, 13, 32, 3, 40),
+                                  (1, 864, 9, 11, 880, 1, 5), (3, 1600, 5, 6, 864, 3, 64)],
+                         ids=lambda d: "x".join(map(str, d)))
+def test_strided_gradients_of_many_channels_on_odd_planes(cp4, dims):
+    N, C, H, W, T, Y, R = dims
+    gen = torch.Generator(device="cuda").manual_seed(sum(dims))
+    x = torch.randn((N, C, H, W), device="cuda", generator=gen)
+    fac = [torch.randn((d, R), device="cuda", generator=gen) for d in (T, C, Y, Y)]
+    s = cp4.capi.shape_for(x.shape, *fac, 0)
+    geom = cp4.geometry(s, 2, "same")
+    dy = torch.randn((N, T, geom.out_h, geom.out_w), device="cuda", generator=gen)
+    dx, grads, _ = cp4.capi.layer_backward(s, geom, x, None, dy, *fac, None, True, True, False)
+    assert cp4.capi.layer_last_backward_route() == cp4.capi.ROUTE_DX_FROM_G1    # (not the stride-1 canvas)
+    _, dxd, gd = dense_reference(x, dy, fac, geom)
+    # sums of T and C channels, of the taps and of the pixels, signs at random: n roundings of 2^-24
+    # grow as sqrt(n), as the sum itself; times 4 for the five stages one after the other
+    bound = 4 * 2.0 ** -24 * (T + C + N * H * W) ** 0.5
+    for name, got, want in zip(("x",) + FACTORS, (dx, *grads), (dxd, *gd)):
+        err = np.linalg.norm(got.cpu().double().numpy() - want) / np.linalg.norm(want)
+        assert err <= bound, (name, err, bound)
