@@ -2254,13 +2254,15 @@ hipError_t bwd_filter_mfma_strided_launch(const BwdFilterArgs& a, const Geometry
     e = contract_one(dy, a.FK, G3, Cc, a.T, N, R, l.ps.RP, HWo, st);
     if (e != hipSuccess) return e;
   }
-  // (room for the partial sums of sixteen waves, of which the limit on the planes counts four)
-  const size_t tsm = strided_taps_lds(a.H, a.W, g.Ho, g.Wo, a.Y, a.X) + 12 * (a.Y + a.X) * sizeof(float);
   // a thread for some six pixels of the input's plane: threads that take one or two are mostly set-up
   // (us with 256, 512 and 1024 threads: N64 14x14 R32 13.4, 20.5, 40.6; N32 28x28 R16 7.7, 8.1, 11.8;
   // N16 55x55 R32 15.8, 13.6, 18.6; N4 112x112 R16 33.6, 20.5, 17.0; N8 150x150 R8 55, 32, 23.5)
   const int tap_threads = HW <= 1536 ? 256 : HW <= 6144 || a.Y == 7 ? 512 : 1024;
   const bool fast = a.Y == a.X && (a.Y == 1 || a.Y == 3 || a.Y == 5 || a.Y == 7);
+  // (the limit on the planes counts the partial sums of four waves; up to sixteen here, of at most
+  // fourteen taps: 672 bytes beyond its 150 KB.  The general kernel has four, of any filter)
+  const size_t lds = strided_taps_lds(a.H, a.W, g.Ho, g.Wo, a.Y, a.X);
+  const size_t tsm = lds + (fast ? (size_t)(tap_threads / 64 - 4) * (a.Y + a.X) * sizeof(float) : 0);
 #define CP4_STRIDED_TAPS(FS_)                                                                    \
   {                                                                                              \
     e = hipFuncSetAttribute(reinterpret_cast<const void*>(taps_strided_fast_kernel<FS_>),        \

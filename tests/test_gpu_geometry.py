@@ -246,3 +246,27 @@ def test_strided_gradients_of_many_channels_on_odd_planes(cp4, dims):
     for name, got, want in zip(("x",) + FACTORS, (dx, *grads), (dxd, *gd)):
         err = np.linalg.norm(got.cpu().double().numpy() - want) / np.linalg.norm(want)
         assert err <= bound, (name, err, bound)
+
+
+# N, C, H, W, T, Y, R: both planes, the taps and their partial sums just below the 150 KB of LDS that
+# admit a layer - the general tap kernel with its largest filters, the fast one with sixteen waves
+@pytest.mark.parametrize("dims", [(1, 2, 172, 172, 2, 127, 2), (1, 16, 174, 174, 16, 45, 1),
+                                  (2, 16, 174, 174, 16, 5, 3)], ids=lambda d: "x".join(map(str, d)))
+def test_strided_taps_at_the_lds_bound(cp4, dims):
+    N, C, H, W, T, Y, R = dims
+    gen = torch.Generator(device="cuda").manual_seed(sum(dims))
+    x = torch.randn((N, C, H, W), device="cuda", generator=gen)
+    fac = [torch.randn((d, R), device="cuda", generator=gen) for d in (T, C, Y, Y)]
+    geom = cp4.geometry(cp4.capi.shape_for(x.shape, *fac, 0), 2, "same")
+    lds = 4 * (H * W + geom.out_h * geom.out_w + 10 * Y)
+    assert 147 * 1024 < lds <= 150 * 1024
+    dy = torch.randn((N, T, geom.out_h, geom.out_w), device="cuda", generator=gen)
+    dx, grads, _ = cp4.capi.layer_backward(cp4.capi.shape_for(x.shape, *fac, 0), geom, x, None, dy, *fac,
+                                           None, True, True, False)
+    assert cp4.capi.layer_last_backward_route() == cp4.capi.ROUTE_DX_FROM_G1
+    _, dxd, gd = dense_reference(x, dy, fac, geom)
+    # as above; a tap's gradient sums the pixels behind Y taps
+    bound = 4 * 2.0 ** -24 * (T + C + N * H * W + 2 * Y) ** 0.5
+    for name, got, want in zip(("x",) + FACTORS, (dx, *grads), (dxd, *gd)):
+        err = np.linalg.norm(got.cpu().double().numpy() - want) / np.linalg.norm(want)
+        assert err <= bound, (name, err, bound)
