@@ -1157,6 +1157,13 @@ __global__ __launch_bounds__(kCT) void grad_gemm_kernel(GradArgs a) {
 // that a wait covers one of them; all threads take a share of Z.  N32 C128 28x28 R16 bf16 17.0 ->
 // 8.9 us, N64 C256 14x14 R64 16.0 -> 14.9, one operand of N32 C256 56x56 R32 30.2 -> 26.2.  (Three
 // chunks in flight: 9.4, 15.0 and 27.9; more splits of the pixels move as much more in partial sets.)
+// The waves decide as well: with one rank block three or four workgroups fit a compute unit (fp32
+// 95 + 32 registers, 99 + 32 with the bias sums, 16-bit 72 + 16 to 82 + 16).  The last chunks as steps
+// of their own, which request nothing past the last, took 124 to 143 + 48: two.  And waves past the last
+// channel only take their share of Z: requesting the last row in place of theirs took the memory's
+// time.  Both together, whole backward-filter or step: N8 C64 224x224 R8 122 -> 107 us, R1 104 -> 90, N16
+// C64 112x112 R8 f16 step 107 -> 97, N5 C434 T3 78x146 R3 77.5 -> 76.7; with an odd number of chunks a
+// split, whose last is requested twice, N32 C256 56x56 R32 109.9 -> 110.4.
 constexpr int kLdS = 36;   // LDS row stride (floats) of the activation tile: 16-byte aligned rows
 
 // How rows move: as 16 bytes (kRowsVec: H*W a multiple of 4, operands on 16-byte boundaries), as
@@ -1174,7 +1181,8 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
   __shared__ u32x4 Zf[2][RB * 2 * 3 * 2 * 32];
   const int which = blockIdx.z;
   const int D = a.D[which], R = a.R, HW = a.HW[which], PS = a.PS[which], cps = a.cps[which];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hi = lane >> 5;
   const int d0 = blockIdx.y * 128 + wave * 32;
   if ((int)blockIdx.y * 128 >= D || (int)blockIdx.x >= a.S[which]) return;
@@ -1219,11 +1227,12 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
     }
   };
   // (rows past D: the last one again, which is not stored; ranks past R count as zero below)
-  auto load_tiles = [&](int slot, int ch) {
+  auto load_tiles = [&](auto live, int slot, int ch) {
     const int p = ch * 32 + acol;
+    if constexpr (decltype(live)::value)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      load4(av[slot][j], actn + (size_t)min(d0 + 8 * j + arow, D - 1) * HW, p);
+      for (int j = 0; j < 4; ++j)
+        load4(av[slot][j], actn + (size_t)min(d0 + 8 * j + arow, D - 1) * HW, p);
     const int pz = ch * 32 + 4 * zq;
 #pragma unroll
     for (int j = 0; j < NZ; ++j) load4(zv[slot][j], zn + (size_t)min(zr, R - 1) * HW, pz + 4 * j);
@@ -1241,30 +1250,36 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
     o.w = 0.f;
     return o;
   };
-  auto store_tiles = [&](int slot, int ch, int buf) {
-    float4 ra[4], rz[NZ];
+  auto store_tiles = [&](auto live, int slot, int ch, int buf) {
+    constexpr bool LIVE = decltype(live)::value;
+    [[maybe_unused]] float4 ra[4];
+    float4 rz[NZ];
+    if constexpr (LIVE)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const act_vec t = av[slot][j];
-      ra[j] = make_float4(act_to_f32(t[0]), act_to_f32(t[1]), act_to_f32(t[2]), act_to_f32(t[3]));
-    }
+      for (int j = 0; j < 4; ++j) {
+        const act_vec t = av[slot][j];
+        ra[j] = make_float4(act_to_f32(t[0]), act_to_f32(t[1]), act_to_f32(t[2]), act_to_f32(t[3]));
+      }
 #pragma unroll
     for (int j = 0; j < NZ; ++j) {
       const z_vec t = zv[slot][j];
       rz[j] = zr < R ? make_float4(t[0], t[1], t[2], t[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
     if (ch * 32 + 32 > HW) {                            // the row's last chunk
+      if constexpr (LIVE)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) ra[j] = settle(ra[j], ch * 32 + acol);
+        for (int j = 0; j < 4; ++j) ra[j] = settle(ra[j], ch * 32 + acol);
 #pragma unroll
       for (int j = 0; j < NZ; ++j) rz[j] = settle(rz[j], ch * 32 + 4 * (zq + j));
     }
+    if constexpr (LIVE) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      *reinterpret_cast<float4*>(&As[wave][(8 * j + arow) * kLdS + acol]) = ra[j];
-    if (sums) {
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<float4*>(&As[wave][(8 * j + arow) * kLdS + acol]) = ra[j];
+      if (sums) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) bs[j] += (ra[j].x + ra[j].y) + (ra[j].z + ra[j].w);
+        for (int j = 0; j < 4; ++j) bs[j] += (ra[j].x + ra[j].y) + (ra[j].z + ra[j].w);
+      }
     }
     // fragment (rank block zr/32, step zq/4, part, half (zq/2)&1, rank zr%32), four pixels a quad
     u32x2* dst = reinterpret_cast<u32x2*>(
@@ -1291,13 +1306,14 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
 #pragma unroll
   for (int mb = 0; mb < RB; ++mb) small[mb] = (f32x16)(0.f);
 #endif
-  auto step = [&](int ch, int slot, bool more) {
+  auto step = [&](auto live, int ch, int slot, bool more) __attribute__((always_inline)) {
     const int buf = (ch - ch0) & 1;
-    store_tiles(slot, ch, buf);
+    store_tiles(live, slot, ch, buf);
     if (ch - ch0 < 3) { BSTAMP(a.dbg, 1, dwg, 4, 1 + (ch - ch0)) }
     __syncthreads();        // Z fragments of this chunk are complete; the other buffer is free
-    if (more) load_tiles(slot, RB == 1 ? ch + 2 : min(ch + 2, ch1 - 1));
+    if (more) load_tiles(live, slot, min(ch + 2, ch1 - 1));
     __builtin_amdgcn_sched_barrier(0);      // (requested here, not behind the products)
+    if constexpr (decltype(live)::value)
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
       const float* ap = &As[wave][l32 * kLdS + 16 * st + 8 * hi];
@@ -1346,35 +1362,24 @@ __global__ __launch_bounds__(kCT) void grad_split_kernel(GradArgs a) {
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  if (ch0 < ch1) {
-    // Every wait with a known number of loads in flight.  With one rank block the last one to three
-    // chunks have steps of their own, of which only those that need it request; with two that
-    // costs registers, and chunks past the last are that one again.
-    load_tiles(0, ch0);
-    load_tiles(1, min(ch0 + 1, ch1 - 1));
+  // Every wait with a known number of loads in flight: chunks past the last are that one again.
+  auto sweep = [&](auto live) {
+    load_tiles(live, 0, ch0);
+    load_tiles(live, 1, min(ch0 + 1, ch1 - 1));
     int ch = ch0;
-    if constexpr (RB == 1) {
-      for (; ch + 4 <= ch1; ch += 2) {
-        step(ch, 0, true);
-        step(ch + 1, 1, true);
-      }
-      if (ch + 3 == ch1) {
-        step(ch, 0, true);
-        step(ch + 1, 1, false);
-        step(ch + 2, 0, false);
-      } else {
-        step(ch, 0, false);
-        if (ch + 1 < ch1) step(ch + 1, 1, false);
-      }
-    } else {
-      for (; ch + 2 < ch1; ch += 2) {
-        step(ch, 0, true);
-        step(ch + 1, 1, true);
-      }
-      step(ch, 0, false);
-      if (ch + 1 < ch1) step(ch + 1, 1, false);
+    for (; ch + 2 < ch1; ch += 2) {
+      step(live, ch, 0, true);
+      step(live, ch + 1, 1, true);
     }
+    step(live, ch, 0, false);
+    if (ch + 1 < ch1) step(live, ch + 1, 1, false);
+  };
+  // (waves past the last row take their share of Z and meet the barriers)
+  if (ch0 < ch1) {
+    if (d0 < D) sweep(std::true_type{});
+    else sweep(std::false_type{});
   }
+  if (d0 >= D) return;
   BSTAMP(a.dbg, 1, dwg, 4, 4)
 #ifndef CP4_BWF_IO16
 #pragma unroll
