@@ -8,6 +8,7 @@
 #include <tuple>
 
 #include "cp4_internal.h"
+#include "store_policy.h"
 
 namespace {
 
@@ -260,6 +261,7 @@ FwdArgs wide_pass_args(const FwdArgs& a, const WidePass& p, bool first) {
   b.x = a.x + (size_t)p.c0 * a.H * a.W;
   b.Fin += (size_t)p.c0 * a.R + p.r0; b.Fout += p.r0; b.FH += p.r0; b.FW += p.r0;
   b.accumulate = !first;
+  if (p.r0 + p.rn < a.R || p.c0 + p.cn < a.Cin) b.reread = cp4::kStreamBytesPass;
   return b;
 }
 bool fwd_pipe64_passes_supported(const FwdArgs& a) {
@@ -932,6 +934,7 @@ cp4_status cp4_conv2d_forward_bias_act(const cp4_shape* shape, const float* x,
       return CP4_OK;
     }
   }
+  plain.reread = cp4::kNeverStreamed;
   rc = run_choice(plain, c, st);
   if (rc != CP4_OK) return rc;
   CP4_HIP(cp4::bias_act_launch(y, bias, activation, shape->N, shape->T,

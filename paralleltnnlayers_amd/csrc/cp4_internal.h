@@ -35,6 +35,9 @@ struct FwdArgs {
   int ldf;
   size_t ldx;
   int accumulate;
+  // Not 0: the launch that follows reads y back (a later pass, the bias / activation kernel); y
+  // leaves the caches only from so many bytes on.
+  size_t reread;
   // 2-D-tap build of the producer / consumer kernel only: depthwise filter
   // [Y, X, R] used instead of the outer product FH x FW (FH, FW unused then).
   const float* taps2d;

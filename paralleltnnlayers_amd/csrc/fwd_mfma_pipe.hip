@@ -1526,7 +1526,8 @@ hipError_t launch_as(const FwdArgs& a, const PipePlan& pl, hipStream_t st) {
 #ifdef CP4_PIPE_EPILOGUE
     const int policy = store_policy(a.y, plane, bytes, kStreamBytesLayer);
 #else
-    const int policy = store_policy(a.y, plane, bytes, kStreamBytes);
+    const int policy = a.reread ? store_policy(a.y, plane, bytes, a.reread, a.reread)
+                                : store_policy(a.y, plane, bytes, kStreamBytes);
 #endif
 #if !defined(CP4_PIPE_IO16) && !defined(CP4_PIPE_STRIDED)
     if (policy == kStoreStreamed) return launch_stored<FS, CPQ, KR, NQ, PAIR, kStoreStreamed>(a, pl, st);

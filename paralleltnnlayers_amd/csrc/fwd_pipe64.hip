@@ -611,7 +611,8 @@ bool plan(const FwdArgs& a, Plan64* best) {
 template <int FS, int CPQ, int NCH>
 hipError_t launch_as(const FwdArgs& a, const Plan64& pl, hipStream_t st) {
   const size_t plane = (size_t)a.H * a.W * sizeof(float);
-  const int store = store_policy(a.y, plane, plane * a.N * a.Cout, kStreamBytes);
+  const int store = a.reread ? store_policy(a.y, plane, plane * a.N * a.Cout, a.reread, a.reread)
+                             : store_policy(a.y, plane, plane * a.N * a.Cout, kStreamBytes);
   auto k = a.accumulate             ? fwd_pipe64_kernel<FS, CPQ, NCH, true, kStorePlain>
            : store == kStoreStreamed ? fwd_pipe64_kernel<FS, CPQ, NCH, false, kStoreStreamed>
            : store == kStoreThrough  ? fwd_pipe64_kernel<FS, CPQ, NCH, false, kStoreThrough>

@@ -12,6 +12,10 @@
 // written.
 // Behind a layer's activation results from 96 to 128 MB are stored plainly: N32 C256 56x56 R32's training
 // step 217 us with a streamed y, 215 with one that goes through, 211.
+// A result that the next launch reads again is streamed from 128 MB on if that is another pass of the
+// layer (R128, us, through / streamed: N32 C256 56x56 155 / 171, N44 237 / 231, N52 293 / 285; R96 N36 145 /
+// 182, N48 263 / 249), never if it is the bias / activation kernel (R64: N32 100 / 116, N44 149 / 156, N50
+// 156 / 170).
 // Plain where planes start inside a cache line and the result is not small: parts of lines then
 // go to memory one by one (N8 C64 130x130, 35 MB, rotating buffers: 28 us, through 35; N8 C64 66x70,
 // 9 MB, 11.1 and 10.3).
@@ -31,12 +35,16 @@ enum StorePolicy { kStorePlain, kStoreThrough, kStoreStreamed };
 // inside cache lines.
 constexpr size_t kStreamBytesLayer = (size_t)128 << 20, kStreamBytes = (size_t)96 << 20;
 constexpr size_t kThroughOffLine = (size_t)16 << 20;
+// ... where another pass of the layer follows; and bytes up to which a result goes through.
+constexpr size_t kStreamBytesPass = (size_t)128 << 20, kNeverStreamed = ~(size_t)0;
+constexpr size_t kThroughBytes = kStreamBytes;
 
 // For planes of `plane` bytes, `bytes` in all.
-inline int store_policy(const void* dst, size_t plane, size_t bytes, size_t stream_from) {
+inline int store_policy(const void* dst, size_t plane, size_t bytes, size_t stream_from,
+                        size_t through_to = kThroughBytes) {
   const bool lines = plane % 128 == 0 && (reinterpret_cast<uintptr_t>(dst) & 127) == 0;
   if (!lines) return bytes <= kThroughOffLine ? kStoreThrough : kStorePlain;
-  return bytes >= stream_from ? kStoreStreamed : bytes >= kStreamBytes ? kStorePlain : kStoreThrough;
+  return bytes >= stream_from ? kStoreStreamed : bytes <= through_to ? kStoreThrough : kStorePlain;
 }
 
 template <class T>
