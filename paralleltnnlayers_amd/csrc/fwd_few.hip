@@ -524,8 +524,8 @@ bool plan_uncached(const FwdArgs& a, FewPlan* best) {
 template <int FS, int NCH, int RING, int OCC, int NW>
 hipError_t launch_as(const FwdArgs& a, const FewPlan& pl, hipStream_t st) {
   const size_t plane = (size_t)a.H * a.W * sizeof(float);
-  const int store = store_policy(a.y, plane, plane * a.N * a.Cout,
-                                 a.bias || a.act ? kStreamBytesLayer : kStreamBytes);
+  const size_t from = a.bias || a.act ? kStreamBytesFewLayer : kStreamBytes;
+  const int store = store_policy(a.y, plane, plane * a.N * a.Cout, from, from);
 #define CP4_FEW(BIAS_)                                                                        \
   (store == kStoreStreamed  ? fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStoreStreamed>   \
    : store == kStoreThrough ? fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStoreThrough>    \

@@ -85,9 +85,12 @@ def test_layer_backward(cp4, dims, dtype):
         assert ((g - w).abs() <= 4 * 2.0 ** -24 * (N * H * W) ** 0.5 * t).all()
 
 
-# results that the next launch reads again - another pass, the bias kernel -, at either side of the lines
+# results that the next launch reads again - another pass, the bias kernel -, at either side of the lines;
+# strips of three, five and eight rows, small, large and too large to go through
 @pytest.mark.parametrize("bias", [False, True], ids=["plain", "bias"])
 @pytest.mark.parametrize("dims", [(36, 64, 56, 56, 256, 1, 128), (44, 64, 56, 56, 256, 1, 96),
-                                  (33, 64, 56, 56, 256, 1, 64), (44, 64, 56, 56, 256, 3, 48)], ids=lambda d: "x".join(map(str, d)))
+                                  (33, 64, 56, 56, 256, 1, 64), (44, 64, 56, 56, 256, 3, 48),
+                                  (12, 64, 56, 56, 256, 3, 32), (20, 64, 56, 56, 256, 3, 32),
+                                  (26, 64, 56, 56, 256, 3, 32)], ids=lambda d: "x".join(map(str, d)))
 def test_forward_read_again(cp4, dims, bias):
     test_forward(cp4, dims, bias)
