@@ -245,7 +245,15 @@ __device__ __forceinline__ void contract_split(const ContractArgs& a, const int 
   constexpr int kRing = MASK ? kSplitRing / 2 : kSplitRing;     // (as many loads in flight)
   extern __shared__ float Fs[];
   u32x4* Fb = reinterpret_cast<u32x4*>(Fs);
-  const int mb = blockIdx.z;
+  // two rank tiles: those of the same items eight workgroups apart, on one die and at about the same
+  // time, so that the second reads the activations from the L2 (training step of N32 C256 56x56 R40 361 us
+  // with all of the first tile's before the second's and either storing the masked dy, 344 with the
+  // first alone storing it, 305 with both; N32 C256 28x28 R64 bf16 135, 134 and 128)
+  int mb = 0, wg = blockIdx.x;
+  if (a.RP > 32) {
+    mb = (wg >> 3) & 1;
+    wg = (wg >> 4) * 8 + (wg & 7);
+  }
   const int Cin = a.Cin[which], R = a.R, HW = a.HW[which], npb = a.npb[which], items = a.items[which];
   const float* F = a.F[which];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -254,10 +262,10 @@ __device__ __forceinline__ void contract_split(const ContractArgs& a, const int 
   // This wave's item; waves past the end keep a valid (clamped) item for their
   // loads and skip the store, so that every wave reaches the barrier.
   const int ks = a.ks[which];
-  if ((int)blockIdx.x * (kSW / 64) >= items * ks) return;         // whole workgroup
-  [[maybe_unused]] const int dwg = (blockIdx.z * 2 + blockIdx.y) * gridDim.x + blockIdx.x;
+  if (wg * (kSW / 64) >= items * ks) return;         // whole workgroup
+  [[maybe_unused]] const int dwg = blockIdx.y * gridDim.x + blockIdx.x;
   BSTAMP(a.dbg, 0, dwg, 8, 0)
-  const int slot = blockIdx.x * (kSW / 64) + wave;        // (item, channel split)
+  const int slot = wg * (kSW / 64) + wave;        // (item, channel split)
   const int item_raw = slot / ks, part = slot - item_raw * ks;   // item = (image, 32-pixel block)
   const bool has_item = item_raw < items;
   const int item = has_item ? item_raw : items - 1;
@@ -299,9 +307,9 @@ __device__ __forceinline__ void contract_split(const ContractArgs& a, const int 
   const size_t at = ((size_t)n * (a.ldc[which] ? a.ldc[which] : Cin) + 16 * c0) * HW;
   constexpr unsigned kEl = sizeof(act_t);
   const unsigned voff = (unsigned)(8 * hi * HW + pc) * kEl;
-  auto chunk_of = [&](const act_t* base, int ch) {
+  auto chunk_of = [&](const act_t* base, int ch, bool any = true) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<act_t*>(base + at + (size_t)(16 * ch) * HW), 0,
-                                             16 * HW * (int)kEl, 0x00020000);
+                                             any ? 16 * HW * (int)kEl : 0, 0x00020000);
   };
 #ifdef CP4_BWF_IO16
   using ring_t = unsigned;     // raw 16-bit values, zero-extended
@@ -327,12 +335,12 @@ __device__ __forceinline__ void contract_split(const ContractArgs& a, const int 
       for (int e = 0; e < 8; ++e) yb[slot][e] = load1(ry, e);
     }
   };
-  // the chunk of a ring slot behind the activation, and that into memory.  (Lanes and waves past
-  // the end hold the last pixel's or item's values and store those once more, and so do the waves
-  // of further rank tiles.)
+  // the chunk of a ring slot behind the activation, and that into memory from the first rank tile.
+  // (Lanes and waves past the end hold the last pixel's or item's values and store those once more.
+  // The second tile's descriptor is empty: its stores go nowhere.)
   auto mask_chunk = [&](int slot, int ch) {
     if constexpr (MASK) {
-      const __amdgpu_buffer_rsrc_t ro = chunk_of(a.masked, ch);
+      const __amdgpu_buffer_rsrc_t ro = chunk_of(a.masked, ch, mb == 0);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         xb[slot][e] = masked_act(xb[slot][e], yb[slot][e]);
@@ -1546,6 +1554,12 @@ bool split_contraction(int C, int T) {
   return (C & 15) == 0 && (T & 15) == 0 && (size_t)(C > T ? C : T) * 192 <= 160 * 1024;
 }
 
+// Workgroups of the split contraction for `waves` waves a rank tile.
+unsigned split_workgroups(long waves, int RP) {
+  const unsigned wgs = (unsigned)((waves + kSW / 64 - 1) / (kSW / 64));
+  return RP > 32 ? 2 * ((wgs + 7) / 8 * 8) : wgs;
+}
+
 // The split contractions of `operands` planes of HW[i] pixels in one launch (ContractArgs::npb,
 // items and ks are filled in here): 32-pixel blocks, fragments of 6 bytes per factor entry.
 hipError_t launch_contract_split(ContractArgs c, int operands, hipStream_t st) {
@@ -1575,7 +1589,7 @@ hipError_t launch_contract_split(ContractArgs c, int operands, hipStream_t st) {
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (e != hipSuccess) return e;
-  k<<<dim3((unsigned)((most + kSW / 64 - 1) / (kSW / 64)), operands, c.RP / 32), kSW, smem, st>>>(c);
+  k<<<dim3(split_workgroups(most, c.RP), operands), kSW, smem, st>>>(c);
   return hipGetLastError();
 }
 
@@ -1606,8 +1620,7 @@ hipError_t contract_slices(const float* src, const float* F, float* Z, float* sl
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(contract_split_kernel),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (e != hipSuccess) return e;
-    contract_split_kernel<<<dim3((unsigned)((c.items[0] + kSW / 64 - 1) / (kSW / 64)), 1, RP / 32), kSW,
-                            smem, st>>>(c);
+    contract_split_kernel<<<split_workgroups(c.items[0], RP), kSW, smem, st>>>(c);
     if (c0) {
       e = add_f32_launch(Z, slice, (size_t)N * R * HW, st);
       if (e != hipSuccess) return e;
