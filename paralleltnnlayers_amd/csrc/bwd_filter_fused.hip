@@ -20,6 +20,7 @@
 //      form the tap gradients from the A window they already hold.
 //   3. reduce_fused_kernel: fixed-order sum of the partials (bit-reproducible; no
 //      floating-point atomics anywhere).
+#include <algorithm>
 #include <cstdint>
 #include <type_traits>
 
@@ -106,11 +107,15 @@ __device__ __forceinline__ void contract_all(const ContractAllArgs& a, const int
     if constexpr (MASK) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) xb[slot][e] *= yb[slot][e] > 0.f ? 1.f : 0.f;
-      if (ch < nch && valid) {
-        float* out = a.masked + ((size_t)n * Cin + 16 * (c0 + ch) + 8 * hi) * HW + p;
+      // (lanes past the plane and chunks past the wave's last: outside the descriptor, not branched
+      // around, so that the waits for the loads behind them know their number)
+      const __amdgpu_buffer_rsrc_t mrs = __builtin_amdgcn_make_buffer_rsrc(
+          a.masked + (size_t)n * Cin * HW, 0, ch < nch ? Cin * HW * 4 : 0, 0x00020000);
+      const unsigned soff = sbase + (unsigned)(16 * ch) * (unsigned)HW * 4u;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) out[(size_t)e * HW] = xb[slot][e];
-      }
+      for (int e = 0; e < 8; ++e)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(xb[slot][e]), mrs, valid ? voff : 0x80000000u,
+                                              soff + (unsigned)e * HW * 4u, 0);
     }
   };
   // the first activation chunks are requested before the factor tile is built
@@ -722,6 +727,20 @@ struct FusedPlan {
   size_t plane, part_elems;   // floats
 };
 
+// Waves that share an item of the contraction: 32-pixel blocks of x and of dy are the wave items; with few
+// of them 2 or 4 take a slice of the channels each until there are about three waves per compute unit.
+// Where dy's mask rides along: a second one below 1536 items of it with more than 256 channels (kernel,
+// us, one and two waves an item: N32 C64 T512 28x28 R16 62 and 47; four, 128 channels each, N64 C512 T512
+// 14x14 R32 cost its step 10 %).
+int channel_splits(long items, int C, int T, bool masked) {
+  const int nch_min = (C < T ? C : T) >> 4;
+  auto splits = [&](int ks) { return (C >> 4) % ks == 0 && (T >> 4) % ks == 0 && nch_min / ks >= 2; };
+  int ks = 1;
+  while (ks < 4 && 2 * items * ks < 3L * num_compute_units() && splits(2 * ks)) ks *= 2;
+  if (masked && ks == 1 && T > 256 && items < 1536 && splits(2)) ks = 2;
+  return ks;
+}
+
 FusedPlan make_fused_plan(const cp4_shape& s) {
   FusedPlan p{};
   const int N = s.N, C = s.C, T = s.T, H = s.H, W = s.W, FS = s.Y, R = s.Rank;
@@ -767,17 +786,10 @@ FusedPlan make_fused_plan(const cp4_shape& s) {
   const size_t tail_gemm = (size_t)8 * p.RB * 16 * 64 * 4, tail_taps = (size_t)2 * FS * 512 * 4;
   if (p.lds < tail_gemm) p.lds = tail_gemm;
   if (p.lds < tail_taps) p.lds = tail_taps;
-  // contraction: 32-pixel blocks of x and of dy are the wave items; with few of them
-  // 2 or 4 waves share an item (a slice of the channels each) until there are about
-  // three waves per compute unit, and a workgroup is four waves (one per SIMD, an
-  // eight-chunk load ring) unless the items alone fill the chip twice over
-  const int npb = (HW + 31) / 32;
-  const long wave_items = 2L * N * npb;
-  p.ks = 1;
-  const int nch_min = (C < T ? C : T) >> 4;
-  while (p.ks < 4 && wave_items * p.ks < 3L * cus && ((C >> 4) % (2 * p.ks)) == 0 &&
-         ((T >> 4) % (2 * p.ks)) == 0 && nch_min / (2 * p.ks) >= 2)
-    p.ks *= 2;
+  // contraction: a workgroup is four waves (one per SIMD, an eight-chunk load ring) unless the
+  // items alone fill the chip twice over
+  const long wave_items = 2L * N * ((HW + 31) / 32);
+  p.ks = channel_splits(wave_items / 2, C, T, false);
   p.nw = wave_items * p.ks <= 5L * cus ? 4 : 8;
   p.ring = p.nw == 4 ? 8 : 4;
   p.lds_contract = ((size_t)dmax / 16 + 1) * p.RB * kFragBytes;   // + the zero block
@@ -835,6 +847,12 @@ size_t bwd_filter_fused_workspace_bytes(const cp4_shape& s) {
   return (2 * p.plane + p.part_elems) * sizeof(float);
 }
 
+// (as bwd_filter_mfma_mask_pays)
+bool bwd_filter_fused_mask_pays(const cp4_shape& s) {
+  const long items = (long)s.N * ((s.H * s.W + 31) / 32);
+  const int ks = channel_splits(items, (int)s.C, (int)s.T, true);
+  return (int)s.T / ks <= 256 || items * ks >= 1536 || (size_t)s.N * s.T * s.H * s.W <= (size_t)4 << 20;
+}
 int bwd_filter_fused_bias_sets(const cp4_shape& s) { return make_fused_plan(s).S; }
 
 hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
@@ -859,7 +877,9 @@ hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
   c.through = store_policy(A, HW * sizeof(float), (size_t)N * R * HW * sizeof(float), ~(size_t)0) == kStoreThrough &&
               store_policy(G3, HW * sizeof(float), (size_t)N * R * HW * sizeof(float), ~(size_t)0) == kStoreThrough;
   c.vecfill = (R & 3) == 0 && ((reinterpret_cast<uintptr_t>(a.FC) | reinterpret_cast<uintptr_t>(a.FK)) & 15) == 0;
-  const long slots = (long)c.items * p.ks;
+  const int ks = c.y ? channel_splits(c.items, a.C, a.T, true) : p.ks;
+  const size_t lds_contract = ks > 1 ? std::max(p.lds_contract, (size_t)p.nw * p.RB * 16 * 64 * 4) : p.lds_contract;
+  const long slots = (long)c.items * ks;
   const dim3 cgrid((unsigned)((slots + p.nw - 1) / p.nw), 2);
   hipError_t e;
 #define CP4_CONTRACT(RB_, KS_, RING_)                                                          \
@@ -867,14 +887,14 @@ hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
     auto k = c.y ? contract_all_kernel<RB_, KS_, RING_, true>                                  \
                  : contract_all_kernel<RB_, KS_, RING_, false>;                                \
     e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),                                  \
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds_contract);  \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_contract);  \
     if (e != hipSuccess) return e;                                                             \
-    k<<<cgrid, p.nw * 64, p.lds_contract, st>>>(c);                                            \
+    k<<<cgrid, p.nw * 64, lds_contract, st>>>(c);                                            \
   }
 #define CP4_CONTRACT_KS(RB_, RING_)                                                            \
   {                                                                                            \
-    if (p.ks == 1) CP4_CONTRACT(RB_, 1, RING_)                                                 \
-    else if (p.ks == 2) CP4_CONTRACT(RB_, 2, RING_)                                            \
+    if (ks == 1) CP4_CONTRACT(RB_, 1, RING_)                                                 \
+    else if (ks == 2) CP4_CONTRACT(RB_, 2, RING_)                                            \
     else CP4_CONTRACT(RB_, 4, RING_)                                                           \
   }
   if (p.RB == 1) {

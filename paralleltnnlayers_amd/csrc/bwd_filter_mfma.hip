@@ -1560,6 +1560,27 @@ unsigned split_workgroups(long waves, int RP) {
   return RP > 32 ? 2 * ((wgs + 7) / 8 * 8) : wgs;
 }
 
+// Waves that share an item of the split contraction, for `waves` items of all rank tiles: with
+// few items 2 or 4, each on a slice of the channels, until there are about 512 waves (every
+// workgroup builds the whole factor tile, so more splits than that cost more than they hide; a
+// slice keeps >= 2 chunks).  A wave that moves the mask's operands too moves three times the bytes:
+// until there are 1024 where slices of 128 channels are left or the other operand's planes are the
+// larger (`smaller`: that one's waves start first), 1536 with more than 256 channels a wave.  Kernel, us,
+// with less of it / now: 512 and 1024 waves, N8 T256 55x55 R16 36.7 / 33.1, bf16 N64 T256 14x14 13.2 / 12.9,
+// but slices of 96 channels N24 T192 27x27 R32 17.0 / 19.0, of 32 N8 T64 55x55 R8 9.3 / 11.2, bf16 of 64 N32
+// T128 28x28 11.4 / 12.1; beside larger planes N16 T256 28x28 21.8 / 20.8, N32 41.5 / 38.8, N64 T512
+// 14x14 49.4 / 38.4, N16 T128 28x28 12.6 / 10.7; 800 and 1600 waves, bf16 N32 T512 28x28 R32 43.4 / 39.0.
+int channel_splits(int Cin, long waves, bool masked, bool smaller) {
+  const int nch = Cin >> 4;
+  int ks = 1;
+  while (ks < 4 && nch % (2 * ks) == 0 && nch / (2 * ks) >= 2 &&
+         waves * ks < (!masked ? kKsWaves
+                       : Cin / ks > 256 ? 3 * kKsWaves
+                       : Cin / ks == 256 || smaller ? 2 * kKsWaves : kKsWaves))
+    ks *= 2;
+  return ks;
+}
+
 // The split contractions of `operands` planes of HW[i] pixels in one launch (ContractArgs::npb,
 // items and ks are filled in here): 32-pixel blocks, fragments of 6 bytes per factor entry.
 hipError_t launch_contract_split(ContractArgs c, int operands, hipStream_t st) {
@@ -1570,18 +1591,8 @@ hipError_t launch_contract_split(ContractArgs c, int operands, hipStream_t st) {
     c.items[i] = c.N * c.npb[i];
     const size_t plane = (size_t)c.HW[i] * sizeof(float);
     c.through[i] = store_policy(c.Z[i], plane, plane * c.N * c.R, ~(size_t)0) == kStoreThrough;
-    // few items: 2 or 4 waves per item, each on a slice of the channels, until
-    // there are about 512 waves (every workgroup builds the whole factor tile,
-    // so more splits than that cost more than they hide; a slice keeps >= 2 chunks),
-    // 1024 where a wave moves the mask's operands too (N16 T256 28x28 R32 beside C128 55x55: 18.9 -> 16.8
-    // us; in 16 bits 11.3 -> 12.0)
-    const long waves = i == 1 && c.y ? kKsWaves * (long)sizeof(act_t) / 2 : kKsWaves;
-    const int nch = c.Cin[i] >> 4;
-    int& ks = c.ks[i];
-    ks = 1;
-    while (ks < 4 && (long)c.items[i] * (c.RP / 32) * ks < waves && nch % (2 * ks) == 0 &&
-           nch / (2 * ks) >= 2)
-      ks *= 2;
+    c.ks[i] = channel_splits(c.Cin[i], (long)c.items[i] * (c.RP / 32), i == 1 && c.y, c.HW[1] < c.HW[0]);
+    const int ks = c.ks[i];
     most = std::max(most, (long)c.items[i] * ks);
     smem = std::max(smem, std::max((size_t)c.Cin[i] * 192, ks > 1 ? (size_t)kSW * 16 * sizeof(float) : 0));
   }
@@ -1667,6 +1678,15 @@ bool bwd_filter_mfma_supported(const cp4_shape& s) {
 bool bwd_filter_mfma_masks(const cp4_shape& s, bool aligned16) {
   const size_t HW = (size_t)s.H * s.W;
   return split_contraction((int)s.C, (int)s.T) && ((HW & 1) || ((HW & 3) == 0 && aligned16));
+}
+// Whether that pays: with more than 256 channels a wave and few waves the pass of its own over dy and y is
+// the quicker (training steps, us, inside / on its own: N8 C768 T768 40x40 R16 191 / 184, N16 C400 T400 45x45
+// R16 169 / 164; but with 1568 waves N16 C384 T384 56x56 R16 194 / 218), unless dy is so small that its
+// launch counts (N4 C512 T512 40x40 R32, 13 MB, 100 / 104).  s: the shape with dy's planes.
+bool bwd_filter_mfma_mask_pays(const cp4_shape& s, bool smaller) {
+  const long waves = (long)s.N * ((s.H * s.W + 31) / 32) * (s.Rank <= 32 ? 1 : 2);
+  const int ks = channel_splits((int)s.T, waves, true, smaller);
+  return (int)s.T / ks <= 256 || waves * ks >= 3 * kKsWaves || (size_t)s.N * s.T * s.H * s.W <= (size_t)4 << 20;
 }
 int bwd_filter_mfma_bias_sets(const cp4_shape& s) {
   return make_plan(s.N, s.C, s.T, s.H, s.W, s.Y, s.X, s.Rank, s.pad).S;

@@ -1708,12 +1708,13 @@ int layer_filter_takes_mask(const cp4_shape& s, const cp4_geometry* g, int dtype
     return (gg.sh > 1 || gg.sw > 1) && bwd_filter_mfma_strided_supported(s, gg) &&
            bwd_filter_mfma_strided_masks(s, gg, aligned16);
   }
-  if (dtype != CP4_DTYPE_F32) return bwd_filter_mfma_io16_supported(s);
+  if (dtype != CP4_DTYPE_F32) return bwd_filter_mfma_io16_supported(s) && bwd_filter_mfma_mask_pays(s, false);
   const FilterRoutes routes = filter_routes(s, (bits & 7) == 0, aligned16,
                                             (reinterpret_cast<uintptr_t>(workspace) & 255) == 0);
   if (routes.tiles_ok || filter_pad_route(s)) return 0;
   const int variant = default_filter_variant(s, routes);
-  return variant == 2 || (variant == 1 && bwd_filter_mfma_masks(s, aligned16)) ? variant : 0;
+  if (variant == 2) return bwd_filter_fused_mask_pays(s) ? 2 : 0;
+  return variant == 1 && bwd_filter_mfma_masks(s, aligned16) && bwd_filter_mfma_mask_pays(s, false) ? 1 : 0;
 }
 
 size_t layer_bias_sets(const cp4_shape& s, const cp4_geometry* g) {

@@ -239,6 +239,7 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs&, hipStream_t);
 // 16-byte boundaries or not), and the partial sets of the bias gradient they leave.
 bool bwd_filter_mfma_masks(const cp4_shape&, bool aligned16);
 bool bwd_filter_mfma_strided_masks(const cp4_shape&, const Geometry&, bool aligned16);
+bool bwd_filter_mfma_mask_pays(const cp4_shape& dy_planes, bool smaller_than_x);
 int bwd_filter_mfma_bias_sets(const cp4_shape&);
 // The same with the layer's activation mask and bias gradient in it (BwdFilterArgs::act_y,
 // dbias, mask_ws); operands on 16-byte boundaries.
@@ -258,6 +259,7 @@ bool bwd_filter_fused_supported(const cp4_shape&);
 // time is launches and first-load latencies rather than bandwidth).
 bool bwd_filter_fused_preferred(const cp4_shape&);
 size_t bwd_filter_fused_workspace_bytes(const cp4_shape&);
+bool bwd_filter_fused_mask_pays(const cp4_shape&);
 int bwd_filter_fused_bias_sets(const cp4_shape&);      // takes BwdFilterArgs::act_y and dbias throughout
 hipError_t bwd_filter_fused_launch(const BwdFilterArgs&, hipStream_t);
 // Few channels on both sides (square filters of 1, 3, 5 taps; T * C up to 256 with plain

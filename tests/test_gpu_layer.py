@@ -192,6 +192,58 @@ def test_mask_and_bias_gradient_inside_the_passes(capi, case, dtype, relu):
     assert torch.equal(dx, dx2) and all(torch.equal(a, b) for a, b in zip(grads, grads2))
 
 
+def layer_reference(x, dy, fac, k, stride, geometry):
+    """(dx, dFK, dFC, dFH, dFW) of dy by autograd over the four contractions in float64."""
+    N, C, H, W = x.shape
+    x = x.double().requires_grad_()
+    FK, FC, FH, FW = f = [t.double().requires_grad_() for t in fac]
+    A = torch.matmul(FC.t(), x.flatten(2)).view(N, -1, H, W)
+    sh, top, left = (stride, geometry.pad_top, geometry.pad_left) if geometry else (1, k // 2, k // 2)
+    oh, ow = dy.shape[2:]
+    A = torch.nn.functional.pad(A, (left, k + sh, top, k + sh))
+    rows = lambda t, i, n: t.narrow(2, i, sh * (n - 1) + 1)[:, :, ::sh]
+    B = sum(FH[i].view(1, -1, 1, 1) * rows(A, i, oh) for i in range(k))
+    Z = sum(FW[j].view(1, -1, 1, 1) * rows(B.transpose(2, 3), j, ow).transpose(2, 3) for j in range(k))
+    y = torch.matmul(FK, Z.flatten(2)).view(N, -1, oh, ow)
+    return torch.autograd.grad(y, [x] + f, dy.double())
+
+
+# (N, C, H, W, T, k, R, stride), inside: channels a wave, waves and bytes at either side of where the mask rides
+# along, in the three-launch and the four-launch variant; two rank tiles, strides
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("case,inside", [
+    ((12, 64, 28, 28, 512, 3, 16, 1), True), ((12, 80, 28, 28, 528, 1, 16, 1), False),
+    ((2, 80, 28, 28, 528, 3, 40, 1), True), ((12, 32, 27, 27, 640, 3, 8, 1), True),
+    ((12, 32, 27, 27, 656, 3, 8, 1), False),
+    ((7, 512, 29, 29, 512, 1, 64, 1), True), ((4, 64, 64, 64, 96, 3, 64, 1), True),
+    ((6, 32, 56, 56, 320, 3, 40, 2), True)], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else v)
+def test_mask_inside_wide_layers(capi, case, inside, dtype):
+    N, C, H, W, T, k, R, stride = case
+    if stride > 1 and dtype != torch.float32:
+        pytest.skip("a layer with a stride takes fp32 activations")
+    gen = torch.Generator(device="cuda").manual_seed(N + C + H + W + R)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, fac = mk(N, C, H, W).to(dtype), [mk(d, R) for d in (T, C, k, k)]
+    s = capi.shape_for(x.shape, *fac, k // 2)
+    g = capi.geometry(s, stride, "same") if stride > 1 else None
+    y = capi.layer_forward(s, g, x, *fac, mk(T), "relu")
+    dy = mk(*y.shape).to(dtype)
+    dx, grads, dbias = capi.layer_backward(s, g, x, y, dy, *fac, "relu")
+    assert capi.layer_last_backward_mask_inside() == inside
+    masked = dy * (y > 0)
+    want = layer_reference(x, masked, fac, k, stride, g)
+    # sums of T and C channels, R ranks, the taps and the pixels, signs at random: n roundings of 2^-24
+    # grow as sqrt(n), as the sum itself; times 4 for the stages one after the other.  dx is rounded to
+    # the layer's type.
+    pixels = N * masked.shape[2] * masked.shape[3]
+    bound = 4 * 2.0 ** -24 * (T + C + R + 2 * k + pixels) ** 0.5
+    for name, got, w in zip(("x", "FK", "FC", "FH", "FW"), (dx, *grads), want):
+        err = ((got.double() - w).norm() / w.norm()).item()
+        assert err <= bound + (2.0 ** -8 if name == "x" and dtype == torch.bfloat16 else 0), (name, err, bound)
+    tol = 4 * 2.0 ** -24 * ((masked.double() ** 2).sum(dim=(0, 2, 3)) * pixels).sqrt()
+    assert ((dbias.double() - masked.double().sum(dim=(0, 2, 3))).abs() <= tol).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16],
                          ids=["f32", "bf16", "f16"])
 def test_non_finite_gradient_is_seen_inside_the_passes(capi, dtype):
