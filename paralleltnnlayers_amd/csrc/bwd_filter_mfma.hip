@@ -1469,11 +1469,12 @@ struct ReduceArgs {
   float* out[5];
   int count[5], S[5];
 };
-// A workgroup owns 64 consecutive outputs; its waves (sixteen, four below 128 sets) each
+// A workgroup owns 64 consecutive outputs; its waves (sixteen, four below 192 sets) each
 // sum a part of the S partials in index order (eight loads in flight, added as a tree), then the
 // parts are added in wave order: the result does not depend on timing.  Bound by the latency of
 // those loads: N16 C128 T256 55x55 R32 stride 2, 224 and 64 sets, 4.6 us with four waves, 3.9 with sixteen;
-// N64 C256 T256 14x14 R64, 64 sets, 3.95 and 4.7.
+// N64 C256 T256 14x14 R64, 64 sets, 3.95 and 4.7; N16 C400 T400 45x45 R16, 128 sets, 4.0 and 4.4; N32 C512
+// T512 28x28 R32 in 16 bits, 128 sets, 4.1 and 7.0; N32 C256 56x56 R32, 256 sets, 7.3 and 6.5.
 constexpr int kReduceWaves = 16;
 __global__ __launch_bounds__(64 * kReduceWaves) void reduce_sets_kernel(ReduceArgs a) {
   __shared__ float part[kReduceWaves][64];
@@ -1650,7 +1651,7 @@ hipError_t launch_reduce(const float* const (&parts)[5], float* const (&outs)[5]
     r.part[i] = parts[i]; r.out[i] = outs[i]; r.count[i] = counts[i]; r.S[i] = Ss[i];
     if (counts[i] > most) most = counts[i];
   }
-  reduce_sets_kernel<<<dim3((most + 63) / 64, counts[4] ? 5 : 4), sets >= 128 ? 64 * kReduceWaves : 256, 0,
+  reduce_sets_kernel<<<dim3((most + 63) / 64, counts[4] ? 5 : 4), sets >= 192 ? 64 * kReduceWaves : 256, 0,
                        st>>>(r);
   return hipGetLastError();
 }
