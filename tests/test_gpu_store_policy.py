@@ -55,6 +55,16 @@ def test_forward(cp4, dims, bias):
     assert ((y[ends].double() - want).abs() <= 4 * (C + 2 * k + R) ** 0.5 * 2.0 ** -24 * terms).all()
 
 
+def factor_gradients(x, dy, fac, k):
+    """dFK, dFC, dFH, dFW of the layer without an epilogue by autograd in float64."""
+    (N, C, H, W), P = x.shape, k // 2
+    FK, FC, FH, FW = f = [t.double().requires_grad_() for t in fac]
+    A = torch.nn.functional.pad(torch.matmul(FC.t(), x.double().flatten(2)).view(N, -1, H, W), (P, P, P, P))
+    B = sum(FH[i].view(1, -1, 1, 1) * A[:, :, i:i + H] for i in range(k))
+    Z = sum(FW[j].view(1, -1, 1, 1) * B[..., j:j + W] for j in range(k))
+    return torch.autograd.grad(torch.matmul(FK, Z.flatten(2)), f, dy.double().flatten(2))
+
+
 # the input gradient beside the factors': dx streamed, through and off the lines
 @pytest.mark.parametrize("dims", [(36, 256, 56, 56, 64, 3, 16), (8, 64, 56, 56, 64, 3, 64),
                                   (40, 64, 58, 58, 64, 3, 64), (2, 64, 36, 36, 64, 3, 64)],
@@ -77,7 +87,12 @@ def test_layer_backward(cp4, dims, dtype):
     eps = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
     bound = 4 * (T + 2 * k + R) ** 0.5 * 2.0 ** -24 * terms + eps * want.abs()
     assert ((dx[ends].double() - want).abs() <= bound).all()
-    # the factor gradients' intermediates: the same call without dx and bias computes them again
+    # the factor gradients in float64: n roundings of 2^-24 grow as sqrt(n), as sums of n terms with signs at
+    # random do; times 4 for the stages one after the other
+    near = 4 * 2.0 ** -24 * (T + C + R + 2 * k + N * H * W) ** 0.5
+    for g, w in zip(grads, factor_gradients(x, masked, fac, k)):
+        assert (g.double() - w).norm() <= near * w.norm()
+    # and their intermediates: the same call without dx and bias computes them again
     alone = capi.layer_backward(s, None, x, None, masked, *fac, None, False, True, False)[1]
     mags = capi.layer_backward(s, None, x.abs(), None, masked.abs(), *[f.abs() for f in fac], None, False,
                                True, False)[1]
