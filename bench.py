@@ -48,7 +48,7 @@ FACTORS = ("FK", "FC", "FH", "FW")
 # workload AND the plan the counters were taken on (variant, strip rows, workgroups): a
 # launch that runs another plan reports null rather than another kernel's bytes.
 MEASURED_TRAFFIC = {
-    # fwd_pipe_kernel<3,4,2,4>: 107.1 MB fetched + 102.8 MB written
+    # fwd_pipe_kernel<3,4,2,4,false,2> (results streamed): 107.1 MB fetched + 102.9 MB written
     ("C3", "mfma_bf16x3_pipe", 8, 224): 209.9e6,
 }
 
