@@ -1171,7 +1171,8 @@ __global__ __launch_bounds__(kCT) void grad_gemm_kernel(GradArgs a) {
 // channel only take their share of Z: requesting the last row in place of theirs took the memory's
 // time.  Both together, whole backward-filter or step: N8 C64 224x224 R8 122 -> 107 us, R1 104 -> 90, N16
 // C64 112x112 R8 f16 step 107 -> 97, N5 C434 T3 78x146 R3 77.5 -> 76.7; with an odd number of chunks a
-// split, whose last is requested twice, N32 C256 56x56 R32 109.9 -> 110.4.
+// split, whose last is requested twice, N32 C256 56x56 R32 109.9 -> 110.4, and N16 C128 T256 55x55 R32 stride
+// 2's two operands 13.7 -> 16.4 us (six layers of stride 1 on odd planes take the same with either).
 constexpr int kLdS = 36;   // LDS row stride (floats) of the activation tile: 16-byte aligned rows
 
 // How rows move: as 16 bytes (kRowsVec: H*W a multiple of 4, operands on 16-byte boundaries), as
