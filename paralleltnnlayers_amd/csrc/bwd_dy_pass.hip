@@ -20,7 +20,8 @@
 // 248 registers with four waves and more; with two or three (64 and 96 channels), where a thread
 // also holds two pieces of Cc, 256 and six of them in scratch memory.
 // N32 T256 56x56 R32 (206 MB) in a training step, by kernel traces: 63 us, 3.3 TB/s of rows in 256-byte
-// pieces; 66.9 with plain stores of G3, 69.9 with the factor's loads in branches as well.
+// pieces; 66.9 with plain stores of G3, 69.9 with the factor's loads in branches as well.  With y's
+// signs from the forward pass (BITS; 3 MB instead of y's 103) 50.7 us.
 #include <algorithm>
 #include <cstdint>
 
@@ -42,13 +43,15 @@ constexpr int kFrag = 4 * 3 * 2 * 32;    // 16-byte fragments of a chunk of Cc: 
 
 struct DyPassArgs {
   const float *dy, *y, *FK, *Cc;
+  const unsigned short* bits;            // FwdArgs::save_mask of the forward; null: y
   float *G3, *partK, *partB;             // partB null: no bias gradient
   int T, R, HW, cpi, chunks;             // chunks per image and in all
   int lines;                             // G3's planes are whole cache lines
 };
 
 // KZ: (rank, octet) pairs of Cc a thread loads and splits (256 of them a chunk).
-template <int KZ>
+// BITS: y's signs from the forward pass, 16 channels of a pixel in 16 bits, instead of y.
+template <int KZ, bool BITS>
 __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5;
@@ -78,7 +81,8 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
 
   // ---- loads: row 4 j + lane / 16 of the wave's channels, four pixels a lane ----
   const int lrow = lane >> 4, lcol = 4 * (lane & 15);
-  float4 dv[8], yv[8], zv[KZ][2];
+  float4 dv[8], yv[BITS ? 1 : 8], zv[KZ][2];
+  uint2 bits[2];                     // BITS: the lane's four pixels, channels 4 j + lrow with even and with odd j
   // (clamped, not branched; values outside are dropped where they are used.  Cc's first: its
   // fragments are made before the rows are waited for)
   auto load_z = [&](int i) {
@@ -99,7 +103,14 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
   };
   auto load_row = [&](size_t at, int j) {
     dv[j] = *reinterpret_cast<const float4*>(a.dy + at + (size_t)(4 * j) * HW);
-    yv[j] = *reinterpret_cast<const float4*>(a.y + at + (size_t)(4 * j) * HW);
+    if constexpr (!BITS) yv[j] = *reinterpret_cast<const float4*>(a.y + at + (size_t)(4 * j) * HW);
+  };
+  auto load_bits = [&](int i) {
+    const int n = i / a.cpi;
+    const int p = (i - n * a.cpi) * kPix + lcol;
+    const unsigned short* m = a.bits + ((size_t)n * (T >> 5) + wave) * 2 * HW + (p < HW ? p : 0);
+    bits[0] = *reinterpret_cast<const uint2*>(m);
+    bits[1] = *reinterpret_cast<const uint2*>(m + HW);
   };
   auto deposit_z = [&](int i) {
 #pragma unroll
@@ -135,6 +146,7 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
   {                                  // (every workgroup has a chunk)
     load_z(i0);
     const size_t at = row_at(i0);
+    if constexpr (BITS) load_bits(i0);
 #pragma unroll
     for (int j = 0; j < 8; ++j) load_row(at, j);
   }
@@ -156,14 +168,25 @@ __global__ __launch_bounds__(512, 2) void dy_pass_kernel(DyPassArgs a) {
     const int inext = i + 1 < i1 ? i + 1 : i;
     const size_t next = row_at(inext);
     load_z(inext);
+    [[maybe_unused]] const uint2 held[2] = {bits[0], bits[1]};
+    if constexpr (BITS) load_bits(inext);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       float4 m = dv[j];
       // (a product, as dy * (y > 0): a non-finite dy at a clipped output stays visible)
-      m.x *= yv[j].x > 0.f ? 1.f : 0.f;
-      m.y *= yv[j].y > 0.f ? 1.f : 0.f;
-      m.z *= yv[j].z > 0.f ? 1.f : 0.f;
-      m.w *= yv[j].w > 0.f ? 1.f : 0.f;
+      if constexpr (BITS) {
+        // channel 4 j + lrow: bit 4 (j / 2) + lrow of its half's 16
+        const unsigned sh = 4 * (j >> 1) + lrow;
+        m.x *= (float)((held[j & 1].x >> sh) & 1u);
+        m.y *= (float)((held[j & 1].x >> (sh + 16)) & 1u);
+        m.z *= (float)((held[j & 1].y >> sh) & 1u);
+        m.w *= (float)((held[j & 1].y >> (sh + 16)) & 1u);
+      } else {
+        m.x *= yv[j].x > 0.f ? 1.f : 0.f;
+        m.y *= yv[j].y > 0.f ? 1.f : 0.f;
+        m.z *= yv[j].z > 0.f ? 1.f : 0.f;
+        m.w *= yv[j].w > 0.f ? 1.f : 0.f;
+      }
       m.x = in ? m.x : 0.f;
       m.y = in ? m.y : 0.f;
       m.z = in ? m.z : 0.f;
@@ -283,19 +306,20 @@ bool bwd_dy_pass_supported(int N, int T, int R, int HW) {
 }
 int bwd_dy_pass_sets(int N, int T, int HW) { return grid_of(N, T, HW); }
 
-hipError_t bwd_dy_pass_launch(const float* dy, const float* y, const float* FK, const float* Cc,
-                              float* G3, float* partK, float* partB, int N, int T, int R, int HW,
-                              hipStream_t st) {
+hipError_t bwd_dy_pass_launch(const float* dy, const float* y, const unsigned short* bits,
+                              const float* FK, const float* Cc, float* G3, float* partK, float* partB,
+                              int N, int T, int R, int HW, hipStream_t st) {
   if (!y) return hipErrorInvalidValue;
   DyPassArgs a{};
-  a.dy = dy; a.y = y; a.FK = FK; a.Cc = Cc; a.G3 = G3; a.partK = partK; a.partB = partB;
+  a.dy = dy; a.y = y; a.bits = bits; a.FK = FK; a.Cc = Cc; a.G3 = G3; a.partK = partK; a.partB = partB;
   a.T = T; a.R = R; a.HW = HW;
   a.lines = store_policy(G3, HW * sizeof(float), (size_t)N * R * HW * sizeof(float), ~(size_t)0) == kStoreThrough;
   a.cpi = (HW + kPix - 1) / kPix;
   a.chunks = N * a.cpi;
   const int waves = T / 32;
   const size_t lds = (size_t)waves * kTile * sizeof(float) + kFrag * 16;
-  auto k = waves >= 4 ? dy_pass_kernel<1> : dy_pass_kernel<2>;
+  auto k = bits ? (waves >= 4 ? dy_pass_kernel<1, true> : dy_pass_kernel<2, true>)
+                : (waves >= 4 ? dy_pass_kernel<1, false> : dy_pass_kernel<2, false>);
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

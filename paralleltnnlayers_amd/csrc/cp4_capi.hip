@@ -878,6 +878,20 @@ cp4_status cp4_conv2d_forward_bias_act(const cp4_shape* shape, const float* x,
                                        const float* FH, const float* FW,
                                        const float* bias, int activation, float* y,
                                        cp4_stream stream) {
+  int parts = 0;
+  return cp4::layer_forward_keeping(shape, x, FK, FC, FH, FW, bias, activation, y, cp4::Kept{}, &parts,
+                                    stream);
+}
+
+}  // extern "C"
+
+namespace cp4 {
+cp4_status layer_forward_keeping(const cp4_shape* shape, const float* x, const float* FK,
+                                 const float* FC, const float* FH, const float* FW,
+                                 const float* bias, int activation, float* y, const Kept& kept,
+                                 int* parts, cp4_stream stream) {
+  const int want = *parts;
+  *parts = 0;
   if (activation != CP4_ACT_NONE && activation != CP4_ACT_RELU)
     return fail(CP4_ERR_UNSUPPORTED, "activation must be CP4_ACT_NONE or CP4_ACT_RELU");
   if (!bias && activation == CP4_ACT_NONE)
@@ -901,6 +915,18 @@ cp4_status cp4_conv2d_forward_bias_act(const cp4_shape* shape, const float* x,
   if (c.variant < 0) return fail(CP4_ERR_UNSUPPORTED, "no kernel variant supports this shape");
   if (is_variant(c.variant, "mfma_bf16x3_pipe")) {
     FwdArgs e = with_tile(a, c);
+    if ((want & CP4_KEEP_MASK) && cp4::fwd_pipe_save_supported(e)) {
+      e.save_mask = kept.mask;
+      *parts = CP4_KEEP_MASK;
+      if ((want & CP4_KEEP_PLANES) && cp4::fwd_pipe_save_planes(e)) {
+        e.save_A = kept.A;
+        e.save_C = kept.Cc;
+        *parts |= CP4_KEEP_PLANES;
+      }
+      CP4_ARM(e);
+      CP4_HIP(cp4::fwd_pipe_save_launch(e, st));
+      return CP4_OK;
+    }
     if (cp4::fwd_pipe_epi_supported(e)) {
       CP4_ARM(e);
       CP4_HIP(cp4::fwd_pipe_epi_launch(e, st));
@@ -930,6 +956,10 @@ cp4_status cp4_conv2d_forward_bias_act(const cp4_shape* shape, const float* x,
   if (is_variant(c.variant, "mfma_bf16x3_few")) {
     FwdArgs e = with_tile(a, c);
     if (cp4::fwd_few_supported(e)) {
+      if (want & CP4_KEEP_MASK) {
+        e.save_mask = kept.mask;
+        *parts = CP4_KEEP_MASK;
+      }
       CP4_HIP(cp4::fwd_few_launch(e, st));          // the same
       return CP4_OK;
     }
@@ -941,6 +971,19 @@ cp4_status cp4_conv2d_forward_bias_act(const cp4_shape* shape, const float* x,
                                (size_t)shape->H * shape->W, st));
   return CP4_OK;
 }
+
+int layer_forward_keeps(const cp4_shape& s) {
+  FwdArgs a = forward_args(s, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+  const Choice c = choose(a);
+  if (c.variant < 0) return 0;
+  a = with_tile(a, c);
+  if (is_variant(c.variant, "mfma_bf16x3_pipe") && fwd_pipe_save_supported(a))
+    return CP4_KEEP_MASK | (fwd_pipe_save_planes(a) ? CP4_KEEP_PLANES : 0);
+  return is_variant(c.variant, "mfma_bf16x3_few") && fwd_few_supported(a) ? CP4_KEEP_MASK : 0;
+}
+}  // namespace cp4
+
+extern "C" {
 
 cp4_status cp4_conv2d_backward_data(const cp4_shape* shape, const float* dy,
                                     const float* FK, const float* FC,
@@ -1743,7 +1786,7 @@ cp4_status layer_backward_filter_masked(int variant, const cp4_shape* shape, con
                                         const float* act_y, const float* dy, const float* FK, const float* FC,
                                         const float* FH, const float* FW, float* dFK, float* dFC,
                                         float* dFH, float* dFW, float* dx, float* dbias,
-                                        float* bias_part, float* mask_ws, void* workspace,
+                                        float* bias_part, float* mask_ws, const Kept& kept, void* workspace,
                                         size_t workspace_bytes, cp4_stream stream) {
   if (!FK || !FC || !FH || !FW || !dFK || !dFC || !dFH || !dFW)
     return fail(CP4_ERR_NULL_POINTER, "a factor or gradient pointer is NULL");
@@ -1758,6 +1801,8 @@ cp4_status layer_backward_filter_masked(int variant, const cp4_shape* shape, con
   a.Y = s.Y; a.X = s.X; a.R = s.Rank;
   a.dx = dx;
   a.act_y = act_y; a.dbias = dbias; a.bias_part = bias_part; a.mask_ws = mask_ws;
+  a.act_bits = act_y ? kept.mask : nullptr;
+  a.kept_A = kept.A; a.kept_Cc = kept.Cc;
   if (variant == 3) CP4_HIP(bwd_filter_dense_tiles_launch(a, as_stream(stream)));
   else CP4_HIP(bwd_filter_mfma_masked_launch(a, as_stream(stream)));
   return CP4_OK;

@@ -66,24 +66,78 @@ BackwardPlan make_backward_plan(const cp4_shape& s, const cp4_geometry* g, int d
   return p;
 }
 
+using PlanKey = std::array<unsigned, 19>;
+PlanKey plan_key(const cp4_shape& s, const cp4_geometry* g, int dtype, int act, int wanted) {
+  const cp4_geometry none{0, 0, 0, 0, 0, 0};
+  const cp4_geometry& gg = g ? *g : none;
+  return {s.N, s.H, s.W, s.pad, s.T, s.C, s.Y, s.X, s.Rank, gg.stride_h, gg.stride_w,
+          gg.pad_top, gg.pad_left, gg.out_h, gg.out_w, (unsigned)dtype, (unsigned)act,
+          (unsigned)wanted, (unsigned)cp4::num_compute_units()};
+}
+template <class Plan, class Make>
+Plan remembered(std::mutex& mu, std::map<PlanKey, Plan>& plans, const PlanKey& key, Make make) {
+  std::lock_guard<std::mutex> lk(mu);
+  auto it = plans.find(key);
+  if (it != plans.end()) return it->second;
+  if (plans.size() > 4096) plans.clear();
+  return plans[key] = make();
+}
+
 // The plan of a call, remembered: planning asks the backward-filter kernels for theirs,
 // several microseconds of host time that every step of a small layer would wait for.  (It
 // depends on the device by its compute units.)
 BackwardPlan backward_plan(const cp4_shape& s, const cp4_geometry* g, int dtype, int act,
                            int wanted) {
-  using Key = std::array<unsigned, 19>;
   static std::mutex mu;
-  static std::map<Key, BackwardPlan> plans;
-  const cp4_geometry none{0, 0, 0, 0, 0, 0};
-  const cp4_geometry& gg = g ? *g : none;
-  const Key key{s.N, s.H, s.W, s.pad, s.T, s.C, s.Y, s.X, s.Rank, gg.stride_h, gg.stride_w,
-                gg.pad_top, gg.pad_left, gg.out_h, gg.out_w, (unsigned)dtype, (unsigned)act,
-                (unsigned)wanted, (unsigned)cp4::num_compute_units()};
-  std::lock_guard<std::mutex> lk(mu);
-  auto it = plans.find(key);
-  if (it != plans.end()) return it->second;
-  if (plans.size() > 4096) plans.clear();
-  return plans[key] = make_backward_plan(s, g, dtype, act, wanted);
+  static std::map<PlanKey, BackwardPlan> plans;
+  return remembered(mu, plans, plan_key(s, g, dtype, act, wanted),
+                    [&] { return make_backward_plan(s, g, dtype, act, wanted); });
+}
+
+// Where the parts of what a forward call leaves lie (byte offsets).
+struct KeepPlan {
+  int parts;
+  size_t A_at, Cc_at, total;
+};
+KeepPlan make_keep_plan(const cp4_shape& s, const cp4_geometry* g, int dtype, int act, int wanted) {
+  KeepPlan k{};
+  const bool filter = wanted & CP4_WANT_FACTORS, dx = wanted & CP4_WANT_DX;
+  if (g || dtype != CP4_DTYPE_F32 || act != CP4_ACT_RELU || !filter || s.N == 0) return k;
+  // (operands on 16-byte boundaries; a call whose are not may take another route and leave them)
+  const int variant = cp4::layer_filter_masks(s, nullptr, nullptr, nullptr, nullptr,
+                                              reinterpret_cast<const float*>(256), dx);
+  // (a first layer's step waits for the host up to some 64 MB of y, and memory for the signs is 4 us more
+  // of that: N2 and N4 C3 K64 224x224 R16, 26 and 51 MB, 62 and 61 us without, 68 and 66 with; N8 and N16
+  // 100 and 147 without, 75 and 130 with)
+  if (!variant || (variant == 3 && elements(s, s.T) < (size_t)16 << 20)) return k;
+  k.parts = cp4::layer_forward_keeps(s) & (variant == 1 ? CP4_KEEP_MASK | CP4_KEEP_PLANES : CP4_KEEP_MASK);
+  if (!k.parts) return k;
+  const size_t plane = (size_t)s.H * s.W;
+  k.total = align256((size_t)s.N * ((s.T + 31) / 32) * plane * 4);
+  if (k.parts & CP4_KEEP_PLANES) {
+    const size_t planes = align256((size_t)s.N * s.Rank * plane * 4);
+    k.A_at = k.total;
+    k.Cc_at = k.A_at + planes;
+    k.total = k.Cc_at + planes;
+  }
+  return k;
+}
+// (remembered as the backward plan is; what a call takes up is decided by its operands)
+KeepPlan keep_plan(const cp4_shape& s, const cp4_geometry* g, int dtype, int act, int wanted) {
+  static std::mutex mu;
+  static std::map<PlanKey, KeepPlan> plans;
+  return remembered(mu, plans, plan_key(s, g, dtype, act, wanted),
+                    [&] { return make_keep_plan(s, g, dtype, act, wanted); });
+}
+cp4::Kept kept_parts(const KeepPlan& k, int parts, const void* kept) {
+  unsigned char* p = static_cast<unsigned char*>(const_cast<void*>(kept));
+  cp4::Kept r{};
+  if (parts & CP4_KEEP_MASK) r.mask = reinterpret_cast<unsigned short*>(p);
+  if (parts & CP4_KEEP_PLANES) {
+    r.A = reinterpret_cast<float*>(p + k.A_at);
+    r.Cc = reinterpret_cast<float*>(p + k.Cc_at);
+  }
+  return r;
 }
 
 thread_local int g_route = 0;      // of this thread's last cp4_layer_backward
@@ -151,6 +205,34 @@ cp4_status cp4_layer_forward(const cp4_shape* shape, const cp4_geometry* g, int 
   return CP4_OK;
 }
 
+size_t cp4_layer_kept_bytes(const cp4_shape* shape, const cp4_geometry* g, int dtype, int activation,
+                            int wanted) {
+  if (check_layer(shape, g, dtype, activation) != CP4_OK || shape->N == 0) return 0;
+  return keep_plan(*shape, g, dtype, activation, wanted).total;
+}
+
+cp4_status cp4_layer_forward_keeping(const cp4_shape* shape, const cp4_geometry* g, int dtype,
+                                     const void* x, const float* FK, const float* FC,
+                                     const float* FH, const float* FW, const float* bias,
+                                     int activation, int wanted, void* y, void* kept,
+                                     size_t kept_bytes, int* parts, void* workspace,
+                                     size_t workspace_bytes, cp4_stream stream) {
+  if (!parts) return cp4::fail_with(CP4_ERR_NULL_POINTER, "parts is NULL");
+  *parts = 0;
+  CP4_TRY(check_layer(shape, g, dtype, activation));
+  if (kept && shape->N && !(reinterpret_cast<uintptr_t>(kept) & 255)) {
+    const KeepPlan k = keep_plan(*shape, g, dtype, activation, wanted);
+    if (k.parts && kept_bytes >= k.total) {
+      *parts = k.parts;
+      return cp4::layer_forward_keeping(shape, static_cast<const float*>(x), FK, FC, FH, FW, bias,
+                                        activation, static_cast<float*>(y),
+                                        kept_parts(k, k.parts, kept), parts, stream);
+    }
+  }
+  return cp4_layer_forward(shape, g, dtype, x, FK, FC, FH, FW, bias, activation, y, workspace,
+                           workspace_bytes, stream);
+}
+
 size_t cp4_layer_backward_workspace_bytes(const cp4_shape* shape, const cp4_geometry* g, int dtype,
                                           int activation, int wanted) {
   if (check_layer(shape, g, dtype, activation) != CP4_OK || shape->N == 0) return 0;
@@ -163,6 +245,16 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* g, int
                               void* dx, float* dFK, float* dFC, float* dFH, float* dFW,
                               float* dbias, void* workspace, size_t workspace_bytes,
                               cp4_stream stream) {
+  return cp4_layer_backward_kept(shape, g, dtype, x, y, dy, FK, FC, FH, FW, activation, dx, dFK, dFC,
+                                 dFH, dFW, dbias, nullptr, 0, 0, workspace, workspace_bytes, stream);
+}
+
+cp4_status cp4_layer_backward_kept(const cp4_shape* shape, const cp4_geometry* g, int dtype,
+                                   const void* x, const void* y, const void* dy, const float* FK,
+                                   const float* FC, const float* FH, const float* FW, int activation,
+                                   void* dx, float* dFK, float* dFC, float* dFH, float* dFW,
+                                   float* dbias, const void* kept, size_t kept_bytes, int parts_kept,
+                                   void* workspace, size_t workspace_bytes, cp4_stream stream) {
   g_route = g_mask_inside = 0;
   CP4_TRY(check_layer(shape, g, dtype, activation));
   const cp4_shape& s = *shape;
@@ -203,9 +295,17 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* g, int
     const int variant = cp4::layer_filter_masks(s, xf, yf, dyf, ws + p.pass_at, mask_ws, dx != nullptr);
     if (variant) {
       g_route = variant == 3 ? CP4_ROUTE_MASKED_TILES : CP4_ROUTE_DY_PASS | (dx ? CP4_ROUTE_DX_FROM_G1 : 0);
+      cp4::Kept left{};
+      if (kept && parts_kept && !(reinterpret_cast<uintptr_t>(kept) & 255)) {
+        const KeepPlan k = keep_plan(s, g, dtype, activation, wanted);
+        if ((k.parts & parts_kept) == parts_kept && kept_bytes >= k.total)
+          left = kept_parts(k, parts_kept, kept);
+        if (variant == 3) left.A = left.Cc = nullptr;
+        g_route |= (left.mask ? CP4_ROUTE_KEPT_MASK : 0) | (left.A ? CP4_ROUTE_KEPT_PLANES : 0);
+      }
       return cp4::layer_backward_filter_masked(variant, shape, xf, yf, dyf, FK, FC, FH, FW, dFK, dFC,
                                                dFH, dFW, static_cast<float*>(dx), dbias, parts, mask_ws,
-                                               ws + p.pass_at, p.pass_bytes, stream);
+                                               left, ws + p.pass_at, p.pass_bytes, stream);
     }
   }
   // or one whose contraction masks dy as it reads it and leaves it in memory for the others

@@ -66,7 +66,8 @@ struct FewPlan {
 // FS: filter size; NCH: 16-channel chunks of the input (1, 2 or 4); RING: chunk loads in
 // flight per lane, a multiple of NCH; OCC: waves per SIMD the register budget is set for.
 // BIAS: a branch on it per group cost layers without one 2 to 4 %.  STORE: a StorePolicy for y.
-template <int FS, int NCH, int RING, int OCC, int NW, bool BIAS, int STORE>
+// KEEP: the signs of the results leave with them (FwdArgs::save_mask).
+template <int FS, int NCH, int RING, int OCC, int NW, bool BIAS, int STORE, bool KEEP>
 __global__ __launch_bounds__(64 * NW, OCC) void fwd_few_kernel(FwdArgs a, FewPlan pl) {
   constexpr int kWaves = NW;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
@@ -385,6 +386,22 @@ __global__ __launch_bounds__(64 * NW, OCC) void fwd_few_kernel(FwdArgs a, FewPla
             acc1[4 * v4] += bv.x; acc1[4 * v4 + 1] += bv.y; acc1[4 * v4 + 2] += bv.z; acc1[4 * v4 + 3] += bv.w;
           }
         }
+        if constexpr (KEEP) {
+          // bit v of a pixel's 16: accumulator element v, channel 8*(v >> 2) + 4*hi + (v & 3) of the block
+          unsigned m0 = 0, m1 = 0;
+#pragma unroll
+          for (int v = 15; v >= 0; --v) {
+            m0 = m0 + m0 + (acc0[v] > 0.f);
+            m1 = m1 + m1 + (acc1[v] > 0.f);
+          }
+          unsigned short* mp = a.save_mask + (((size_t)n * nkb + kb) * 2 + hi) * HW + (size_t)h * W + w;
+          if ((W & 1) == 0) {                                    // (both pixels or neither)
+            if (in0) *reinterpret_cast<unsigned*>(mp) = m0 | (m1 << 16);
+          } else {
+            if (in0) mp[0] = (unsigned short)m0;
+            if (in1) mp[1] = (unsigned short)m1;
+          }
+        }
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const int kk = 32 * kb + 8 * (v >> 2) + (v & 3);       // + 4*hi is in the lane offset
@@ -526,11 +543,12 @@ hipError_t launch_as(const FwdArgs& a, const FewPlan& pl, hipStream_t st) {
   const size_t plane = (size_t)a.H * a.W * sizeof(float);
   const size_t from = a.bias || a.act ? kStreamBytesFewLayer : kStreamBytes;
   const int store = store_policy(a.y, plane, plane * a.N * a.Cout, from, from);
-#define CP4_FEW(BIAS_)                                                                        \
-  (store == kStoreStreamed  ? fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStoreStreamed>   \
-   : store == kStoreThrough ? fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStoreThrough>    \
-                            : fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStorePlain>)
-  auto k = a.bias ? CP4_FEW(true) : CP4_FEW(false);
+#define CP4_FEW(BIAS_, KEEP_)                                                                       \
+  (store == kStoreStreamed  ? fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStoreStreamed, KEEP_>  \
+   : store == kStoreThrough ? fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStoreThrough, KEEP_>   \
+                            : fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStorePlain, KEEP_>)
+  auto k = a.save_mask ? (a.bias ? CP4_FEW(true, true) : CP4_FEW(false, true))
+                       : (a.bias ? CP4_FEW(true, false) : CP4_FEW(false, false));
 #undef CP4_FEW
   const size_t lds = pl.lds_bytes + (a.bias ? (size_t)pl.nkb * 32 * sizeof(float) : 0);
   if (lds > 64 * 1024) {

@@ -228,6 +228,7 @@ struct LayerSpec {
   cp4_geometry geometry;
   bool has_geometry, has_bias;
   int dtype, activation;
+  int kept_parts;                               // what the forward pass left in the last saved tensor
   const cp4_geometry* g() const { return has_geometry ? &geometry : nullptr; }
 };
 
@@ -236,13 +237,25 @@ Tensor as_f32(const Tensor& t) {
   return t.contiguous().to(at::kFloat);
 }
 
-Tensor layer_forward(const LayerSpec& l, const Tensor& x, const Factors& f, const Tensor& bias) {
+// wanted: CP4_WANT_* of the backward pass that will follow (0: none); kept and parts: what the forward
+// pass leaves for it, the memory of which outlives the call as the saved tensors do.
+Tensor layer_forward(const LayerSpec& l, const Tensor& x, const Factors& f, const Tensor& bias,
+                     int wanted = 0, Tensor* kept = nullptr, int* parts = nullptr) {
   const cp4_shape& s = l.shape;
   const int64_t oh = l.has_geometry ? l.geometry.out_h : s.H, ow = l.has_geometry ? l.geometry.out_w : s.W;
   Tensor y = empty({s.N, s.T, oh, ow}, x.scalar_type(), x);
   const size_t need = l.dtype == CP4_DTYPE_F32
                           ? 0 : cp4_layer_forward_workspace_bytes(&s, l.g(), l.dtype);
   const Tensor ws = scratch(need, x);
+  if (const size_t room = wanted ? cp4_layer_kept_bytes(&s, l.g(), l.dtype, l.activation, wanted) : 0) {
+    *kept = scratch(room, x);
+    check(cp4_layer_forward_keeping(&s, l.g(), l.dtype, x.data_ptr(), f32(f.FK), f32(f.FC), f32(f.FH),
+                                    f32(f.FW), bias.defined() ? f32(bias) : nullptr, l.activation,
+                                    wanted, y.data_ptr(), kept->data_ptr(), room, parts, ptr(ws), need,
+                                    c10::hip::getCurrentHIPStream(x.device().index()).stream()));
+    if (!*parts) *kept = Tensor();
+    return y;
+  }
   check(cp4_layer_forward(&s, l.g(), l.dtype, x.data_ptr(), f32(f.FK), f32(f.FC), f32(f.FH),
                           f32(f.FW), bias.defined() ? f32(bias) : nullptr, l.activation,
                           y.data_ptr(), ptr(ws), need,
@@ -256,9 +269,15 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
                         const std::optional<Tensor>& bias, LayerSpec l) {
     const Factors f{as_f32(FK), as_f32(FC), as_f32(FH), as_f32(FW)};
     const Tensor b = bias ? as_f32(*bias) : Tensor();
-    Tensor y = layer_forward(l, x, f, b);
+    const bool factors = FK.requires_grad() || FC.requires_grad() || FH.requires_grad() || FW.requires_grad();
+    const int wanted = (x.requires_grad() ? CP4_WANT_DX : 0) | (factors ? CP4_WANT_FACTORS : 0) |
+                       (bias && bias->requires_grad() ? CP4_WANT_BIAS : 0);
+    Tensor kept;
+    Tensor y = layer_forward(l, x, f, b, factors ? wanted : 0, &kept, &l.kept_parts);
     const bool relu = l.activation == CP4_ACT_RELU;
-    ctx->save_for_backward({x, f.FK, f.FC, f.FH, f.FW, relu ? y : Tensor()});
+    torch::autograd::variable_list saved{x, f.FK, f.FC, f.FH, f.FW, relu ? y : Tensor()};
+    if (kept.defined()) saved.push_back(kept);
+    ctx->save_for_backward(std::move(saved));
     ctx->saved_data["spec"] = c10::IValue(std::string(reinterpret_cast<const char*>(&l), sizeof l));
     return y;
   }
@@ -294,11 +313,16 @@ struct LayerFunction : torch::autograd::Function<LayerFunction> {
         cp4_layer_backward_workspace_bytes(&l.shape, l.g(), l.dtype, l.activation, wanted);
     const Tensor ws = scratch(need, x);
     void* st = c10::hip::getCurrentHIPStream(x.device().index()).stream();
-    check(cp4_layer_backward(&l.shape, l.g(), l.dtype, x.data_ptr(), ptr(saved[5]), dy.data_ptr(),
+    // (what hooks on saved tensors give back in another form than bytes on this device is left alone)
+    const Tensor kept = saved.size() > 6 && saved[6].defined() && saved[6].device() == x.device() &&
+                                saved[6].scalar_type() == at::kByte && saved[6].is_contiguous()
+                            ? saved[6] : Tensor();
+    check(cp4_layer_backward_kept(&l.shape, l.g(), l.dtype, x.data_ptr(), ptr(saved[5]), dy.data_ptr(),
                              f32(FK), f32(FC), f32(FH), f32(FW), l.activation, ptr(dx),
                              static_cast<float*>(ptr(grads[0])), static_cast<float*>(ptr(grads[1])),
                              static_cast<float*>(ptr(grads[2])), static_cast<float*>(ptr(grads[3])),
-                             static_cast<float*>(ptr(dbias)), ptr(ws), need, st));
+                             static_cast<float*>(ptr(dbias)), ptr(kept),
+                             kept.defined() ? (size_t)kept.numel() : 0, l.kept_parts, ptr(ws), need, st));
     if (g_check_backward.load(std::memory_order_relaxed)) check(cp4_device_status(st, nullptr));
     if (bias_graph) {
       const Tensor d = saved[5].defined() ? grad[0] * (saved[5] > 0) : grad[0];
