@@ -22,8 +22,9 @@
 //   3. dense_fold_kernel: the chain rule, a workgroup per 32 ranks and gradient.
 // No atomics: bit-reproducible.  Plain fp32 multiply-adds, or exact fp32 products from bf16
 // parts on the matrix cores.
-#include "cp4_internal.h"
 #include <atomic>
+
+#include "dense_tiles.h"
 #include "split_bf16.h"
 
 namespace cp4 {
@@ -56,25 +57,6 @@ struct DensePlan {
   int grid;
   size_t lds_bytes;
 };
-
-// A workgroup's tiles.  Workgroups go to the chip's eight dies in turn (blockIdx & 7), each die
-// with an L2 of its own: a die takes one contiguous eighth of the tiles and its workgroups
-// stride through it, so that tiles which share halo rows and columns run on the same die at
-// about the same time (tile t, t + 1 on neighbouring dies: every halo cell is fetched once
-// per die that needs it, 1.7 - 1.9 times the input in all).
-struct TileRange {
-  int first, end, step;
-};
-__device__ __forceinline__ TileRange tiles_of_workgroup(int ntiles) {
-  const int dies = gridDim.x < 8 ? (int)gridDim.x : 8;            // (fewer than eight workgroups: a range each)
-  const int die = blockIdx.x % dies, slot = blockIdx.x / dies;
-  const int on_die = ((int)gridDim.x - die + dies - 1) / dies;     // workgroups on this die
-  TileRange r;
-  r.first = (int)((long)ntiles * die / dies) + slot;
-  r.end = (int)((long)ntiles * (die + 1) / dies);
-  r.step = on_die;
-  return r;
-}
 
 template <int FS, int KB>
 __global__ __launch_bounds__(kThreads) void dense_tiles_kernel(BwdFilterArgs a, DensePlan pl,
@@ -1284,6 +1266,20 @@ bool use_mfma(const cp4_shape& s) {
 
 }  // namespace
 
+// Partial sets of the kernel that takes dy straight from memory (bwd_filter_dense_direct.hip), 0 where
+// it does not run: it is the faster one wherever it takes the shape (rows of a multiple of four, operands
+// on 16-byte boundaries, up to 15 blocks of 16 x 16 entries of dK, 80 columns of them).
+static int direct_sets(const cp4_shape& s, bool aligned16, bool masked) {
+  if (g_forced_tile_kernel.load() >= 0 || !use_mfma(s)) return 0;
+  const int sets = dense_direct_sets(s, aligned16);
+  // (the workspace has room for the partial sets of the other's plans)
+  MfmaPlan plain;
+  int room = 0;
+  for (const bool al : {false, true})
+    if (mfma_plan(s, al, &plain)) room = std::max(room, plain.grid);
+  return sets < room ? sets : room;
+}
+
 bool bwd_filter_dense_tiles_supported(const cp4_shape& s) { return valu_ok(s) || mfma_ok(s); }
 
 bool bwd_filter_dense_tiles_masks(const cp4_shape& s) {
@@ -1364,7 +1360,11 @@ hipError_t bwd_filter_dense_tiles_launch(const BwdFilterArgs& a, hipStream_t st)
   const bool aligned16 = ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.dy) |
                            reinterpret_cast<uintptr_t>(a.act_y)) & 15) == 0;
   const bool masked = a.act_y || a.dbias;
-  if (masked || use_mfma(s)) {
+  const int direct = direct_sets(s, aligned16, masked);
+  if (direct) {
+    sets = direct;
+    e = dense_direct_launch(a, partial, sets, st);
+  } else if (masked || use_mfma(s)) {
     MfmaPlan pl;
     if (!mfma_plan(s, aligned16, &pl, masked) && !mfma_plan(s, false, &pl, masked))
       return hipErrorInvalidValue;
