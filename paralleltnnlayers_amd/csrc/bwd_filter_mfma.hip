@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "cp4_internal.h"
+#include "reduce_sets.h"
 #ifdef CP4_DEBUG_PHASES
 #include "cp4_debug.h"
 #endif
@@ -1464,54 +1465,15 @@ __global__ __launch_bounds__(256) void tap_grad_kernel(const float* __restrict__
   }
 }
 
-// ---- 4. out[i] = sum_s partial[s][i], up to five segments in one launch ------
-struct ReduceArgs {
-  const float* part[5];
-  float* out[5];
-  int count[5], S[5];
-};
-// A workgroup owns 64 consecutive outputs; its waves (sixteen, four below 192 sets) each
-// sum a part of the S partials in index order (eight loads in flight, added as a tree), then the
-// parts are added in wave order: the result does not depend on timing.  Bound by the latency of
-// those loads: N16 C128 T256 55x55 R32 stride 2, 224 and 64 sets, 4.6 us with four waves, 3.9 with sixteen;
+// ---- 4. out[i] = sum_s partial[s][i], up to five segments in one launch (reduce_sets.h) ------
+// Sixteen waves a workgroup, four below 192 sets.  Bound by the latency of their loads: N16 C128 T256
+// 55x55 R32 stride 2, 224 and 64 sets, 4.6 us with four waves, 3.9 with sixteen;
 // N64 C256 T256 14x14 R64, 64 sets, 3.95 and 4.7; N16 C400 T400 45x45 R16, 128 sets, 4.0 and 4.4; N32 C512
 // T512 28x28 R32 in 16 bits, 128 sets, 4.1 and 7.0; N32 C256 56x56 R32, 256 sets, 7.3 and 6.5.
 constexpr int kReduceWaves = 16;
 __global__ __launch_bounds__(64 * kReduceWaves) void reduce_sets_kernel(ReduceArgs a) {
   __shared__ float part[kReduceWaves][64];
-  const int seg = blockIdx.y, waves = blockDim.x >> 6;
-  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-  const int i = blockIdx.x * 64 + lane;
-  const int count = a.count[seg], S = a.S[seg];
-  if ((int)blockIdx.x * 64 >= count) return;               // whole workgroup
-  const int k0 = (int)((long)S * q / waves), k1 = (int)((long)S * (q + 1) / waves);
-  float s = 0.f;
-  if (i < count) {
-    const float* p = a.part[seg] + i;
-    const size_t stride = count;
-    int k = k0;
-    for (; k + 8 <= k1; k += 8) {
-      float v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = p[(size_t)(k + u) * stride];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] += v[u + 4];
-      s += (v[0] + v[2]) + (v[1] + v[3]);
-    }
-    // (the rest together too, the last set in place of those past it)
-    float v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = p[(size_t)(k + u < k1 ? k + u : k1 - 1 > 0 ? k1 - 1 : 0) * stride];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) s += k + u < k1 ? v[u] : 0.f;
-  }
-  part[q][lane] = s;
-  __syncthreads();
-  if (q == 0 && i < count) {
-    float t = part[0][lane];
-    for (int w = 1; w < waves; ++w) t += part[w][lane];
-    a.out[seg][i] = t;
-  }
+  reduce_sets_block(a, blockIdx.y, blockIdx.x, blockDim.x >> 6, part);
 }
 
 struct Plan {
@@ -1643,13 +1605,19 @@ hipError_t contract_slices(const float* src, const float* F, float* Z, float* sl
 }
 #endif
 
-hipError_t launch_reduce(const float* const (&parts)[5], float* const (&outs)[5],
-                         const int (&counts)[5], const int (&Ss)[5], hipStream_t st) {
+ReduceArgs reduce_args(const float* const (&parts)[5], float* const (&outs)[5],
+                       const int (&counts)[5], const int (&Ss)[5]) {
   ReduceArgs r{};
-  int most = 0, sets = 0;
   for (int i = 0; i < 5; ++i) {
-    if (counts[i] > 0) sets = std::max(sets, Ss[i]);
     r.part[i] = parts[i]; r.out[i] = outs[i]; r.count[i] = counts[i]; r.S[i] = Ss[i];
+  }
+  return r;
+}
+hipError_t launch_reduce(const ReduceArgs& r, hipStream_t st) {
+  int most = 0, sets = 0;
+  const int (&counts)[5] = r.count;
+  for (int i = 0; i < 5; ++i) {
+    if (counts[i] > 0) sets = std::max(sets, r.S[i]);
     if (counts[i] > most) most = counts[i];
   }
   reduce_sets_kernel<<<dim3((most + 63) / 64, counts[4] ? 5 : 4), sets >= 192 ? 64 * kReduceWaves : 256, 0,
@@ -1832,25 +1800,22 @@ hipError_t bwd_filter_mfma_launch(const BwdFilterArgs& a, hipStream_t st) {
 #endif
   if (e != hipSuccess) return e;
 
-  // (after the GEMMs, whose operands its stores would push out of the cache)
-  if (a.dx) {
-#ifdef CP4_BWF_HALF
-    constexpr int kDtype = CP4_DTYPE_F16;
-#elif defined(CP4_BWF_IO16)
-    constexpr int kDtype = CP4_DTYPE_BF16;
-#else
-    constexpr int kDtype = CP4_DTYPE_F32;
-#endif
-    e = rank_expand_launch(a.FC, G1, a.dx, kDtype, N, a.C, HW, R, st);
-    if (e != hipSuccess) return e;
-  }
-
   const float* parts[5] = {pK, pC, pH, pW, a.bias_part};
   float* outs[5] = {a.dFK, a.dFC, a.taps2d ? a.dtaps2d : a.dFH, a.dFW, a.dbias};
   const int counts[5] = {a.T * R, a.C * R, a.taps2d ? a.Y * a.X * R : a.Y * R,
                          a.taps2d ? 0 : a.X * R, a.dbias ? a.T : 0};
   const int Ss[5] = {p.S, p.S, a.taps2d ? N : p.St, p.St, p.S};
-  return launch_reduce(parts, outs, counts, Ss, st);
+  const ReduceArgs sums = reduce_args(parts, outs, counts, Ss);
+  if (!a.dx) return launch_reduce(sums, st);
+#ifdef CP4_BWF_HALF
+  constexpr int kDtype = CP4_DTYPE_F16;
+#elif defined(CP4_BWF_IO16)
+  constexpr int kDtype = CP4_DTYPE_BF16;
+#else
+  constexpr int kDtype = CP4_DTYPE_F32;
+#endif
+  // (after the GEMMs, whose operands its stores would push out of the cache)
+  return rank_expand_reduce_launch(a.FC, G1, a.dx, kDtype, N, a.C, HW, R, sums, st);
 }
 
 #ifndef CP4_BWF_IO16
@@ -2217,15 +2182,13 @@ hipError_t bwd_filter_mfma_masked_launch(const BwdFilterArgs& a, hipStream_t st)
 #undef CP4_TAPS
   e = grad_one(a.x, G1, pC, a.C, N, R, p, HW, ws, st);
   if (e != hipSuccess) return e;
-  if (a.dx) {
-    e = rank_expand_launch(a.FC, G1, a.dx, CP4_DTYPE_F32, N, a.C, HW, R, st);
-    if (e != hipSuccess) return e;
-  }
   const float* parts[5] = {pK, pC, pH, pW, pB};
   float* outs[5] = {a.dFK, a.dFC, a.dFH, a.dFW, a.dbias};
   const int counts[5] = {a.T * R, a.C * R, a.Y * R, a.X * R, a.dbias ? a.T : 0};
   const int Ss[5] = {sets, p.S, p.St, p.St, sets};
-  return launch_reduce(parts, outs, counts, Ss, st);
+  const ReduceArgs sums = reduce_args(parts, outs, counts, Ss);
+  return a.dx ? rank_expand_reduce_launch(a.FC, G1, a.dx, CP4_DTYPE_F32, N, a.C, HW, R, sums, st)
+              : launch_reduce(sums, st);
 }
 
 namespace {
@@ -2361,15 +2324,13 @@ hipError_t bwd_filter_mfma_strided_launch(const BwdFilterArgs& a, const Geometry
     e = grad_one(a.x, G1, pC, a.C, N, R, l.pf, HW, ws, st);
   }
   if (e != hipSuccess) return e;
-  if (a.dx) {
-    e = rank_expand_launch(a.FC, G1, a.dx, CP4_DTYPE_F32, N, a.C, HW, R, st);
-    if (e != hipSuccess) return e;
-  }
   const float* parts[5] = {pK, pC, pH, pW, a.bias_part};
   float* outs[5] = {a.dFK, a.dFC, a.dFH, a.dFW, a.dbias};
   const int counts[5] = {a.T * R, a.C * R, a.Y * R, a.X * R, a.dbias ? a.T : 0};
   const int Ss[5] = {l.ps.S, l.pf.S, N, N, l.ps.S};
-  return launch_reduce(parts, outs, counts, Ss, st);
+  const ReduceArgs sums = reduce_args(parts, outs, counts, Ss);
+  return a.dx ? rank_expand_reduce_launch(a.FC, G1, a.dx, CP4_DTYPE_F32, N, a.C, HW, R, sums, st)
+              : launch_reduce(sums, st);
 }
 #endif  // !CP4_BWF_IO16
 

@@ -227,10 +227,6 @@ hipError_t act_grad_launch(const void* y, const void* dy, void* out, int dtype, 
 hipError_t convert_launch(const void* src, int src_dtype, void* dst, int dst_dtype, size_t n,
                           hipStream_t);
 
-// dst[n,c,p] = sum_r F[c,r] Z[n,r,p] (ranks up to 64), dst of a cp4_dtype.
-hipError_t rank_expand_launch(const float* F, const float* Z, void* dst, int dtype, int N, int C,
-                              int HW, int R, hipStream_t);
-
 // Backward-filter (factor gradients).
 struct BwdFilterArgs {
   const float *x, *dy, *FK, *FC, *FH, *FW;

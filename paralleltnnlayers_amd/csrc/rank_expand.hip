@@ -22,6 +22,7 @@
 #include <cstdint>
 
 #include "cp4_internal.h"
+#include "reduce_sets.h"
 #include "split_bf16.h"
 #include "store_policy.h"
 
@@ -40,7 +41,14 @@ struct ExpandArgs {
   int cblocks;                 // blocks of 32 channels a wave takes
   int slices;                  // waves a block of pixels is shared by
   long pixels, items;          // N * HW; blocks of pixels * slices
+  int rblocks;                 // workgroups in front that add partial sets up (a multiple of eight)
 };
+
+int reduce_blocks(const ReduceArgs& r) {
+  int n = 0;
+  for (int i = 0; i < 5; ++i) n += (r.count[i] + 63) / 64;
+  return n;
+}
 
 struct ToF32 {
   using raw = float;
@@ -64,7 +72,23 @@ struct ToF16 {
 // (planes start at any address then, and a wider access off its own boundary is the slower:
 // N16 C128 55x55 R32 28 us against 10.7).
 template <class Out, int KC, int PX, bool VEC, int STORE>
-__global__ __launch_bounds__(kThreads, 2) void rank_expand_kernel(ExpandArgs a) {
+__global__ __launch_bounds__(kThreads, 2) void rank_expand_kernel(ExpandArgs a, ReduceArgs sums) {
+  // The factor gradients' partial sets, which the GEMM before left: in a launch of their own they waited for
+  // loads while nothing else ran (us, expansion + sums, and both together: N32 C256 56x56 R32 26.5 + 6.8,
+  // 28.7; N16 C128 T256 55x55 R32 stride 2 12.0 + 4.0, 13.1; N32 C128 28x28 R16 bf16 4.2 + 4.2, 4.5).
+  __shared__ float part[kThreads / 64][64];
+  if ((int)blockIdx.x < a.rblocks) {
+    int block = blockIdx.x;
+    for (int seg = 0; seg < 5; ++seg) {
+      const int n = (sums.count[seg] + 63) >> 6;
+      if (block < n) {
+        reduce_sets_block(sums, seg, block, kThreads / 64, part);
+        return;
+      }
+      block -= n;
+    }
+    return;
+  }
   using raw = typename Out::raw;
   typedef float ZV __attribute__((ext_vector_type(PX)));
   typedef raw OV __attribute__((ext_vector_type(PX)));
@@ -72,8 +96,9 @@ __global__ __launch_bounds__(kThreads, 2) void rank_expand_kernel(ExpandArgs a) 
   constexpr int NP = VEC ? 1 : PX;                           // accesses a row takes
   const int lane = threadIdx.x & 63, l32 = lane & 31, hi = lane >> 5;
   // workgroups of a die: consecutive ones
-  const unsigned die = blockIdx.x & 7, per = gridDim.x >> 3, rest = gridDim.x & 7;
-  const unsigned wg = die * per + (die < rest ? die : rest) + (blockIdx.x >> 3);
+  const unsigned bid = blockIdx.x - a.rblocks, grid = gridDim.x - a.rblocks;
+  const unsigned die = bid & 7, per = grid >> 3, rest = grid & 7;
+  const unsigned wg = die * per + (die < rest ? die : rest) + (bid >> 3);
   const long item = (long)wg * (kThreads / 64) + (threadIdx.x >> 6);
   if (item >= a.items) return;
   const int slice = (int)(item % a.slices);
@@ -205,7 +230,7 @@ __global__ __launch_bounds__(kThreads, 2) void rank_expand_kernel(ExpandArgs a) 
 }
 
 template <class Out>
-hipError_t launch(ExpandArgs a, hipStream_t st) {
+hipError_t launch(ExpandArgs a, const ReduceArgs& sums, hipStream_t st) {
   // four pixels a lane while the parts of its ranks leave room for four accumulators
   const int px = a.R <= 32 ? 4 : 2;
   const long blocks = (a.pixels + 32 * px - 1) / (32 * px);
@@ -230,7 +255,7 @@ hipError_t launch(ExpandArgs a, hipStream_t st) {
              : store == kStoreStreamed ? rank_expand_kernel<Out, KC_, PX_, true, wide ? kStoreStreamed : kStorePlain> \
              : store == kStoreThrough ? rank_expand_kernel<Out, KC_, PX_, true, wide ? kStoreThrough : kStorePlain>   \
                                       : rank_expand_kernel<Out, KC_, PX_, true, kStorePlain>;              \
-    k<<<grid, kThreads, 0, st>>>(a);                                                     \
+    k<<<a.rblocks + grid, kThreads, 0, st>>>(a, sums);                                                   \
   }
   if (a.R <= 16) CP4_EXPAND(1, 4)
   else if (a.R <= 32) CP4_EXPAND(2, 4)
@@ -242,16 +267,17 @@ hipError_t launch(ExpandArgs a, hipStream_t st) {
 
 }  // namespace
 
-hipError_t rank_expand_launch(const float* F, const float* Z, void* dst, int dtype, int N, int C,
-                              int HW, int R, hipStream_t st) {
+hipError_t rank_expand_reduce_launch(const float* F, const float* Z, void* dst, int dtype, int N, int C,
+                                     int HW, int R, const ReduceArgs& sums, hipStream_t st) {
   if (R > 64) return hipErrorInvalidValue;         // (four chunks of ranks)
   ExpandArgs a{};
   a.F = F; a.Z = Z; a.dst = dst;
   a.C = C; a.R = R; a.HW = HW;
   a.pixels = (long)N * HW;
-  if (dtype == CP4_DTYPE_BF16) return launch<ToBF16>(a, st);
-  if (dtype == CP4_DTYPE_F16) return launch<ToF16>(a, st);
-  return launch<ToF32>(a, st);
+  a.rblocks = (reduce_blocks(sums) + 7) / 8 * 8;
+  if (dtype == CP4_DTYPE_BF16) return launch<ToBF16>(a, sums, st);
+  if (dtype == CP4_DTYPE_F16) return launch<ToF16>(a, sums, st);
+  return launch<ToF32>(a, sums, st);
 }
 
 }  // namespace cp4
