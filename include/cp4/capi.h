@@ -493,7 +493,8 @@ cp4_status cp4_layer_backward_kept(const cp4_shape* shape, const cp4_geometry* g
 enum {
   CP4_ROUTE_MASKED_TILES = 1, /* mask and bias gradient inside the dense-gradient tile kernel */
   CP4_ROUTE_DY_PASS = 2,      /* one pass over dy for mask, bias gradient, G3 and dFK */
-  CP4_ROUTE_DX_FROM_G1 = 4,   /* the input gradient from the factor gradients' G1 plane */
+  CP4_ROUTE_DX_FROM_G1 = 4,   /* the input gradient from the factor gradients' G1 plane (not where it is
+                               * formed for that alone: cp4_layer_last_backward_dx_beside) */
   CP4_ROUTE_KEPT_MASK = 8,    /* the signs of y that the forward call left */
   CP4_ROUTE_KEPT_PLANES = 16  /* its rank planes */
 };
@@ -501,6 +502,8 @@ int cp4_layer_last_backward_route(void);
 /* 1 if its mask and bias gradient ran inside the contraction and the gradient GEMM of the factor
  * gradients' passes on their own, without a pass of theirs; else 0. */
 int cp4_layer_last_backward_mask_inside(void);
+/* 1 if its input gradient came beside the factor gradients, without a pass over dy of its own; else 0. */
+int cp4_layer_last_backward_dx_beside(void);
 
 /* ---- 3-factor CP sibling op ------------------------------------------------
  * Stands where the reference registers its TensorFlow op Conv2dCpFusedNchw

@@ -22,9 +22,11 @@
 //      floating-point atomics anywhere).
 #include <algorithm>
 #include <cstdint>
+#include <cstring>
 #include <type_traits>
 
 #include "cp4_internal.h"
+#include "reduce_sets.h"
 #include "split_bf16.h"
 #include "store_policy.h"
 
@@ -330,6 +332,7 @@ struct FusedArgs {
   float *part0, *part1;         // [S][D][R]
   float *partH, *partW;         // [S * TG][FS][R]
   float* partB;                 // [S][D0] sums of dy's rows, the layer's bias gradient; may be null
+  float* G1;                    // [N][R][HW]: the adjoint taps' results, for the input gradient; may be null
   int D0, D1;
   int N, R, H, W, P, HW;
   int TG;                     // channel groups of dFK that share the tap gradients (1 or 2)
@@ -567,6 +570,11 @@ __global__ __launch_bounds__(512) void grad_fused_kernel(FusedArgs a) {
         const float v = j < k ? call[j] : call[j + 2 * Q];
         out[j] = (qb + j < q1) ? v : 0.f;
       }
+      if (which && cg == 0 && a.G1 && r < R) {         // (strips end on multiples of four pixels)
+        float* g = a.G1 + ((size_t)n * R + r) * HW + qb;
+        *reinterpret_cast<float4*>(g) = make_float4(out[0], out[1], out[2], out[3]);
+        if (qb + 4 < q1) *reinterpret_cast<float4*>(g + 4) = make_float4(out[4], out[5], out[6], out[7]);
+      }
       u32x4 ph, pm, pl;
       split8(out, ph, pm, pl);
       dst[0] = ph;
@@ -680,39 +688,11 @@ __global__ __launch_bounds__(512) void grad_fused_kernel(FusedArgs a) {
   }
 }
 
-// ---- 3. out[i] = sum_s partial[s][i], up to five segments in one launch -------------------
-struct ReduceFusedArgs {
-  const float* part[5];
-  float* out[5];
-  int count[5], S[5];
-};
-// A workgroup owns 64 consecutive outputs; its four waves each sum a quarter of the
-// S partials in index order, then the quarter sums are added in wave order.
-__global__ __launch_bounds__(256) void reduce_fused_kernel(ReduceFusedArgs a) {
-  __shared__ float quarter[4][64];
-  const int seg = blockIdx.y;
-  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-  const int i = blockIdx.x * 64 + lane;
-  const int count = a.count[seg], S = a.S[seg];
-  if ((int)blockIdx.x * 64 >= count) return;           // whole workgroup
-  const int k0 = (int)((long)S * q / 4), k1 = (int)((long)S * (q + 1) / 4);
-  float s = 0.f;
-  if (i < count) {
-    const float* p = a.part[seg] + i;
-    const size_t stride = count;
-    // sixteen loads in flight (one round trip for up to 64 partial sets), summed in index order
-    for (int k = k0; k < k1; k += 16) {
-      float v[16];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) v[u] = k + u < k1 ? p[(size_t)(k + u) * stride] : 0.f;
-#pragma unroll
-      for (int u = 0; u < 16; ++u) s += v[u];
-    }
-  }
-  quarter[q][lane] = s;
-  __syncthreads();
-  if (q == 0 && i < count)
-    a.out[seg][i] = ((quarter[0][lane] + quarter[1][lane]) + quarter[2][lane]) + quarter[3][lane];
+// ---- 3. out[i] = sum_s partial[s][i], up to five segments in one launch (reduce_sets.h) -----
+// (four waves, as beside dx: the same sums with dx and without)
+__global__ __launch_bounds__(256) void reduce_fused_kernel(ReduceArgs a) {
+  __shared__ float part[4][64];
+  reduce_sets_block(a, blockIdx.y, blockIdx.x, 4, part);
 }
 
 // ---- host side -----------------------------------------------------------------------
@@ -741,7 +721,22 @@ int channel_splits(long items, int C, int T, bool masked) {
   return ks;
 }
 
+FusedPlan make_fused_plan_uncached(const cp4_shape& s);
+// The plan of the last shape asked for, per thread: a call asks several times (whether the variant takes
+// the shape, for its workspace, then with what), and the search goes over every strip height.
 FusedPlan make_fused_plan(const cp4_shape& s) {
+  static thread_local cp4_shape last_shape{};
+  static thread_local FusedPlan last_plan{};
+  static thread_local int last_cus = 0;
+  const int cus = num_compute_units();
+  if (last_cus != cus || memcmp(&last_shape, &s, sizeof(s))) {
+    last_plan = make_fused_plan_uncached(s);
+    last_shape = s;
+    last_cus = cus;
+  }
+  return last_plan;
+}
+FusedPlan make_fused_plan_uncached(const cp4_shape& s) {
   FusedPlan p{};
   const int N = s.N, C = s.C, T = s.T, H = s.H, W = s.W, FS = s.Y, R = s.Rank;
   const int HW = H * W;
@@ -863,7 +858,7 @@ hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
   if (!p.ok) return hipErrorInvalidValue;
   const int HW = a.H * a.W, R = a.R, N = a.N, FS = a.Y;
   float* ws = static_cast<float*>(a.workspace);
-  float *A = ws, *G3 = ws + p.plane, *part = ws + 2 * p.plane;
+  float *A = ws, *G3 = ws + p.plane, *G1 = a.g1_ws, *part = ws + 2 * p.plane;
   float* pK = part;
   float* pC = pK + (size_t)p.S * a.T * R;
   float* pH = pC + (size_t)p.S * a.C * R;
@@ -910,6 +905,7 @@ hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
   g.act1 = a.x; g.Zsrc1 = G3; g.part1 = pC; g.D1 = a.C;
   g.FH = a.FH; g.FW = a.FW; g.partH = pH; g.partW = pW;
   g.partB = a.dbias ? a.bias_part : nullptr;
+  g.G1 = a.dx ? G1 : nullptr;
   g.N = N; g.R = R; g.H = a.H; g.W = a.W; g.P = a.pad; g.HW = HW;
   g.TG = p.TG; g.TH = p.TH; g.NS = p.NS; g.items = p.items; g.S = p.S; g.MT = p.MT;
   g.Wp = p.Wp; g.PSt = p.PSt; g.KSmax = p.KSmax;
@@ -934,7 +930,7 @@ hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
 #undef CP4_FUSED_FS
 #undef CP4_FUSED
 
-  ReduceFusedArgs r{};
+  ReduceArgs r{};
   const float* parts[5] = {pK, pC, pH, pW, a.bias_part};
   float* outs[5] = {a.dFK, a.dFC, a.dFH, a.dFW, a.dbias};
   const int counts[5] = {a.T * R, a.C * R, FS * R, FS * R, a.dbias ? a.T : 0};
@@ -944,6 +940,10 @@ hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
     r.part[i] = parts[i]; r.out[i] = outs[i]; r.count[i] = counts[i]; r.S[i] = Ss[i];
     if (counts[i] > maxc) maxc = counts[i];
   }
+  // dx = FC G1 beside the sums (N16 C64 32x32 R16: the pass over dy of its own took 7.5 us, the sums 3.9;
+  // together 4.1; the layer backwards of nine layers of C and T 16-512, R 8-64, 1x1 and 3x3, 14x14 to
+  // 56x56 1.12 to 1.37 times as fast)
+  if (a.dx) return rank_expand_reduce_launch(a.FC, G1, a.dx, CP4_DTYPE_F32, N, a.C, HW, R, r, st);
   reduce_fused_kernel<<<dim3((maxc + 63) / 64, a.dbias ? 5 : 4), 256, 0, st>>>(r);
   return hipGetLastError();
 }

@@ -743,7 +743,22 @@ FilterPadLayout filter_pad_layout(const cp4_shape& s, const cp4_shape& t) {
 }
 
 // One workspace size serves every backward-filter variant.
+size_t filter_workspace_uncached(const cp4_shape& s);
+// The size of the last shape asked for, per thread: every call checks its workspace against it, and every
+// variant plans for it.  (It depends on the device by its compute units.)
 size_t filter_workspace(const cp4_shape& s) {
+  static thread_local cp4_shape last{};
+  static thread_local int last_cus = 0;
+  static thread_local size_t bytes = 0;
+  const int cus = cp4::num_compute_units();
+  if (cus != last_cus || memcmp(&last, &s, sizeof(s))) {
+    bytes = filter_workspace_uncached(s);
+    last = s;
+    last_cus = cus;
+  }
+  return bytes;
+}
+size_t filter_workspace_uncached(const cp4_shape& s) {
   if (filter_pad_route(s)) {
     const cp4_shape t = filter_padded_shape(s);
     const size_t general = cp4::bwd_filter_workspace_bytes(s);
@@ -1158,6 +1173,7 @@ void set_mask(cp4::BwdFilterArgs& a, const cp4::LayerMask& m) {
 
 // (dx not null: the input gradient as well where the matrix-core variant runs on the layer as
 // it is, *dx_done)
+thread_local int g_dx_variant = 0;      // of this thread's last call that brought dx along
 cp4_status backward_filter_f32(const cp4_shape* shape, const float* x, const float* dy,
                                const float* FK, const float* FC, const float* FH, const float* FW,
                                float* dFK, float* dFC, float* dFH, float* dFW, void* workspace,
@@ -1266,9 +1282,14 @@ cp4_status backward_filter_f32(const cp4_shape* shape, const float* x, const flo
     }
     return CP4_OK;
   }
-  if (variant == 1 && dx && s.Y == s.X && 2 * s.pad + 1 == s.Y) {
+  // (the three-launch variant forms G1 for dx only: where the workspace has room for it behind its own)
+  const size_t own = align256(filter_workspace(s)), g1 = (size_t)s.N * s.Rank * s.H * s.W * sizeof(float);
+  if ((variant == 1 || (variant == 2 && workspace_bytes >= own + g1)) && dx && s.Y == s.X &&
+      2 * s.pad + 1 == s.Y) {
     a.dx = dx;
+    a.g1_ws = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + own);
     *dx_done = true;
+    g_dx_variant = variant;
   }
   if (variant == 2) CP4_HIP(cp4::bwd_filter_fused_launch(a, st));
   else if (variant == 1) CP4_HIP(cp4::bwd_filter_mfma_launch(a, st));
@@ -1727,6 +1748,7 @@ cp4_status layer_backward_filter(const cp4_shape* s, const cp4_geometry* g, int 
                                  void* workspace, size_t workspace_bytes, void* dx, bool* dx_done,
                                  int variant, const LayerMask* mask, cp4_stream stream) {
   *dx_done = false;
+  g_dx_variant = 0;
   const float *xf = static_cast<const float*>(x), *dyf = static_cast<const float*>(dy);
   if (g)
     return backward_filter_geometry(s, g, xf, dyf, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
@@ -1739,6 +1761,8 @@ cp4_status layer_backward_filter(const cp4_shape* s, const cp4_geometry* g, int 
   return backward_filter_16(s, x, dy, FK, FC, FH, FW, dFK, dFC, dFH, dFW, workspace,
                             workspace_bytes, dtype == CP4_DTYPE_F16, dx, mask, stream);
 }
+
+int layer_dx_variant() { return g_dx_variant; }
 
 int layer_filter_takes_mask(const cp4_shape& s, const cp4_geometry* g, int dtype, const void* x,
                             const void* dy, const void* workspace) {

@@ -124,6 +124,8 @@ cp4_status layer_backward_filter(const cp4_shape*, const cp4_geometry*, int dtyp
                                  const float* FW, float* dFK, float* dFC, float* dFH, float* dFW,
                                  void* workspace, size_t workspace_bytes, void* dx, bool* dx_done,
                                  int variant, const LayerMask* mask, cp4_stream);
+// The fp32 variant in which this thread's last such call wrote dx; 0: another pass, or none did.
+int layer_dx_variant();
 // The backward-filter variant (strided and 16-bit layers: any number above 0) that such a call
 // runs with the mask and the bias gradient in it; 0: none does.
 int layer_filter_takes_mask(const cp4_shape&, const cp4_geometry*, int dtype, const void* x,
@@ -237,9 +239,11 @@ struct BwdFilterArgs {
   // of FH x FW and its gradient (FH, FW, dFH, dFW unused then).
   const float* taps2d;
   float* dtaps2d;
-  // Matrix-core variant only: not null, the input gradient too, dx = FC G1 (in the type of
+  // Matrix-core and three-launch variants: not null, the input gradient too, dx = FC G1 (in the type of
   // x; the forward's adjoint only where 2 * pad = Y - 1 = X - 1 or with a geometry).
   void* dx;
+  // Three-launch variant: room for G1, [N, R, H, W], which it forms for dx only.
+  float* g1_ws;
   // Where the variant's _masks function says so: dy counts where act_y > 0 (null: everywhere) and
   // dbias[t], its sum over images and pixels, comes along; all null: neither.  Scratch:
   // bias_part, T floats per compute unit (dense gradient) or partial set (_bias_sets), mask_ws, N * T * H * W

@@ -62,6 +62,9 @@ BackwardPlan make_backward_plan(const cp4_shape& s, const cp4_geometry* g, int d
   p.pass_at = at;
   if (g) p.pass_bytes = dx || filter ? cp4_conv2d_backward_ex_workspace_bytes(&s, g) : 0;
   else p.pass_bytes = filter ? cp4_conv2d_backward_filter_workspace_bytes(&s) : 0;
+  // (room for G1, from which the three-launch variant then brings dx along)
+  if (!g && !half && dx && filter && cp4::bwd_filter_fused_supported(s))
+    p.pass_bytes = align256(p.pass_bytes) + (size_t)s.N * s.Rank * s.H * s.W * 4;
   p.total = at + align256(p.pass_bytes);
   return p;
 }
@@ -141,7 +144,7 @@ cp4::Kept kept_parts(const KeepPlan& k, int parts, const void* kept) {
 }
 
 thread_local int g_route = 0;      // of this thread's last cp4_layer_backward
-thread_local int g_mask_inside = 0;
+thread_local int g_mask_inside = 0, g_dx_beside = 0;
 
 cp4_status check_layer(const cp4_shape* s, const cp4_geometry* g, int dtype, int act) {
   cp4_status rc = g ? cp4::check_layer_geometry(s, g) : cp4::check_layer_shape(s);
@@ -255,7 +258,7 @@ cp4_status cp4_layer_backward_kept(const cp4_shape* shape, const cp4_geometry* g
                                    void* dx, float* dFK, float* dFC, float* dFH, float* dFW,
                                    float* dbias, const void* kept, size_t kept_bytes, int parts_kept,
                                    void* workspace, size_t workspace_bytes, cp4_stream stream) {
-  g_route = g_mask_inside = 0;
+  g_route = g_mask_inside = g_dx_beside = 0;
   CP4_TRY(check_layer(shape, g, dtype, activation));
   const cp4_shape& s = *shape;
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -294,6 +297,7 @@ cp4_status cp4_layer_backward_kept(const cp4_shape* shape, const cp4_geometry* g
     float* mask_ws = p.act16 ? reinterpret_cast<float*>(ws + p.act16_at) : nullptr;
     const int variant = cp4::layer_filter_masks(s, xf, yf, dyf, ws + p.pass_at, mask_ws, dx != nullptr);
     if (variant) {
+      g_dx_beside = variant != 3 && dx;
       g_route = variant == 3 ? CP4_ROUTE_MASKED_TILES : CP4_ROUTE_DY_PASS | (dx ? CP4_ROUTE_DX_FROM_G1 : 0);
       cp4::Kept left{};
       if (kept && parts_kept && !(reinterpret_cast<uintptr_t>(kept) & 255)) {
@@ -334,7 +338,10 @@ cp4_status cp4_layer_backward_kept(const cp4_shape* shape, const cp4_geometry* g
                                        dFH, dFW, pass_ws, p.pass_bytes, dx, &dx_done,
                                        inside && !half && !g ? inside : -1, inside ? &mask : nullptr,
                                        stream));
-    if (dx && dx_done) g_route |= CP4_ROUTE_DX_FROM_G1;
+    if (dx && dx_done) {
+      g_dx_beside = 1;
+      if (cp4::layer_dx_variant() != 2) g_route |= CP4_ROUTE_DX_FROM_G1;
+    }
     dx_done = dx_done || !dx;
   } else if (filter) {
     float* x32 = reinterpret_cast<float*>(ws + p.x32_at);
@@ -361,5 +368,6 @@ cp4_status cp4_layer_backward_kept(const cp4_shape* shape, const cp4_geometry* g
 
 int cp4_layer_last_backward_route(void) { return g_route; }
 int cp4_layer_last_backward_mask_inside(void) { return g_mask_inside; }
+int cp4_layer_last_backward_dx_beside(void) { return g_dx_beside; }
 
 }  // extern "C"
