@@ -22,10 +22,10 @@
 //      floating-point atomics anywhere).
 #include <algorithm>
 #include <cstdint>
-#include <cstring>
 #include <type_traits>
 
 #include "cp4_internal.h"
+#include "plan_memo.h"
 #include "reduce_sets.h"
 #include "split_bf16.h"
 #include "store_policy.h"
@@ -722,19 +722,11 @@ int channel_splits(long items, int C, int T, bool masked) {
 }
 
 FusedPlan make_fused_plan_uncached(const cp4_shape& s);
-// The plan of the last shape asked for, per thread: a call asks several times (whether the variant takes
-// the shape, for its workspace, then with what), and the search goes over every strip height.
 FusedPlan make_fused_plan(const cp4_shape& s) {
-  static thread_local cp4_shape last_shape{};
-  static thread_local FusedPlan last_plan{};
-  static thread_local int last_cus = 0;
-  const int cus = num_compute_units();
-  if (last_cus != cus || memcmp(&last_shape, &s, sizeof(s))) {
-    last_plan = make_fused_plan_uncached(s);
-    last_shape = s;
-    last_cus = cus;
-  }
-  return last_plan;
+  using Key = std::array<unsigned, 10>;
+  static thread_local PlanMemo<Key, FusedPlan> memo;
+  return memo.get(Key{s.N, s.H, s.W, s.pad, s.T, s.C, s.Y, s.X, s.Rank, (unsigned)num_compute_units()},
+                  [&] { return make_fused_plan_uncached(s); });
 }
 FusedPlan make_fused_plan_uncached(const cp4_shape& s) {
   FusedPlan p{};

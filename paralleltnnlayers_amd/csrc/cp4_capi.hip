@@ -1,5 +1,6 @@
 // C ABI entry points: argument checks, kernel-variant choice, the PROFCOUNT
 // timing loops and the device allocator / copy helpers.
+#include <array>
 #include <atomic>
 #include <cstdio>
 #include <cstring>
@@ -8,6 +9,7 @@
 #include <tuple>
 
 #include "cp4_internal.h"
+#include "plan_memo.h"
 #include "store_policy.h"
 
 namespace {
@@ -628,7 +630,20 @@ int heuristic_variant(const FwdArgs& a) {
 // every kernel for its plan, several microseconds of host time that a small layer's launch
 // (5 us on the device) would otherwise wait for.
 std::map<std::tuple<TuneKey, unsigned>, int> g_heuristic_picks;
+// (g_choices counts the changes of either table)
+std::atomic<unsigned> g_choices{0};
+Choice choose_uncached(const FwdArgs& a);
 Choice choose(const FwdArgs& a) {
+  using Key = std::array<unsigned, 12>;
+  static thread_local cp4::PlanMemo<Key, Choice> memo;
+  return memo.get(Key{(unsigned)a.N, (unsigned)a.Cin, (unsigned)a.Cout, (unsigned)a.H, (unsigned)a.W,
+                      (unsigned)a.pad, (unsigned)a.Y, (unsigned)a.X, (unsigned)a.R, (unsigned)a.flip,
+                      (unsigned)((reinterpret_cast<uintptr_t>(a.x) & 15) << 4 |
+                                 (reinterpret_cast<uintptr_t>(a.y) & 15)),
+                      g_choices.load()},
+                  [&] { return choose_uncached(a); });
+}
+Choice choose_uncached(const FwdArgs& a) {
   const std::tuple<TuneKey, unsigned> hk(
       key_of(a), (unsigned)((reinterpret_cast<uintptr_t>(a.x) & 15) << 4 |
                             (reinterpret_cast<uintptr_t>(a.y) & 15)));
@@ -744,19 +759,14 @@ FilterPadLayout filter_pad_layout(const cp4_shape& s, const cp4_shape& t) {
 
 // One workspace size serves every backward-filter variant.
 size_t filter_workspace_uncached(const cp4_shape& s);
-// The size of the last shape asked for, per thread: every call checks its workspace against it, and every
-// variant plans for it.  (It depends on the device by its compute units.)
+using ShapeKey = std::array<unsigned, 11>;
+ShapeKey shape_key(const cp4_shape& s, unsigned flags) {
+  return {s.N, s.H, s.W, s.pad, s.T, s.C, s.Y, s.X, s.Rank, flags, (unsigned)cp4::num_compute_units()};
+}
+// (every call checks its workspace against it, and every variant plans for it)
 size_t filter_workspace(const cp4_shape& s) {
-  static thread_local cp4_shape last{};
-  static thread_local int last_cus = 0;
-  static thread_local size_t bytes = 0;
-  const int cus = cp4::num_compute_units();
-  if (cus != last_cus || memcmp(&last, &s, sizeof(s))) {
-    bytes = filter_workspace_uncached(s);
-    last = s;
-    last_cus = cus;
-  }
-  return bytes;
+  static thread_local cp4::PlanMemo<ShapeKey, size_t> memo;
+  return memo.get(shape_key(s, 0), [&] { return filter_workspace_uncached(s); });
 }
 size_t filter_workspace_uncached(const cp4_shape& s) {
   if (filter_pad_route(s)) {
@@ -1120,7 +1130,13 @@ struct FilterRoutes {
   bool tiles_ok, mfma_ok, fused_ok;
   bool dense_ok;      // variant 3: the dense filter gradient over tiles, then the chain rule
 };
+FilterRoutes filter_routes_uncached(const cp4_shape& s, bool aligned8, bool aligned16, bool ws256);
 FilterRoutes filter_routes(const cp4_shape& s, bool aligned8, bool aligned16, bool ws256) {
+  static thread_local cp4::PlanMemo<ShapeKey, FilterRoutes> memo;
+  return memo.get(shape_key(s, aligned8 | aligned16 << 1 | ws256 << 2),
+                  [&] { return filter_routes_uncached(s, aligned8, aligned16, ws256); });
+}
+FilterRoutes filter_routes_uncached(const cp4_shape& s, bool aligned8, bool aligned16, bool ws256) {
   FilterRoutes r;
   r.tiles_ok = filter_rank_tiles_supported(s) && aligned8 && ws256;
   r.mfma_ok = (cp4::bwd_filter_mfma_supported(s) && aligned8) || r.tiles_ok;
@@ -1964,6 +1980,7 @@ cp4_status tune_forward_like(const FwdArgs& a, unsigned warmup, unsigned profcou
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tuned[key_of(a)] = best;
+    ++g_choices;
   }
   if (best_variant) *best_variant = best.variant;
   if (best_us) *best_us = best_t;
@@ -2112,6 +2129,7 @@ cp4_status cp4_set_tuned_choice(const cp4_shape* shape, int backward_data, int v
     return fail(CP4_ERR_UNSUPPORTED, "the variant does not take this shape with this tile");
   std::lock_guard<std::mutex> lk(g_tune_mu);
   g_tuned[key_of(a)] = c;
+  ++g_choices;
   return CP4_OK;
 }
 
@@ -2195,6 +2213,7 @@ void cp4_tune_clear(void) {
   g_tuned.clear();
   g_tuned_filter.clear();
   g_heuristic_picks.clear();
+  ++g_choices;
 }
 
 cp4_status cp4_device_status(cp4_stream stream, int* detail) {

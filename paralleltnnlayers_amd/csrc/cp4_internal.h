@@ -14,7 +14,7 @@ namespace cp4 {
 // Operands of one forward-shaped launch.  Backward-data is the same kernel
 // with x<-dy, Cin<-T, Cout<-C, Fin<-FK, Fout<-FC and flipped taps
 // (Cuda_kernels/cp4Conv2dBackwardData.cu:79-87,98-108).
-struct FwdArgs {
+struct FwdKernelArgs {
   const float* x;     // [N, Cin, H, W]
   const float* Fin;   // [Cin, R]
   const float* Fout;  // [Cout, R]
@@ -35,19 +35,10 @@ struct FwdArgs {
   int ldf;
   size_t ldx;
   int accumulate;
-  // Not 0: the launch that follows reads y back (a later pass, the bias / activation kernel); y
-  // leaves the caches only from so many bytes on.
-  size_t reread;
   // 2-D-tap build of the producer / consumer kernel only: depthwise filter
   // [Y, X, R] used instead of the outer product FH x FW (FH, FW unused then).
   const float* taps2d;
-  // Producer / consumer kernel: a tuned strip height (tile height in the tiled
-  // build), log2 of the tile width (tiled build) and role split (1: off) that
-  // replace the planner's choice; 0 leaves it to the planner.
-  int tune_th, tune_lgwt, tune_split2;
-  // Producer / consumer kernel: polls before a wait between waves gives up
-  // (0: the default) and the device's fault record, four ints (may be null).
-  int spin_limit;
+  // Producer / consumer kernel: the device's fault record, four ints (may be null).
   int* fault;
   // Layer geometry beyond the reference's (stride 1, `pad` zeros before the image,
   // an H x W output): output pixel (ho, wo) reads x at (sh*ho + i - pt, sw*wo + j - pl),
@@ -73,6 +64,19 @@ struct FwdArgs {
   // Recomposed-filter kernel only: the dense filter [Cout, Cin, Y, X] itself, taps in
   // the order the pass reads them; the four factors are unused then.
   const float* dense;
+};
+// ... with what the launchers alone read (a launch costs by the bytes of its arguments, too: 2.6 us of
+// host time with 60 of them, 3.0 with 360).
+struct FwdArgs : FwdKernelArgs {
+  // Not 0: the launch that follows reads y back (a later pass, the bias / activation kernel); y
+  // leaves the caches only from so many bytes on.
+  size_t reread;
+  // Producer / consumer kernel: a tuned strip height (tile height in the tiled
+  // build), log2 of the tile width (tiled build) and role split (1: off) that
+  // replace the planner's choice; 0 leaves it to the planner.
+  int tune_th, tune_lgwt, tune_split2;
+  // Producer / consumer kernel: polls before a wait between waves gives up (0: the default).
+  int spin_limit;
 };
 
 // The geometry of a launch with the defaults filled in.

@@ -6,6 +6,7 @@
 #include <mutex>
 
 #include "cp4_internal.h"
+#include "plan_memo.h"
 
 namespace {
 
@@ -79,11 +80,14 @@ PlanKey plan_key(const cp4_shape& s, const cp4_geometry* g, int dtype, int act, 
 }
 template <class Plan, class Make>
 Plan remembered(std::mutex& mu, std::map<PlanKey, Plan>& plans, const PlanKey& key, Make make) {
-  std::lock_guard<std::mutex> lk(mu);
-  auto it = plans.find(key);
-  if (it != plans.end()) return it->second;
-  if (plans.size() > 4096) plans.clear();
-  return plans[key] = make();
+  static thread_local cp4::PlanMemo<PlanKey, Plan> memo;
+  return memo.get(key, [&] {
+    std::lock_guard<std::mutex> lk(mu);
+    auto it = plans.find(key);
+    if (it != plans.end()) return it->second;
+    if (plans.size() > 4096) plans.clear();
+    return plans[key] = make();
+  });
 }
 
 // The plan of a call, remembered: planning asks the backward-filter kernels for theirs,

@@ -51,7 +51,7 @@ struct DensePlan {
 
 // SW: the filter does not fit LDS and streams by channel chunk (DensePlan::stream_w).
 template <int FS, int KO, bool SW>
-__global__ __launch_bounds__(kThreads) void fwd_dense_small_kernel(FwdArgs a, DensePlan pl) {
+__global__ __launch_bounds__(kThreads) void fwd_dense_small_kernel(FwdKernelArgs a, DensePlan pl) {
   extern __shared__ float lds[];
   const int Cin = a.Cin, R = a.R, H = a.H, W = a.W;
   // Workgroup b runs on XCD b % 8, each with an L2 of its own: tile ids are permuted

@@ -68,7 +68,7 @@ struct FewPlan {
 // BIAS: a branch on it per group cost layers without one 2 to 4 %.  STORE: a StorePolicy for y.
 // KEEP: the signs of the results leave with them (FwdArgs::save_mask).
 template <int FS, int NCH, int RING, int OCC, int NW, bool BIAS, int STORE, bool KEEP>
-__global__ __launch_bounds__(64 * NW, OCC) void fwd_few_kernel(FwdArgs a, FewPlan pl) {
+__global__ __launch_bounds__(64 * NW, OCC) void fwd_few_kernel(FwdKernelArgs a, FewPlan pl) {
   constexpr int kWaves = NW;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   float4* As4 = reinterpret_cast<float4*>(lds_raw);                  // [quads][QA]

@@ -19,7 +19,7 @@ namespace {
 constexpr int kTH = 8, kTW = 32, kThreads = kTH * kTW;
 
 template <int RB>
-__global__ __launch_bounds__(kThreads) void fwd_general_kernel(FwdArgs a, Geometry g) {
+__global__ __launch_bounds__(kThreads) void fwd_general_kernel(FwdKernelArgs a, Geometry g) {
   extern __shared__ float lds[];
   // input cells under a tile of kTH x kTW outputs: rows, columns
   const int HT = g.sh * (kTH - 1) + a.Y, WT = g.sw * (kTW - 1) + a.X;

@@ -50,7 +50,7 @@ struct LightPlan {
 
 // STORE: a StorePolicy for y.
 template <int FS, int NW, int STORE>
-__global__ __launch_bounds__(64 * NW) void fwd_light_kernel(FwdArgs a, LightPlan pl) {
+__global__ __launch_bounds__(64 * NW) void fwd_light_kernel(FwdKernelArgs a, LightPlan pl) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   float4* As4 = reinterpret_cast<float4*>(lds_raw);                  // [quads][QA]
   unsigned char* Cf = lds_raw + pl.cf_off;   // plane ((part*nc + c)*2 + hi)*2 + parity: [pixel >> 1] x 16 B

@@ -65,7 +65,7 @@ __device__ __forceinline__ f32x16 mfma32(float a, float b, f32x16 c) {
 // FS: square filter size known at compile time (1, 3, 5, 7), 0 = any Y, X.
 // NS: Cin / 2 known at compile time (P1 fully unrolled), 0 = any even Cin.
 template <int RB, int FS, int NS>
-__global__ __launch_bounds__(kThreads) void fwd_mfma_strip_kernel(FwdArgs a, StripPlan pl) {
+__global__ __launch_bounds__(kThreads) void fwd_mfma_strip_kernel(FwdKernelArgs a, StripPlan pl) {
   constexpr int RP = 32 * RB;
   constexpr int kRing = 32 / RB;   // channel pairs in flight per lane
   extern __shared__ float lds[];

@@ -77,6 +77,7 @@
 #include <type_traits>
 
 #include "cp4_internal.h"
+#include "plan_memo.h"
 #include "split_bf16.h"
 #include "pipe_wait.h"
 #include "store_policy.h"
@@ -166,7 +167,7 @@ struct PipePlan {
 // STORE: how y goes to memory, a StorePolicy (builds of their own: two kinds of store in one cost ten
 // registers that there are not).
 template <int FS, int CPQ, int KR, int NQ = 4, bool PAIR = false, int STORE = kStorePlain>
-__global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdArgs a, PipePlan pl) {
+__global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, PipePlan pl) {
   extern __shared__ float lds[];
   // A plane: [rank quad][QA cells] of four fp32 each (the quad's ranks side by side:
   // one 16-byte LDS access moves a cell's four ranks)
@@ -1489,7 +1490,7 @@ bool layout_strided(const FwdArgs& a, int TH, PipePlan* pl) {
   pl->lds_bytes = bytes;
   return true;
 }
-bool plan(const FwdArgs& a, PipePlan* best) {
+bool plan_uncached(const FwdArgs& a, PipePlan* best) {
   double best_cost = 0;
   bool found = false;
   if (a.tune_th > 0) return a.tune_th <= a.Ho && layout_strided(a, a.tune_th, best);
@@ -1536,7 +1537,7 @@ bool layout_tiled(const FwdArgs& a, int TH, int lgWt, PipePlan* pl) {
   pl->lds_bytes = bytes;
   return true;
 }
-bool plan(const FwdArgs& a, PipePlan* best) {
+bool plan_uncached(const FwdArgs& a, PipePlan* best) {
   double best_cost = 0;
   bool found = false;
   // a tuned tile (cp4_tune_forward) replaces the cost model
@@ -1564,7 +1565,7 @@ bool plan(const FwdArgs& a, PipePlan* best) {
 }
 #endif
 #if !defined(CP4_PIPE_TILED) && !defined(CP4_PIPE_STRIDED)
-bool plan(const FwdArgs& a, PipePlan* best) {
+bool plan_uncached(const FwdArgs& a, PipePlan* best) {
   double best_cost = 0;
   bool found = false;
   // a tuned strip height (cp4_tune_forward) replaces the cost model
@@ -1590,6 +1591,25 @@ bool plan(const FwdArgs& a, PipePlan* best) {
   return found;
 }
 #endif
+
+struct PlanAnswer {
+  bool ok = false;
+  PipePlan plan;
+};
+bool plan(const FwdArgs& a, PipePlan* best) {
+  using Key = std::array<int, 23>;
+  static thread_local PlanMemo<Key, PlanAnswer> memo;
+  const PlanAnswer& r = memo.get(
+      Key{a.N, a.Cin, a.Cout, a.H, a.W, a.pad, a.Y, a.X, a.R, a.accumulate, a.tune_th, a.tune_lgwt,
+          a.tune_split2, a.sh, a.sw, a.pt, a.pl, a.Ho, a.Wo, a.transposed, a.ty, a.tx, num_compute_units()},
+      [&] {
+        PlanAnswer n;
+        n.ok = plan_uncached(a, &n.plan);
+        return n;
+      });
+  if (r.ok) *best = r.plan;
+  return r.ok;
+}
 
 template <int FS, int CPQ, int KR, int NQ, bool PAIR, int STORE>
 hipError_t launch_stored(const FwdArgs& a, const PipePlan& pl, hipStream_t st) {

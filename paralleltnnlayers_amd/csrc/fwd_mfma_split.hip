@@ -99,7 +99,7 @@ __device__ __forceinline__ f32x16 mfma_split(u32x4 ah, u32x4 am, u32x4 al, u32x4
 }
 
 template <int FS>
-__global__ __launch_bounds__(kThreads) void fwd_split_kernel(FwdArgs a, SplitPlan pl) {
+__global__ __launch_bounds__(kThreads) void fwd_split_kernel(FwdKernelArgs a, SplitPlan pl) {
   extern __shared__ float lds[];
   float* As = lds;                                      // [32][QA] fp32
   unsigned char* R2 = reinterpret_cast<unsigned char*>(lds + pl.r2_off);

@@ -79,7 +79,7 @@ struct Plan64 {
 // channels, 2: up to 256); NCH: 16-rank chunks (3: up to 48 ranks, 4: up to 64).
 // ACC: a later pass, y += (FwdArgs::accumulate); STORE: a StorePolicy for y.
 template <int FS, int CPQ, int NCH, bool ACC, int STORE>
-__global__ __launch_bounds__(kThreads) void fwd_pipe64_kernel(FwdArgs a, Plan64 pl) {
+__global__ __launch_bounds__(kThreads) void fwd_pipe64_kernel(FwdKernelArgs a, Plan64 pl) {
   extern __shared__ float lds[];
   // A plane: [rank quad][QA cells] of four fp32 each
   f32x4* As4 = reinterpret_cast<f32x4*>(lds);

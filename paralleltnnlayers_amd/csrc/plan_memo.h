@@ -1,0 +1,31 @@
+// The last few answers of a planner, per thread: a launch asks its kernel's planner several times (does it
+// take the shape, with what grid), a training step the same few shapes over and over, and a search
+// over strip heights is a microsecond of host time that a small layer's launch would wait for.
+#ifndef CP4_PLAN_MEMO_H
+#define CP4_PLAN_MEMO_H
+
+#include <array>
+
+namespace cp4 {
+
+// Key: what the answer depends on, a std::array of integers (compute units of the device included).
+template <class Key, class Answer, int kEntries = 4>
+struct PlanMemo {
+  Key keys[kEntries];
+  Answer answers[kEntries];
+  int used = 0, next = 0;
+  template <class Make>
+  const Answer& get(const Key& key, Make make) {
+    for (int i = 0; i < used; ++i)
+      if (keys[i] == key) return answers[i];
+    const int at = next;
+    answers[at] = make();          // (before the key: make may throw)
+    keys[at] = key;
+    next = (next + 1) % kEntries;
+    if (used < kEntries) ++used;
+    return answers[at];
+  }
+};
+
+}  // namespace cp4
+#endif
