@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "cp4_internal.h"
+#include "die_order.h"
 #include "plan_memo.h"
 #include "reduce_sets.h"
 #include "split_bf16.h"
@@ -53,6 +54,7 @@ struct ContractAllArgs {
   const float* y;          // masked build: dy counts where y > 0 ...
   float* masked;           // ... and is written so to here
   int through;             // A and G3 go through the L2
+  DieOrder order;          // of an operand's workgroups
 };
 
 // x / dy and the factor are read through buffer descriptors: an address is
@@ -70,7 +72,9 @@ __device__ __forceinline__ void contract_all(const ContractAllArgs& a, const int
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nthr >> 6;
   const int l32 = lane & 31, hi = lane >> 5;
   // This wave's (item, channel split); waves past the end do nothing but reach the barriers.
-  const int slot = blockIdx.x * nw + wave;
+  const int place = die_place(blockIdx.x, a.order);
+  if (place < 0) return;                               // whole workgroup
+  const int slot = place * nw + wave;
   const int item = slot / KS, part = slot - item * KS;
   const bool has_item = item < a.items;
   const int n = has_item ? item / a.npb : 0, pb = has_item ? item - n * a.npb : 0;
@@ -332,10 +336,12 @@ struct FusedArgs {
   float *part0, *part1;         // [S][D][R]
   float *partH, *partW;         // [S * TG][FS][R]
   float* partB;                 // [S][D0] sums of dy's rows, the layer's bias gradient; may be null
-  float* G1;                    // [N][R][HW]: the adjoint taps' results, for the input gradient; may be null
+  float* G1;                    // [N][R][HW]: the adjoint taps' results, for the input gradient
   int D0, D1;
   int N, R, H, W, P, HW;
   int TG;                     // channel groups of dFK that share the tap gradients (1 or 2)
+  int per, rest;              // items a workgroup takes, and how many take one more
+  DieOrder order;             // of the workgroups
   int TH, NS, items, S, MT;   // strip rows, strips per image, items = N * NS, workgroups per
                               // (gradient, channel group), 32-channel tiles per workgroup (4 or 8)
   int Wp, PSt, KSmax;         // padded row pitch, plane stride (odd), 16-pixel steps per strip
@@ -345,7 +351,9 @@ struct FusedArgs {
 // Workgroup: 512 threads.  LDS: [RP][PSt] plane | [RB][KSmax] fragment steps.
 // Square odd filters with "same" padding P = (FS-1)/2, so the zero border of the
 // plane is Q = P cells on every side and both chains read the same window.
-template <int FS, int RB>
+// LEAVE: G1 goes to memory as well (FusedArgs::G1), a build of its own (a test of the pointer cost the
+// others 1 to 4 %: N64 C128 T256 28x28 R48 54.3 us, 56.8).
+template <int FS, int RB, bool LEAVE>
 __global__ __launch_bounds__(512) void grad_fused_kernel(FusedArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   constexpr int RP = 32 * RB;
@@ -353,10 +361,13 @@ __global__ __launch_bounds__(512) void grad_fused_kernel(FusedArgs a) {
   constexpr int NX = 8 + 2 * Q;        // window positions that can hold a pixel of the octet
   constexpr int WN = NX + FS - 1;      // window columns read per tap row
   constexpr int kRing = 4;             // 16-pixel steps in flight per wave
-  const int which = blockIdx.z, cg = blockIdx.y, sidx = blockIdx.x;
+  const int which = blockIdx.z, cg = blockIdx.y;
+  const int sidx = die_place(blockIdx.x, a.order);
   const int D = which ? a.D1 : a.D0, R = a.R, H = a.H, W = a.W, HW = a.HW;
   const int MT = a.MT, KH = 8 / MT;
-  if (cg * 32 * MT >= D) return;                       // whole workgroup
+  if (cg * 32 * MT >= D || sidx < 0) return;           // whole workgroup
+  // a contiguous range of the items (a division here would be a microsecond of a small layer's launch)
+  const int item0 = sidx * a.per + min(sidx, a.rest), item1 = item0 + a.per + (sidx < a.rest);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hi = lane >> 5;
@@ -392,7 +403,7 @@ __global__ __launch_bounds__(512) void grad_fused_kernel(FusedArgs a) {
   const float* Zs = which ? a.Zsrc1 : a.Zsrc0;
   const float* act = which ? a.act1 : a.act0;
 
-  for (int item = sidx; item < a.items; item += a.S) {
+  for (int item = item0; item < item1; ++item) {
     const int n = item / a.NS, st = item - n * a.NS;
     const int h0 = st * a.TH, h1 = min(H, h0 + a.TH);
     const int q0 = h0 * W, q1 = h1 * W;
@@ -463,7 +474,7 @@ __global__ __launch_bounds__(512) void grad_fused_kernel(FusedArgs a) {
     // this wave's first activation steps, requested behind the plane so that the plane arrives first
 #pragma unroll
     for (int u = 0; u < kRing; ++u) issue(ring[u], kh + u * KH);
-    if (item == sidx) {
+    if (item == item0) {
       // the tap weights, requested behind the first loads and first used in the tap
       // step; padding ranks read rank 0's weights: their plane rows are all zero
 #pragma unroll
@@ -570,11 +581,12 @@ __global__ __launch_bounds__(512) void grad_fused_kernel(FusedArgs a) {
         const float v = j < k ? call[j] : call[j + 2 * Q];
         out[j] = (qb + j < q1) ? v : 0.f;
       }
-      if (which && cg == 0 && a.G1 && r < R) {         // (strips end on multiples of four pixels)
-        float* g = a.G1 + ((size_t)n * R + r) * HW + qb;
-        *reinterpret_cast<float4*>(g) = make_float4(out[0], out[1], out[2], out[3]);
-        if (qb + 4 < q1) *reinterpret_cast<float4*>(g + 4) = make_float4(out[4], out[5], out[6], out[7]);
-      }
+      if constexpr (LEAVE)
+        if (which && cg == 0 && r < R) {               // (strips end on multiples of four pixels)
+          float* g = a.G1 + ((size_t)n * R + r) * HW + qb;
+          *reinterpret_cast<float4*>(g) = make_float4(out[0], out[1], out[2], out[3]);
+          if (qb + 4 < q1) *reinterpret_cast<float4*>(g + 4) = make_float4(out[4], out[5], out[6], out[7]);
+        }
       u32x4 ph, pm, pl;
       split8(out, ph, pm, pl);
       dst[0] = ph;
@@ -867,7 +879,16 @@ hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
   const int ks = c.y ? channel_splits(c.items, a.C, a.T, true) : p.ks;
   const size_t lds_contract = ks > 1 ? std::max(p.lds_contract, (size_t)p.nw * p.RB * 16 * 64 * 4) : p.lds_contract;
   const long slots = (long)c.items * ks;
-  const dim3 cgrid((unsigned)((slots + p.nw - 1) / p.nw), 2);
+  const long wgs = (slots + p.nw - 1) / p.nw;
+  // Die order, and contiguous items for a workgroup of the gradients, which then finds x (and dy, where
+  // nothing masks it) in its L2: 28 layers of C 64-512, R 16-64, N 1-100 1.02 times as fast on the mean.
+  // Not for a few images, which every die shares (N1 C256 28x28 R32 18.8 us in turn, 19.3 in order), nor for
+  // strips of a row or two with two rank blocks, whose neighbours request the same lines of the planes at
+  // the same time (N4 C256 28x28 R64 26.5 / 29.0, N8 28.4 / 29.9; but N16 28x28, strips of 448 bytes,
+  // 33.4 / 31.7, N4 56x56 34.3 / 32.9, and N12 28x28 R32 28.4 / 27.1).
+  const bool dies = N >= 4 && (p.RB == 1 || p.TH * a.W * (int)sizeof(float) >= 448);
+  c.order = die_order(wgs, dies);
+  const dim3 cgrid(dies ? die_grid(wgs) : (unsigned)wgs, 2);
   hipError_t e;
 #define CP4_CONTRACT(RB_, KS_, RING_)                                                          \
   {                                                                                            \
@@ -899,16 +920,19 @@ hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
   g.partB = a.dbias ? a.bias_part : nullptr;
   g.G1 = a.dx ? G1 : nullptr;
   g.N = N; g.R = R; g.H = a.H; g.W = a.W; g.P = a.pad; g.HW = HW;
+  g.per = p.items / p.S; g.rest = p.items % p.S;
+  g.order = die_order(p.S, dies);
   g.TG = p.TG; g.TH = p.TH; g.NS = p.NS; g.items = p.items; g.S = p.S; g.MT = p.MT;
   g.Wp = p.Wp; g.PSt = p.PSt; g.KSmax = p.KSmax;
   g.wmagic = (unsigned)(0x100000000ull / (unsigned)a.W) + 1u;
-  const dim3 ggrid(p.S, p.ncg, 2);
+  const dim3 ggrid(dies ? die_grid(p.S) : p.S, p.ncg, 2);
 #define CP4_FUSED(FS_, RB_)                                                                   \
   {                                                                                           \
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(grad_fused_kernel<FS_, RB_>),       \
+    auto k = g.G1 ? grad_fused_kernel<FS_, RB_, true> : grad_fused_kernel<FS_, RB_, false>;   \
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),                                 \
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds);          \
     if (e != hipSuccess) return e;                                                            \
-    grad_fused_kernel<FS_, RB_><<<ggrid, 512, p.lds, st>>>(g);                                \
+    k<<<ggrid, 512, p.lds, st>>>(g);                                                          \
   }
 #define CP4_FUSED_FS(FS_)                                 \
   {                                                       \

@@ -14,8 +14,8 @@ struct ReduceArgs {
   int count[5], S[5];
 };
 
-// A workgroup owns 64 consecutive outputs of segment `seg`, from 64 * block on; its `waves` waves each
-// sum a part of the S partials in index order (sixteen loads in flight, eight added as a tree), then the
+// A workgroup owns 64 consecutive outputs of segment `seg`, from 64 * block on; its `waves` waves (4 or
+// 16) each sum a part of the S partials in index order (sixteen loads in flight, eight added as a tree), then the
 // parts are added in wave order: the result does not depend on timing.  part: 64 floats a wave.
 __device__ __forceinline__ void reduce_sets_block(const ReduceArgs& a, int seg, int block, int waves,
                                                   float (*part)[64]) {
@@ -23,7 +23,8 @@ __device__ __forceinline__ void reduce_sets_block(const ReduceArgs& a, int seg, 
   const int i = block * 64 + lane;
   const int count = a.count[seg], S = a.S[seg];
   if (block * 64 >= count) return;                         // whole workgroup
-  const int k0 = (int)((long)S * q / waves), k1 = (int)((long)S * (q + 1) / waves);
+  const int shift = waves == 4 ? 2 : 4;                    // (a division is a third of a small sum's time)
+  const int k0 = (int)((unsigned)S * q >> shift), k1 = (int)((unsigned)S * (q + 1) >> shift);
   float s = 0.f;
   if (i < count) {
     const float* p = a.part[seg] + i;
@@ -51,12 +52,14 @@ __device__ __forceinline__ void reduce_sets_block(const ReduceArgs& a, int seg, 
       s += (v[0] + v[2]) + (v[1] + v[3]);
     }
     s += s1;
-    // (the rest together too, the last set in place of those past it)
-    float v[8];
+    // (the rest together too, the last set in place of those past it; none left: the same for a wave)
+    if (k < k1) {
+      float v[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = p[(size_t)(k + u < k1 ? k + u : k1 - 1 > 0 ? k1 - 1 : 0) * stride];
+      for (int u = 0; u < 8; ++u) v[u] = p[(size_t)(k + u < k1 ? k + u : k1 - 1) * stride];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) s += k + u < k1 ? v[u] : 0.f;
+      for (int u = 0; u < 8; ++u) s += k + u < k1 ? v[u] : 0.f;
+    }
   }
   part[q][lane] = s;
   __syncthreads();
