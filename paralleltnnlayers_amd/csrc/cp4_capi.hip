@@ -661,6 +661,53 @@ Choice choose_uncached(const FwdArgs& a) {
   return Choice{pick, 0, 0, 0};
 }
 
+// 16-bit activations.  The producer / consumer kernel decides which shapes are taken; the
+// few-channel and the recomposed-filter kernel take over by the fp32 layers' rules (150 layers of 1 to
+// 64 channels on either side, and 74 of planes from 56x56 to 225x225: 1.27 and 1.20 times as fast on the
+// mean, up to 10 times).  But where a row leaves much of a 32-column tile empty and there are many of them
+// the strips of whole rows are quicker: N60 65x65 R4 C16 K16 5x5 19.3 us against 25.3, C32 K64 3x3 27
+// against 32; N16 the other way round, 12.1 and 11.5, 18.4 and 12.1.
+constexpr long kFew16RaggedMaxPixels = 1l << 17;
+bool few16_wastes_columns(const FwdArgs& a) {
+  return (a.W + 31) / 32 * 32 * 10l > 14l * a.W && (long)a.N * a.H * a.W >= kFew16RaggedMaxPixels;
+}
+enum class Kernel16 { kNone, kPipe, kFew, kDense };
+Kernel16 pick16_uncached(const FwdArgs& a, bool half) {
+  if (!(half ? cp4::fwd_pipe_iof16_supported(a) : cp4::fwd_pipe_io16_supported(a))) return Kernel16::kNone;
+  const bool dense = (half ? cp4::fwd_dense_small_iof16_supported(a) : cp4::fwd_dense_small_io16_supported(a)) &&
+                     dense_small_estimate(a) <= kMatrixSmallChannelEstimate && !dense_small_loses_to_matrix(a);
+  if ((half ? cp4::fwd_few_iof16_supported(a) : cp4::fwd_few_io16_supported(a)) &&
+      few_preferred(a, dense) && !(few16_wastes_columns(a) && !dense))
+    return Kernel16::kFew;
+  return dense ? Kernel16::kDense : Kernel16::kPipe;
+}
+cp4_status run_16(FwdArgs a, int dtype, hipStream_t st) {
+  const bool half = dtype == CP4_DTYPE_F16;
+  using Key = std::array<unsigned, 12>;
+  static thread_local cp4::PlanMemo<Key, Kernel16> memo;
+  const Kernel16 k = memo.get(
+      Key{(unsigned)a.N, (unsigned)a.Cin, (unsigned)a.Cout, (unsigned)a.H, (unsigned)a.W, (unsigned)a.pad,
+          (unsigned)a.Y, (unsigned)a.X, (unsigned)a.R, (unsigned)half,
+          (unsigned)((reinterpret_cast<uintptr_t>(a.x) & 15) << 4 | (reinterpret_cast<uintptr_t>(a.y) & 15)),
+          (unsigned)cp4::num_compute_units()},
+      [&] { return pick16_uncached(a, half); });
+  switch (k) {
+    case Kernel16::kFew:
+      CP4_HIP(half ? cp4::fwd_few_iof16_launch(a, st) : cp4::fwd_few_io16_launch(a, st));
+      return CP4_OK;
+    case Kernel16::kDense:
+      CP4_HIP(half ? cp4::fwd_dense_small_iof16_launch(a, st) : cp4::fwd_dense_small_io16_launch(a, st));
+      return CP4_OK;
+    case Kernel16::kPipe:
+      CP4_ARM(a);
+      CP4_HIP(half ? cp4::fwd_pipe_iof16_launch(a, st) : cp4::fwd_pipe_io16_launch(a, st));
+      return CP4_OK;
+    default:
+      return fail(CP4_ERR_UNSUPPORTED, half ? "half-precision I/O: shape not taken by the producer/consumer kernel"
+                                            : "bfloat16 I/O: shape not taken by the producer/consumer kernel");
+  }
+}
+
 FwdArgs with_tile(const FwdArgs& a, const Choice& c) {
   FwdArgs b = a;
   b.tune_th = c.th;
@@ -1053,11 +1100,7 @@ cp4_status cp4_conv2d_forward_bf16(const cp4_shape* shape, const void* x_bf16,
                            static_cast<float*>(y_bf16));
   a.bias = bias;
   a.act = activation;
-  CP4_ARM(a);
-  if (!cp4::fwd_pipe_io16_supported(a))
-    return fail(CP4_ERR_UNSUPPORTED, "bfloat16 I/O: shape not taken by the producer/consumer kernel");
-  CP4_HIP(cp4::fwd_pipe_io16_launch(a, as_stream(stream)));
-  return CP4_OK;
+  return run_16(a, CP4_DTYPE_BF16, as_stream(stream));
 }
 
 cp4_status cp4_conv2d_backward_data_bf16(const cp4_shape* shape, const void* dy_bf16,
@@ -1071,11 +1114,7 @@ cp4_status cp4_conv2d_backward_data_bf16(const cp4_shape* shape, const void* dy_
   if (rc != CP4_OK) return rc;
   FwdArgs a = backward_data_args(*shape, static_cast<const float*>(dy_bf16), FK, FC, FH, FW,
                                  static_cast<float*>(dx_bf16));
-  CP4_ARM(a);
-  if (!cp4::fwd_pipe_io16_supported(a))
-    return fail(CP4_ERR_UNSUPPORTED, "bfloat16 I/O: shape not taken by the producer/consumer kernel");
-  CP4_HIP(cp4::fwd_pipe_io16_launch(a, as_stream(stream)));
-  return CP4_OK;
+  return run_16(a, CP4_DTYPE_BF16, as_stream(stream));
 }
 
 cp4_status cp4_conv2d_forward_f16(const cp4_shape* shape, const void* x_f16,
@@ -1095,11 +1134,7 @@ cp4_status cp4_conv2d_forward_f16(const cp4_shape* shape, const void* x_f16,
                            static_cast<float*>(y_f16));
   a.bias = bias;
   a.act = activation;
-  CP4_ARM(a);
-  if (!cp4::fwd_pipe_iof16_supported(a))
-    return fail(CP4_ERR_UNSUPPORTED, "half-precision I/O: shape not taken by the producer/consumer kernel");
-  CP4_HIP(cp4::fwd_pipe_iof16_launch(a, as_stream(stream)));
-  return CP4_OK;
+  return run_16(a, CP4_DTYPE_F16, as_stream(stream));
 }
 
 cp4_status cp4_conv2d_backward_data_f16(const cp4_shape* shape, const void* dy_f16,
@@ -1113,11 +1148,7 @@ cp4_status cp4_conv2d_backward_data_f16(const cp4_shape* shape, const void* dy_f
   if (rc != CP4_OK) return rc;
   FwdArgs a = backward_data_args(*shape, static_cast<const float*>(dy_f16), FK, FC, FH, FW,
                                  static_cast<float*>(dx_f16));
-  CP4_ARM(a);
-  if (!cp4::fwd_pipe_iof16_supported(a))
-    return fail(CP4_ERR_UNSUPPORTED, "half-precision I/O: shape not taken by the producer/consumer kernel");
-  CP4_HIP(cp4::fwd_pipe_iof16_launch(a, as_stream(stream)));
-  return CP4_OK;
+  return run_16(a, CP4_DTYPE_F16, as_stream(stream));
 }
 
 namespace {

@@ -204,6 +204,15 @@ hipError_t fwd_pipe_io16_launch(const FwdArgs&, hipStream_t);
 // The same with IEEE half-precision x and y in memory.
 bool fwd_pipe_iof16_supported(const FwdArgs&);
 hipError_t fwd_pipe_iof16_launch(const FwdArgs&, hipStream_t);
+// The few-channel and the recomposed-filter kernel likewise (the latter for filters up to 7 x 7).
+bool fwd_few_io16_supported(const FwdArgs&);
+hipError_t fwd_few_io16_launch(const FwdArgs&, hipStream_t);
+bool fwd_few_iof16_supported(const FwdArgs&);
+hipError_t fwd_few_iof16_launch(const FwdArgs&, hipStream_t);
+bool fwd_dense_small_io16_supported(const FwdArgs&);
+hipError_t fwd_dense_small_io16_launch(const FwdArgs&, hipStream_t);
+bool fwd_dense_small_iof16_supported(const FwdArgs&);
+hipError_t fwd_dense_small_iof16_launch(const FwdArgs&, hipStream_t);
 // The same kernel honouring FwdArgs::ldf and FwdArgs::accumulate (rank passes).
 bool fwd_pipe_rankpass_supported(const FwdArgs&);
 hipError_t fwd_pipe_rankpass_launch(const FwdArgs&, hipStream_t);

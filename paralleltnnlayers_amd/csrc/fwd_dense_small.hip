@@ -28,6 +28,13 @@
 //   epilogue  one float4 store per output channel where alignment allows
 // Tap order follows FwdArgs::flip (backward-data reads the taps in reverse,
 // Cuda_kernels/cp4Conv2dBackwardData.cu:79-87).
+//
+// Compiled with CP4_IO16 the activations are 16-bit (act_io.h; entry points
+// fwd_dense_small_io16_* and _iof16_*, filters up to 7 x 7); the arithmetic stays fp32.
+// The producer / consumer kernel pays for 32 x 32 tiles and a workgroup per strip whatever
+// the channel counts: N56 C3 K1 304x342 bf16 406 us there, 39 here, N2 C3 K3 507x507 66 and 11.5,
+// N81 C2 K2 73x73 R28 f16 59 and 10.3.
+#include "act_io.h"
 #include "cp4_internal.h"
 
 namespace cp4 {
@@ -108,9 +115,10 @@ __global__ __launch_bounds__(kThreads) void fwd_dense_small_kernel(FwdKernelArgs
   const int ty = tid >> 4, tx = tid & 15;             // row of the tile, group of four columns
   const int WT = pl.tile_w;
   const int left = a.pad;                             // halo cells left of the tile (pad <= FS - 1)
-  const bool vec_in = (W & 3) == 0 && w0 + kTW <= W && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0;
-  const bool vec_out = (W & 3) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
-  const float* xn = a.x + (size_t)n * Cin * HW;
+  // (four pixels at once: sixteen bytes of floats, eight of a 16-bit type)
+  const bool vec_in = (W & 3) == 0 && w0 + kTW <= W && (reinterpret_cast<uintptr_t>(a.x) & (4 * kIoBytes - 1)) == 0;
+  const bool vec_out = (W & 3) == 0 && (reinterpret_cast<uintptr_t>(a.y) & (4 * kIoBytes - 1)) == 0;
+  const io_t* xn = reinterpret_cast<const io_t*>(a.x) + (size_t)n * Cin * HW;
 
   for (int tr = 0; tr < pl.tpw; ++tr) {
     const int h0 = (by * pl.tpw + tr) * kTH;
@@ -140,8 +148,16 @@ __global__ __launch_bounds__(kThreads) void fwd_dense_small_kernel(FwdKernelArgs
           const int c = rowid / HT, row = rowid - c * HT;
           const int gh = h0 + row - a.pad;
           float4 val = make_float4(0.f, 0.f, 0.f, 0.f);
-          if (gh >= 0 && gh < H)
-            val = *reinterpret_cast<const float4*>(xn + (size_t)(c0 + c) * HW + (size_t)gh * W + w0 + 4 * v);
+          if (gh >= 0 && gh < H) {
+            const io_t* src = xn + (size_t)(c0 + c) * HW + (size_t)gh * W + w0 + 4 * v;
+#ifdef CP4_IO16
+            const uint2 u = *reinterpret_cast<const uint2*>(src);
+            val = make_float4(from_io((io_t)u.x), from_io((io_t)(u.x >> 16)), from_io((io_t)u.y),
+                              from_io((io_t)(u.y >> 16)));
+#else
+            val = *reinterpret_cast<const float4*>(src);
+#endif
+          }
           float* dst = tile + rowid * WT + left + 4 * v;
           dst[0] = val.x;
           dst[1] = val.y;
@@ -156,7 +172,7 @@ __global__ __launch_bounds__(kThreads) void fwd_dense_small_kernel(FwdKernelArgs
           const int col = e < left ? e : kTW + e;     // cell of the row: left halo, then right halo
           const int gh = h0 + row - a.pad, gw = w0 + col - left;
           float v = 0.f;
-          if (gh >= 0 && gh < H && gw >= 0 && gw < W) v = xn[(size_t)(c0 + c) * HW + (size_t)gh * W + gw];
+          if (gh >= 0 && gh < H && gw >= 0 && gw < W) v = from_io(xn[(size_t)(c0 + c) * HW + (size_t)gh * W + gw]);
           tile[rowid * WT + col] = v;
         }
       } else {
@@ -165,7 +181,7 @@ __global__ __launch_bounds__(kThreads) void fwd_dense_small_kernel(FwdKernelArgs
           const int c = rowid / HT, row = rowid - c * HT;
           const int gh = h0 + row - a.pad, gw = w0 + col - left;
           float v = 0.f;
-          if (gh >= 0 && gh < H && gw >= 0 && gw < W) v = xn[(size_t)(c0 + c) * HW + (size_t)gh * W + gw];
+          if (gh >= 0 && gh < H && gw >= 0 && gw < W) v = from_io(xn[(size_t)(c0 + c) * HW + (size_t)gh * W + gw]);
           tile[rowid * WT + col] = v;
         }
       }
@@ -196,12 +212,12 @@ __global__ __launch_bounds__(kThreads) void fwd_dense_small_kernel(FwdKernelArgs
 
     const int h = h0 + ty, w = w0 + kPX * tx;
     if (h < H && w < W) {
-      float* yp = a.y + ((size_t)n * a.Cout + k0) * HW + (size_t)h * W + w;
+      io_t* yp = reinterpret_cast<io_t*>(a.y) + ((size_t)n * a.Cout + k0) * HW + (size_t)h * W + w;
       const bool vec = vec_out && w + kPX <= W;
 #pragma unroll
       for (int k = 0; k < KO; ++k) {
         if (k < Cout) {
-          float* dst = yp + (size_t)k * HW;
+          io_t* dst = yp + (size_t)k * HW;
           // y = act(conv + bias[k]) as the values are stored (FwdArgs::bias / act)
           const float bk = a.bias ? a.bias[k0 + k] : 0.f;
           float o[kPX];
@@ -211,11 +227,15 @@ __global__ __launch_bounds__(kThreads) void fwd_dense_small_kernel(FwdKernelArgs
             o[p] = (a.act != 0 && t < 0.f) ? 0.f : t;
           }
           if (vec) {
+#ifdef CP4_IO16
+            *reinterpret_cast<uint2*>(dst) = make_uint2(io_pair(o[0], o[1]), io_pair(o[2], o[3]));
+#else
             *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
+#endif
           } else {
 #pragma unroll
             for (int p = 0; p < kPX; ++p)
-              if (w + p < W) dst[p] = o[p];
+              if (w + p < W) dst[p] = to_io(o[p]);
           }
         }
       }
@@ -226,6 +246,9 @@ __global__ __launch_bounds__(kThreads) void fwd_dense_small_kernel(FwdKernelArgs
 bool plan(const FwdArgs& a, DensePlan* pl) {
   if (a.Y != a.X || !(a.Y & 1) || a.Y > 17 || a.pad > a.Y - 1) return false;
   if (a.ldf || a.accumulate || a.sh) return false;
+#ifdef CP4_IO16
+  if (a.Y > 7 || a.dense) return false;
+#endif
   const int kgrp = a.Cout < 8 ? a.Cout : 8;           // output channels of a workgroup
   const long ngrp = (a.Cout + 7) / 8;
   long nw = (long)kgrp * a.Cin * a.Y * a.X;
@@ -282,7 +305,10 @@ hipError_t launch_sw(const FwdArgs& a, const DensePlan& pl, hipStream_t st) {
 }
 template <int FS, int KO>
 hipError_t launch_as(const FwdArgs& a, const DensePlan& pl, hipStream_t st) {
-  return pl.stream_w ? launch_sw<FS, KO, true>(a, pl, st) : launch_sw<FS, KO, false>(a, pl, st);
+#ifndef CP4_IO16
+  if (pl.stream_w) return launch_sw<FS, KO, true>(a, pl, st);    // (given filters only)
+#endif
+  return launch_sw<FS, KO, false>(a, pl, st);
 }
 
 template <int FS>
@@ -295,11 +321,20 @@ hipError_t launch_ko(const FwdArgs& a, const DensePlan& pl, hipStream_t st) {
 
 }  // namespace
 
+#if defined(CP4_IO16) && CP4_IO16 == 2
+#define fwd_dense_small_supported fwd_dense_small_iof16_supported
+#define fwd_dense_small_launch fwd_dense_small_iof16_launch
+#elif defined(CP4_IO16)
+#define fwd_dense_small_supported fwd_dense_small_io16_supported
+#define fwd_dense_small_launch fwd_dense_small_io16_launch
+#endif
+
 bool fwd_dense_small_supported(const FwdArgs& a) {
   DensePlan pl;
   return plan(a, &pl);
 }
 
+#ifndef CP4_IO16
 bool fwd_dense_small_plan_info(const FwdArgs& a, long* tiles, size_t* lds_bytes) {
   DensePlan pl;
   if (!plan(a, &pl)) return false;
@@ -307,6 +342,7 @@ bool fwd_dense_small_plan_info(const FwdArgs& a, long* tiles, size_t* lds_bytes)
   *lds_bytes = pl.lds_bytes;
   return true;
 }
+#endif
 
 hipError_t fwd_dense_small_launch(const FwdArgs& a, hipStream_t st) {
   DensePlan pl;
@@ -316,12 +352,17 @@ hipError_t fwd_dense_small_launch(const FwdArgs& a, hipStream_t st) {
     case 3: return launch_ko<3>(a, pl, st);
     case 5: return launch_ko<5>(a, pl, st);
     case 7: return launch_ko<7>(a, pl, st);
+#ifdef CP4_IO16
+    default: return hipErrorInvalidValue;
+  }
+#else
     case 9: return launch_ko<9>(a, pl, st);
     case 11: return launch_ko<11>(a, pl, st);
     case 13: return launch_ko<13>(a, pl, st);
     case 15: return launch_ko<15>(a, pl, st);
     default: return launch_ko<17>(a, pl, st);
   }
+#endif
 }
 
 }  // namespace cp4

@@ -26,8 +26,17 @@
 //     stores with the bias / activation epilogue;
 //   * barrier (the plane is free for the next tile).
 // Out-of-image cells are zeros in the plane, so the tap step needs no masks.
+//
+// Compiled with CP4_IO16 (act_io.h; entry points fwd_few_io16_* and _iof16_*) x and y are
+// 16-bit: a bfloat16 is one of the three parts of a split, a half two of them, so three or
+// five of the six products per chunk remain; A, the taps and the output contraction are as in
+// the fp32 build.  Against the producer / consumer kernel, which took these layers: N16 C3 K64
+// 224x224 R16 bf16 63 -> 42 us (77 MB written, 1.9 TB/s), C16 K16 R4 f16 45 -> 22, C32 K64 5x5 R4
+// 92 -> 51.  (A half is split into its two parts by hand: the general split's third, zero as it is,
+// kept 70 to 160 more registers alive than there are.)
 #include <cstring>
 
+#include "act_io.h"
 #include "cp4_internal.h"
 #include "split_bf16.h"
 #include "store_policy.h"
@@ -148,7 +157,11 @@ __global__ __launch_bounds__(64 * NW, OCC) void fwd_few_kernel(FwdKernelArgs a, 
   // ... padded to whole turns of the ring, so that a step of any tile has the same slot;
   // the padding steps load the tile's last chunk again and are not used
   auto padded = [&](int nsteps) { return (nsteps + RING - 1) / RING * RING; };
+#ifdef CP4_IO16
+  unsigned xb[RING][8];                                 // 16-bit values, zero-extended
+#else
   float xb[RING][8];
+#endif
   int cellv[RING];     // the slot's LDS cell; bit 30: outside the image (zero); -1: not a cell
   auto issue = [&](int slot, const Tile& tl, int step, int c) {   // c == step % NCH, given statically
     const int rows = tl.first ? PH : pl.TH, prow0 = tl.first ? 0 : FS - 1;
@@ -159,17 +172,23 @@ __global__ __launch_bounds__(64 * NW, OCC) void fwd_few_kernel(FwdKernelArgs a, 
     const bool cell = pr < rows;
     const bool inside = h >= 0 && h < H && w >= 0 && w < W;
     const int hc = h < 0 ? 0 : (h > H - 1 ? H - 1 : h), wc = w < 0 ? 0 : (w > W - 1 ? W - 1 : w);
-    const unsigned voff = (unsigned)(8 * hi * HW + hc * W + wc) * 4u;
+    const unsigned voff = (unsigned)(8 * hi * HW + hc * W + wc) * (unsigned)kIoBytes;
     // x through a buffer descriptor over the tile's image: reads past its last channel return 0
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(a.x + (size_t)tl.n * Cin * HW), 0, Cin * HW * 4, 0x00020000);
-    const unsigned soff = (unsigned)(16 * c) * (unsigned)HW * 4u;
+        const_cast<io_t*>(reinterpret_cast<const io_t*>(a.x) + (size_t)tl.n * Cin * HW), 0,
+        Cin * HW * kIoBytes, 0x00020000);
+    const unsigned soff = (unsigned)(16 * c) * (unsigned)HW * (unsigned)kIoBytes;
 #pragma unroll
     for (int e = 0; e < 8; ++e)
+#ifdef CP4_IO16
+      xb[slot][e] = (unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(
+          xrs, voff, __builtin_amdgcn_readfirstlane(soff + (unsigned)e * HW * 2u), 0);
+#else
       xb[slot][e] = __builtin_bit_cast(          // (the scalar offset said to be wave-uniform: held in
           float,                                   // a vector register it would cost a loop per load)
           __builtin_amdgcn_raw_buffer_load_b32(
               xrs, voff, __builtin_amdgcn_readfirstlane(soff + (unsigned)e * HW * 4u), 0));
+#endif
     int ring_row = tl.slot0 + prow;
     ring_row = ring_row >= PH ? ring_row - PH : ring_row;
     cellv[slot] = !cell ? -1 : (ring_row * PS + pc) | (inside ? 0 : 0x40000000);
@@ -271,10 +290,33 @@ __global__ __launch_bounds__(64 * NW, OCC) void fwd_few_kernel(FwdKernelArgs a, 
           const int c = u % NCH;
           if (s0 + u < nsteps) {                        // (the same for all lanes)
             if (c == 0) acc = (f32x16)(0.f);
+            const u32x4 th = frag[(c * 3 + 0) * 64 + lane], tm = frag[(c * 3 + 1) * 64 + lane],
+                        tl = frag[(c * 3 + 2) * 64 + lane];
+#if !defined(CP4_IO16)
             u32x4 xh, xm, xl;
             split8(xb[u], xh, xm, xl);
-            acc = mfma_split(frag[(c * 3 + 0) * 64 + lane], frag[(c * 3 + 1) * 64 + lane],
-                             frag[(c * 3 + 2) * 64 + lane], xh, xm, xl, acc);
+            acc = mfma_split(th, tm, tl, xh, xm, xl, acc);
+#elif CP4_IO16 == 2
+            u32x4 xh, xm;                               // (11 significant bits: two parts)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+              const float p = from_io((io_t)xb[u][2 * d]), q = from_io((io_t)xb[u][2 * d + 1]);
+              xh[d] = pack_hi16(p, q);
+              xm[d] = pack_hi16(p - trunc_bf16(p), q - trunc_bf16(q));
+            }
+            acc = mfma16(tl, xh, acc);
+            acc = mfma16(tm, xm, acc);
+            acc = mfma16(tm, xh, acc);
+            acc = mfma16(th, xm, acc);
+            acc = mfma16(th, xh, acc);
+#else
+            u32x4 xh;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) xh[d] = xb[u][2 * d] | (xb[u][2 * d + 1] << 16);
+            acc = mfma16(tl, xh, acc);
+            acc = mfma16(tm, xh, acc);
+            acc = mfma16(th, xh, acc);
+#endif
             if (c == NCH - 1 && cellv[u] >= 0) {
               const int cell = cellv[u] & 0x3fffffff;
               const bool valid = !(cellv[u] & 0x40000000);
@@ -302,8 +344,8 @@ __global__ __launch_bounds__(64 * NW, OCC) void fwd_few_kernel(FwdKernelArgs a, 
 
     // ---- P2 + P3: taps in registers, rank -> output-channel contraction ------------
     const __amdgpu_buffer_rsrc_t yrs = __builtin_amdgcn_make_buffer_rsrc(
-        a.y + (size_t)n * Cout * HW, 0, Cout * HW * 4, 0x00020000);
-    const bool pair_ok = (W & 1) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 7) == 0;
+        reinterpret_cast<io_t*>(a.y) + (size_t)n * Cout * HW, 0, Cout * HW * kIoBytes, 0x00020000);
+    const bool pair_ok = (W & 1) == 0 && (reinterpret_cast<uintptr_t>(a.y) & (2 * kIoBytes - 1)) == 0;
     for (int g = wave; g < pl.ngroups; g += kWaves) {
       const int p0 = 64 * g + 2 * l32;                 // the lane's pixels p0, p0 + 1 of the tile
       const int row = p0 >> pl.lgTW, col = p0 & (TW - 1);
@@ -360,8 +402,8 @@ __global__ __launch_bounds__(64 * NW, OCC) void fwd_few_kernel(FwdKernelArgs a, 
       // Stores through a buffer descriptor over the image's output planes: a store past its
       // range is dropped, so channels past the last one need no test, and a pixel outside
       // the image gets an offset past the range.
-      const unsigned vo = (unsigned)(4 * hi * HW + h * W + w) * 4u;
-      const unsigned vo0 = in0 ? vo : 0x80000000u, vo1 = in1 ? vo + 4u : 0x80000000u;
+      const unsigned vo = (unsigned)(4 * hi * HW + h * W + w) * (unsigned)kIoBytes;
+      const unsigned vo0 = in0 ? vo : 0x80000000u, vo1 = in1 ? vo + (unsigned)kIoBytes : 0x80000000u;
       const bool relu = a.act == 1;
       for (int kb = 0; kb < nkb; ++kb) {
         const u32x4 kh = frag[((NCH + kb) * 3 + 0) * 64 + lane];
@@ -411,7 +453,15 @@ __global__ __launch_bounds__(64 * NW, OCC) void fwd_few_kernel(FwdKernelArgs a, 
               o0 = o0 < 0.f ? 0.f : o0;
               o1 = o1 < 0.f ? 0.f : o1;
             }
-            const unsigned so = __builtin_amdgcn_readfirstlane((unsigned)kk * (unsigned)HW * 4u);
+            const unsigned so = __builtin_amdgcn_readfirstlane((unsigned)kk * (unsigned)HW * (unsigned)kIoBytes);
+#ifdef CP4_IO16
+            if (pair_ok) {
+              __builtin_amdgcn_raw_buffer_store_b32(io_pair(o0, o1), yrs, vo0, so, buffer_policy(STORE));
+            } else {
+              __builtin_amdgcn_raw_buffer_store_b16(to_io(o0), yrs, vo0, so, 0);
+              __builtin_amdgcn_raw_buffer_store_b16(to_io(o1), yrs, vo1, so, 0);
+            }
+#else
             if (pair_ok) {                                       // (W even: both pixels or neither)
               u32x2 o = {__float_as_uint(o0), __float_as_uint(o1)};
               __builtin_amdgcn_raw_buffer_store_b64(o, yrs, vo0, so, buffer_policy(STORE));
@@ -419,6 +469,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void fwd_few_kernel(FwdKernelArgs a, 
               __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o0), yrs, vo0, so, 0);
               __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o1), yrs, vo1, so, 0);
             }
+#endif
           }
         }
       }
@@ -540,15 +591,19 @@ bool plan_uncached(const FwdArgs& a, FewPlan* best) {
 
 template <int FS, int NCH, int RING, int OCC, int NW>
 hipError_t launch_as(const FwdArgs& a, const FewPlan& pl, hipStream_t st) {
-  const size_t plane = (size_t)a.H * a.W * sizeof(float);
+  const size_t plane = (size_t)a.H * a.W * kIoBytes;
   const size_t from = a.bias || a.act ? kStreamBytesFewLayer : kStreamBytes;
   const int store = store_policy(a.y, plane, plane * a.N * a.Cout, from, from);
 #define CP4_FEW(BIAS_, KEEP_)                                                                       \
   (store == kStoreStreamed  ? fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStoreStreamed, KEEP_>  \
    : store == kStoreThrough ? fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStoreThrough, KEEP_>   \
                             : fwd_few_kernel<FS, NCH, RING, OCC, NW, BIAS_, kStorePlain, KEEP_>)
+#ifdef CP4_IO16
+  auto k = a.bias ? CP4_FEW(true, false) : CP4_FEW(false, false);
+#else
   auto k = a.save_mask ? (a.bias ? CP4_FEW(true, true) : CP4_FEW(false, true))
                        : (a.bias ? CP4_FEW(true, false) : CP4_FEW(false, false));
+#endif
 #undef CP4_FEW
   const size_t lds = pl.lds_bytes + (a.bias ? (size_t)pl.nkb * 32 * sizeof(float) : 0);
   if (lds > 64 * 1024) {
@@ -568,6 +623,14 @@ hipError_t launch_fs(const FwdArgs& a, const FewPlan& pl, hipStream_t st) {
 
 }  // namespace
 
+#if defined(CP4_IO16) && CP4_IO16 == 2
+#define fwd_few_supported fwd_few_iof16_supported
+#define fwd_few_launch fwd_few_iof16_launch
+#elif defined(CP4_IO16)
+#define fwd_few_supported fwd_few_io16_supported
+#define fwd_few_launch fwd_few_io16_launch
+#endif
+
 bool fwd_few_supported(const FwdArgs& a) {
   if (a.R > kMaxRank || a.Cin > 64 || a.sh || a.dense || a.taps2d || a.ldf || a.ldx || a.accumulate)
     return false;
@@ -575,11 +638,12 @@ bool fwd_few_supported(const FwdArgs& a) {
   if (!fits_int_indexing(a.N, a.H, a.W) || (size_t)a.Cin * a.H * a.W >= (1u << 28) ||
       (size_t)a.Cout * a.H * a.W >= (1u << 28))          // 32-bit buffer offsets, stores past the range dropped
     return false;
-  if (a.x && (reinterpret_cast<uintptr_t>(a.x) & 3)) return false;
+  if (a.x && (reinterpret_cast<uintptr_t>(a.x) & (kIoBytes - 1))) return false;
   FewPlan pl;
   return plan(a, &pl);
 }
 
+#ifndef CP4_IO16
 bool fwd_few_plan(const FwdArgs& a, int* rows, int* cols, int* workgroups) {
   FewPlan pl;
   if (!fwd_few_supported(a) || !plan(a, &pl)) return false;
@@ -588,6 +652,7 @@ bool fwd_few_plan(const FwdArgs& a, int* rows, int* cols, int* workgroups) {
   *workgroups = pl.grid;
   return true;
 }
+#endif
 
 hipError_t fwd_few_launch(const FwdArgs& a, hipStream_t st) {
   FewPlan pl;
