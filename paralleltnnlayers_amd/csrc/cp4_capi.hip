@@ -1278,22 +1278,26 @@ cp4_status backward_filter_f32(const cp4_shape* shape, const float* x, const flo
       float* w = static_cast<float*>(workspace);
       const size_t hw = (size_t)s.H * s.W;
       const float *xp = x, *dyp = dy;
+      cp4::PadJob jobs[cp4::kMaxPadJobs];
+      int njobs = 0;
       if (t.C != s.C) {
-        CP4_HIP(cp4::pad_rows_launch(x, w + l.x, s.N, s.C, t.C, hw, st));
+        jobs[njobs++] = {x, w + l.x, s.N, s.C, t.C, hw};
         xp = w + l.x;
       }
       if (t.T != s.T) {
-        CP4_HIP(cp4::pad_rows_launch(dy, w + l.dy, s.N, s.T, t.T, hw, st));
+        jobs[njobs++] = {dy, w + l.dy, s.N, s.T, t.T, hw};
         dyp = w + l.dy;
       }
-      CP4_HIP(cp4::pad_rows_launch(FC, w + l.fc, 1, s.C, t.C, s.Rank, st));
-      CP4_HIP(cp4::pad_rows_launch(FK, w + l.fk, 1, s.T, t.T, s.Rank, st));
+      jobs[njobs++] = {FC, w + l.fc, 1, s.C, t.C, s.Rank};
+      jobs[njobs++] = {FK, w + l.fk, 1, s.T, t.T, s.Rank};
+      CP4_HIP(cp4::pad_rows_launch(jobs, njobs, st));
       rc = backward_filter_f32(&t, xp, dyp, w + l.fk, w + l.fc, FH, FW, w + l.gfk, w + l.gfc, dFH,
                                dFW, w + l.head, workspace_bytes - l.head * sizeof(float), -1,
                                t.C == s.C ? dx : nullptr, dx_done, nullptr, stream);
       if (rc != CP4_OK) return rc;
-      CP4_HIP(cp4::copy_f32_launch(dFC, w + l.gfc, (size_t)s.C * s.Rank, st));
-      CP4_HIP(cp4::copy_f32_launch(dFK, w + l.gfk, (size_t)s.T * s.Rank, st));
+      const cp4::PadJob back[2] = {{w + l.gfc, dFC, 1, 1, 1, (size_t)s.C * s.Rank},
+                                   {w + l.gfk, dFK, 1, 1, 1, (size_t)s.T * s.Rank}};
+      CP4_HIP(cp4::pad_rows_launch(back, 2, st));
       return CP4_OK;
     }
   }

@@ -66,21 +66,42 @@ __global__ __launch_bounds__(256) void copy_f32x4_kernel(
     dst[i] = src[i];
 }
 // dst[g][r][e] = r < rows ? src[g][r][e] : 0 for r < rows_padded: matrices or image
-// stacks with zero rows (channels) appended.  V = float4 when rows are whole quads.
-template <class V>
-__global__ __launch_bounds__(256) void pad_rows_kernel(V* __restrict__ dst,
-                                                       const V* __restrict__ src, size_t groups,
-                                                       size_t rows, size_t rows_padded,
-                                                       size_t row_elems) {
-  const size_t total = groups * rows_padded * row_elems;
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total;
-       i += (size_t)gridDim.x * 256) {
-    const size_t e = i % row_elems, gr = i / row_elems;
-    const size_t r = gr % rows_padded, g = gr / rows_padded;
+// stacks with zero rows (channels) appended, up to four of them in one launch: each on its own range
+// of workgroups, in quads of floats where rows are whole quads, with 32-bit indices where they suffice.
+// (The factor gradients of a layer of ragged channels have four of them in front and two plain
+// copies behind, up to four launches; each was a launch of 4 to 10 us, most of it the start and 64-bit
+// divisions.  Whole pass: N64 C33 K35 27x27 R8 53.4 -> 39.0 us, N16 C100 K99 28x28 R16 39.7 -> 33.9, N24
+// C480 K31 47x51 R46 120.8 -> 112.4.)
+struct PadGrid {
+  PadJob j[kMaxPadJobs];
+  unsigned first[kMaxPadJobs + 1];     // workgroups of job i: first[i] ... first[i + 1] - 1
+};
+template <class V, class I>
+__device__ __forceinline__ void pad_rows(const PadJob& p, unsigned block, unsigned blocks) {
+  constexpr int kPer = sizeof(V) / sizeof(float);
+  const V* src = reinterpret_cast<const V*>(p.src);
+  V* dst = reinterpret_cast<V*>(p.dst);
+  const I elems = (I)(p.row_elems / kPer), rows = (I)p.rows, padded = (I)p.rows_padded;
+  const I total = (I)p.groups * padded * elems;
+  for (size_t at = (size_t)block * 256 + threadIdx.x; at < total; at += (size_t)blocks * 256) {
+    const I i = (I)at, gr = i / elems, e = i - gr * elems, g = gr / padded, r = gr - g * padded;
     V v{};
-    if (r < rows) v = src[(g * rows + r) * row_elems + e];
+    if (r < rows) v = src[(g * rows + r) * elems + e];
     dst[i] = v;
   }
+}
+__global__ __launch_bounds__(256) void pad_rows_kernel(PadGrid pg) {
+  int k = 0;
+  while (k + 1 < kMaxPadJobs && blockIdx.x >= pg.first[k + 1]) ++k;
+  const PadJob& p = pg.j[k];
+  const unsigned block = blockIdx.x - pg.first[k], blocks = pg.first[k + 1] - pg.first[k];
+  const bool quads = (p.row_elems & 3) == 0 && ((reinterpret_cast<uintptr_t>(p.dst) |
+                                                 reinterpret_cast<uintptr_t>(p.src)) & 15) == 0;
+  const bool small = p.groups * p.rows_padded * p.row_elems < (1ull << 32);
+  if (quads && small) pad_rows<float4, unsigned>(p, block, blocks);
+  else if (quads) pad_rows<float4, size_t>(p, block, blocks);
+  else if (small) pad_rows<float, unsigned>(p, block, blocks);
+  else pad_rows<float, size_t>(p, block, blocks);
 }
 __global__ __launch_bounds__(256) void add_f32_kernel(float* __restrict__ dst,
                                                       const float* __restrict__ src, size_t n) {
@@ -389,17 +410,16 @@ hipError_t transpose_f32_launch(const float* src, float* dst, int rows, int cols
   return hipGetLastError();
 }
 
-hipError_t pad_rows_launch(const float* src, float* dst, size_t groups, size_t rows,
-                           size_t rows_padded, size_t row_elems, hipStream_t st) {
-  const size_t total = groups * rows_padded * row_elems;
-  if (total == 0) return hipSuccess;
-  if ((row_elems & 3) == 0 && (((uintptr_t)dst | (uintptr_t)src) & 15) == 0)
-    pad_rows_kernel<float4><<<grid_for(total / 4, 2048), 256, 0, st>>>(
-        reinterpret_cast<float4*>(dst), reinterpret_cast<const float4*>(src), groups, rows,
-        rows_padded, row_elems / 4);
-  else
-    pad_rows_kernel<float><<<grid_for(total, 2048), 256, 0, st>>>(dst, src, groups, rows,
-                                                                  rows_padded, row_elems);
+hipError_t pad_rows_launch(const PadJob* jobs, int n, hipStream_t st) {
+  if (n > kMaxPadJobs) return hipErrorInvalidValue;
+  PadGrid pg{};
+  for (int k = 0; k < kMaxPadJobs; ++k) {
+    if (k < n) pg.j[k] = jobs[k];
+    const size_t total = k < n ? jobs[k].groups * jobs[k].rows_padded * jobs[k].row_elems : 0;
+    pg.first[k + 1] = pg.first[k] + (total ? grid_for((total + 3) / 4, 2048) : 0);
+  }
+  if (!pg.first[kMaxPadJobs]) return hipSuccess;
+  pad_rows_kernel<<<pg.first[kMaxPadJobs], 256, 0, st>>>(pg);
   return hipGetLastError();
 }
 
