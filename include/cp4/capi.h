@@ -465,15 +465,13 @@ cp4_status cp4_layer_backward(const cp4_shape* shape, const cp4_geometry* geomet
                               void* dx, float* dFK, float* dFC, float* dFH, float* dFW,
                               float* dbias, void* workspace, size_t workspace_bytes,
                               cp4_stream stream);
-/* A training step's forward call may leave what its backward call would otherwise read or form
- * again: the signs of y, one bit an output (the backward reads them instead of y), and the layer's rank
- * planes before and after the taps, [N, R, H, W] each.  cp4_layer_kept_bytes: the room for what helps
- * the backward call that `wanted` describes (0: nothing does).  cp4_layer_forward_keeping is
- * cp4_layer_forward and says in *parts which of CP4_KEEP_* it left in `kept` (device memory on a
- * 256-byte boundary; 0 if a kernel ran that leaves none, or there is no room).  cp4_layer_backward_kept
- * is cp4_layer_backward given those; x, y and the factors must be those of the forward call.  The
- * same results but for the rounding of sums. */
-enum { CP4_KEEP_MASK = 1, CP4_KEEP_PLANES = 2 };
+/* A training step's forward call may leave the signs of y, one bit an output, which its backward call
+ * then reads instead of y.  cp4_layer_kept_bytes: the room for what helps the backward call that
+ * `wanted` describes (0: nothing does).  cp4_layer_forward_keeping is cp4_layer_forward and says in
+ * *parts what of CP4_KEEP_* it left in `kept` (device memory on a 256-byte boundary; 0 if a kernel ran
+ * that leaves nothing, or there is no room).  cp4_layer_backward_kept is cp4_layer_backward given it;
+ * y must be that of the forward call.  Both give the results of the calls without, bit for bit. */
+enum { CP4_KEEP_MASK = 1 };
 size_t cp4_layer_kept_bytes(const cp4_shape* shape, const cp4_geometry* geometry, int dtype,
                             int activation, int wanted);
 cp4_status cp4_layer_forward_keeping(const cp4_shape* shape, const cp4_geometry* geometry, int dtype,
@@ -495,8 +493,7 @@ enum {
   CP4_ROUTE_DY_PASS = 2,      /* one pass over dy for mask, bias gradient, G3 and dFK */
   CP4_ROUTE_DX_FROM_G1 = 4,   /* the input gradient from the factor gradients' G1 plane (not where it is
                                * formed for that alone: cp4_layer_last_backward_dx_beside) */
-  CP4_ROUTE_KEPT_MASK = 8,    /* the signs of y that the forward call left */
-  CP4_ROUTE_KEPT_PLANES = 16  /* its rank planes */
+  CP4_ROUTE_KEPT_MASK = 8     /* the signs of y that the forward call left */
 };
 int cp4_layer_last_backward_route(void);
 /* 1 if its mask and bias gradient ran inside the contraction and the gradient GEMM of the factor

@@ -2164,24 +2164,18 @@ hipError_t bwd_filter_mfma_masked_launch(const BwdFilterArgs& a, hipStream_t st)
   float* pW = pH + (size_t)p.St * a.Y * R;
   const int sets = bwd_dy_pass_sets(N, a.T, HW);
   float *pK = a.mask_ws, *pB = pK + (size_t)sets * a.T * R;
-  hipError_t e = hipSuccess;
-  // (A and Cc from the forward pass, or formed here)
-  const bool kept = a.kept_A && a.kept_Cc;
-  const float* Ak = kept ? a.kept_A : A;
-  if (!kept) e = contract_one(a.x, a.FC, A, G1, a.C, N, R, p.RP, HW, st);
+  hipError_t e = contract_one(a.x, a.FC, A, G1, a.C, N, R, p.RP, HW, st);
   if (e != hipSuccess) return e;
 #define CP4_TAPS(PART_)                                                                   \
   switch (a.Y) {                                                                          \
-    case 1: e = launch_taps_column<1, PART_>(Ak, G3, a, Cc, G1, pH, pW, st); break;       \
-    case 3: e = launch_taps_column<3, PART_>(Ak, G3, a, Cc, G1, pH, pW, st); break;       \
-    case 5: e = launch_taps_column<5, PART_>(Ak, G3, a, Cc, G1, pH, pW, st); break;       \
-    default: e = launch_taps_column<7, PART_>(Ak, G3, a, Cc, G1, pH, pW, st); break;       \
+    case 1: e = launch_taps_column<1, PART_>(A, G3, a, Cc, G1, pH, pW, st); break;        \
+    case 3: e = launch_taps_column<3, PART_>(A, G3, a, Cc, G1, pH, pW, st); break;        \
+    case 5: e = launch_taps_column<5, PART_>(A, G3, a, Cc, G1, pH, pW, st); break;        \
+    default: e = launch_taps_column<7, PART_>(A, G3, a, Cc, G1, pH, pW, st); break;       \
   }                                                                                       \
   if (e != hipSuccess) return e;
-  if (!kept) {
-    CP4_TAPS(kTapsCc)
-  }
-  e = bwd_dy_pass_launch(a.dy, a.act_y, a.act_bits, a.FK, kept ? a.kept_Cc : Cc, G3, pK, a.dbias ? pB : nullptr, N, a.T, R, HW, st);
+  CP4_TAPS(kTapsCc)
+  e = bwd_dy_pass_launch(a.dy, a.act_y, a.act_bits, a.FK, Cc, G3, pK, a.dbias ? pB : nullptr, N, a.T, R, HW, st);
   if (e != hipSuccess) return e;
   CP4_TAPS(kTapsRest)
 #undef CP4_TAPS

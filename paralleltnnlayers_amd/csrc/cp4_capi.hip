@@ -951,7 +951,7 @@ cp4_status cp4_conv2d_forward_bias_act(const cp4_shape* shape, const float* x,
                                        const float* bias, int activation, float* y,
                                        cp4_stream stream) {
   int parts = 0;
-  return cp4::layer_forward_keeping(shape, x, FK, FC, FH, FW, bias, activation, y, cp4::Kept{}, &parts,
+  return cp4::layer_forward_keeping(shape, x, FK, FC, FH, FW, bias, activation, y, nullptr, &parts,
                                     stream);
 }
 
@@ -960,9 +960,8 @@ cp4_status cp4_conv2d_forward_bias_act(const cp4_shape* shape, const float* x,
 namespace cp4 {
 cp4_status layer_forward_keeping(const cp4_shape* shape, const float* x, const float* FK,
                                  const float* FC, const float* FH, const float* FW,
-                                 const float* bias, int activation, float* y, const Kept& kept,
+                                 const float* bias, int activation, float* y, unsigned short* mask,
                                  int* parts, cp4_stream stream) {
-  const int want = *parts;
   *parts = 0;
   if (activation != CP4_ACT_NONE && activation != CP4_ACT_RELU)
     return fail(CP4_ERR_UNSUPPORTED, "activation must be CP4_ACT_NONE or CP4_ACT_RELU");
@@ -987,16 +986,11 @@ cp4_status layer_forward_keeping(const cp4_shape* shape, const float* x, const f
   if (c.variant < 0) return fail(CP4_ERR_UNSUPPORTED, "no kernel variant supports this shape");
   if (is_variant(c.variant, "mfma_bf16x3_pipe")) {
     FwdArgs e = with_tile(a, c);
-    if ((want & CP4_KEEP_MASK) && cp4::fwd_pipe_save_supported(e)) {
-      e.save_mask = kept.mask;
-      *parts = CP4_KEEP_MASK;
-      if ((want & CP4_KEEP_PLANES) && cp4::fwd_pipe_save_planes(e)) {
-        e.save_A = kept.A;
-        e.save_C = kept.Cc;
-        *parts |= CP4_KEEP_PLANES;
-      }
+    if (mask && cp4::fwd_pipe_save_supported(e)) {
+      e.save_mask = mask;
       CP4_ARM(e);
       CP4_HIP(cp4::fwd_pipe_save_launch(e, st));
+      *parts = CP4_KEEP_MASK;
       return CP4_OK;
     }
     if (cp4::fwd_pipe_epi_supported(e)) {
@@ -1028,11 +1022,9 @@ cp4_status layer_forward_keeping(const cp4_shape* shape, const float* x, const f
   if (is_variant(c.variant, "mfma_bf16x3_few")) {
     FwdArgs e = with_tile(a, c);
     if (cp4::fwd_few_supported(e)) {
-      if (want & CP4_KEEP_MASK) {
-        e.save_mask = kept.mask;
-        *parts = CP4_KEEP_MASK;
-      }
+      e.save_mask = mask;
       CP4_HIP(cp4::fwd_few_launch(e, st));          // the same
+      *parts = mask ? CP4_KEEP_MASK : 0;
       return CP4_OK;
     }
   }
@@ -1044,14 +1036,13 @@ cp4_status layer_forward_keeping(const cp4_shape* shape, const float* x, const f
   return CP4_OK;
 }
 
-int layer_forward_keeps(const cp4_shape& s) {
+bool layer_forward_keeps(const cp4_shape& s) {
   FwdArgs a = forward_args(s, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
   const Choice c = choose(a);
-  if (c.variant < 0) return 0;
+  if (c.variant < 0) return false;
   a = with_tile(a, c);
-  if (is_variant(c.variant, "mfma_bf16x3_pipe") && fwd_pipe_save_supported(a))
-    return CP4_KEEP_MASK | (fwd_pipe_save_planes(a) ? CP4_KEEP_PLANES : 0);
-  return is_variant(c.variant, "mfma_bf16x3_few") && fwd_few_supported(a) ? CP4_KEEP_MASK : 0;
+  return (is_variant(c.variant, "mfma_bf16x3_pipe") && fwd_pipe_save_supported(a)) ||
+         (is_variant(c.variant, "mfma_bf16x3_few") && fwd_few_supported(a));
 }
 }  // namespace cp4
 
@@ -1861,7 +1852,7 @@ cp4_status layer_backward_filter_masked(int variant, const cp4_shape* shape, con
                                         const float* act_y, const float* dy, const float* FK, const float* FC,
                                         const float* FH, const float* FW, float* dFK, float* dFC,
                                         float* dFH, float* dFW, float* dx, float* dbias,
-                                        float* bias_part, float* mask_ws, const Kept& kept, void* workspace,
+                                        float* bias_part, float* mask_ws, const unsigned short* bits, void* workspace,
                                         size_t workspace_bytes, cp4_stream stream) {
   if (!FK || !FC || !FH || !FW || !dFK || !dFC || !dFH || !dFW)
     return fail(CP4_ERR_NULL_POINTER, "a factor or gradient pointer is NULL");
@@ -1876,8 +1867,7 @@ cp4_status layer_backward_filter_masked(int variant, const cp4_shape* shape, con
   a.Y = s.Y; a.X = s.X; a.R = s.Rank;
   a.dx = dx;
   a.act_y = act_y; a.dbias = dbias; a.bias_part = bias_part; a.mask_ws = mask_ws;
-  a.act_bits = act_y ? kept.mask : nullptr;
-  a.kept_A = kept.A; a.kept_Cc = kept.Cc;
+  a.act_bits = act_y ? bits : nullptr;
   if (variant == 3) CP4_HIP(bwd_filter_dense_tiles_launch(a, as_stream(stream)));
   else CP4_HIP(bwd_filter_mfma_masked_launch(a, as_stream(stream)));
   return CP4_OK;

@@ -55,12 +55,11 @@ struct FwdKernelArgs {
   // Strided build only, set by its own entry points: a filter of ty x tx taps that runs as
   // the square window of Y = X taps around it (even and rectangular filters); 0: Y, X.
   int ty, tx;
-  // What a training step's backward pass would form again (the saving build of the producer /
-  // consumer kernel, the few-channel kernel; null: not wanted): one bit an output, y > 0, as
+  // For a training step's backward pass (the saving build of the producer / consumer kernel, the
+  // few-channel kernel; null: not wanted): one bit an output, y > 0, as
   // [N][blocks of 32 output channels][2][H * W] of 16 bits - half h, bit 4 a + b is channel 8 a + 4 h + b of
-  // the block -, and the rank planes [N, R, H, W] before and after the taps.
+  // the block.
   unsigned short* save_mask;
-  float *save_A, *save_C;
   // Recomposed-filter kernel only: the dense filter [Cout, Cin, Y, X] itself, taps in
   // the order the pass reads them; the four factors are unused then.
   const float* dense;
@@ -105,18 +104,13 @@ struct LayerMask {
   float *dbias, *bias_part;
 };
 
-// What a layer's forward pass leaves for its backward pass (FwdArgs::save_mask, save_A, save_C).
-struct Kept {
-  unsigned short* mask;
-  float *A, *Cc;
-};
-// The forward pass of a layer, leaving what *parts (CP4_KEEP_*) names of `kept` where the kernel that runs
-// can; *parts says what it left.
+// The forward pass of a layer, leaving y's signs (FwdArgs::save_mask) in `mask` (null: not wanted) where
+// the kernel that runs can; *parts says whether (CP4_KEEP_MASK) or not (0).
 cp4_status layer_forward_keeping(const cp4_shape*, const float* x, const float* FK, const float* FC,
                                  const float* FH, const float* FW, const float* bias, int activation,
-                                 float* y, const Kept& kept, int* parts, cp4_stream);
-// What of CP4_KEEP_* the kernel of a layer's forward pass can leave (aligned operands).
-int layer_forward_keeps(const cp4_shape&);
+                                 float* y, unsigned short* mask, int* parts, cp4_stream);
+// Whether the kernel of a layer's forward pass can leave them (aligned operands).
+bool layer_forward_keeps(const cp4_shape&);
 
 // The backward-filter entry points with the input gradient beside the factors' where the
 // variant that runs has it at hand (`dx` may be null; *dx_done says whether it was written).
@@ -140,7 +134,7 @@ cp4_status layer_backward_filter_masked(int variant, const cp4_shape*, const flo
                                         const float* dy, const float* FK, const float* FC,
                                         const float* FH, const float* FW, float* dFK, float* dFC,
                                         float* dFH, float* dFW, float* dx, float* dbias,
-                                        float* bias_part, float* mask_ws, const Kept& kept, void* workspace,
+                                        float* bias_part, float* mask_ws, const unsigned short* bits, void* workspace,
                                         size_t workspace_bytes, cp4_stream);
 
 // The backward-filter variant that an fp32 layer's factor gradients (and, want_dx, its input
@@ -193,9 +187,8 @@ bool fwd_pipe64_plan(const FwdArgs&, int* rows, int* workgroups);
 // The same kernel compiled with the bias / activation epilogue in its stores.
 bool fwd_pipe_epi_supported(const FwdArgs&);
 hipError_t fwd_pipe_epi_launch(const FwdArgs&, hipStream_t);
-// ... and with FwdArgs::save_mask, save_A and save_C (both planes or neither, where _planes says so).
+// ... and with FwdArgs::save_mask: the same y, bit for bit, and its signs.
 bool fwd_pipe_save_supported(const FwdArgs&);
-bool fwd_pipe_save_planes(const FwdArgs&);
 hipError_t fwd_pipe_save_launch(const FwdArgs&, hipStream_t);
 // The same kernel with bfloat16 x and y in memory (FwdArgs::x / y point at
 // 16-bit elements; factors and bias stay fp32), epilogue included.
@@ -263,10 +256,9 @@ struct BwdFilterArgs {
   // elements (matrix cores: dy behind the activation or, in the masked launch, partial sets).
   const float* act_y;
   float *dbias, *bias_part, *mask_ws;
-  // What the layer's forward pass left (FwdArgs::save_mask, save_A, save_C; null: it did not): the dense
-  // gradient and the masked launch read the signs instead of act_y, the masked launch takes the planes.
+  // y's signs from the layer's forward pass (FwdArgs::save_mask; null: it left none), which the dense
+  // gradient and the masked launch read instead of act_y.
   const unsigned short* act_bits;
-  const float *kept_A, *kept_Cc;
 };
 // general (VALU, any shape) and matrix-core variants
 size_t bwd_filter_workspace_bytes(const cp4_shape&);

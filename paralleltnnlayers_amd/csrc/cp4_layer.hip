@@ -101,50 +101,25 @@ BackwardPlan backward_plan(const cp4_shape& s, const cp4_geometry* g, int dtype,
                     [&] { return make_backward_plan(s, g, dtype, act, wanted); });
 }
 
-// Where the parts of what a forward call leaves lie (byte offsets).
-struct KeepPlan {
-  int parts;
-  size_t A_at, Cc_at, total;
-};
-KeepPlan make_keep_plan(const cp4_shape& s, const cp4_geometry* g, int dtype, int act, int wanted) {
-  KeepPlan k{};
+// Bytes of y's signs that a forward call leaves for its backward call; 0: none.
+size_t make_keep_plan(const cp4_shape& s, const cp4_geometry* g, int dtype, int act, int wanted) {
   const bool filter = wanted & CP4_WANT_FACTORS, dx = wanted & CP4_WANT_DX;
-  if (g || dtype != CP4_DTYPE_F32 || act != CP4_ACT_RELU || !filter || s.N == 0) return k;
+  if (g || dtype != CP4_DTYPE_F32 || act != CP4_ACT_RELU || !filter || s.N == 0) return 0;
   // (operands on 16-byte boundaries; a call whose are not may take another route and leave them)
   const int variant = cp4::layer_filter_masks(s, nullptr, nullptr, nullptr, nullptr,
                                               reinterpret_cast<const float*>(256), dx);
   // (a first layer's step waits for the host up to some 64 MB of y, and memory for the signs is 4 us more
   // of that: N2 and N4 C3 K64 224x224 R16, 26 and 51 MB, 62 and 61 us without, 68 and 66 with; N8 and N16
   // 100 and 147 without, 75 and 130 with)
-  if (!variant || (variant == 3 && elements(s, s.T) < (size_t)16 << 20)) return k;
-  k.parts = cp4::layer_forward_keeps(s) & (variant == 1 ? CP4_KEEP_MASK | CP4_KEEP_PLANES : CP4_KEEP_MASK);
-  if (!k.parts) return k;
-  const size_t plane = (size_t)s.H * s.W;
-  k.total = align256((size_t)s.N * ((s.T + 31) / 32) * plane * 4);
-  if (k.parts & CP4_KEEP_PLANES) {
-    const size_t planes = align256((size_t)s.N * s.Rank * plane * 4);
-    k.A_at = k.total;
-    k.Cc_at = k.A_at + planes;
-    k.total = k.Cc_at + planes;
-  }
-  return k;
+  if (!variant || (variant == 3 && elements(s, s.T) < (size_t)16 << 20)) return 0;
+  return cp4::layer_forward_keeps(s) ? align256((size_t)s.N * ((s.T + 31) / 32) * s.H * s.W * 4) : 0;
 }
 // (remembered as the backward plan is; what a call takes up is decided by its operands)
-KeepPlan keep_plan(const cp4_shape& s, const cp4_geometry* g, int dtype, int act, int wanted) {
+size_t keep_plan(const cp4_shape& s, const cp4_geometry* g, int dtype, int act, int wanted) {
   static std::mutex mu;
-  static std::map<PlanKey, KeepPlan> plans;
+  static std::map<PlanKey, size_t> plans;
   return remembered(mu, plans, plan_key(s, g, dtype, act, wanted),
                     [&] { return make_keep_plan(s, g, dtype, act, wanted); });
-}
-cp4::Kept kept_parts(const KeepPlan& k, int parts, const void* kept) {
-  unsigned char* p = static_cast<unsigned char*>(const_cast<void*>(kept));
-  cp4::Kept r{};
-  if (parts & CP4_KEEP_MASK) r.mask = reinterpret_cast<unsigned short*>(p);
-  if (parts & CP4_KEEP_PLANES) {
-    r.A = reinterpret_cast<float*>(p + k.A_at);
-    r.Cc = reinterpret_cast<float*>(p + k.Cc_at);
-  }
-  return r;
 }
 
 thread_local int g_route = 0;      // of this thread's last cp4_layer_backward
@@ -215,7 +190,7 @@ cp4_status cp4_layer_forward(const cp4_shape* shape, const cp4_geometry* g, int 
 size_t cp4_layer_kept_bytes(const cp4_shape* shape, const cp4_geometry* g, int dtype, int activation,
                             int wanted) {
   if (check_layer(shape, g, dtype, activation) != CP4_OK || shape->N == 0) return 0;
-  return keep_plan(*shape, g, dtype, activation, wanted).total;
+  return keep_plan(*shape, g, dtype, activation, wanted);
 }
 
 cp4_status cp4_layer_forward_keeping(const cp4_shape* shape, const cp4_geometry* g, int dtype,
@@ -228,13 +203,11 @@ cp4_status cp4_layer_forward_keeping(const cp4_shape* shape, const cp4_geometry*
   *parts = 0;
   CP4_TRY(check_layer(shape, g, dtype, activation));
   if (kept && shape->N && !(reinterpret_cast<uintptr_t>(kept) & 255)) {
-    const KeepPlan k = keep_plan(*shape, g, dtype, activation, wanted);
-    if (k.parts && kept_bytes >= k.total) {
-      *parts = k.parts;
+    const size_t room = keep_plan(*shape, g, dtype, activation, wanted);
+    if (room && kept_bytes >= room)
       return cp4::layer_forward_keeping(shape, static_cast<const float*>(x), FK, FC, FH, FW, bias,
                                         activation, static_cast<float*>(y),
-                                        kept_parts(k, k.parts, kept), parts, stream);
-    }
+                                        static_cast<unsigned short*>(kept), parts, stream);
   }
   return cp4_layer_forward(shape, g, dtype, x, FK, FC, FH, FW, bias, activation, y, workspace,
                            workspace_bytes, stream);
@@ -303,17 +276,17 @@ cp4_status cp4_layer_backward_kept(const cp4_shape* shape, const cp4_geometry* g
     if (variant) {
       g_dx_beside = variant != 3 && dx;
       g_route = variant == 3 ? CP4_ROUTE_MASKED_TILES : CP4_ROUTE_DY_PASS | (dx ? CP4_ROUTE_DX_FROM_G1 : 0);
-      cp4::Kept left{};
-      if (kept && parts_kept && !(reinterpret_cast<uintptr_t>(kept) & 255)) {
-        const KeepPlan k = keep_plan(s, g, dtype, activation, wanted);
-        if ((k.parts & parts_kept) == parts_kept && kept_bytes >= k.total)
-          left = kept_parts(k, parts_kept, kept);
-        if (variant == 3) left.A = left.Cc = nullptr;
-        g_route |= (left.mask ? CP4_ROUTE_KEPT_MASK : 0) | (left.A ? CP4_ROUTE_KEPT_PLANES : 0);
+      const unsigned short* bits = nullptr;
+      if (kept && parts_kept == CP4_KEEP_MASK && !(reinterpret_cast<uintptr_t>(kept) & 255)) {
+        const size_t room = keep_plan(s, g, dtype, activation, wanted);
+        if (room && kept_bytes >= room) {
+          bits = static_cast<const unsigned short*>(kept);
+          g_route |= CP4_ROUTE_KEPT_MASK;
+        }
       }
       return cp4::layer_backward_filter_masked(variant, shape, xf, yf, dyf, FK, FC, FH, FW, dFK, dFC,
                                                dFH, dFW, static_cast<float*>(dx), dbias, parts, mask_ws,
-                                               left, ws + p.pass_at, p.pass_bytes, stream);
+                                               bits, ws + p.pass_at, p.pass_bytes, stream);
     }
   }
   // or one whose contraction masks dy as it reads it and leaves it in memory for the others

@@ -67,12 +67,13 @@
 // plane the sh*(TH-1) + Y input rows under them; the tap step of output pixel
 // (ho, wo) reads the plane at row sh*ho, column sw*wo - pl, so only the kept
 // outputs are filtered, contracted and stored; entry points fwd_pipe_strided_*;
-// and with CP4_PIPE_SAVE (and the epilogue), for a layer's forward pass in a training step: what
-// the backward pass would otherwise form again leaves with y - one bit an output, y > 0
-// (FwdArgs::save_mask), written by the contraction waves, and the rank planes A and Cc
-// (FwdArgs::save_A, save_C), which the tap waves hold in registers; entry points fwd_pipe_save_*.
-// N32 C256 K256 56x56 R32: 29 MB more to write, 56 -> 63 us, and the backward pass does without the
-// contraction of x (21 us), the taps on A (8) and the way of y's 103 MB (13): the step 211 -> 170.
+// and with CP4_PIPE_SAVE (and the epilogue), for a layer's forward pass in a training step: one
+// bit an output, y > 0 (FwdArgs::save_mask), leaves with y, written by the contraction waves, so that
+// the backward pass need not read y; y itself is bit for bit the epilogue build's; entry points
+// fwd_pipe_save_*.  N32 C256 K256 56x56 R32: 3 MB more to write; the backward's pass over dy does without
+// y's 103 MB (13 us).  (The rank planes before and after the taps, which the tap waves hold, could leave
+// too.  The backward pass forms them again: its own sums round less - dFK from the planes of this kernel 2.5 %
+// further from float64 over 40 layers - and they are 2 R words a pixel for as long as y lives.)
 #include <cstdlib>
 #include <type_traits>
 
@@ -324,13 +325,6 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, Pip
     // sweep, already split: lane holds rank l32, channels 16*(cpq*cq+c) + 8*hi + e.
     constexpr int NF = FLDS ? 1 : CPQ;
     u32x4 fh[NF], fm[NF], fl[NF];
-#ifdef CP4_PIPE_SAVE
-    // Every other quarter contracts with the factor negated and its partial sums are subtracted: the
-    // matrix cores' sums come out low by a little whatever their sign, which the factor gradients' sums
-    // over all pixels of A and Cc bring to the front.  In the other block of a round the other quarters
-    // do, for channel counts whose quarters are not alike.
-    const float sign = !FLDS && NQ == 4 && ((cq + bsel) & 1) ? -1.f : 1.f;
-#endif
     if (!FLDS) {
       // (two copies of the loop on purpose: with whole chunks of channels the loads of
       // a slice sit under one condition and go out together - the start of every
@@ -342,10 +336,6 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, Pip
 #pragma unroll
           for (int e = 0; e < 8; ++e)
             v[e] = l32 < R ? a.Fin[(size_t)(cg0 + 16 * c + e) * ldf + l32] : 0.f;
-#ifdef CP4_PIPE_SAVE
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] *= sign;
-#endif
           split8(v, fh[c], fm[c], fl[c]);
         }
       } else {
@@ -357,10 +347,6 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, Pip
             v[e] = (l32 < R && cg0 + 16 * c + e < Cin)
                        ? a.Fin[(size_t)(cg0 + 16 * c + e) * ldf + l32]
                        : 0.f;
-#ifdef CP4_PIPE_SAVE
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] *= sign;
-#endif
           split8(v, fh[c], fm[c], fl[c]);
         }
       }
@@ -437,12 +423,6 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, Pip
       const unsigned xpn = geom(r + 1 < nrounds ? r + 1 : r, jn, qan, validn, exn);
       f32x16 acc = (f32x16)(0.f);
       [[maybe_unused]] f32x16 acc2 = (f32x16)(0.f);      // PAIR: the odd pixels
-#ifdef CP4_PIPE_SAVE
-      // (planes that leave: the products of the high parts apart from the small ones, so that a chunk
-      // rounds once at the sum's magnitude)
-      constexpr bool kApart = !FLDS && NQ == 4;
-      f32x16 acch = (f32x16)(0.f);
-#endif
       auto step = [&](int ch, int u) {
 #if CP4_PIPE_IO16 == 2
         // half-precision activations: 11 significand bits are two bfloat16 parts
@@ -537,15 +517,6 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, Pip
         if (FLDS) {
           const u32x4* fp = fbase + (size_t)(ch + u) * (6 * 32);
           acc = mfma_split(fp[0], fp[64], fp[128], xh, xm, xl, acc);
-#ifdef CP4_PIPE_SAVE
-        } else if constexpr (kApart) {
-          acc = mfma16(fl[FLDS ? 0 : ch + u], xh, acc);
-          acc = mfma16(fm[FLDS ? 0 : ch + u], xm, acc);
-          acc = mfma16(fh[FLDS ? 0 : ch + u], xl, acc);
-          acch = mfma16(fh[FLDS ? 0 : ch + u], xh, acch);
-          acc = mfma16(fm[FLDS ? 0 : ch + u], xh, acc);
-          acc = mfma16(fh[FLDS ? 0 : ch + u], xm, acc);
-#endif
         } else {
           acc = mfma_split(fh[FLDS ? 0 : ch + u], fm[FLDS ? 0 : ch + u], fl[FLDS ? 0 : ch + u], xh,
                            xm, xl, acc);
@@ -572,9 +543,6 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, Pip
           for (int u = 0; u < KR; ++u) step(ch, u);
         }
       }
-#ifdef CP4_PIPE_SAVE
-      if constexpr (kApart) acc += acch;
-#endif
       if (j < nblk) {
         // add this quarter's partial sums after the lower quarters
         int* bf = &flags[j];
@@ -620,14 +588,9 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, Pip
         if (cq == 0) {
 #pragma unroll
           for (int g = 0; g < 4; ++g)
-            if (g < ng) {
-              const f32x4 part = {acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
-#ifdef CP4_PIPE_SAVE
-              dst[(2 * g) * QA] = valid ? sign * part : f32x4{0.f, 0.f, 0.f, 0.f};
-#else
-              dst[(2 * g) * QA] = valid ? part : f32x4{0.f, 0.f, 0.f, 0.f};
-#endif
-            }
+            if (g < ng)
+              dst[(2 * g) * QA] = valid ? f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]}
+                                        : f32x4{0.f, 0.f, 0.f, 0.f};
         } else {
           wait_ge(bf, cq, backoff, wx, 1);
           // read, add, write two quads at a time: one LDS round trip per half
@@ -640,13 +603,8 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, Pip
 #pragma unroll
             for (int g = 0; g < 2; ++g) {
               const int v = 4 * (2 * half + g);
-              const f32x4 part = {acc[v], acc[v + 1], acc[v + 2], acc[v + 3]};
-#ifdef CP4_PIPE_SAVE
-              const f32x4 sum = old[g] + sign * part;
-#else
-              const f32x4 sum = old[g] + part;
-#endif
-              dst[(2 * (2 * half + g)) * QA] = valid ? sum : old[g];
+              dst[(2 * (2 * half + g)) * QA] =
+                  valid ? old[g] + f32x4{acc[v], acc[v + 1], acc[v + 2], acc[v + 3]} : old[g];
             }
           }
         }
@@ -918,11 +876,7 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, Pip
     // fragment tile cb.  wa / wb: the quad's weights (2-D taps: wa[rank][row][col];
     // else rows wa[rank][row] and columns wb[rank][col]).
     auto tap_quad = [&](const TapPos& tp, int q, const auto& wa, [[maybe_unused]] const auto& wb,
-                        unsigned char* cb, [[maybe_unused]] int g) {
-#ifdef CP4_PIPE_SAVE
-      const bool saves = a.save_A && blockIdx.y == 0;
-      f32x4 centre = {0.f, 0.f, 0.f, 0.f};
-#endif
+                        unsigned char* cb) {
       // (a quad past the last rank has zero weights; it reads quad 0's cells, the
       // plane may end before its own, and writes zeros)
       const bool live = 4 * q < R;
@@ -937,9 +891,6 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, Pip
         for (int ti = 0; ti < FS; ++ti)
 #pragma unroll
           for (int j = 0; j < FS; ++j) av[ti][j] = ab[tp.roff[ti] + tp.off[j]];
-#ifdef CP4_PIPE_SAVE
-        centre = av[FS / 2][FS / 2];
-#endif
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
           float s = 0.f;
@@ -982,22 +933,6 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, Pip
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) o[rr] = live ? s[rr] : 0.f;
       }
-#ifdef CP4_PIPE_SAVE
-      // the quad's rows of A and Cc at the group's pixels (256 bytes a rank, whole lines where the
-      // planes are)
-      if (saves && live) {
-        const int p = 64 * g - gshift + lane;
-        if (p >= 0 && p < nvalid) {
-          const size_t at = ((size_t)n * R + 4 * q) * HW + (size_t)h0 * W + p;
-#pragma unroll
-          for (int rr = 0; rr < 4; ++rr)
-            if (4 * q + rr < R) {
-              store_through(a.save_A + at + (size_t)rr * HW, centre[rr]);
-              store_through(a.save_C + at + (size_t)rr * HW, o[rr]);
-            }
-        }
-      }
-#endif
       // exact split of the four values: two dwords per part
       u32x2 ph, pm, pl2;
 #pragma unroll
@@ -1031,9 +966,9 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, Pip
 #pragma unroll
       for (int qi = 0; qi < decltype(ntq_c)::value; ++qi) {
 #ifdef CP4_PIPE_TAPS2D
-        tap_quad(tp, wq + 4 * qi, w2[qi], w2[qi], cb, g);
+        tap_quad(tp, wq + 4 * qi, w2[qi], w2[qi], cb);
 #else
-        tap_quad(tp, wq + 4 * qi, fh[qi], fw[qi], cb, g);
+        tap_quad(tp, wq + 4 * qi, fh[qi], fw[qi], cb);
 #endif
       }
       STAMPX(3 + 4 * i)
@@ -1245,7 +1180,7 @@ __global__ __launch_bounds__(kThreads) void fwd_pipe_kernel(FwdKernelArgs a, Pip
               qw[rr][j] = r < R ? a.FW[tap * ldf + r] : 0.f;
 #endif
             }
-          tap_quad(tp, q, qh, qw, cb, g);
+          tap_quad(tp, q, qh, qw, cb);
         }
         STAMPX(3 + 4 * (i >> 3))
         // (the tile is this wave's own: its LDS writes and reads stay in order)
@@ -1758,7 +1693,7 @@ bool fwd_pipe_supported(const FwdArgs& a_in) {
   if ((size_t)a.Cin * a.H * a.W * sizeof(io_t) >= (1ull << 31)) return false;   // buffer offsets
   if (a.Y != a.X || !(a.Y == 1 || a.Y == 3 || a.Y == 5 || a.Y == 7)) return false;
 #ifdef CP4_PIPE_SAVE
-  if (a.Y > 3 || 2 * a.pad + 1 != a.Y) return false;    // (5x5: 46 registers in scratch; a pixel's own cell is the centre tap)
+  if (a.Y > 3 || 2 * a.pad + 1 != a.Y) return false;    // (what the pass over dy takes, filters up to 3x3)
 #endif
 #ifdef CP4_PIPE_TAPS2D
   if (!a.taps2d || a.Y > 3) return false;        // 4 * Y * X weights per wave in registers
@@ -1780,15 +1715,6 @@ bool fwd_pipe_strip_plan(const FwdArgs& a, int* rows, int* workgroups) {
 }
 #endif
 
-#ifdef CP4_PIPE_SAVE
-// Whether A and Cc may leave with y: where the producers split the channels four ways, so that
-// alternate quarters balance the matrix cores' drift (launch_fs, launch_cpq).
-bool fwd_pipe_save_planes(const FwdArgs& a) {
-  PipePlan pl;
-  return a.Cin > 16 && a.Cin <= 256 && plan(a, &pl) && (a.Cin > 64 || pl.nblk < kWholeBlockMin);
-}
-#endif
-
 hipError_t fwd_pipe_launch(const FwdArgs& a_in, hipStream_t st) {
 #ifdef CP4_PIPE_STRIDED
   const FwdArgs a = in_window(a_in);
@@ -1807,7 +1733,7 @@ hipError_t fwd_pipe_launch(const FwdArgs& a_in, hipStream_t st) {
     case 1: return launch_fs<1>(a, pl, st);
     case 3: return launch_fs<3>(a, pl, st);
 #if defined(CP4_PIPE_TAPS2D) || defined(CP4_PIPE_SAVE)
-    default: return hipErrorInvalidValue;          // larger filters: the weights would spill
+    default: return hipErrorInvalidValue;          // (2-D taps: larger filters' weights would spill)
 #else
     case 5: return launch_fs<5>(a, pl, st);
     default: return launch_fs<7>(a, pl, st);

@@ -1,6 +1,6 @@
 """What a training step's forward call leaves for its backward call (cp4_layer_forward_keeping,
-cp4_layer_backward_kept): the signs of y and the rank planes, against float64 and against the
-backward call that reads y and forms the planes itself."""
+cp4_layer_backward_kept): the signs of y, against the backward call that reads y itself and against
+float64.  Keeping them changes no bit of y nor of any gradient."""
 import ctypes
 
 import pytest
@@ -9,8 +9,8 @@ import torch.nn.functional as F
 
 pytestmark = pytest.mark.gpu
 
-MASK, PLANES = 1, 2                       # CP4_KEEP_*
-KEPT_MASK, KEPT_PLANES = 8, 16            # CP4_ROUTE_*
+MASK = 1                                  # CP4_KEEP_*
+KEPT_MASK = 8                             # CP4_ROUTE_*
 
 
 @pytest.fixture(scope="module")
@@ -80,54 +80,60 @@ def _backward(capi, s, x, y, dy, fac, wanted, kept, parts):
 # of pairs and odd ones, every filter.
 TILES = [(5, 3, 352, 360, 33, 3, 4), (4, 3, 351, 353, 34, 3, 16), (17, 8, 180, 182, 32, 1, 8),
          (6, 3, 224, 228, 64, 5, 16)]
-# The pass over dy: signs and planes where the producers split the channels (whole and ragged
-# quarters, one rank quad past a half, 2 to 8 blocks of output channels), signs alone with few.
-PASSES = [((12, 256, 56, 56, 256, 3, 32), MASK | PLANES), ((48, 80, 52, 60, 96, 3, 17), MASK | PLANES),
-          ((40, 128, 40, 44, 256, 1, 20), MASK | PLANES), ((24, 64, 80, 80, 256, 1, 32), MASK),
-          ((40, 16, 60, 64, 128, 3, 8), MASK)]
+# The pass over dy: producers that split the channels (whole and ragged quarters, one rank quad past a
+# half, 2 to 8 blocks of output channels) and, with few channels, whole blocks.
+PASSES = [(12, 256, 56, 56, 256, 3, 32), (48, 80, 52, 60, 96, 3, 17), (40, 128, 40, 44, 256, 1, 20),
+          (24, 64, 80, 80, 256, 1, 32), (40, 16, 60, 64, 128, 3, 8)]
 
 
-@pytest.mark.parametrize("dims,parts", [(d, MASK) for d in TILES] + PASSES,
-                         ids=["x".join(map(str, d)) for d in TILES] + ["x".join(map(str, d)) for d, _ in PASSES])
-def test_backward_from_what_the_forward_left(capi, dims, parts):
+@pytest.mark.parametrize("dims", TILES + PASSES, ids=lambda d: "x".join(map(str, d)))
+def test_backward_from_what_the_forward_left(capi, dims):
     N, C, H, W, T, k, R = dims
     x, dy, fac, bias = _inputs(*dims)
     s = capi.shape_for(x.shape, *fac, k // 2)
     wanted = 6 if dims in TILES else 7            # factors and bias; dx too
     y, kept, left = _forward(capi, s, x, fac, bias, wanted)
-    assert left == parts
+    assert left == MASK
     # the signs: 16 bits a pixel and half, bit 4 a + b of half h is channel 8 a + 4 h + b
     nkb = (T + 31) // 32
     bits = kept[:N * nkb * H * W * 4].view(torch.int16).view(N, nkb, 2, H * W)
     for c in {0, 3, 4, 8, T // 2, T - 1}:
         word = bits[:, c // 32, c // 4 % 2].int()
         assert torch.equal(word >> (4 * (c % 32 // 8) + c % 4) & 1, (y[:, c].view(N, -1) > 0).int())
-    # y is what the call that keeps nothing gives, up to the order of the sums over the channels
-    plain = capi.layer_forward(s, None, x, *fac, bias, "relu")
-    terms = (C + R + 2 * k) * 2.0 ** -24
-    assert (y - plain).norm() <= terms ** 0.5 * 2.0 ** -12 * plain.norm()
+    # y is what the call that keeps nothing gives
+    assert torch.equal(y, capi.layer_forward(s, None, x, *fac, bias, "relu"))
     got = _backward(capi, s, x, y, dy, fac, wanted, kept, left)
     want = _backward(capi, s, x, y, dy, fac, wanted, kept, 0)
-    assert got[3] == want[3] | (KEPT_MASK if left & MASK else 0) | (KEPT_PLANES if left & PLANES else 0)
+    assert got[3] == want[3] | KEPT_MASK
+    # nothing but where the mask comes from differs
     assert torch.equal(got[2], want[2])
-    if left == MASK:                              # nothing but where the mask comes from differs
-        assert got[0] is None or torch.equal(got[0], want[0])
-        assert all(torch.equal(a, b) for a, b in zip(got[1], want[1]))
-        return
+    assert got[0] is None or torch.equal(got[0], want[0])
+    assert all(torch.equal(a, b) for a, b in zip(got[1], want[1]))
+    if dims in TILES or T // 32 % 2:              # (an odd number of blocks of output channels leaves one
+        return                                    # block's share of the matrix cores' drift in G3: 1.3e-6)
     exact = _exact(x, dy * (y > 0), *fac, k)
     # exact products; each sum rounds by 2^-24 a term, which over the C + T + R channels and ranks and 2 k taps
-    # of an entry add up as a random walk.  (An odd number of blocks of output channels leaves one block's
-    # share of the matrix cores' drift in G3, whatever A and Cc come from: 96 channels, three blocks,
-    # 1.3e-6 without anything kept.  No further off than that then.)
+    # of an entry add up as a random walk
     tol = 2.0 ** -24 * (C + T + R + 2 * k) ** 0.5
-    for a, p, b in zip([got[0]] + got[1], [want[0]] + want[1], (exact[0],) + exact[1]):
-        off, off_plain = (a.double() - b).norm(), (p.double() - b).norm()
-        assert off <= tol * b.norm() or (T // 32 % 2 and off <= 1.1 * off_plain)
+    for a, b in zip([got[0]] + got[1], (exact[0],) + exact[1]):
+        assert (a.double() - b).norm() <= tol * b.norm()
+
+
+@pytest.mark.parametrize("dims", TILES + PASSES, ids=lambda d: "x".join(map(str, d)))
+def test_a_training_steps_output_is_that_of_inference(capi, dims):
+    from paralleltnnlayers_amd import torch_ops
+    N, C, H, W, T, k, R = dims
+    x, _, fac, bias = _inputs(*dims)
+    layer = torch_ops.CP4Conv2d(C, T, k, R, bias=True, activation="relu")
+    with torch.no_grad():
+        for p, f in zip((layer.FK, layer.FC, layer.FH, layer.FW, layer.bias), fac + [bias]):
+            p.copy_(f)
+        want = layer(x)
+    assert torch.equal(layer(x.clone().requires_grad_(dims in PASSES)).detach(), want)
 
 
 def test_layer_under_hooks_on_saved_tensors(capi):
-    """What hooks give back - moved and returned, or as another type - changes no gradient but by the
-    order of the sums."""
+    """What hooks give back - moved and returned, or as another type - changes no gradient."""
     from paralleltnnlayers_amd import torch_ops
     N, C, H, W, T, k, R = 12, 256, 56, 56, 256, 3, 32
     x, dy, fac, bias = _inputs(N, C, H, W, T, k, R)
@@ -147,5 +153,4 @@ def test_layer_under_hooks_on_saved_tensors(capi):
         assert all(torch.equal(a, b) for a, b in zip(grads(), want))
     with torch.autograd.graph.saved_tensors_hooks(lambda t: t.float(), lambda t: t):
         got = grads()                             # (the bytes as floats: not taken up)
-    for a, b in zip(got, want):
-        assert (a - b).norm() <= 2.0 ** -23 * (C + T + R + 2 * k) ** 0.5 * b.norm()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
