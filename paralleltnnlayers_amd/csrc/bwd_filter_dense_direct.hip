@@ -12,6 +12,10 @@
 // puts the B fragments of its row together (five dwords a part, shifted where a column starts on an odd
 // cell), then block by block of output channels masks, splits and multiplies the held dy and requests
 // the same block of the next tile; x of the next tile is split into the other buffer; one barrier.
+// The loop has no branch of its own in all this: behind the last tile its x is staged once more, into the
+// buffer that nobody reads, and whether dy's sums are wanted is a build (SUMS).  Where a branch stood, code that
+// reads a product or overwrites its addend could land right behind it, and the compiler leaves no wait for
+// the matrix cores on such an edge; tests/test_matrix_waits_cpu.py walks the listing for it.
 // A tile's products are added up apart and go to the accumulators in one correctly rounded
 // addition, with x's sign reversed every other tile: the matrix cores' sums come out low by a little
 // whatever their sign.
@@ -22,7 +26,7 @@
 // 1.14 times as fast on the mean, none slower by more than the runs differ.
 //
 // MASK: dy counts everywhere (0) or where y > 0 - y itself (1) or its signs from the forward pass (2).  Its
-// sums per channel may leave as the bias gradient's partial sets.
+// sums per channel may leave as the bias gradient's partial sets (SUMS; always there in the masked builds).
 #include "dense_tiles.h"
 #include "split_bf16.h"
 
@@ -54,7 +58,7 @@ __device__ __forceinline__ f32x4 load16(__amdgpu_buffer_rsrc_t r, unsigned voff,
 }
 
 // FS: filter; RB: blocks of 16 output channels; CB: blocks of 16 columns (c, i, j).
-template <int FS, int RB, int CB, int MASK>
+template <int FS, int RB, int CB, int MASK, bool SUMS>
 __global__ __launch_bounds__(kThreads, 2) void dense_direct_kernel(BwdFilterArgs a, DirectPlan pl,
                                                                    float* partial) {
   constexpr int PH = kTH + FS - 1, LEAD = FS > 1 ? 4 : 0, XS = kTW + 2 * LEAD;
@@ -92,8 +96,7 @@ __global__ __launch_bounds__(kThreads, 2) void dense_direct_kernel(BwdFilterArgs
   for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const bool sums = a.dbias != nullptr;              // the bias gradient comes along
-  float bs[RB];
+  [[maybe_unused]] float bs[RB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) bs[rb] = 0.f;
 
@@ -179,7 +182,7 @@ __global__ __launch_bounds__(kThreads, 2) void dense_direct_kernel(BwdFilterArgs
   for (int t = tr.first; t < tr.end; t += tr.step) {
     const bool more = t + tr.step < tr.end;
     const Tile nxt = tile_at(more ? t + tr.step : t);
-    if (more) load_x(nxt);
+    load_x(nxt);
     // ---- B: cells off ... off + 7 of each plane, the dwords from off / 2 shifted by its parity ----
     u32x4 bh[CB], bm[CB], bl[CB];
     const unsigned* xp = reinterpret_cast<const unsigned*>(lds) + (buf * 3 * pl.plane >> 1);
@@ -224,7 +227,10 @@ __global__ __launch_bounds__(kThreads, 2) void dense_direct_kernel(BwdFilterArgs
         for (int e = 0; e < 8; ++e)
           v[e] *= (float)__builtin_amdgcn_ubfe(held[rb >> 1][e >> 1], at + 16 * (e & 1), 1);
       }
-      if (sums) bs[rb] += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+      if constexpr (SUMS) bs[rb] += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+      // (the blocks' loads stay apart: moved about, a step of N16 C3 K64 224x224 took 117 us instead of 111; beside
+      // many accumulators arithmetic may move, or 40 registers go to scratch)
+      __builtin_amdgcn_sched_barrier(RB * CB > 9 ? 15 : 0);
       u32x4 ah, am, al;
       split::split8(v, ah, am, al);
       load_block(nxt, more, rb);
@@ -248,13 +254,13 @@ __global__ __launch_bounds__(kThreads, 2) void dense_direct_kernel(BwdFilterArgs
     }
     sign = -sign;
     buf ^= 1;
-    if (more) deposit_x(buf, sign);
+    deposit_x(buf, sign);
     __syncthreads();
   }
 
   // ---- the waves' sums, in order through LDS: one partial set per workgroup ----
   float* red = reinterpret_cast<float*>(lds);
-  if (sums) {
+  if (SUMS && a.dbias) {
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
       float s = bs[rb];
@@ -318,8 +324,9 @@ template <int FS, int RB, int CB>
 hipError_t launch_blocks(const BwdFilterArgs& a, const DirectPlan& pl, float* partial, int sets, hipStream_t st) {
   const int bytes = kWaves * CB * 256 * 4;
   const size_t lds = pl.stage > bytes ? pl.stage : bytes;
-  auto k = a.act_bits ? dense_direct_kernel<FS, RB, CB, 2>
-           : a.act_y  ? dense_direct_kernel<FS, RB, CB, 1> : dense_direct_kernel<FS, RB, CB, 0>;
+  auto k = a.act_bits ? dense_direct_kernel<FS, RB, CB, 2, true>
+           : a.act_y  ? dense_direct_kernel<FS, RB, CB, 1, true>
+           : a.dbias  ? dense_direct_kernel<FS, RB, CB, 0, true> : dense_direct_kernel<FS, RB, CB, 0, false>;
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

@@ -19,6 +19,9 @@ def capi():
 CASES = [(3, 1, 3, 4, 1, 1), (2, 3, 9, 36, 17, 3), (1, 4, 8, 32, 64, 1), (2, 5, 17, 28, 48, 3),
          (3, 3, 33, 20, 17, 5), (2, 8, 15, 64, 33, 3), (1, 1, 40, 100, 64, 5), (5, 2, 130, 132, 16, 3),
          (2, 16, 24, 40, 64, 1), (3, 3, 257, 260, 48, 5)]
+# one block of columns and many tiles a workgroup: one channel under 3x3, under 1x1, one to four blocks of rows
+CASES += [(6, 1, 260, 252, 16, 3), (6, 1, 257, 252, 64, 1), (7, 1, 256, 256, 1, 3), (5, 1, 264, 260, 33, 3),
+          (5, 9, 250, 244, 16, 1)]
 
 
 @pytest.mark.parametrize("how", ["relu", "bias", "plain"])
@@ -62,4 +65,14 @@ def test_repeats_bit_for_bit(capi):
     mk = lambda *s: torch.randn(*s, device="cuda")
     x, dy, fac = mk(N, C, H, W), mk(N, T, H, W), [mk(d, R) for d in (T, C, k, k)]
     runs = [capi.conv2d_backward_filter(x, dy, *fac, pad=1, variant=3) for _ in range(3)]
+    assert all(torch.equal(a, b) for r in runs[1:] for a, b in zip(r, runs[0]))
+
+
+@pytest.mark.parametrize("case", [(6, 1, 260, 252, 16, 3), (6, 1, 250, 252, 64, 1), (6, 1, 256, 256, 33, 3)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_one_block_of_columns_repeats_bit_for_bit(capi, case):
+    N, C, H, W, T, k = case
+    mk = lambda *s: torch.randn(*s, device="cuda")
+    x, dy, fac = mk(N, C, H, W), mk(N, T, H, W), [mk(d, 7) for d in (T, C, k, k)]
+    runs = [capi.conv2d_backward_filter(x, dy, *fac, pad=k // 2, variant=3) for _ in range(5)]
     assert all(torch.equal(a, b) for r in runs[1:] for a, b in zip(r, runs[0]))
