@@ -134,7 +134,9 @@ __global__ __launch_bounds__(kThreads, 2) void dense_direct_kernel(BwdFilterArgs
       yv[rb][1] = load16(yrs, v1, soff);
     }
     if constexpr (MASK == 2) {
-      if ((rb & 1) == 0) {                           // (past the row's end dy is zero, whatever the signs)
+      // (past the row's end dy is zero, whatever the signs; past the image's last sign the descriptor's range is
+      // checked dword by dword, so that the half of a load that lies before it arrives)
+      if ((rb & 1) == 0) {
         const __amdgpu_buffer_rsrc_t brs = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<unsigned short*>(a.act_bits + (size_t)tl.n * bits_image), 0, bits_image * 2, 0x00020000);
         bits[rb >> 1] = __builtin_bit_cast(

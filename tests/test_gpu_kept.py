@@ -80,6 +80,10 @@ def _backward(capi, s, x, y, dy, fac, wanted, kept, parts):
 # of pairs and odd ones, every filter.
 TILES = [(5, 3, 352, 360, 33, 3, 4), (4, 3, 351, 353, 34, 3, 16), (17, 8, 180, 182, 32, 1, 8),
          (6, 3, 224, 228, 64, 5, 16)]
+# ... and for the direct filter gradient rows of an odd number of fours, whose last signs are half a load,
+# down to the image's last row; one, two and four blocks of 16 channels, one to four of columns
+TILES += [(6, 3, 227, 228, 64, 3, 16), (24, 4, 214, 220, 16, 3, 8), (13, 4, 203, 212, 32, 3, 8),
+          (28, 6, 213, 220, 13, 1, 4), (8, 1, 225, 236, 64, 5, 5), (11, 2, 229, 236, 31, 5, 6)]
 # The pass over dy: producers that split the channels (whole and ragged quarters, one rank quad past a
 # half, 2 to 8 blocks of output channels) and, with few channels, whole blocks.
 PASSES = [(12, 256, 56, 56, 256, 3, 32), (48, 80, 52, 60, 96, 3, 17), (40, 128, 40, 44, 256, 1, 20),
