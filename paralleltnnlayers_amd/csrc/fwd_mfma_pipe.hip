@@ -1534,7 +1534,7 @@ struct PlanAnswer {
 bool plan(const FwdArgs& a, PipePlan* best) {
   using Key = std::array<int, 23>;
   static thread_local PlanMemo<Key, PlanAnswer> memo;
-  const PlanAnswer& r = memo.get(
+  const PlanAnswer r = memo.get(
       Key{a.N, a.Cin, a.Cout, a.H, a.W, a.pad, a.Y, a.X, a.R, a.accumulate, a.tune_th, a.tune_lgwt,
           a.tune_split2, a.sh, a.sw, a.pt, a.pl, a.Ho, a.Wo, a.transposed, a.ty, a.tx, num_compute_units()},
       [&] {

@@ -8,22 +8,24 @@
 
 namespace cp4 {
 
-// Key: what the answer depends on, a std::array of integers (compute units of the device included).
+// Key: what the answer depends on, a std::array of integers (compute units of the device included).  make()
+// may ask the same memo for something else, as the workspace of a layer on padded channels does: the answer is
+// put away, and given out as a copy, only when there is one.
 template <class Key, class Answer, int kEntries = 4>
 struct PlanMemo {
   Key keys[kEntries];
   Answer answers[kEntries];
   int used = 0, next = 0;
   template <class Make>
-  const Answer& get(const Key& key, Make make) {
+  Answer get(const Key& key, Make make) {
     for (int i = 0; i < used; ++i)
       if (keys[i] == key) return answers[i];
-    const int at = next;
-    answers[at] = make();          // (before the key: make may throw)
-    keys[at] = key;
+    const Answer answer = make();
+    answers[next] = answer;
+    keys[next] = key;
     next = (next + 1) % kEntries;
     if (used < kEntries) ++used;
-    return answers[at];
+    return answer;
   }
 };
 
