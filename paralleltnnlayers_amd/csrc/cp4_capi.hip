@@ -626,27 +626,27 @@ int heuristic_variant(const FwdArgs& a) {
   return pick;
 }
 
-// The heuristic's pick per shape and operand alignment, remembered: evaluating it asks
-// every kernel for its plan, several microseconds of host time that a small layer's launch
+// The heuristic's pick per shape, operand alignment and device size, remembered: evaluating it
+// asks every kernel for its plan, several microseconds of host time that a small layer's launch
 // (5 us on the device) would otherwise wait for.
-std::map<std::tuple<TuneKey, unsigned>, int> g_heuristic_picks;
+std::map<std::tuple<TuneKey, unsigned, int>, int> g_heuristic_picks;
 // (g_choices counts the changes of either table)
 std::atomic<unsigned> g_choices{0};
 Choice choose_uncached(const FwdArgs& a);
 Choice choose(const FwdArgs& a) {
-  using Key = std::array<unsigned, 12>;
+  using Key = std::array<unsigned, 13>;
   static thread_local cp4::PlanMemo<Key, Choice> memo;
   return memo.get(Key{(unsigned)a.N, (unsigned)a.Cin, (unsigned)a.Cout, (unsigned)a.H, (unsigned)a.W,
                       (unsigned)a.pad, (unsigned)a.Y, (unsigned)a.X, (unsigned)a.R, (unsigned)a.flip,
                       (unsigned)((reinterpret_cast<uintptr_t>(a.x) & 15) << 4 |
                                  (reinterpret_cast<uintptr_t>(a.y) & 15)),
-                      g_choices.load()},
+                      (unsigned)cp4::num_compute_units(), g_choices.load()},
                   [&] { return choose_uncached(a); });
 }
 Choice choose_uncached(const FwdArgs& a) {
-  const std::tuple<TuneKey, unsigned> hk(
+  const std::tuple<TuneKey, unsigned, int> hk(
       key_of(a), (unsigned)((reinterpret_cast<uintptr_t>(a.x) & 15) << 4 |
-                            (reinterpret_cast<uintptr_t>(a.y) & 15)));
+                            (reinterpret_cast<uintptr_t>(a.y) & 15)), cp4::num_compute_units());
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tuned.find(key_of(a));
