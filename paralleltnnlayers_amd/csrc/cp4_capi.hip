@@ -630,7 +630,7 @@ int heuristic_variant(const FwdArgs& a) {
 // asks every kernel for its plan, several microseconds of host time that a small layer's launch
 // (5 us on the device) would otherwise wait for.
 std::map<std::tuple<TuneKey, unsigned, int>, int> g_heuristic_picks;
-// (g_choices counts the changes of either table)
+// (g_choices counts the changes of the tables)
 std::atomic<unsigned> g_choices{0};
 Choice choose_uncached(const FwdArgs& a);
 Choice choose(const FwdArgs& a) {
@@ -1805,6 +1805,10 @@ cp4_status layer_backward_filter(const cp4_shape* s, const cp4_geometry* g, int 
 }
 
 int layer_dx_variant() { return g_dx_variant; }
+bool layer_filter_forms_g1(const cp4_shape& s) {
+  return bwd_filter_fused_supported(s) && default_filter_variant(s, filter_routes(s, true, true, true)) == 2;
+}
+unsigned tuned_choices() { return g_choices.load(); }
 
 int layer_filter_takes_mask(const cp4_shape& s, const cp4_geometry* g, int dtype, const void* x,
                             const void* dy, const void* workspace) {
@@ -2068,6 +2072,7 @@ cp4_status cp4_tune_backward_filter(const cp4_shape* shape, const float* x, cons
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tuned_filter[key_of(*shape)] = best;
+    ++g_choices;
   }
   if (best_variant) *best_variant = best;
   if (best_us) *best_us = best_t;
@@ -2230,6 +2235,7 @@ cp4_status cp4_set_tuned_filter_choice(const cp4_shape* shape, int variant) {
   // (a choice the shape or the caller's alignment does not allow is ignored at launch)
   std::lock_guard<std::mutex> lk(g_tune_mu);
   g_tuned_filter[key_of(*shape)] = variant;
+  ++g_choices;
   return CP4_OK;
 }
 

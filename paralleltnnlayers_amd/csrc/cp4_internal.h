@@ -122,6 +122,11 @@ cp4_status layer_backward_filter(const cp4_shape*, const cp4_geometry*, int dtyp
                                  const float* FW, float* dFK, float* dFC, float* dFH, float* dFW,
                                  void* workspace, size_t workspace_bytes, void* dx, bool* dx_done,
                                  int variant, const LayerMask* mask, cp4_stream);
+// Whether such a call of a layer with aligned operands forms G1 for dx (the three-launch variant): it does
+// where its workspace has N * R * H * W floats more.
+bool layer_filter_forms_g1(const cp4_shape&);
+// Counts the changes of the tuned choices.
+unsigned tuned_choices();
 // The fp32 variant in which this thread's last such call wrote dx; 0: another pass, or none did.
 int layer_dx_variant();
 // The backward-filter variant (strided and 16-bit layers: any number above 0) that such a call

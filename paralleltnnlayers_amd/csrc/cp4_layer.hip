@@ -22,6 +22,7 @@ struct BackwardPlan {
   size_t x32_at, dx32_at;    // widened x, fp32 dx before it is rounded
   size_t bias_at, pass_at;   // partial bias sums, the passes' own workspace
   size_t pass_bytes, total;
+  size_t g1_bytes;           // of the passes' workspace, at its end: the call runs without them too
 };
 
 size_t elements(const cp4_shape& s, unsigned channels) {
@@ -63,20 +64,23 @@ BackwardPlan make_backward_plan(const cp4_shape& s, const cp4_geometry* g, int d
   p.pass_at = at;
   if (g) p.pass_bytes = dx || filter ? cp4_conv2d_backward_ex_workspace_bytes(&s, g) : 0;
   else p.pass_bytes = filter ? cp4_conv2d_backward_filter_workspace_bytes(&s) : 0;
-  // (room for G1, from which the three-launch variant then brings dx along)
-  if (!g && !half && dx && filter && cp4::bwd_filter_fused_supported(s))
-    p.pass_bytes = align256(p.pass_bytes) + (size_t)s.N * s.Rank * s.H * s.W * 4;
   p.total = at + align256(p.pass_bytes);
+  // (room for G1 where the three-launch variant runs, which then brings dx along)
+  if (!g && !half && dx && filter && cp4::layer_filter_forms_g1(s)) {
+    p.pass_bytes = align256(p.pass_bytes);
+    p.g1_bytes = align256((size_t)s.N * s.Rank * s.H * s.W * 4);
+    p.total += p.g1_bytes;
+  }
   return p;
 }
 
-using PlanKey = std::array<unsigned, 19>;
+using PlanKey = std::array<unsigned, 20>;
 PlanKey plan_key(const cp4_shape& s, const cp4_geometry* g, int dtype, int act, int wanted) {
   const cp4_geometry none{0, 0, 0, 0, 0, 0};
   const cp4_geometry& gg = g ? *g : none;
   return {s.N, s.H, s.W, s.pad, s.T, s.C, s.Y, s.X, s.Rank, gg.stride_h, gg.stride_w,
           gg.pad_top, gg.pad_left, gg.out_h, gg.out_w, (unsigned)dtype, (unsigned)act,
-          (unsigned)wanted, (unsigned)cp4::num_compute_units()};
+          (unsigned)wanted, (unsigned)cp4::num_compute_units(), cp4::tuned_choices()};
 }
 template <class Plan, class Make>
 Plan remembered(std::mutex& mu, std::map<PlanKey, Plan>& plans, const PlanKey& key, Make make) {
@@ -92,7 +96,7 @@ Plan remembered(std::mutex& mu, std::map<PlanKey, Plan>& plans, const PlanKey& k
 
 // The plan of a call, remembered: planning asks the backward-filter kernels for theirs,
 // several microseconds of host time that every step of a small layer would wait for.  (It
-// depends on the device by its compute units.)
+// depends on the device by its compute units, and on which variants were tuned.)
 BackwardPlan backward_plan(const cp4_shape& s, const cp4_geometry* g, int dtype, int act,
                            int wanted) {
   static std::mutex mu;
@@ -254,10 +258,12 @@ cp4_status cp4_layer_backward_kept(const cp4_shape* shape, const cp4_geometry* g
   const int wanted =
       (dx ? CP4_WANT_DX : 0) | (filter ? CP4_WANT_FACTORS : 0) | (dbias ? CP4_WANT_BIAS : 0);
   const BackwardPlan p = backward_plan(s, g, dtype, activation, wanted);
-  if (p.total && (!workspace || workspace_bytes < p.total ||
-                  (reinterpret_cast<uintptr_t>(workspace) & 255)))
+  const size_t least = p.total - p.g1_bytes;
+  if (least && (!workspace || workspace_bytes < least ||
+                (reinterpret_cast<uintptr_t>(workspace) & 255)))
     return cp4::fail_with(CP4_ERR_WORKSPACE, "workspace smaller than "
                           "cp4_layer_backward_workspace_bytes or not on a 256-byte boundary");
+  const size_t pass_bytes = p.pass_bytes + (workspace_bytes >= p.total ? p.g1_bytes : 0);
   unsigned char* ws = static_cast<unsigned char*>(workspace);
   const size_t plane = out_elements(s, g) / ((size_t)s.N * s.T);
   const int N = (int)s.N, T = (int)s.T;
@@ -286,7 +292,7 @@ cp4_status cp4_layer_backward_kept(const cp4_shape* shape, const cp4_geometry* g
       }
       return cp4::layer_backward_filter_masked(variant, shape, xf, yf, dyf, FK, FC, FH, FW, dFK, dFC,
                                                dFH, dFW, static_cast<float*>(dx), dbias, parts, mask_ws,
-                                               bits, ws + p.pass_at, p.pass_bytes, stream);
+                                               bits, ws + p.pass_at, pass_bytes, stream);
     }
   }
   // or one whose contraction masks dy as it reads it and leaves it in memory for the others
@@ -312,7 +318,7 @@ cp4_status cp4_layer_backward_kept(const cp4_shape* shape, const cp4_geometry* g
   bool dx_done = !dx;
   if (filter && (!half || p.filter16)) {
     CP4_TRY(cp4::layer_backward_filter(shape, g, dtype, x, inside ? dy : dya, FK, FC, FH, FW, dFK, dFC,
-                                       dFH, dFW, pass_ws, p.pass_bytes, dx, &dx_done,
+                                       dFH, dFW, pass_ws, pass_bytes, dx, &dx_done,
                                        inside && !half && !g ? inside : -1, inside ? &mask : nullptr,
                                        stream));
     if (dx && dx_done) {
@@ -324,13 +330,13 @@ cp4_status cp4_layer_backward_kept(const cp4_shape* shape, const cp4_geometry* g
     float* x32 = reinterpret_cast<float*>(ws + p.x32_at);
     CP4_LAUNCH(cp4::convert_launch(x, dtype, x32, CP4_DTYPE_F32, elements(s, s.C), st));
     CP4_TRY(cp4_conv2d_backward_filter(shape, x32, dy32, FK, FC, FH, FW, dFK, dFC, dFH, dFW, pass_ws,
-                                       p.pass_bytes, stream));
+                                       pass_bytes, stream));
   }
   if (dx_done) return CP4_OK;
   // 3. the input gradient on its own
   if (g)
     return cp4_conv2d_backward_data_ex(shape, g, static_cast<const float*>(dya), FK, FC, FH, FW,
-                                       static_cast<float*>(dx), pass_ws, p.pass_bytes, stream);
+                                       static_cast<float*>(dx), pass_ws, pass_bytes, stream);
   if (!half)
     return cp4_conv2d_backward_data(shape, static_cast<const float*>(dya), FK, FC, FH, FW,
                                     static_cast<float*>(dx), stream);

@@ -223,3 +223,33 @@ def test_backward_filter_workspace_sizes_over_random_shapes():
                        Rank=rng.choice((1, 2, 7, 16, 32, 33, 64, 65, 130)))
         need = L.cp4_conv2d_backward_filter_workspace_bytes(ctypes.byref(s))
         assert need > 0, s
+
+
+def test_layer_backward_workspace_holds_g1_where_it_is_formed(L):
+    """Room for the plane that the three-launch factor gradients leave for dx: where that variant runs, by
+    rule or as tuned, and nowhere else."""
+    from paralleltnnlayers_amd import capi
+
+    formed = set()
+
+    def holds(s):
+        need = lambda wanted: L.cp4_layer_backward_workspace_bytes(ctypes.byref(s), None, 0, 0, wanted)
+        fused = capi.plan_query(s, "backward_filter")["variant"] == "mfma_fused_taps"
+        plane = (s.N * s.Rank * s.H * s.W * 4 + 255) // 256 * 256
+        assert need(3) - need(2) == (plane if fused else 0), s     # dx and the factors, the factors alone
+        formed.add(fused)
+        return fused
+
+    for N, C, T, hw, R in ((16, 64, 64, 32, 16), (32, 256, 256, 56, 32), (64, 256, 256, 14, 64), (8, 8, 8, 256, 16),
+                           (1, 16, 16, 6, 5), (4, 48, 32, 20, 40)):
+        s = capi.Shape(N=N, H=hw, W=hw, pad=1, T=T, C=C, Y=3, X=3, Rank=R)
+        by_rule = holds(s)
+        try:
+            capi.set_tuned_filter_choice(s, 0)
+            assert not holds(s)
+            capi.set_tuned_filter_choice(s, 2)
+            assert holds(s) or not by_rule           # (a choice that the shape does not allow is ignored)
+        finally:
+            capi.tune_clear()
+        assert holds(s) == by_rule
+    assert formed == {False, True}
