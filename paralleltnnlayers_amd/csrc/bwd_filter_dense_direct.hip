@@ -324,18 +324,22 @@ bool make_direct_plan(const cp4_shape& s, DirectPlan* pl) {
 
 template <int FS, int RB, int CB>
 hipError_t launch_blocks(const BwdFilterArgs& a, const DirectPlan& pl, float* partial, int sets, hipStream_t st) {
-  const int bytes = kWaves * CB * 256 * 4;
-  const size_t lds = pl.stage > bytes ? pl.stage : bytes;
-  auto k = a.act_bits ? dense_direct_kernel<FS, RB, CB, 2, true>
-           : a.act_y  ? dense_direct_kernel<FS, RB, CB, 1, true>
-           : a.dbias  ? dense_direct_kernel<FS, RB, CB, 0, true> : dense_direct_kernel<FS, RB, CB, 0, false>;
-  if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
+  if constexpr (RB * CB > kMaxBlocks) {
+    return hipErrorInvalidValue;                     // (make_direct_plan refuses them)
+  } else {
+    const int bytes = kWaves * CB * 256 * 4;
+    const size_t lds = pl.stage > bytes ? pl.stage : bytes;
+    auto k = a.act_bits ? dense_direct_kernel<FS, RB, CB, 2, true>
+             : a.act_y  ? dense_direct_kernel<FS, RB, CB, 1, true>
+             : a.dbias  ? dense_direct_kernel<FS, RB, CB, 0, true> : dense_direct_kernel<FS, RB, CB, 0, false>;
+    if (lds > 64 * 1024) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (e != hipSuccess) return e;
+    }
+    k<<<sets, kThreads, lds, st>>>(a, pl, partial);
+    return hipGetLastError();
   }
-  k<<<sets, kThreads, lds, st>>>(a, pl, partial);
-  return hipGetLastError();
 }
 template <int FS, int CB>
 hipError_t launch_cb(const BwdFilterArgs& a, const DirectPlan& pl, float* partial, int sets, hipStream_t st) {

@@ -1269,7 +1269,7 @@ bool use_mfma(const cp4_shape& s) {
 // Partial sets of the kernel that takes dy straight from memory (bwd_filter_dense_direct.hip), 0 where
 // it does not run: it is the faster one wherever it takes the shape (rows of a multiple of four, operands
 // on 16-byte boundaries, up to 15 blocks of 16 x 16 entries of dK, 80 columns of them).
-static int direct_sets(const cp4_shape& s, bool aligned16, bool masked) {
+static int direct_sets(const cp4_shape& s, bool aligned16) {
   if (g_forced_tile_kernel.load() >= 0 || !use_mfma(s)) return 0;
   const int sets = dense_direct_sets(s, aligned16);
   // (the workspace has room for the partial sets of the other's plans)
@@ -1360,7 +1360,7 @@ hipError_t bwd_filter_dense_tiles_launch(const BwdFilterArgs& a, hipStream_t st)
   const bool aligned16 = ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.dy) |
                            reinterpret_cast<uintptr_t>(a.act_y)) & 15) == 0;
   const bool masked = a.act_y || a.dbias;
-  const int direct = direct_sets(s, aligned16, masked);
+  const int direct = direct_sets(s, aligned16);
   if (direct) {
     sets = direct;
     e = dense_direct_launch(a, partial, sets, st);

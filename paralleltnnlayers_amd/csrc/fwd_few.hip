@@ -47,6 +47,11 @@ namespace {
 using namespace split;
 
 constexpr int kMaxRank = 16;
+#ifdef CP4_IO16
+constexpr int kMaxCin = 32;      // (more: the producer / consumer kernel's, as in fp32 unless asked for)
+#else
+constexpr int kMaxCin = 64;
+#endif
 
 struct FewPlan {
   int TH, TW, lgTW;
@@ -617,8 +622,10 @@ hipError_t launch_as(const FwdArgs& a, const FewPlan& pl, hipStream_t st) {
 template <int FS>
 hipError_t launch_fs(const FwdArgs& a, const FewPlan& pl, hipStream_t st) {
   if (a.Cin <= 16) return pl.nw == 8 ? launch_as<FS, 1, 2, 4, 8>(a, pl, st) : launch_as<FS, 1, 2, 4, 4>(a, pl, st);
-  if (a.Cin <= 32) return pl.nw == 8 ? launch_as<FS, 2, 2, 4, 8>(a, pl, st) : launch_as<FS, 2, 2, 4, 4>(a, pl, st);
-  return pl.nw == 8 ? launch_as<FS, 4, 4, 4, 8>(a, pl, st) : launch_as<FS, 4, 4, 4, 4>(a, pl, st);
+#ifndef CP4_IO16
+  if (a.Cin > 32) return pl.nw == 8 ? launch_as<FS, 4, 4, 4, 8>(a, pl, st) : launch_as<FS, 4, 4, 4, 4>(a, pl, st);
+#endif
+  return pl.nw == 8 ? launch_as<FS, 2, 2, 4, 8>(a, pl, st) : launch_as<FS, 2, 2, 4, 4>(a, pl, st);
 }
 
 }  // namespace
@@ -632,7 +639,7 @@ hipError_t launch_fs(const FwdArgs& a, const FewPlan& pl, hipStream_t st) {
 #endif
 
 bool fwd_few_supported(const FwdArgs& a) {
-  if (a.R > kMaxRank || a.Cin > 64 || a.sh || a.dense || a.taps2d || a.ldf || a.ldx || a.accumulate)
+  if (a.R > kMaxRank || a.Cin > kMaxCin || a.sh || a.dense || a.taps2d || a.ldf || a.ldx || a.accumulate)
     return false;
   if (a.Y != a.X || !(a.Y == 1 || a.Y == 3 || a.Y == 5) || a.pad > a.Y - 1) return false;
   if (!fits_int_indexing(a.N, a.H, a.W) || (size_t)a.Cin * a.H * a.W >= (1u << 28) ||
