@@ -395,6 +395,9 @@ cp4_status cp4_tuned_choice(const cp4_shape* shape, int backward_data, int* vari
  * (reference/kernels/cp4Conv2dForward.cu:183-198). */
 cp4_status cp4_plan_query(const cp4_shape* shape, int pass, int* variant, int* strip_rows,
                           int* workgroups);
+/* The same for the 16-bit entry points (dtype CP4_DTYPE_BF16 or _F16; pass 0 or 1, operands on 16-byte
+ * boundaries): `variant` indexes cp4_forward_variant_name, -1 where they refuse the shape. */
+cp4_status cp4_plan_query_16(const cp4_shape* shape, int dtype, int pass, int* variant);
 /* Enters a choice into the table as cp4_tune_forward / cp4_tune_backward_data
  * would (one saved from an earlier process, say), in cp4_tuned_choice's terms.
  * `tile_cols` is 0, 32, 64, 128 or 256 (which of them a variant takes is its own matter).

@@ -157,6 +157,7 @@ def lib():
                                                  ctypes.POINTER(ctypes.c_float), ctypes.c_void_p]
     L.cp4_tuned_choice.argtypes = [_S, ctypes.c_int] + [ctypes.POINTER(ctypes.c_int)] * 4
     L.cp4_plan_query.argtypes = [_S, ctypes.c_int] + [ctypes.POINTER(ctypes.c_int)] * 3
+    L.cp4_plan_query_16.argtypes = [_S, ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
     L.cp4_set_tuned_choice.argtypes = [_S] + [ctypes.c_int] * 5
     L.cp4_tuned_count.restype = ctypes.c_int
     L.cp4_tuned_entry.argtypes = [ctypes.c_int, _S] + [ctypes.POINTER(ctypes.c_int)] * 5
@@ -764,10 +765,15 @@ def tuned_choice(s, backward_data=False):
     return dict(zip(("variant", "tile_rows", "tile_cols", "role_split"), (i.value for i in v)))
 
 
-def plan_query(s, pass_="forward"):
+def plan_query(s, pass_="forward", dtype=torch.float32):
     """{'variant' (its name), 'strip_rows', 'workgroups'} a launch of this pass would run with
-    now; rows and workgroups are 0 unless the whole-row strip kernel takes the shape."""
+    now; rows and workgroups are 0 unless the whole-row strip kernel takes the shape.  With a 16-bit
+    dtype, {'variant'} of the forward or backward-data entry point of that type, None if it refuses."""
     idx = ("forward", "backward_data", "backward_filter").index(pass_)
+    if dtype != torch.float32:
+        v = ctypes.c_int()
+        check(lib().cp4_plan_query_16(ctypes.byref(s), _DTYPES[dtype], idx, ctypes.byref(v)))
+        return {"variant": {i: n for i, n, _ in forward_variants()}.get(v.value)}
     v = [ctypes.c_int() for _ in range(3)]
     check(lib().cp4_plan_query(ctypes.byref(s), idx, *[ctypes.byref(i) for i in v]))
     if idx == 2:

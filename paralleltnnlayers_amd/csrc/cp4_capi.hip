@@ -681,17 +681,19 @@ Kernel16 pick16_uncached(const FwdArgs& a, bool half) {
     return Kernel16::kFew;
   return dense ? Kernel16::kDense : Kernel16::kPipe;
 }
-cp4_status run_16(FwdArgs a, int dtype, hipStream_t st) {
-  const bool half = dtype == CP4_DTYPE_F16;
+Kernel16 pick16(const FwdArgs& a, bool half) {
   using Key = std::array<unsigned, 12>;
   static thread_local cp4::PlanMemo<Key, Kernel16> memo;
-  const Kernel16 k = memo.get(
+  return memo.get(
       Key{(unsigned)a.N, (unsigned)a.Cin, (unsigned)a.Cout, (unsigned)a.H, (unsigned)a.W, (unsigned)a.pad,
           (unsigned)a.Y, (unsigned)a.X, (unsigned)a.R, (unsigned)half,
           (unsigned)((reinterpret_cast<uintptr_t>(a.x) & 15) << 4 | (reinterpret_cast<uintptr_t>(a.y) & 15)),
           (unsigned)cp4::num_compute_units()},
       [&] { return pick16_uncached(a, half); });
-  switch (k) {
+}
+cp4_status run_16(FwdArgs a, int dtype, hipStream_t st) {
+  const bool half = dtype == CP4_DTYPE_F16;
+  switch (pick16(a, half)) {
     case Kernel16::kFew:
       CP4_HIP(half ? cp4::fwd_few_iof16_launch(a, st) : cp4::fwd_few_io16_launch(a, st));
       return CP4_OK;
@@ -2133,6 +2135,26 @@ cp4_status cp4_plan_query(const cp4_shape* shape, int pass, int* variant, int* s
   if (variant) *variant = v;
   if (strip_rows) *strip_rows = rows;
   if (workgroups) *workgroups = wgs;
+  return CP4_OK;
+}
+
+cp4_status cp4_plan_query_16(const cp4_shape* shape, int dtype, int pass, int* variant) {
+  cp4_status rc = check_shape(shape);
+  if (rc != CP4_OK) return rc;
+  if (dtype != CP4_DTYPE_BF16 && dtype != CP4_DTYPE_F16)
+    return fail(CP4_ERR_UNSUPPORTED, "dtype must be CP4_DTYPE_BF16 or CP4_DTYPE_F16");
+  if (pass < 0 || pass > 1) return fail(CP4_ERR_SHAPE, "pass must be 0 or 1");
+  const FwdArgs a = pass == 1
+      ? backward_data_args(*shape, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr)
+      : forward_args(*shape, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+  int v = -1;
+  switch (pick16(a, dtype == CP4_DTYPE_F16)) {
+    case Kernel16::kFew: v = variant_named("mfma_bf16x3_few"); break;
+    case Kernel16::kDense: v = variant_named("dense_small_valu"); break;
+    case Kernel16::kPipe: v = variant_named("mfma_bf16x3_pipe"); break;
+    default: break;
+  }
+  if (variant) *variant = v;
   return CP4_OK;
 }
 

@@ -16,14 +16,24 @@ pytestmark = pytest.mark.gpu
 TYPES = {"bf16": (torch.bfloat16, 2.0 ** -8, capi.conv2d_forward_bf16, capi.conv2d_backward_data_bf16),
          "f16": (torch.float16, 2.0 ** -11, capi.conv2d_forward_f16, capi.conv2d_backward_data_f16)}
 
+FEW, DENSE, PIPE = "mfma_bf16x3_few", "dense_small_valu", "mfma_bf16x3_pipe"
+
+# (shape, the kernel of the forward pass, that of the input gradient)
 SHAPES = [
     # few-channel kernel: one, two rows of tiles; odd and even rows; one chunk of channels and two
-    (9, 5, 14, 97, 83, 3, 6), (8, 16, 16, 96, 128, 3, 16), (2, 32, 33, 200, 161, 3, 16),
-    (5, 17, 31, 120, 130, 5, 3), (61, 3, 64, 33, 32, 3, 16), (70, 12, 5, 47, 47, 1, 9),
-    (1, 1, 1, 260, 260, 5, 1), (3, 31, 64, 151, 138, 1, 16), (20, 4, 64, 57, 56, 5, 8),
+    ((9, 5, 14, 97, 83, 3, 6), FEW, FEW), ((8, 16, 16, 96, 128, 3, 16), FEW, FEW),
+    ((2, 32, 33, 200, 161, 3, 16), FEW, PIPE), ((5, 17, 31, 120, 130, 5, 3), FEW, FEW),
+    ((61, 3, 64, 33, 32, 3, 16), FEW, PIPE), ((70, 12, 5, 47, 47, 1, 9), FEW, FEW),
+    ((3, 31, 64, 151, 138, 1, 16), FEW, PIPE), ((20, 4, 64, 57, 56, 5, 8), FEW, PIPE),
     # recomposed filter: whole tiles of 64 columns and ragged ones, groups of eight channels, ranks past 16
-    (2, 2, 7, 240, 240, 3, 20), (3, 1, 9, 88, 107, 3, 21), (9, 3, 2, 128, 64, 7, 20),
-    (4, 4, 3, 130, 70, 5, 30), (2, 12, 1, 300, 101, 1, 27), (1, 16, 4, 500, 128, 3, 24),
+    ((1, 1, 1, 260, 260, 5, 1), DENSE, DENSE), ((2, 2, 7, 240, 240, 3, 20), DENSE, PIPE),
+    ((3, 1, 9, 88, 107, 3, 21), DENSE, PIPE), ((9, 3, 2, 128, 64, 7, 20), DENSE, DENSE),
+    ((9, 2, 11, 41, 128, 1, 30), DENSE, DENSE), ((2, 1, 9, 136, 181, 1, 27), DENSE, DENSE),
+    ((8, 9, 1, 146, 128, 3, 27), DENSE, DENSE), ((5, 9, 1, 195, 170, 5, 30), DENSE, DENSE),
+    ((7, 1, 2, 30, 76, 5, 20), DENSE, DENSE),
+    # on the other side of the rules
+    ((4, 4, 3, 130, 70, 5, 30), PIPE, PIPE), ((2, 12, 1, 300, 101, 1, 27), PIPE, DENSE),
+    ((1, 16, 4, 500, 128, 3, 24), PIPE, PIPE),
 ]
 
 
@@ -34,11 +44,15 @@ def _inputs(N, C, T, H, W, k, R, seed):
 
 
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
-@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("shape,forward_kernel,backward_kernel", SHAPES,
+                         ids=["x".join(map(str, s[0])) for s in SHAPES])
 @pytest.mark.parametrize("bias", [False, True])
-def test_passes_over_activations(shape, kind, bias):
+def test_passes_over_activations(shape, forward_kernel, backward_kernel, kind, bias):
     N, C, T, H, W, k, R = shape
     dtype, ulp, forward, backward_data = TYPES[kind]
+    s = capi.Shape(N=N, H=H, W=W, pad=k // 2, T=T, C=C, Y=k, X=k, Rank=R)
+    assert capi.plan_query(s, "forward", dtype)["variant"] == forward_kernel
+    assert capi.plan_query(s, "backward_data", dtype)["variant"] == backward_kernel
     gen, f, K = _inputs(*shape, seed=7)
     fd = [v.cuda() for v in f]
     x = torch.randn(N, C, H, W, generator=gen).to(dtype)
