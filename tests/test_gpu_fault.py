@@ -10,6 +10,8 @@ forces that from the host by setting the bound to one poll
 Also here: argument errors that need device tensors (an undersized workspace of
 another dtype) and the documented behaviour on non-finite inputs.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -160,6 +162,33 @@ def _build_cases(cp4, oracle):
     b3 = rng.standard_normal(64).astype(np.float32)
     add("epilogue", lambda: cp4.conv2d_forward_bias_act(dev(x3), *[dev(v) for v in f3], dev(b3), "relu", pad=1),
         lambda: np.maximum(oracle.forward(x3, *f3, 1) + b3[None, :, None, None], 0))
+    # ... that leaves the signs of y for a training step's backward: y itself is the output looked at
+    s5 = cp4.capi.Shape(N=24, H=80, W=80, pad=0, T=256, C=64, Y=1, X=1, Rank=32)
+    x5 = torch.from_numpy(rng.standard_normal((24, 64, 80, 80)).astype(np.float32)).cuda()
+    f5 = [dev(v) for v in _factors(rng, 256, 64, 1, 32)]
+    b5 = dev(rng.standard_normal(256).astype(np.float32))
+
+    def keeping():
+        L, F32, RELU, all_gradients = cp4.capi.lib(), 0, 1, 7
+        L.cp4_layer_kept_bytes.restype = ctypes.c_size_t
+        room = L.cp4_layer_kept_bytes(ctypes.byref(s5), None, F32, RELU, all_gradients)
+        kept = torch.empty(room, dtype=torch.uint8, device="cuda")
+        y = torch.empty(24, 256, 80, 80, device="cuda")
+        parts = ctypes.c_int(0)
+        p = lambda t: ctypes.c_void_p(t.data_ptr())
+        cp4.capi.check(L.cp4_layer_forward_keeping(
+            ctypes.byref(s5), None, F32, p(x5), *map(p, f5), p(b5), RELU, all_gradients, p(y), p(kept),
+            ctypes.c_size_t(room), ctypes.byref(parts), None, ctypes.c_size_t(0), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        assert parts.value == 1
+        return y
+
+    def kept_want():
+        FK, FC, FH, FW = (v.cpu().double() for v in f5)
+        K = torch.einsum("tr,cr,r,r->tc", FK, FC, FH[0], FW[0])
+        y = torch.nn.functional.conv2d(x5.cpu().double(), K[:, :, None, None], b5.cpu().double())
+        return y.clamp(min=0).numpy()
+
+    add("epilogue, signs kept", keeping, kept_want)
     # 16-bit activations
     xb = torch.from_numpy(x3).cuda().to(torch.bfloat16)
     add("bfloat16", lambda: cp4.conv2d_forward_bf16(xb, *[dev(v) for v in f3], pad=1).float(),
@@ -185,9 +214,10 @@ def _build_cases(cp4, oracle):
 
 
 def test_wait_timeout_is_reported_in_every_build(cp4, oracle):
-    """The wait code is compiled into ten builds of the producer / consumer kernel:
-    with the bound at one poll each of them must report the fault (every wave still
-    ends normally), and with the default bound give the right answer again."""
+    """The wait code is compiled into eleven builds of the producer / consumer kernel - all but the
+    plain one here, which the tests above time out -: with the bound at one poll each of them must
+    report the fault (every wave still ends normally), and with the default bound give the right
+    answer again."""
     for name, launch, want, tol in _build_cases(cp4, oracle):
         assert cp4.device_status_detail()[0] == cp4.capi.OK, name
         cp4.set_spin_limit(1)
