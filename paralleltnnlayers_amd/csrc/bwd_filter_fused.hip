@@ -885,7 +885,7 @@ hipError_t bwd_filter_fused_launch(const BwdFilterArgs& a, hipStream_t st) {
   // Not for a few images, which every die shares (N1 C256 28x28 R32 18.8 us in turn, 19.3 in order), nor for
   // strips of a row or two with two rank blocks, whose neighbours request the same lines of the planes at
   // the same time (N4 C256 28x28 R64 26.5 / 29.0, N8 28.4 / 29.9; but N16 28x28, strips of 448 bytes,
-  // 33.4 / 31.7, N4 56x56 34.3 / 32.9, and N12 28x28 R32 28.4 / 27.1).
+  // 33.4 / 31.7, N4 56x56 34.3 / 32.9, and N12 28x28 R32 28.4 / 27.1; these six are what the 448 bytes rest on).
   const bool dies = N >= 4 && (p.RB == 1 || p.TH * a.W * (int)sizeof(float) >= 448);
   c.order = die_order(wgs, dies);
   const dim3 cgrid(dies ? die_grid(wgs) : (unsigned)wgs, 2);

@@ -666,7 +666,8 @@ Choice choose_uncached(const FwdArgs& a) {
 // 64 channels on either side, and 74 of planes from 56x56 to 225x225: 1.27 and 1.20 times as fast on the
 // mean, up to 10 times).  But where a row leaves much of a 32-column tile empty and there are many of them
 // the strips of whole rows are quicker: N60 65x65 R4 C16 K16 5x5 19.3 us against 25.3, C32 K64 3x3 27
-// against 32; N16 the other way round, 12.1 and 11.5, 18.4 and 12.1.
+// against 32; N16 the other way round, 12.1 and 11.5, 18.4 and 12.1.  (Rows of that one width were timed, in two
+// batch sizes: where the line lies between widths is an estimate.)
 constexpr long kFew16RaggedMaxPixels = 1l << 17;
 bool few16_wastes_columns(const FwdArgs& a) {
   return (a.W + 31) / 32 * 32 * 10l > 14l * a.W && (long)a.N * a.H * a.W >= kFew16RaggedMaxPixels;

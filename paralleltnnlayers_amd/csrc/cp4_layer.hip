@@ -114,7 +114,7 @@ size_t make_keep_plan(const cp4_shape& s, const cp4_geometry* g, int dtype, int 
                                               reinterpret_cast<const float*>(256), dx);
   // (a first layer's step waits for the host up to some 64 MB of y, and memory for the signs is 4 us more
   // of that: N2 and N4 C3 K64 224x224 R16, 26 and 51 MB, 62 and 61 us without, 68 and 66 with; N8 and N16
-  // 100 and 147 without, 75 and 130 with)
+  // 100 and 147 without, 75 and 130 with.  That layer alone was timed, on either side of the line.)
   if (!variant || (variant == 3 && elements(s, s.T) < (size_t)16 << 20)) return 0;
   return cp4::layer_forward_keeps(s) ? align256((size_t)s.N * ((s.T + 31) / 32) * s.H * s.W * 4) : 0;
 }
