@@ -392,10 +392,7 @@ __device__ __forceinline__ void split4(const float (&v)[4], u32x2& h, u32x2& m, 
 // added up apart and go to the accumulators in one correctly rounded addition.  N16 C16 K48 112x112 3x3
 // R16, distance from float64 in the 2-norm: dFK 5.8e-7 without, 2.2e-7 with, 4.3e-7 in the plain
 // build; dFH 9.4e-7, 2.6e-7, 6.7e-7; 4 to 6 % of the pass's time.
-//
-// BITS (masked builds): y's signs from the forward pass (BwdFilterArgs::act_bits) instead of y, 16
-// channels of a pixel in 16 bits (the layer above 90 -> 74 us, its step 147 -> 130).
-template <int FS, int MB, bool M16, bool MASK, bool BALANCE, bool BITS = false>
+template <int FS, int MB, bool M16, bool MASK, bool BALANCE>
 __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kernel(BwdFilterArgs a, MfmaPlan pl,
                                                                   float* partial) {
   // blocks of BW x BW entries of dK, steps of 2^SPLG pixels, NV accumulator registers a block
@@ -445,8 +442,6 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
   const int xgroups = pl.nx >> 2, groups = xgroups + (pl.nd >> 2);
   unsigned rel[SLOTS];
   int rc[SLOTS];
-  [[maybe_unused]] unsigned mrel[BITS ? SLOTS : 1];   // the group's cells in the signs' planes
-  [[maybe_unused]] int mshift[BITS ? SLOTS : 1];      // ... and its channel's bit
 #pragma unroll
   for (int q = 0; q < SLOTS; ++q) {
     const int g = tid + THREADS * q;
@@ -456,24 +451,18 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
       const int pr = (int)__umulhi((unsigned)r2, pl.xsmagic), pc = r2 - pr * pl.XS;
       rel[q] = (unsigned)(c * HW + pr * W + pc);
       rc[q] = r2 < pl.PHXS ? (pr << 16) | pc : -1;
-      if constexpr (BITS) mrel[q] = 0, mshift[q] = -1;
     } else {
       const int e = 4 * (g - xgroups);
       const int k = (int)__umulhi((unsigned)e, pl.dsmagic), r2 = e - k * pl.DS;
       const int pr = r2 >> pl.lgTW, pc = r2 & (pl.TW - 1);
       rel[q] = (unsigned)(k * HW + pr * W + pc);
       rc[q] = g < groups && pr < pl.TH ? (pr << 16) | pc : -1;
-      if constexpr (BITS) {
-        mrel[q] = (unsigned)(((k >> 5) * 2 + ((k >> 2) & 1)) * HW + pr * W + pc);
-        mshift[q] = 4 * ((k & 31) >> 3) + (k & 3);
-      }
     }
   }
 
   const int tiles_per_image = pl.tilesX * pl.tilesY;
   const int lgcw = pl.lgTW - SPLG, nsteps = (pl.TH * pl.TW) >> SPLG;
-  float4 held[SLOTS], act[MASK && !BITS ? SLOTS : 1];
-  [[maybe_unused]] uint2 bits[BITS ? SLOTS : 1];      // two pixels' 16 bits a word
+  float4 held[SLOTS], act[MASK ? SLOTS : 1];
   float bsum[MASK ? SLOTS : 1];
   if constexpr (MASK)
 #pragma unroll
@@ -487,8 +476,6 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
     const float* xn = a.x + (size_t)n * a.C * HW;
     const float* dn = a.dy + (size_t)n * a.T * HW;
     const float* yn = MASK && a.act_y ? a.act_y + (size_t)n * a.T * HW : nullptr;
-    [[maybe_unused]] const unsigned short* mn =
-        BITS ? a.act_bits + (size_t)n * ((a.T + 31) >> 5) * 2 * HW : nullptr;
 #pragma unroll
     for (int q = 0; q < SLOTS; ++q) {
       const int g = tid + THREADS * q;
@@ -499,21 +486,7 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
       const bool row_in = rc[q] >= 0 && (unsigned)h < (unsigned)H;
       const long at = (long)rel[q] + (long)h0 * W + w0;
       float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      if constexpr (BITS) {
-        uint2 m = make_uint2(0u, 0u);
-        if (!isx && row_in) {
-          const unsigned short* src16 = mn + (long)mrel[q] + (long)h0 * W + w0;
-          if (pl.vec) {
-            if ((unsigned)w < (unsigned)W) m = *reinterpret_cast<const uint2*>(src16);
-          } else {
-            if ((unsigned)w < (unsigned)W) m.x = src16[0];
-            if ((unsigned)(w + 1) < (unsigned)W) m.x |= (unsigned)src16[1] << 16;
-            if ((unsigned)(w + 2) < (unsigned)W) m.y = src16[2];
-            if ((unsigned)(w + 3) < (unsigned)W) m.y |= (unsigned)src16[3] << 16;
-          }
-        }
-        bits[q] = m;
-      } else if constexpr (MASK) {
+      if constexpr (MASK) {
         float4 yv = make_float4(1.f, 1.f, 1.f, 1.f);
         if (yn && !isx && row_in) {
           if (pl.vec) {
@@ -555,22 +528,14 @@ __global__ __launch_bounds__(M16 ? 1024 : 512, M16 ? 4 : 2) void dense_mfma_kern
         float v[4] = {held[q].x, held[q].y, held[q].z, held[q].w};
         if constexpr (MASK) {
           // (a product, as dy * (y > 0): a non-finite dy at a clipped output stays visible)
+          const float yv[4] = {act[q].x, act[q].y, act[q].z, act[q].w};
           float one = 1.f;
           if constexpr (BALANCE) {
             const int st = ((rc[q] >> 16) << lgcw) + ((rc[q] & 0xffff) >> SPLG);
             if (!isx && (st >= nsteps / 2) != (index & 1)) one = -1.f;
           }
-          if constexpr (BITS) {
-            // (x's cells are not masked)
-            const unsigned b0 = bits[q].x >> (mshift[q] & 31), b1 = bits[q].y >> (mshift[q] & 31);
-            const unsigned on[4] = {b0, b0 >> 16, b1, b1 >> 16};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] *= isx || (on[i] & 1u) ? one : 0.f;
-          } else {
-            const float yv[4] = {act[q].x, act[q].y, act[q].z, act[q].w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] *= yv[i] > 0.f ? one : 0.f;
-          }
+          for (int i = 0; i < 4; ++i) v[i] *= yv[i] > 0.f ? one : 0.f;
           bsum[q] += one * ((v[0] + v[1]) + (v[2] + v[3]));
         }
         u32x2 h, m, l;
@@ -1195,11 +1160,7 @@ hipError_t launch_mfma_fs(const BwdFilterArgs& a, const MfmaPlan& pl, bool balan
   auto k1 = dense_mfma_kernel<FS, 1, false, false, false>;
   auto k2 = dense_mfma_kernel<FS, 2, false, false, false>;
   auto k = pl.m16 ? (pl.MB == 2 ? k02 : k0) : (pl.MB == 2 ? k2 : k1);
-  if (a.act_bits && balance)
-    k = pl.MB == 2 ? dense_mfma_kernel<FS, 2, true, true, true, true> : dense_mfma_kernel<FS, 1, true, true, true, true>;
-  else if (a.act_bits)
-    k = pl.MB == 2 ? dense_mfma_kernel<FS, 2, true, true, false, true> : dense_mfma_kernel<FS, 1, true, true, false, true>;
-  else if ((a.act_y || a.dbias) && balance)
+  if ((a.act_y || a.dbias) && balance)
     k = pl.MB == 2 ? dense_mfma_kernel<FS, 2, true, true, true> : dense_mfma_kernel<FS, 1, true, true, true>;
   else if (a.act_y || a.dbias)
     k = pl.MB == 2 ? dense_mfma_kernel<FS, 2, true, true, false> : dense_mfma_kernel<FS, 1, true, true, false>;
@@ -1279,6 +1240,8 @@ static int direct_sets(const cp4_shape& s, bool aligned16) {
     if (mfma_plan(s, al, &plain)) room = std::max(room, plain.grid);
   return sets < room ? sets : room;
 }
+
+bool bwd_filter_dense_tiles_reads_signs(const cp4_shape& s, bool aligned16) { return direct_sets(s, aligned16) > 0; }
 
 bool bwd_filter_dense_tiles_supported(const cp4_shape& s) { return valu_ok(s) || mfma_ok(s); }
 

@@ -261,7 +261,7 @@ struct BwdFilterArgs {
   // elements (matrix cores: dy behind the activation or, in the masked launch, partial sets).
   const float* act_y;
   float *dbias, *bias_part, *mask_ws;
-  // y's signs from the layer's forward pass (FwdArgs::save_mask; null: it left none), which the dense
+  // y's signs from the layer's forward pass (FwdArgs::save_mask; null: it left none), which the direct filter
   // gradient and the masked launch read instead of act_y.
   const unsigned short* act_bits;
 };
@@ -310,6 +310,9 @@ size_t bwd_filter_dense_tiles_workspace_bytes(const cp4_shape&);
 hipError_t bwd_filter_dense_tiles_launch(const BwdFilterArgs&, hipStream_t);
 // The route takes the layer's activation mask and bias gradient with it (BwdFilterArgs::act_y).
 bool bwd_filter_dense_tiles_masks(const cp4_shape&);
+// Whether it reads y's signs (BwdFilterArgs::act_bits) where they are at hand; aligned16: x, dy and act_y on
+// 16-byte boundaries.
+bool bwd_filter_dense_tiles_reads_signs(const cp4_shape&, bool aligned16);
 // 0: the plain multiply-add tile kernel, 1: the matrix-core one, wherever both can run the
 // shape; anything else: the route's own choice.
 void bwd_filter_dense_tiles_force_kernel(int which);

@@ -115,7 +115,12 @@ size_t make_keep_plan(const cp4_shape& s, const cp4_geometry* g, int dtype, int 
   // (a first layer's step waits for the host up to some 64 MB of y, and memory for the signs is 4 us more
   // of that: N2 and N4 C3 K64 224x224 R16, 26 and 51 MB, 62 and 61 us without, 68 and 66 with; N8 and N16
   // 100 and 147 without, 75 and 130 with.  That layer alone was timed, on either side of the line.)
-  if (!variant || (variant == 3 && elements(s, s.T) < (size_t)16 << 20)) return 0;
+  // (nor where the tile kernel runs instead of the direct one: on rows off the multiples of four it would read the
+  // signs one by one, N16 C3 K64 225x225 R16 241 us without, 248 with, and on others they gain nothing beyond
+  // what the forward pays, N20 C3 K64 5x5 148x148 115.5 and 116.5, 224x224 184 and 179)
+  if (!variant || (variant == 3 && (elements(s, s.T) < (size_t)16 << 20 ||
+                                    !cp4::bwd_filter_dense_tiles_reads_signs(s, true))))
+    return 0;
   return cp4::layer_forward_keeps(s) ? align256((size_t)s.N * ((s.T + 31) / 32) * s.H * s.W * 4) : 0;
 }
 // (remembered as the backward plan is; what a call takes up is decided by its operands)
@@ -283,7 +288,10 @@ cp4_status cp4_layer_backward_kept(const cp4_shape* shape, const cp4_geometry* g
       g_dx_beside = variant != 3 && dx;
       g_route = variant == 3 ? CP4_ROUTE_MASKED_TILES : CP4_ROUTE_DY_PASS | (dx ? CP4_ROUTE_DX_FROM_G1 : 0);
       const unsigned short* bits = nullptr;
-      if (kept && parts_kept == CP4_KEEP_MASK && !(reinterpret_cast<uintptr_t>(kept) & 255)) {
+      const uintptr_t at = reinterpret_cast<uintptr_t>(xf) | reinterpret_cast<uintptr_t>(yf) |
+                           reinterpret_cast<uintptr_t>(dyf);
+      if (kept && parts_kept == CP4_KEEP_MASK && !(reinterpret_cast<uintptr_t>(kept) & 255) &&
+          (variant != 3 || cp4::bwd_filter_dense_tiles_reads_signs(s, (at & 15) == 0))) {
         const size_t room = keep_plan(s, g, dtype, activation, wanted);
         if (room && kept_bytes >= room) {
           bits = static_cast<const unsigned short*>(kept);

@@ -76,14 +76,14 @@ def _backward(capi, s, x, y, dy, fac, wanted, kept, parts):
     return dx, grads, dbias, L.cp4_layer_last_backward_route()
 
 
-# First layers (signs alone, from the few-channel kernel): whole and ragged blocks of channels, rows
-# of pairs and odd ones, every filter.
-TILES = [(5, 3, 352, 360, 33, 3, 4), (4, 3, 351, 353, 34, 3, 16), (17, 8, 180, 182, 32, 1, 8),
-         (6, 3, 224, 228, 64, 5, 16)]
-# ... and for the direct filter gradient rows of an odd number of fours, whose last signs are half a load,
-# down to the image's last row; one, two and four blocks of 16 channels, one to four of columns
-TILES += [(6, 3, 227, 228, 64, 3, 16), (24, 4, 214, 220, 16, 3, 8), (13, 4, 203, 212, 32, 3, 8),
-          (28, 6, 213, 220, 13, 1, 4), (8, 1, 225, 236, 64, 5, 5), (11, 2, 229, 236, 31, 5, 6)]
+# First layers, behind which the direct filter gradient reads the signs: whole and ragged blocks of channels,
+# every filter; rows of an odd number of fours, whose last signs are half a load, down to the image's
+# last row; one to four blocks of 16 channels, one to five of columns.
+TILES = [(5, 3, 352, 360, 33, 3, 4), (6, 3, 227, 228, 64, 3, 16), (24, 4, 214, 220, 16, 3, 8), (13, 4, 203, 212, 32, 3, 8),
+         (28, 6, 213, 220, 13, 1, 4), (8, 1, 225, 236, 64, 5, 5), (11, 2, 229, 236, 31, 5, 6), (17, 8, 180, 184, 32, 1, 8),
+         (8, 3, 224, 228, 48, 5, 16)]
+# ... and the tile kernel, which reads y: rows off the multiples of four, more than 15 blocks
+LEFT_OUT = [(4, 3, 351, 353, 34, 3, 16), (17, 8, 180, 182, 32, 1, 8), (6, 3, 224, 228, 64, 5, 16)]
 # The pass over dy: producers that split the channels (whole and ragged quarters, one rank quad past a
 # half, 2 to 8 blocks of output channels) and, with few channels, whole blocks.
 PASSES = [(12, 256, 56, 56, 256, 3, 32), (48, 80, 52, 60, 96, 3, 17), (40, 128, 40, 44, 256, 1, 20),
@@ -123,7 +123,30 @@ def test_backward_from_what_the_forward_left(capi, dims):
         assert (a.double() - b).norm() <= tol * b.norm()
 
 
-@pytest.mark.parametrize("dims", TILES + PASSES, ids=lambda d: "x".join(map(str, d)))
+@pytest.mark.parametrize("dims", LEFT_OUT, ids=lambda d: "x".join(map(str, d)))
+def test_nothing_is_kept_for_the_tile_kernel(capi, dims):
+    x, _, fac, bias = _inputs(*dims)
+    s = capi.shape_for(x.shape, *fac, dims[5] // 2)
+    y, kept, left = _forward(capi, s, x, fac, bias, 6)
+    assert left == 0 and kept.numel() == 1
+    assert torch.equal(y, capi.layer_forward(s, None, x, *fac, bias, "relu"))
+
+
+def test_signs_are_left_alone_where_operands_are_off_their_boundaries(capi):
+    """The direct filter gradient wants 16-byte boundaries; without them the tile kernel reads y."""
+    N, C, H, W, T, k, R = dims = TILES[1]
+    x, dy, fac, bias = _inputs(*dims)
+    s = capi.shape_for(x.shape, *fac, k // 2)
+    y, kept, left = _forward(capi, s, x, fac, bias, 6)
+    assert left == MASK
+    off = torch.empty(dy.numel() + 1, device="cuda")[1:].view_as(dy).copy_(dy)
+    got = _backward(capi, s, x, y, off, fac, 6, kept, left)
+    want = _backward(capi, s, x, y, off, fac, 6, kept, 0)
+    assert got[3] == want[3] and not got[3] & KEPT_MASK
+    assert all(torch.equal(a, b) for a, b in zip([got[2]] + got[1], [want[2]] + want[1]))
+
+
+@pytest.mark.parametrize("dims", TILES + LEFT_OUT + PASSES, ids=lambda d: "x".join(map(str, d)))
 def test_a_training_steps_output_is_that_of_inference(capi, dims):
     from paralleltnnlayers_amd import torch_ops
     N, C, H, W, T, k, R = dims
