@@ -665,12 +665,20 @@ Choice choose_uncached(const FwdArgs& a) {
 // few-channel and the recomposed-filter kernel take over by the fp32 layers' rules (150 layers of 1 to
 // 64 channels on either side, and 74 of planes from 56x56 to 225x225: 1.27 and 1.20 times as fast on the
 // mean, up to 10 times).  But where a row leaves much of a 32-column tile empty and there are many of them
-// the strips of whole rows are quicker: N60 65x65 R4 C16 K16 5x5 19.3 us against 25.3, C32 K64 3x3 27
-// against 32; N16 the other way round, 12.1 and 11.5, 18.4 and 12.1.  (Rows of that one width were timed, in two
-// batch sizes: where the line lies between widths is an estimate.)
+// the strips of whole rows are quicker: from 2^17 pixels on with up to four ranks, whose taps cost them
+// little (us, strips and tiles: N39 C3 K24 66x66 R4 f16 11.7 and 14.9, N111 C3 K16 42x42 R1 bf16 11.8 and 13.2, but
+// N91 C3 K8 65x65 R9 39 and 22), or where the recomposed filter would not do either (N60 65x65 R4 C16 K16 5x5 19.3
+// and 25.3, C32 K64 3x3 27 and 32; N16 12.1 and 11.5, 18.4 and 12.1); and with up to four ranks and more
+// than 32 output channels from 2^16 on (N108 C32 K48 33x33 R2 f16 17.2 and 20.1, N57 C12 K64 40x40 R3 9.9 and 11.0;
+// below, N41 C4 K64 40x40 R3 10.0 and 9.6).  120 such layers of rows of 33 to 68 pixels, ranks 1 to 16, were
+// timed: of those left to the tiles the worst lose 2 to 7 %, on the mean they gain a third.
 constexpr long kFew16RaggedMaxPixels = 1l << 17;
-bool few16_wastes_columns(const FwdArgs& a) {
-  return (a.W + 31) / 32 * 32 * 10l > 14l * a.W && (long)a.N * a.H * a.W >= kFew16RaggedMaxPixels;
+constexpr int kFew16FewRanks = 4;
+bool few16_loses_to_strips(const FwdArgs& a, bool dense) {
+  if ((a.W + 31) / 32 * 32 * 10l <= 14l * a.W) return false;
+  const long pixels = (long)a.N * a.H * a.W;
+  if (pixels >= kFew16RaggedMaxPixels) return !dense || a.R <= kFew16FewRanks;
+  return 2 * pixels >= kFew16RaggedMaxPixels && a.R <= kFew16FewRanks && a.Cout > 32;
 }
 enum class Kernel16 { kNone, kPipe, kFew, kDense };
 Kernel16 pick16_uncached(const FwdArgs& a, bool half) {
@@ -678,8 +686,8 @@ Kernel16 pick16_uncached(const FwdArgs& a, bool half) {
   const bool dense = (half ? cp4::fwd_dense_small_iof16_supported(a) : cp4::fwd_dense_small_io16_supported(a)) &&
                      dense_small_estimate(a) <= kMatrixSmallChannelEstimate && !dense_small_loses_to_matrix(a);
   if ((half ? cp4::fwd_few_iof16_supported(a) : cp4::fwd_few_io16_supported(a)) &&
-      few_preferred(a, dense) && !(few16_wastes_columns(a) && !dense))
-    return Kernel16::kFew;
+      few_preferred(a, dense))
+    return few16_loses_to_strips(a, dense) ? Kernel16::kPipe : Kernel16::kFew;
   return dense ? Kernel16::kDense : Kernel16::kPipe;
 }
 Kernel16 pick16(const FwdArgs& a, bool half) {

@@ -34,6 +34,11 @@ SHAPES = [
     # on the other side of the rules
     ((4, 4, 3, 130, 70, 5, 30), PIPE, PIPE), ((2, 12, 1, 300, 101, 1, 27), PIPE, DENSE),
     ((1, 16, 4, 500, 128, 3, 24), PIPE, PIPE),
+    # rows that leave much of a tile of 32 columns empty: strips of whole rows with up to four ranks, by the
+    # number of pixels and of output channels; tiles with more ranks
+    ((39, 3, 24, 66, 66, 3, 4), PIPE, PIPE), ((39, 3, 24, 66, 66, 3, 5), FEW, PIPE),
+    ((57, 4, 64, 40, 40, 3, 2), PIPE, PIPE), ((40, 4, 64, 40, 40, 3, 2), FEW, PIPE),
+    ((57, 4, 32, 40, 40, 3, 2), FEW, FEW),
 ]
 
 
