@@ -671,7 +671,7 @@ Choice choose_uncached(const FwdArgs& a) {
 // and 25.3, C32 K64 3x3 27 and 32; N16 12.1 and 11.5, 18.4 and 12.1); and with up to four ranks and more
 // than 32 output channels from 2^16 on (N108 C32 K48 33x33 R2 f16 17.2 and 20.1, N57 C12 K64 40x40 R3 9.9 and 11.0;
 // below, N41 C4 K64 40x40 R3 10.0 and 9.6).  120 such layers of rows of 33 to 68 pixels, ranks 1 to 16, were
-// timed: of those left to the tiles the worst lose 2 to 7 %, on the mean they gain a third.
+// timed: of those left to the tiles the worst lose 2 to 8 %, on the mean they gain a third.
 constexpr long kFew16RaggedMaxPixels = 1l << 17;
 constexpr int kFew16FewRanks = 4;
 bool few16_loses_to_strips(const FwdArgs& a, bool dense) {
